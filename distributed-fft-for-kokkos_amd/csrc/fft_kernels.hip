@@ -15,6 +15,7 @@
 
 #include "fft_kernels.hpp"
 #include "fft_line_impl.hpp"
+#include "fft_mixed.hpp"
 
 #include <algorithm>
 #include <cstdint>
@@ -82,7 +83,8 @@ __global__ void __launch_bounds__(kGroupThreads) fft_group_pass(const LinePass* 
 // ---------------------------------------------------------------------------
 // Generic runtime-length kernel (any n): lines staged in LDS, every output of
 // a radix-r stage is a length-r sum with combined twiddles.  Handles lines
-// that cross rank boundaries (per-element addressing).
+// that cross rank boundaries (per-element addressing); lengths without a prime
+// factor above 13 whose lines lie whole in a rank run fft_mixed instead.
 // ---------------------------------------------------------------------------
 struct GenPlan {
   int32_t nst;
@@ -653,7 +655,7 @@ bool line_length_supported(int n, bool fp64) {
 // 2053: 79 / 3.4 ms.  Bluestein is taken where it models at least 20 %
 // cheaper than every other kernel that can run the length.
 bool bluestein_preferred(int n, bool fp64) {
-  if (n < 2 || has_fast_line_kernel(n)) return false;
+  if (n < 2 || has_fast_line_kernel(n) || mixed_length(n, fp64)) return false;
   if (!line_length_supported(n, fp64)) return true;
   auto generic = [](int len) {
     GenPlan g;
@@ -717,9 +719,10 @@ hipError_t launch_bluestein_post(const LinePass& p, int log2m, const void* chirp
 hipError_t launch_line_pass(const LinePass& p, bool fp64, hipStream_t s) {
   if (p.nlines <= 0) return hipSuccess;
   if (p.long_n1 > 0) return fp64 ? launch_long<double>(p, s) : launch_long<float>(p, s);
-  // the compile-time kernel needs the line axis undistributed on both sides
+  // the register kernels need the line axis undistributed on both sides
   const bool fast = has_fast_line_kernel(p.n) && p.in.ntopo[p.axis] == 1 && p.out.ntopo[p.axis] == 1;
   if (fast) return fp64 ? dispatch<double>(p, s) : dispatch<float>(p, s);
+  if (mixed_pass_supported(p, fp64)) return fp64 ? launch_mixed_f64(p, s) : launch_mixed_f32(p, s);
   return fp64 ? launch_generic<double>(p, s) : launch_generic<float>(p, s);
 }
 

@@ -28,7 +28,8 @@ struct LinePass {
   int32_t inverse;                      // 1: exponent +2 pi i jk/n
   int32_t lines_fast;                   // 1: consecutive lanes walk across lines
   int32_t lines_per_block;              // 0: launcher heuristic
-  int32_t values_per_thread;            // 0: default (8); compile-time kernels exist for 4, 8, 16
+  int32_t values_per_thread;            // 0: default (8); compile-time kernels exist for 4, 8, 16,
+                                        // the runtime-radix kernel takes it as an upper bound
   const void* tw;                       // exp(-2 pi i e / n), e in [0, n), Real precision
   double scale;
   // 1: an R2C (forward) or C2R (inverse) pass on the fast kernel transforms

@@ -1,0 +1,629 @@
+// Line passes of any length n = product of radices 2..13, 15, 16 (every n
+// without a prime factor above 13): a Stockham kernel whose radices are read
+// from the launch's plan and whose butterflies are straight-line code on
+// registers.  It serves the lengths without a compile-time kernel
+// (fft_line_impl.hpp), e.g. 36, 50, 100, 162, 250, 360, 375, 384, 1000.
+//
+// Why this shape: the per-element kernel (fft_line_generic) forms every output
+// of a radix-r stage as an r-term sum read from LDS, 4 to 16 LDS reads and
+// complex products per element and stage, and moved 0.25 to 0.6 TB/s.  Here a
+// lane reads a butterfly's r inputs once, so LDS traffic and arithmetic drop
+// by about r and a pass is bound by its line loads and stores (contiguous
+// FP64 lines: 4.7 to 5.5 TB/s read and written) or, in FP32 and in real
+// pairs, by instruction issue (2.4 to 4.7 TB/s).  An LDS index with a shift
+// per element instead of one constant step per exchange cost 5-10 % there.
+// Measured, per-element kernel -> this one (forward + backward unless stated):
+// R2C 384^3 FP64 7.16 -> 1.55 ms, C2C 375x250x162 FP32 forward 1.16 -> 0.29 ms,
+// inverse 2-D of 32x1000x1000 FP64 2.43 -> 0.49 ms, R2C 50x42x36 FP32
+// 124 -> 62 us.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "fft_kernels.hpp"
+#include "fft_line_impl.hpp"
+
+namespace dfft {
+
+constexpr int kMixStages = 8;
+// V: complex values a lane holds at most, and with it the radices a kernel
+// instance knows.  FP32 lanes hold 16.  FP64 lanes hold 10: with 16 (or with
+// radices 12 to 16) the kernel spills registers at the 128 that a block of
+// 1024 lanes leaves it; lengths with a factor 11 or 13 run an instance of
+// their own with up to 13 (a few spill slots).
+template <int V> constexpr bool mix_has(int r) { return r <= V; }
+// butterflies of radix r a lane carries through one stage
+template <int V> constexpr int mix_nb_max() { return V >= 16 ? 4 : 2; }
+template <int V> constexpr int mix_nb(int r) { return V / r < mix_nb_max<V>() ? V / r : mix_nb_max<V>(); }
+// half-spectrum entries a lane handles at most (n/2 + 1 entries over at least n / V lanes)
+template <int V> constexpr int mix_half() { return (V + 1) / 2 + 1; }
+
+struct MixStage {
+  int32_t r;    // radix
+  int32_t nr;   // n / r: butterflies of a line
+  int32_t L;    // product of the radices before
+  int32_t ts;   // n / (L r): twiddle-table step
+  // LDS index of position p in the exchange after a stage: p + pad (p / (L r)).
+  // Both sides of the exchange walk it with one constant step, as the next
+  // stage's n / r is a multiple of L r.
+  int32_t out_group;  // L r + pad: groups of the stage's outputs
+  int32_t in_pad;     // pad of the exchange before
+  int32_t in_step;    // (nr + nr / L * in_pad) * ps: from input j to j + 1
+  FastDiv dL;
+};
+
+struct MixPlan {
+  int32_t nst;
+  int32_t T;         // lanes per line
+  int32_t log2B;     // lanes across lines: B = 1 << log2B lines per block
+  int32_t ps, bs;    // LDS strides (reals) of a position and of a line
+  FastDiv dT;
+  MixStage st[kMixStages];
+};
+
+// ---------------------------------------------------------------------------
+// Butterflies beyond 2, 3, 4, 5 and 8 (exponent -2 pi i jk / r).
+// ---------------------------------------------------------------------------
+template <int r> struct Roots;  // c[k] = cos(2 pi k / r), s[k] = sin(2 pi k / r)
+template <> struct Roots<7> {
+  static constexpr double c[7] = {1.0, 0.623489801858733530525, -0.222520933956314404289, -0.900968867902419126236,
+                                  -0.900968867902419126236, -0.222520933956314404289, 0.623489801858733530525};
+  static constexpr double s[7] = {0.0, 0.781831482468029808708, 0.974927912181823607018, 0.433883739117558120475,
+                                  -0.433883739117558120475, -0.974927912181823607018, -0.781831482468029808708};
+};
+template <> struct Roots<9> {
+  static constexpr double c[5] = {1.0, 0.766044443118978035202, 0.173648177666930348852, -0.5,
+                                  -0.939692620785908384054};
+  static constexpr double s[5] = {0.0, 0.642787609686539326323, 0.984807753012208059367, 0.866025403784438646764,
+                                  0.342020143325668733044};
+};
+template <> struct Roots<11> {
+  static constexpr double c[11] = {1.0, 0.841253532831181168862, 0.415415013001886425529, -0.142314838273285140443,
+                                   -0.654860733945285064056, -0.959492973614497389891, -0.959492973614497389891,
+                                   -0.654860733945285064056, -0.142314838273285140443, 0.415415013001886425529,
+                                   0.841253532831181168862};
+  static constexpr double s[11] = {0.0, 0.540640817455597582108, 0.909631995354518371412, 0.989821441880932732376,
+                                   0.755749574354258283774, 0.281732556841429697711, -0.281732556841429697711,
+                                   -0.755749574354258283774, -0.989821441880932732376, -0.909631995354518371412,
+                                   -0.540640817455597582108};
+};
+template <> struct Roots<13> {
+  static constexpr double c[13] = {1.0, 0.885456025653209895900, 0.568064746731155775490, 0.12053668025532305335,
+                                   -0.354604887042535625970, -0.748510748171101098635, -0.970941817426052027156,
+                                   -0.970941817426052027156, -0.748510748171101098635, -0.354604887042535625970,
+                                   0.12053668025532305335, 0.568064746731155775490, 0.885456025653209895900};
+  static constexpr double s[13] = {0.0, 0.464723172043768546302, 0.82298386589365639458, 0.992708874098054009100,
+                                   0.935016242685414832420, 0.663122658240795206160, 0.23931566428755776715,
+                                   -0.23931566428755776715, -0.663122658240795206160, -0.935016242685414832420,
+                                   -0.992708874098054009100, -0.82298386589365639458, -0.464723172043768546302};
+};
+template <> struct Roots<16> {
+  static constexpr double c[10] = {1.0, 0.923879532511286756128, 0.707106781186547524401, 0.382683432365089771728,
+                                   0.0, -0.382683432365089771728, -0.707106781186547524401, -0.923879532511286756128,
+                                   -1.0, -0.923879532511286756128};
+  static constexpr double s[10] = {0.0, 0.382683432365089771728, 0.707106781186547524401, 0.923879532511286756128,
+                                   1.0, 0.923879532511286756128, 0.707106781186547524401, 0.382683432365089771728,
+                                   0.0, -0.382683432365089771728};
+};
+
+// prime radix: the terms m and p - m share their cosine and sine products
+template <int p, typename C> __device__ __forceinline__ void bfly_prime(C* a) {
+  using R = decltype(a[0].x);
+  constexpr int h = (p - 1) / 2;
+  C s[h], d[h];
+  C sum = a[0];
+#pragma unroll
+  for (int m = 0; m < h; ++m) {
+    s[m] = cadd(a[m + 1], a[p - 1 - m]);
+    d[m] = csub(a[m + 1], a[p - 1 - m]);
+    sum = cadd(sum, s[m]);
+  }
+  const C a0 = a[0];
+  a[0] = sum;
+#pragma unroll
+  for (int k = 1; k <= h; ++k) {
+    C A = a0, B{R(0), R(0)};
+#pragma unroll
+    for (int m = 1; m <= h; ++m) {
+      const R c = static_cast<R>(Roots<p>::c[(k * m) % p]), sn = static_cast<R>(Roots<p>::s[(k * m) % p]);
+      A = C{A.x + c * s[m - 1].x, A.y + c * s[m - 1].y};
+      B = C{B.x + sn * d[m - 1].x, B.y + sn * d[m - 1].y};
+    }
+    const C t = cmul_mi(B);
+    a[k] = cadd(A, t);
+    a[p - k] = csub(A, t);
+  }
+}
+
+template <int r, typename C> __device__ __forceinline__ void mix_bfly(C* a);
+
+// r = r1 * r2, coprime: input r2 i + r1 j and output e1 k1 + e2 k2 (mod r)
+// with e1 = 1 (mod r1), 0 (mod r2) and e2 the other way round need no
+// twiddles between the two dimensions (Good 1958, Thomas 1963)
+template <int r1, int r2, typename C> __device__ __forceinline__ void bfly_coprime(C* a) {
+  constexpr int r = r1 * r2;
+  constexpr int e1 = [] { for (int v = r2;; v += r2) if (v % r1 == 1) return v; }();
+  constexpr int e2 = [] { for (int v = r1;; v += r1) if (v % r2 == 1) return v; }();
+  C g[r2][r1];
+#pragma unroll
+  for (int j = 0; j < r2; ++j) {
+#pragma unroll
+    for (int i = 0; i < r1; ++i) g[j][i] = a[(r2 * i + r1 * j) % r];
+    mix_bfly<r1>(g[j]);
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < r1; ++k1) {
+    C t[r2];
+#pragma unroll
+    for (int j = 0; j < r2; ++j) t[j] = g[j][k1];
+    mix_bfly<r2>(t);
+#pragma unroll
+    for (int k2 = 0; k2 < r2; ++k2) a[(e1 * k1 + e2 * k2) % r] = t[k2];
+  }
+}
+
+// r = q * q: q sub-transforms of the inputs q i + j, a twiddle, q across
+template <int q, typename C> __device__ __forceinline__ void bfly_square(C* a) {
+  using R = decltype(a[0].x);
+  constexpr int r = q * q;
+  C g[q][q];
+#pragma unroll
+  for (int j = 0; j < q; ++j) {
+#pragma unroll
+    for (int i = 0; i < q; ++i) g[j][i] = a[q * i + j];
+    mix_bfly<q>(g[j]);
+#pragma unroll
+    for (int k = 1; k < q; ++k) {
+      if (j > 0) {
+        const R c = static_cast<R>(Roots<r>::c[j * k]), s = static_cast<R>(Roots<r>::s[j * k]);
+        const C x = g[j][k];
+        g[j][k] = C{x.x * c + x.y * s, x.y * c - x.x * s};
+      }
+    }
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < q; ++k1) {
+    C t[q];
+#pragma unroll
+    for (int j = 0; j < q; ++j) t[j] = g[j][k1];
+    mix_bfly<q>(t);
+#pragma unroll
+    for (int k2 = 0; k2 < q; ++k2) a[k1 + q * k2] = t[k2];
+  }
+}
+
+template <int r, typename C> __device__ __forceinline__ void mix_bfly(C* a) {
+  if constexpr (r == 2 || r == 3 || r == 4 || r == 5 || r == 8) bfly<r>(a);
+  else if constexpr (r == 6) bfly_coprime<2, 3>(a);
+  else if constexpr (r == 9) bfly_square<3>(a);
+  else if constexpr (r == 10) bfly_coprime<2, 5>(a);
+  else if constexpr (r == 12) bfly_coprime<4, 3>(a);
+  else if constexpr (r == 15) bfly_coprime<3, 5>(a);
+  else if constexpr (r == 16) bfly_square<4>(a);
+  else bfly_prime<r>(a);
+}
+
+// Twiddle-table entries a butterfly loads: w, and for FP64 also w^4 and w^8,
+// which keeps every power at most two rounded products away from the table
+// (with w alone they are four away, and the error of a 1000-point FP64 line
+// grows from 5.2e-16 to 6.4e-16).  FP32 powers are FP64 products of w.
+template <int r, typename Real> constexpr int mix_ntw() { return sizeof(Real) == 8 ? (r + 3) / 4 : 1; }
+
+// v[j] *= w^j: each power is rounded once to the kernel's precision and used
+// before the next is formed
+template <int r, typename C> __device__ __forceinline__ void mix_twiddle(C* v, const double2* ww) {
+  constexpr bool kTable = sizeof(C) == 16;
+  const double2 w = ww[0];
+  double2 lo[4];
+  lo[1] = w;
+  if constexpr (r > 2) lo[2] = cmul(w, w);
+  if constexpr (r > 3) lo[3] = cmul(lo[2], w);
+#pragma unroll
+  for (int j = 1; j < 4 && j < r; ++j) v[j] = cmul(v[j], to_prec<C>(lo[j]));
+  if constexpr (r > 4) {
+    double2 w4, hi;
+    if constexpr (kTable) hi = w4 = ww[1];
+    else hi = w4 = cmul(lo[2], lo[2]);
+#pragma unroll
+    for (int g = 4; g < r; g += 4) {
+      v[g] = cmul(v[g], to_prec<C>(hi));
+#pragma unroll
+      for (int j = 1; j < 4; ++j)
+        if (g + j < r) v[g + j] = cmul(v[g + j], to_prec<C>(cmul(hi, lo[j])));
+      if (g + 4 < r) {
+        if constexpr (kTable) hi = ww[g / 4 + 1];
+        else hi = cmul(hi, w4);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Stage pieces.  Lane t of a line carries butterflies beta = t + q T of a
+// stage (q < mix_nb<V>(r)); its inputs are positions beta + j nr, its outputs
+// (beta / L) L r + beta % L + j L.
+// ---------------------------------------------------------------------------
+// Real or imaginary halves of the values of one lane through the line's LDS
+// positions (the exchanges always travel in two halves: half the LDS per
+// line, so two blocks of long lines stay resident on a CU)
+template <int r, int V, typename Real>
+__device__ __forceinline__ void mix_gather(Real* v, const MixStage& st, int t, int T, const Real* lds, int ps) {
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      const int g = static_cast<int>(st.dL.div(static_cast<uint32_t>(beta)));
+      const Real* src = lds + (beta + g * st.in_pad) * ps;
+#pragma unroll
+      for (int j = 0; j < r; ++j) v[q * r + j] = src[j * st.in_step];
+    }
+  }
+}
+template <int r, int V, typename Real>
+__device__ __forceinline__ void mix_scatter(const Real* v, const MixStage& st, int t, int T, Real* lds, int ps) {
+  const int step = st.L * ps;
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      const int g = static_cast<int>(st.dL.div(static_cast<uint32_t>(beta)));
+      Real* dst = lds + (beta + g * (st.out_group - st.L)) * ps;
+#pragma unroll
+      for (int j = 0; j < r; ++j) dst[j * step] = v[q * r + j];
+    }
+  }
+}
+// twiddle-table entries of the lane's butterflies of a stage
+template <int r, int V, typename Real>
+__device__ __forceinline__ void mix_tw_load(double2* w, const MixStage& st, int t, int T, const double2* tw) {
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      const int g = static_cast<int>(st.dL.div(static_cast<uint32_t>(beta)));
+      const int e = (beta - g * st.L) * st.ts;
+      constexpr int N = mix_ntw<r, Real>();
+#pragma unroll
+      for (int i = 0; i < N; ++i) w[q * N + i] = twiddle_load(tw + (i == 0 ? e : 4 * i * e));
+    }
+  }
+}
+template <int r, int V, typename Real>
+__device__ __forceinline__ void mix_compute(Real* re, Real* im, const MixStage& st, int t, int T, const double2* w) {
+  using C = cplx_t<Real>;
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    if (t + q * T < st.nr) {
+      C a[r];
+#pragma unroll
+      for (int j = 0; j < r; ++j) a[j] = C{re[q * r + j], im[q * r + j]};
+      if (st.L > 1) mix_twiddle<r>(a, w + q * mix_ntw<r, Real>());
+      mix_bfly<r>(a);
+#pragma unroll
+      for (int j = 0; j < r; ++j) {
+        re[q * r + j] = a[j].x;
+        im[q * r + j] = a[j].y;
+      }
+    }
+  }
+}
+
+// the radix of a stage is uniform over the launch: a scalar branch
+#define DFFT_MIX_SWITCH(radix, CALL) \
+  switch (radix) {                   \
+    case 2: if constexpr (mix_has<V>(2)) { CALL(2); } break; \
+    case 3: if constexpr (mix_has<V>(3)) { CALL(3); } break; \
+    case 4: if constexpr (mix_has<V>(4)) { CALL(4); } break; \
+    case 5: if constexpr (mix_has<V>(5)) { CALL(5); } break; \
+    case 6: if constexpr (mix_has<V>(6)) { CALL(6); } break; \
+    case 7: if constexpr (mix_has<V>(7)) { CALL(7); } break; \
+    case 8: if constexpr (mix_has<V>(8)) { CALL(8); } break; \
+    case 9: if constexpr (mix_has<V>(9)) { CALL(9); } break; \
+    case 10: if constexpr (mix_has<V>(10)) { CALL(10); } break; \
+    case 11: if constexpr (mix_has<V>(11)) { CALL(11); } break; \
+    case 12: if constexpr (mix_has<V>(12)) { CALL(12); } break; \
+    case 13: if constexpr (mix_has<V>(13)) { CALL(13); } break; \
+    case 15: if constexpr (mix_has<V>(15)) { CALL(15); } break; \
+    case 16: if constexpr (mix_has<V>(16)) { CALL(16); } break; \
+    default: break;                  \
+  }
+
+// global loads of the first stage / stores of the last one
+template <int r, int V, bool NT, typename Real>
+__device__ __forceinline__ void mix_load_c2c(Real* re, Real* im, const MixStage& st, int t, int T, const char* ib,
+                                             int64_t is, bool inverse) {
+  using C = cplx_t<Real>;
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      const C* src = reinterpret_cast<const C*>(ib) + beta * is;
+      const int64_t step = st.nr * is;
+      C x[r];
+#pragma unroll
+      for (int j = 0; j < r; ++j) {
+        x[j] = gload_c<NT, Real>(src);
+        src += step;
+      }
+#pragma unroll
+      for (int j = 0; j < r; ++j) {
+        re[q * r + j] = x[j].x;
+        im[q * r + j] = inverse ? -x[j].y : x[j].y;
+      }
+    }
+  }
+}
+template <int r, int V, bool NT, typename Real>
+__device__ __forceinline__ void mix_load_real(Real* v, const MixStage& st, int t, int T, const char* ib, int64_t is) {
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      const Real* src = reinterpret_cast<const Real*>(ib) + beta * is;
+      const int64_t step = st.nr * is;
+#pragma unroll
+      for (int j = 0; j < r; ++j) {
+        v[q * r + j] = gload<NT>(src);
+        src += step;
+      }
+    }
+  }
+}
+template <int r, int V, bool NT, typename Real>
+__device__ __forceinline__ void mix_store_c2c(const Real* re, const Real* im, const MixStage& st, int t, int T,
+                                              char* ob, int64_t os, Real sx, Real sy) {
+  using C = cplx_t<Real>;
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      C* dst = reinterpret_cast<C*>(ob) + beta * os;
+      const int64_t step = st.nr * os;
+#pragma unroll
+      for (int j = 0; j < r; ++j) {
+        gstore_c<NT, Real>(dst, C{re[q * r + j] * sx, im[q * r + j] * sy});
+        dst += step;
+      }
+    }
+  }
+}
+template <int r, int V, bool NT, typename Real>
+__device__ __forceinline__ void mix_store_real(const Real* v, const MixStage& st, int t, int T, char* ob, int64_t os,
+                                               Real s) {
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      Real* dst = reinterpret_cast<Real*>(ob) + beta * os;
+      const int64_t step = st.nr * os;
+#pragma unroll
+      for (int j = 0; j < r; ++j) {
+        gstore<NT>(dst, v[q * r + j] * s);
+        dst += step;
+      }
+    }
+  }
+}
+
+// All radix stages of a line whose stage-0 inputs are in registers; leaves
+// the outputs of the last stage there.
+template <int V, typename Real>
+__device__ __forceinline__ void mix_stages(Real* re, Real* im, const MixPlan& m, int t, Real* lds, const double2* tw) {
+  double2 w[sizeof(Real) == 8 ? 4 : mix_nb_max<V>()];
+  for (int s = 0;; ++s) {
+    const MixStage& st = m.st[s];
+#define DFFT_MIX_CALL(r) mix_compute<r, V, Real>(re, im, st, t, m.T, w)
+    DFFT_MIX_SWITCH(st.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    if (s + 1 >= m.nst) break;
+    const MixStage& nx = m.st[s + 1];
+    __syncthreads();
+#define DFFT_MIX_CALL(r) mix_scatter<r, V, Real>(re, st, t, m.T, lds, m.ps)
+    DFFT_MIX_SWITCH(st.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    __syncthreads();
+    // the next stage's twiddles are on their way during the second half
+#define DFFT_MIX_CALL(r)                             \
+  mix_tw_load<r, V, Real>(w, nx, t, m.T, tw);                 \
+  mix_gather<r, V, Real>(re, nx, t, m.T, lds, m.ps)
+    DFFT_MIX_SWITCH(nx.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    __syncthreads();
+#define DFFT_MIX_CALL(r) mix_scatter<r, V, Real>(im, st, t, m.T, lds, m.ps)
+    DFFT_MIX_SWITCH(st.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    __syncthreads();
+#define DFFT_MIX_CALL(r) mix_gather<r, V, Real>(im, nx, t, m.T, lds, m.ps)
+    DFFT_MIX_SWITCH(nx.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+  }
+}
+
+// KIND kC2C: one complex line per T lanes.  kR2C / kC2R: two real lines 2q,
+// 2q+1 per T lanes as one complex line (PairIO).
+template <typename Real, int V, bool NT, int KIND>
+__global__ void __launch_bounds__(1024) fft_mixed(const LinePass p, const MixPlan m) {
+  using C = cplx_t<Real>;
+  extern __shared__ unsigned char smem_raw[];
+  const int tid = threadIdx.x;
+  const int B = p.lines_per_block, T = m.T, n = p.n;
+  int b, t;
+  if (p.lines_fast) {
+    b = tid & (B - 1);
+    t = tid >> m.log2B;
+  } else {
+    b = static_cast<int>(m.dT.div(static_cast<uint32_t>(tid)));
+    t = tid - b * T;
+  }
+  // lanes beyond the block's lines hold no butterfly (beta < nr never holds)
+  // and touch neither LDS nor global memory; they reach every barrier
+  const bool active = tid < B * T;
+  if (!active) {
+    b = 0;
+    t = 1 << 28;
+  }
+  Real* lds = reinterpret_cast<Real*>(smem_raw) + b * m.bs;
+  const double2* tw = reinterpret_cast<const double2*>(p.tw);
+  const int32_t unit = pass_block(p, blockIdx.x, gridDim.x) * B + b;
+  const MixStage& s0 = m.st[0];
+  const MixStage& sl = m.st[m.nst - 1];
+  Real re[V], im[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    re[j] = Real(0);
+    im[j] = Real(0);
+  }
+
+  if constexpr (KIND == kC2C) {
+    const bool valid = active && unit < p.nlines && !padding_line<Real>(p, unit);
+    LineIO<Real, NT> io;
+    if (valid) {
+      io = make_line_io<Real, NT>(p, unit);
+#define DFFT_MIX_CALL(r) mix_load_c2c<r, V, NT, Real>(re, im, s0, t, T, io.ib, io.is, p.inverse != 0)
+      DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    }
+    mix_stages<V, Real>(re, im, m, t, lds, tw);
+    if (valid) {
+      const Real sy = p.inverse ? -io.scale : io.scale;
+#define DFFT_MIX_CALL(r) mix_store_c2c<r, V, NT, Real>(re, im, sl, t, T, io.ob, io.os, io.scale, sy)
+      DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    }
+  } else if constexpr (KIND == kR2C) {
+    const bool valid = active && 2 * unit < p.nlines;  // paired passes never enumerate padding
+    PairIO<Real, NT> io{};
+    if (valid) {
+      io = make_pair_io<Real, NT>(p, unit);
+#define DFFT_MIX_CALL(r) mix_load_real<r, V, NT, Real>(re, s0, t, T, io.ib[0], io.is[0])
+      DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+      if (io.has_b) {
+#define DFFT_MIX_CALL(r) mix_load_real<r, V, NT, Real>(im, s0, t, T, io.ib[1], io.is[1])
+        DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+      }
+    }
+    mix_stages<V, Real>(re, im, m, t, lds, tw);
+    // spectra of the two lines at k = t + q T <= n/2 from Z_k and Z_{n-k}:
+    // A = (Z_k + conj Z_{n-k}) / 2, B = (Z_k - conj Z_{n-k}) / (2 i)
+    Real ax[mix_half<V>()], by[mix_half<V>()], ay[mix_half<V>()], bx[mix_half<V>()];
+    __syncthreads();
+#define DFFT_MIX_CALL(r) mix_scatter<r, V, Real>(re, sl, t, T, lds, m.ps)
+    DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < mix_half<V>(); ++q) {
+      const int k = t + q * T;
+      if (2 * k <= n) {
+        const Real u = lds[k * m.ps], v = lds[(k == 0 ? 0 : n - k) * m.ps];
+        ax[q] = u + v;
+        by[q] = v - u;
+      }
+    }
+    __syncthreads();
+#define DFFT_MIX_CALL(r) mix_scatter<r, V, Real>(im, sl, t, T, lds, m.ps)
+    DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < mix_half<V>(); ++q) {
+      const int k = t + q * T;
+      if (2 * k <= n) {
+        const Real u = lds[k * m.ps], v = lds[(k == 0 ? 0 : n - k) * m.ps];
+        ay[q] = u - v;
+        bx[q] = u + v;
+      }
+    }
+    if (valid) {
+      C* pa = reinterpret_cast<C*>(io.ob[0]) + t * io.os[0];
+      C* pb = reinterpret_cast<C*>(io.ob[1]) + t * io.os[1];
+#pragma unroll
+      for (int q = 0; q < mix_half<V>(); ++q) {
+        const int k = t + q * T;
+        if (2 * k <= n) {
+          const Real h = Real(0.5) * io.scale * ((k != 0 && 2 * k != n) ? io.hw : Real(1));
+          gstore_c<NT, Real>(pa + static_cast<int64_t>(q) * T * io.os[0], C{ax[q] * h, ay[q] * h});
+          if (io.has_b) gstore_c<NT, Real>(pb + static_cast<int64_t>(q) * T * io.os[1], C{bx[q] * h, by[q] * h});
+        }
+      }
+    }
+  } else {
+    // C2R: the lane that loads entry k <= n/2 of both half spectra forms the
+    // inputs conj(A + i B) at k and at n - k and hands them out through LDS
+    const bool valid = active && 2 * unit < p.nlines;
+    PairIO<Real, NT> io{};
+    Real xk[mix_half<V>()], xm[mix_half<V>()], yk[mix_half<V>()], ym[mix_half<V>()];
+    if (valid) {
+      io = make_pair_io<Real, NT>(p, unit);
+      C A[mix_half<V>()], Bv[mix_half<V>()];
+      const C* pa = reinterpret_cast<const C*>(io.ib[0]) + t * io.is[0];
+      const C* pb = reinterpret_cast<const C*>(io.ib[1]) + t * io.is[1];
+#pragma unroll
+      for (int q = 0; q < mix_half<V>(); ++q) {
+        const int k = t + q * T;
+        A[q] = C{Real(0), Real(0)};
+        Bv[q] = C{Real(0), Real(0)};
+        if (2 * k <= n) {
+          A[q] = gload_c<NT, Real>(pa + static_cast<int64_t>(q) * T * io.is[0]);
+          if (io.has_b) Bv[q] = gload_c<NT, Real>(pb + static_cast<int64_t>(q) * T * io.is[1]);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < mix_half<V>(); ++q) {
+        const int k = t + q * T;
+        const C lo = io.c2r_value(k, true, A[q], Bv[q]);
+        const C hi = io.c2r_value(n - k, false, A[q], Bv[q]);
+        xk[q] = lo.x;
+        yk[q] = lo.y;
+        xm[q] = hi.x;
+        ym[q] = hi.y;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < mix_half<V>(); ++q) xk[q] = xm[q] = yk[q] = ym[q] = Real(0);
+    }
+#pragma unroll
+    for (int q = 0; q < mix_half<V>(); ++q) {
+      const int k = t + q * T;
+      if (2 * k <= n) {
+        lds[k * m.ps] = xk[q];
+        if (k > 0 && 2 * k < n) lds[(n - k) * m.ps] = xm[q];
+      }
+    }
+    __syncthreads();
+#define DFFT_MIX_CALL(r) mix_gather<r, V, Real>(re, s0, t, T, lds, m.ps)
+    DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < mix_half<V>(); ++q) {
+      const int k = t + q * T;
+      if (2 * k <= n) {
+        lds[k * m.ps] = yk[q];
+        if (k > 0 && 2 * k < n) lds[(n - k) * m.ps] = ym[q];
+      }
+    }
+    __syncthreads();
+#define DFFT_MIX_CALL(r) mix_gather<r, V, Real>(im, s0, t, T, lds, m.ps)
+    DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+    mix_stages<V, Real>(re, im, m, t, lds, tw);
+    // w = FFT(conj Z), a + i b = conj(w)
+    if (valid) {
+#define DFFT_MIX_CALL(r) mix_store_real<r, V, NT, Real>(re, sl, t, T, io.ob[0], io.os[0], io.scale)
+      DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+      if (io.has_b) {
+#define DFFT_MIX_CALL(r) mix_store_real<r, V, NT, Real>(im, sl, t, T, io.ob[1], io.os[1], -io.scale)
+        DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
+      }
+    }
+  }
+}
+
+#undef DFFT_MIX_SWITCH
+
+}  // namespace dfft
