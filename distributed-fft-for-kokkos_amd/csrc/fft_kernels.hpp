@@ -76,6 +76,13 @@ struct LinePass {
   // divergence-form Navier-Stokes right-hand side formed as the lines load
   int32_t products;
   int32_t prod_axis;
+  // band > 0: a pass over the kept modes |k| <= band of a dealiased field
+  // (FP64, power-of-two lengths 8..1024; launch_band_pass).  Index i of batch
+  // axis j stands for i + (i > band ? band_shift[j] : 0) (the kept indices of
+  // a whole spectral axis wrap around), inverse lines read the positions
+  // beyond the band as zeros, forward lines store none of them.
+  int32_t band;
+  int32_t band_shift[kMaxDim - 1];
   // Weight of the interior half-spectrum entries (0 < k < n/2) of an R2C /
   // C2R line, applied to the values a C2R line loads or an R2C line stores;
   // 0 means 1.  Adjoint transforms use 1/2 (C2R) and 2 (R2C).
@@ -152,6 +159,10 @@ hipError_t launch_bluestein_post(const LinePass& p, int log2m, const void* chirp
 // of two); hipErrorNotSupported for other passes
 hipError_t launch_products_pass(const LinePass& p, hipStream_t s);
 bool products_pass_supported(int n);
+// a pass with p.band set (and products, if set too): C2C lines, R2C / C2R
+// lines in pairs, undistributed line axis
+hipError_t launch_band_pass(const LinePass& p, hipStream_t s);
+bool band_pass_supported(int n);
 hipError_t launch_remap(const RemapArgs& a, int esize, hipStream_t s);
 
 // Reference-exact pack/unpack of one rank's local array (mapped by `map`)

@@ -273,7 +273,8 @@ template <typename Real, bool NT = false> struct PairIO {
   }
 };
 
-template <typename Real>
+// BAND: a pass over the kept modes of a dealiased field only (LinePass::band)
+template <typename Real, bool BAND = false>
 __device__ __forceinline__ void decode_line(const LinePass& p, int32_t line, int32_t* idx) {
 #pragma unroll
   for (int a = 0; a < kMaxDim; ++a) idx[a] = 0;
@@ -282,26 +283,28 @@ __device__ __forceinline__ void decode_line(const LinePass& p, int32_t line, int
   for (int j = kMaxDim - 2; j >= 0; --j) {
     if (j < p.nbatch) {
       uint32_t q = p.batch_div[j].div(rem);
-      idx[p.batch_axis[j]] = static_cast<int32_t>(rem - q * static_cast<uint32_t>(p.batch_ext[j]));
+      int32_t i = static_cast<int32_t>(rem - q * static_cast<uint32_t>(p.batch_ext[j]));
+      if constexpr (BAND) i += i > p.band ? p.band_shift[j] : 0;
+      idx[p.batch_axis[j]] = i;
       rem = q;
     }
   }
 }
 
 // true if line `line` of a pass enumerated over a padded extent is padding
-template <typename Real>
+template <typename Real, bool BAND = false>
 __device__ __forceinline__ bool padding_line(const LinePass& p, int32_t line) {
   if (p.pad_real <= 0) return false;
   int32_t idx[kMaxDim];
-  decode_line<Real>(p, line, idx);
+  decode_line<Real, BAND>(p, line, idx);
   return idx[p.pad_axis] >= p.pad_real;
 }
 
-template <typename Real, bool NT = false>
+template <typename Real, bool NT = false, bool BAND = false>
 __device__ __forceinline__ LineIO<Real, NT> make_line_io(const LinePass& p, int32_t line) {
   using C = cplx_t<Real>;
   int32_t idx[kMaxDim];
-  decode_line<Real>(p, line, idx);
+  decode_line<Real, BAND>(p, line, idx);
   LineIO<Real, NT> io;
   const int64_t ies = p.kind == kR2C ? sizeof(Real) : sizeof(C);
   const int64_t oes = p.kind == kC2R ? sizeof(Real) : sizeof(C);
@@ -335,7 +338,7 @@ __device__ __forceinline__ const char* product_source(const LinePass& p, const i
   return element_ptr(p.in, j, ies, p.axis, is);
 }
 
-template <typename Real, bool NT, bool PROD = false>
+template <typename Real, bool NT, bool PROD = false, bool BAND = false>
 __device__ __forceinline__ PairIO<Real, NT> make_pair_io(const LinePass& p, int32_t pair) {
   using C = cplx_t<Real>;
   PairIO<Real, NT> io;
@@ -343,7 +346,7 @@ __device__ __forceinline__ PairIO<Real, NT> make_pair_io(const LinePass& p, int3
   const int64_t oes = p.kind == kC2R ? sizeof(Real) : sizeof(C);
   int32_t idx[kMaxDim];
   const int32_t la = 2 * pair;
-  decode_line<Real>(p, la, idx);
+  decode_line<Real, BAND>(p, la, idx);
   if constexpr (PROD) {
     io.ib[0] = product_source(p, idx, ies, io.is[0]);
   } else {
@@ -352,7 +355,7 @@ __device__ __forceinline__ PairIO<Real, NT> make_pair_io(const LinePass& p, int3
   io.ob[0] = element_ptr(p.out, idx, oes, p.axis, io.os[0]);
   io.has_b = la + 1 < p.nlines;
   if (io.has_b) {
-    decode_line<Real>(p, la + 1, idx);
+    decode_line<Real, BAND>(p, la + 1, idx);
     if constexpr (PROD) {
       io.ib[1] = io.ib[0];
       io.is[1] = io.is[0];
@@ -823,7 +826,9 @@ __device__ __forceinline__ void fast_line2_body(const LinePass& p, int32_t blk, 
 // lengths) run the stages on zeros in a spare LDS slot (index B) so every
 // lane reaches every barrier; they load and store nothing.  STAGE (complex64
 // grouped passes) moves contiguous lines 16 bytes per lane through LDS.
-template <typename Real, int N, int RM, bool NT, bool SPLIT, bool STAGE = false>
+// BAND: a C2C pass over kept modes: inverse lines read positions outside the
+// band as zeros, forward lines store only the band.
+template <typename Real, int N, int RM, bool NT, bool SPLIT, bool STAGE = false, bool BAND = false>
 __device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, int B, unsigned char* lds) {
   using C = cplx_t<Real>;
   using Cfg = FastCfg<Real, N, RM>;
@@ -853,11 +858,11 @@ __device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, i
     // spare lanes), so the line index is wave-uniform and the descriptor
     // arithmetic of make_line_io runs once per wave on the scalar unit
     const int32_t wl = __builtin_amdgcn_readfirstlane(line);
-    valid = active && wl < p.nlines && !padding_line<Real>(p, wl);
-    if (valid) io = make_line_io<Real, NT>(p, wl);
+    valid = active && wl < p.nlines && !padding_line<Real, BAND>(p, wl);
+    if (valid) io = make_line_io<Real, NT, BAND>(p, wl);
   } else {
-    valid = active && line < p.nlines && !padding_line<Real>(p, line);
-    if (valid) io = make_line_io<Real, NT>(p, line);
+    valid = active && line < p.nlines && !padding_line<Real, BAND>(p, line);
+    if (valid) io = make_line_io<Real, NT, BAND>(p, line);
   }
 
   C v[R];
@@ -897,6 +902,27 @@ __device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, i
   }
   if (vin) {
     // loaded above, through LDS
+  } else if (BAND && p.inverse) {
+    // positions p.band < pos < N - p.band are zeros: runs of S positions that
+    // lie in there whole are not loaded (a branch on scalars), lanes of the
+    // two runs at its ends repeat the address of the band's edge
+    constexpr int S = N / r0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = C{Real(0), Real(0)};
+    if (valid) {
+#pragma unroll
+      for (int j = 0; j < r0; ++j) {
+        if (j * S > p.band && (j + 1) * S - 1 < N - p.band) continue;
+#pragma unroll
+        for (int q = 0; q < NB0; ++q) {
+          const int pos = t * NB0 + q + j * S;
+          const bool keep = pos <= p.band || pos >= N - p.band;
+          const C x = gload_c<NT, Real>(reinterpret_cast<const C*>(io.ib) +
+                                        static_cast<int64_t>(keep ? pos : p.band) * io.is);
+          v[q * r0 + j] = keep ? cconj(x) : C{Real(0), Real(0)};
+        }
+      }
+    }
   } else if (p.kind == kC2C) {
     // C2C lines are walked with pointer increments (no 64-bit product per
     // element).  One branch around all the loads: a select per load puts
@@ -983,7 +1009,16 @@ __device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, i
   }
 
   if (valid && !vout) {
-    if (p.kind == kC2C) {
+    if (BAND && !p.inverse) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        const int pos = t + j * T;
+        if (j * T > p.band && (j + 1) * T - 1 < N - p.band) continue;
+        if (pos <= p.band || pos >= N - p.band)
+          gstore_c<NT, Real>(reinterpret_cast<C*>(io.ob) + static_cast<int64_t>(pos) * io.os,
+                             C{v[j].x * io.scale, v[j].y * io.scale});
+      }
+    } else if (p.kind == kC2C) {
       C* dst = reinterpret_cast<C*>(io.ob) + static_cast<int64_t>(t) * io.os;
       const int64_t step = static_cast<int64_t>(T) * io.os;
 #pragma unroll
@@ -1005,7 +1040,8 @@ __device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, i
 // (q = blk*B + b) as one complex line; same stage code as fast_line_body.
 // PROD: a products pass (LinePass::products): each loaded real value is the
 // product of the two factor lines' values at that position.
-template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false>
+// BAND: half-spectrum entries above p.band are neither read (zeros) nor stored.
+template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false, bool BAND = false>
 __device__ __forceinline__ void fast_pair_body(const LinePass& p, int32_t blk, int B, unsigned char* lds) {
   using C = cplx_t<Real>;
   using Cfg = FastCfg<Real, N, RM>;
@@ -1035,9 +1071,9 @@ __device__ __forceinline__ void fast_pair_body(const LinePass& p, int32_t blk, i
     // spare lanes), so the pair index is wave-uniform and the descriptor
     // arithmetic of make_pair_io runs once per wave on the scalar unit
     const int32_t wp = __builtin_amdgcn_readfirstlane(pair);
-    if (valid) io = make_pair_io<Real, NT, PROD>(p, wp);
+    if (valid) io = make_pair_io<Real, NT, PROD, BAND>(p, wp);
   } else {
-    if (valid) io = make_pair_io<Real, NT, PROD>(p, pair);
+    if (valid) io = make_pair_io<Real, NT, PROD, BAND>(p, pair);
   }
 
   // Products pass: the block holds whole positions (B is a multiple of 3 and
@@ -1109,27 +1145,47 @@ __device__ __forceinline__ void fast_pair_body(const LinePass& p, int32_t blk, i
         constexpr int JH = r0 / 2;
         const C* la = reinterpret_cast<const C*>(io.ib[0]) + static_cast<int64_t>(beta) * io.is[0];
         const C* lb = reinterpret_cast<const C*>(io.ib[1]) + static_cast<int64_t>(beta) * io.is[1];
-        const bool mid = 2 * (beta + JH * S) <= N;
+        const bool mid = !BAND && 2 * (beta + JH * S) <= N;
         C A[JH + 1], Bv[JH + 1];
 #pragma unroll
         for (int j = 0; j <= JH; ++j) {
           A[j] = C{Real(0), Real(0)};
           Bv[j] = C{Real(0), Real(0)};
         }
-        if (valid) {
+        if constexpr (BAND) {
+          // as in fast_line_body: whole runs above the band are skipped, lanes
+          // beyond its edge repeat the edge's address
 #pragma unroll
-          for (int j = 0; j < JH; ++j) A[j] = gload_c<NT, Real>(la + j * sa);
-          if (mid) A[JH] = gload_c<NT, Real>(la + JH * sa);
-        }
-        if (vb) {
+          for (int j = 0; j < JH; ++j) {
+            if (j * S > p.band) continue;
+            const int pos = beta + j * S;
+            const bool keep = pos <= p.band;
+            const int64_t at = keep ? pos : p.band;
+            if (valid) {
+              const C x = gload_c<NT, Real>(reinterpret_cast<const C*>(io.ib[0]) + at * io.is[0]);
+              A[j] = keep ? x : C{Real(0), Real(0)};
+            }
+            if (vb) {
+              const C x = gload_c<NT, Real>(reinterpret_cast<const C*>(io.ib[1]) + at * io.is[1]);
+              Bv[j] = keep ? x : C{Real(0), Real(0)};
+            }
+          }
+        } else {
+          if (valid) {
 #pragma unroll
-          for (int j = 0; j < JH; ++j) Bv[j] = gload_c<NT, Real>(lb + j * sb);
-          if (mid) Bv[JH] = gload_c<NT, Real>(lb + JH * sb);
+            for (int j = 0; j < JH; ++j) A[j] = gload_c<NT, Real>(la + j * sa);
+            if (mid) A[JH] = gload_c<NT, Real>(la + JH * sa);
+          }
+          if (vb) {
+#pragma unroll
+            for (int j = 0; j < JH; ++j) Bv[j] = gload_c<NT, Real>(lb + j * sb);
+            if (mid) Bv[JH] = gload_c<NT, Real>(lb + JH * sb);
+          }
         }
 #pragma unroll
         for (int j = 0; j <= JH; ++j) {
           const int pos = beta + j * S;
-          if (j < JH || mid) {
+          if (j < JH || mid || BAND) {
             v[q * r0 + j] = io.c2r_value(pos, true, A[j], Bv[j]);
             mirror[q * r0 + j] = io.c2r_value(N - pos, false, A[j], Bv[j]);
           }
@@ -1248,7 +1304,7 @@ __device__ __forceinline__ void fast_pair_body(const LinePass& p, int32_t blk, i
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       const int pos = t + j * T;
-      if (2 * pos <= N) {
+      if (BAND ? pos <= p.band : 2 * pos <= N) {
         C A, Bv;
         io.r2c_values(pos, v[j], w[j], A, Bv);
         gstore_c<NT, Real>(pa, A);
@@ -1282,18 +1338,18 @@ __device__ __forceinline__ int32_t pass_block(const LinePass& p, int32_t b, int3
   return b;
 }
 
-template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false>
+template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false, bool BAND = false>
 __global__ void __launch_bounds__(1024) fft_pair_fast(const LinePass p) {
   extern __shared__ unsigned char smem_raw[];
   const int32_t blk = pass_block(p, blockIdx.x, gridDim.x);
-  fast_pair_body<Real, N, RM, NT, SPLIT, PROD>(p, blk, p.lines_per_block, smem_raw);
+  fast_pair_body<Real, N, RM, NT, SPLIT, PROD, BAND>(p, blk, p.lines_per_block, smem_raw);
 }
 
-template <typename Real, int N, int RM, bool NT, bool SPLIT>
+template <typename Real, int N, int RM, bool NT, bool SPLIT, bool BAND = false>
 __global__ void __launch_bounds__(1024) fft_line_fast(const LinePass p) {
   extern __shared__ unsigned char smem_raw[];
   const int32_t blk = pass_block(p, blockIdx.x, gridDim.x);
-  fast_line_body<Real, N, RM, NT, SPLIT>(p, blk, p.lines_per_block, smem_raw);
+  fast_line_body<Real, N, RM, NT, SPLIT, false, BAND>(p, blk, p.lines_per_block, smem_raw);
 }
 
 template <typename Real, int N, int RM, bool NT, int SPLIT_IN>
@@ -1637,6 +1693,46 @@ hipError_t launch_products(LinePass p, hipStream_t s) {
   return hipGetLastError();
 }
 
+// FP64 passes over kept modes (LinePass::band): 8 values per lane, exchanges
+// in halves; C2C lines, R2C / C2R lines in pairs, products formed at the loads.
+template <int N, bool NT>
+hipError_t launch_band(LinePass p, hipStream_t s) {
+  using Real = double;
+  using Cfg = FastCfg<Real, N, 8>;
+  constexpr int T = Cfg::T;
+  constexpr size_t line_bytes = line_lds_bytes<Real, N, 8, true>();
+  const bool pair = p.kind != kC2C;
+  if (pair && (p.kind == kR2C) == (p.inverse != 0)) return hipErrorInvalidValue;
+  int B = p.lines_per_block;
+  if (p.products) {
+    // whole positions of three pairs each, as launch_products
+    B = 3;
+    while (B * T < 192 || (B * T) % 64) B += 3;
+    while (B > 3 && (B * T > 1024 || static_cast<size_t>(B) * line_bytes > 160 * 1024)) B -= 3;
+    if (p.kind != kR2C || p.nlines % 6 != 0 || p.line_begin % 6 != 0) return hipErrorInvalidConfiguration;
+  } else if (B <= 0) {
+    B = p.lines_fast ? 8 : (T >= 256 ? 1 : 256 / T);
+    while (B * T > 1024) B /= 2;
+  }
+  const size_t smem = static_cast<size_t>(B) * line_bytes;
+  if (B * T > 1024 || smem > 160 * 1024) return hipErrorInvalidConfiguration;
+  p.lines_per_block = B;
+  p.swizzle = 0;
+  const int64_t units = pair ? (static_cast<int64_t>(p.nlines) + 1) / 2 : p.nlines;
+  const dim3 grid(static_cast<unsigned>((units + B - 1) / B)), block(static_cast<unsigned>(T * B));
+  static std::atomic<size_t> limit[3] = {64 * 1024, 64 * 1024, 64 * 1024};
+  const void* fns[3] = {reinterpret_cast<const void*>(&fft_line_fast<Real, N, 8, NT, true, true>),
+                        reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, true, false, true>),
+                        reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, true, true, true>)};
+  const int k = p.products ? 2 : (pair ? 1 : 0);
+  const hipError_t e = raise_lds_limit(limit[k], fns[k], smem);
+  if (e != hipSuccess) return e;
+  if (k == 2) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, true, true>), grid, block, smem, s, p);
+  else if (k == 1) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, false, true>), grid, block, smem, s, p);
+  else hipLaunchKernelGGL((fft_line_fast<Real, N, 8, NT, true, true>), grid, block, smem, s, p);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 // fast-kernel dispatch for one precision and a range of lengths (defined in
@@ -1648,5 +1744,6 @@ hipError_t dispatch_fast_f32_long(const LinePass& p, hipStream_t s);
 hipError_t dispatch_fast_f64_xl(const LinePass& p, hipStream_t s);
 hipError_t dispatch_fast_f32_xl(const LinePass& p, hipStream_t s);
 hipError_t dispatch_products_f64(const LinePass& p, hipStream_t s);
+hipError_t dispatch_band_f64(const LinePass& p, hipStream_t s);
 
 }  // namespace dfft

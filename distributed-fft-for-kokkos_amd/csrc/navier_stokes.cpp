@@ -128,45 +128,61 @@ std::vector<void*> NavierStokes::alloc_set(bool spectral, int nf) {
   return out;
 }
 
+bool NavierStokes::kept_only() const {
+  if (form_ != 0 || !kept_modes_) return false;
+  for (const Plan* p : {plan_b_.get(), plan_f_.get(), plan_f3_.get()})
+    if (!p->band_supported(g_.cutoff)) return false;
+  return true;
+}
+
+void NavierStokes::forward(Plan& p, void* const* in, void* const* out, hipStream_t s) {
+  if (kept_only()) p.execute_band(in, out, DFFT_FORWARD, g_.cutoff, s);
+  else p.execute(in, out, DFFT_FORWARD, s);
+}
+
+void NavierStokes::backward(Plan& p, void* const* in, void* const* out, hipStream_t s) {
+  if (kept_only()) p.execute_band(in, out, DFFT_BACKWARD, g_.cutoff, s);
+  else p.execute(in, out, DFFT_BACKWARD, s);
+}
+
 void NavierStokes::forward_products(void* const* u, hipStream_t s) {
   if (fuse_products_ && plan_f_->products_supported()) {
-    plan_f_->execute_forward_products(u, nl_.data(), s);
+    plan_f_->execute_forward_products(u, nl_.data(), kept_only() ? g_.cutoff : 0, s);
     return;
   }
   for (int r = 0; r < P_; ++r)
     hip_check(ns_products(static_cast<const double*>(u[r]), static_cast<double*>(pf_[r]), phys_pts(r), s),
               "ns_products");
-  plan_f_->execute(pf_.data(), nl_.data(), DFFT_FORWARD, s);
+  forward(*plan_f_, pf_.data(), nl_.data(), s);
 }
 
 void NavierStokes::set_option(const std::string& key, long value) {
-  if (key == "fuse_products") {
-    if (value != 0 && value != 1) throw Error(DFFT_ERROR_INVALID_ARGUMENT, "fuse_products must be 0 or 1");
-    if (graph_exec_) {  // the captured step holds the old launches
-      hip_check(hipStreamSynchronize(graph_stream_), "hipStreamSynchronize");
-      (void)hipGraphExecDestroy(graph_exec_);
-      graph_exec_ = nullptr;
-    }
-    if (graph_) {
-      (void)hipGraphDestroy(graph_);
-      graph_ = nullptr;
-    }
-    fuse_products_ = value != 0;
-    return;
+  bool* flag = key == "fuse_products" ? &fuse_products_ : key == "kept_modes" ? &kept_modes_ : nullptr;
+  if (!flag) throw Error(DFFT_ERROR_INVALID_ARGUMENT, "unknown NS option " + key);
+  if (value != 0 && value != 1) throw Error(DFFT_ERROR_INVALID_ARGUMENT, key + " must be 0 or 1");
+  if (graph_exec_) {  // the captured step holds the old launches
+    hip_check(hipStreamSynchronize(graph_stream_), "hipStreamSynchronize");
+    (void)hipGraphExecDestroy(graph_exec_);
+    graph_exec_ = nullptr;
   }
-  throw Error(DFFT_ERROR_INVALID_ARGUMENT, "unknown NS option " + key);
+  if (graph_) {
+    (void)hipGraphDestroy(graph_);
+    graph_ = nullptr;
+  }
+  *flag = value != 0;
 }
 
 long NavierStokes::get_option(const std::string& key) const {
   if (key == "fuse_products") return fuse_products_ ? 1 : 0;
   if (key == "products_fused") return (form_ == 0 && fuse_products_ && plan_f_->products_supported()) ? 1 : 0;
+  if (key == "kept_modes") return kept_only() ? 1 : 0;
   throw Error(DFFT_ERROR_INVALID_ARGUMENT, "unknown NS option " + key);
 }
 
 void NavierStokes::rk_stage(int stage, hipStream_t s, void* const* u_keep) {
   if (form_ == 0) {
     void* const* u = u_keep ? u_keep : pb_.data();
-    plan_b_->execute(y_.data(), u, DFFT_BACKWARD, s);
+    backward(*plan_b_, y_.data(), u, s);
     forward_products(u, s);
   } else {
     for (int r = 0; r < P_; ++r)
@@ -182,7 +198,7 @@ void NavierStokes::rk_stage(int stage, hipStream_t s, void* const* u_keep) {
     NsStage st{form_, stage, static_cast<const double2*>(nl_[r]), static_cast<double2*>(y_[r]),
                static_cast<double2*>(yc_[r]), static_cast<double2*>(k1_[r]), static_cast<double2*>(k2_[r]),
                static_cast<double2*>(k3_[r])};
-    hip_check(ns_rhs_rk(g_, sblk_[r], st, s), "ns_rhs_rk");
+    hip_check(ns_rhs_rk(g_, sblk_[r], modes(r), st, s), "ns_rhs_rk");
   }
 }
 
@@ -254,8 +270,8 @@ void NavierStokes::autotune(hipStream_t s) {
 
 void NavierStokes::set_physical(void* const* u3, hipStream_t s) {
   Plan* pf = plan_f3_ ? plan_f3_.get() : plan_f_.get();
-  pf->execute(u3, y_.data(), DFFT_FORWARD, s);
-  for (int r = 0; r < P_; ++r)
+  forward(*pf, u3, y_.data(), s);
+  for (int r = 0; r < P_; ++r)  // also clears the modes beyond the cutoff
     hip_check(ns_dealias_project(g_, sblk_[r], static_cast<double2*>(y_[r]), s), "ns_dealias_project");
 }
 

@@ -41,7 +41,7 @@ void NavierStokes::apply_rhs(void* const* y3, void* const* out3, hipStream_t s) 
   for (int r = 0; r < P_; ++r)
     hip_check(ns_dealias(g_, sblk_[r], static_cast<const double2*>(y3[r]), static_cast<double2*>(ym[r]), s),
               "dealias");
-  plan_b_->execute(ym.data(), pb_.data(), DFFT_BACKWARD, s);
+  backward(*plan_b_, ym.data(), pb_.data(), s);
   forward_products(pb_.data(), s);
   for (int r = 0; r < P_; ++r)
     hip_check(ns_rhs_only(g_, sblk_[r], static_cast<const double2*>(nl_[r]), static_cast<const double2*>(ym[r]),
@@ -61,13 +61,13 @@ void NavierStokes::apply_rhs_tangent(void* const* y3, void* const* d3, void* con
     hip_check(ns_dealias(g_, sblk_[r], static_cast<const double2*>(y3[r]), static_cast<double2*>(ym[r]), s),
               "dealias");
   }
-  plan_b_->execute(ym.data(), pb_.data(), DFFT_BACKWARD, s);
-  plan_b_->execute(dm.data(), du.data(), DFFT_BACKWARD, s);
+  backward(*plan_b_, ym.data(), pb_.data(), s);
+  backward(*plan_b_, dm.data(), du.data(), s);
   for (int r = 0; r < P_; ++r)
     hip_check(ns_products_tangent(static_cast<double*>(pb_[r]), static_cast<double*>(du[r]),
                                   static_cast<double*>(pf_[r]), phys_pts(r), s),
               "products_tangent");
-  plan_f_->execute(pf_.data(), nl_.data(), DFFT_FORWARD, s);
+  forward(*plan_f_, pf_.data(), nl_.data(), s);
   for (int r = 0; r < P_; ++r)
     hip_check(ns_rhs_only(g_, sblk_[r], static_cast<const double2*>(nl_[r]), static_cast<const double2*>(dm[r]),
                           static_cast<double2*>(out3[r]), s),
@@ -89,29 +89,29 @@ void NavierStokes::adjoint_core(const void* const* y3, const void* const* l3, co
   std::vector<void*>& ch = aux_s3b_;
   std::vector<void*>& c = aux_p3_;
   for (int r = 0; r < P_; ++r)
-    hip_check(ns_adjoint_prepare(g_, sblk_[r], static_cast<const double2*>(l3[r]), static_cast<double2*>(mu[r]),
+    hip_check(ns_adjoint_prepare(g_, sblk_[r], modes(r), static_cast<const double2*>(l3[r]), static_cast<double2*>(mu[r]),
                                  static_cast<double2*>(nl_[r]), s),
               "adjoint_prepare");
-  plan_f_->execute(nl_.data(), pf_.data(), DFFT_BACKWARD, s);  // S_mj (6 fields)
+  backward(*plan_f_, nl_.data(), pf_.data(), s);  // S_mj (6 fields)
   if (!u3) {
     for (int r = 0; r < P_; ++r)  // D y into ch, which is free until the forward transform of c
       hip_check(ns_dealias(g_, sblk_[r], static_cast<const double2*>(y3[r]), static_cast<double2*>(ch[r]), s),
                 "dealias");
-    plan_b_->execute(ch.data(), pb_.data(), DFFT_BACKWARD, s);  // u = IFFT(D y)
+    backward(*plan_b_, ch.data(), pb_.data(), s);  // u = IFFT(D y)
     u3 = pb_.data();
   }
   for (int r = 0; r < P_; ++r)
     hip_check(ns_adjoint_contract(static_cast<const double*>(u3[r]), static_cast<double*>(pf_[r]),
                                   static_cast<double*>(c[r]), phys_pts(r), s),
               "adjoint_contract");
-  plan_f3_->execute(c.data(), ch.data(), DFFT_FORWARD, s);
+  forward(*plan_f3_, c.data(), ch.data(), s);
   for (int r = 0; r < P_; ++r) {
     const auto* chr = static_cast<const double2*>(ch[r]);
     const auto* mur = static_cast<const double2*>(mu[r]);
     if (f.mode == 0)
       hip_check(ns_adjoint_finish(g_, sblk_[r], chr, mur, static_cast<double2*>(f.out3[r]), s), "adjoint_finish");
     else
-      hip_check(ns_adjoint_finish_rk(g_, sblk_[r], chr, mur, static_cast<double2*>(f.acc[r]),
+      hip_check(ns_adjoint_finish_rk(g_, sblk_[r], modes(r), chr, mur, static_cast<double2*>(f.acc[r]),
                                      static_cast<double2*>(f.lam[r]), f.fb ? static_cast<double2*>(f.fb[r]) : nullptr,
                                      f.a, f.c, f.mode, s),
                 "adjoint_finish_rk");
@@ -187,7 +187,7 @@ double NavierStokes::gradient(int nsteps, int ck, void* const* u0, void* const* 
       for (int st = last - 1; st >= first; --st) {
         const int base = 4 * (st - first);
         for (int r = 0; r < P_; ++r)
-          hip_check(ns_rk_adjoint_init(3 * spec_pts(r), static_cast<const double2*>(lam[r]),
+          hip_check(ns_rk_adjoint_init(sblk_[r], modes(r), static_cast<const double2*>(lam[r]),
                                        static_cast<double2*>(fb[r]), static_cast<double2*>(acc[r]), dt / 6.0, s),
                     "rk_adjoint_init");
         const double a[3] = {1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0}, c[3] = {1.0, 0.5, 0.5};
@@ -205,7 +205,7 @@ double NavierStokes::gradient(int nsteps, int ck, void* const* u0, void* const* 
     for (int r = 0; r < P_; ++r)
       hip_check(ns_dealias_project(g_, sblk_[r], static_cast<double2*>(lam[r]), s), "dealias_project");
     Plan* pb3 = plan_b3_ ? plan_b3_.get() : plan_b_.get();
-    pb3->execute(lam.data(), grad, DFFT_BACKWARD, s);
+    backward(*pb3, lam.data(), grad, s);
     const double n3 = std::pow(static_cast<double>(n_), 3);
     for (int r = 0; r < P_; ++r) hip_check(ns_scale(3 * phys_pts(r), n3, static_cast<double*>(grad[r]), s), "scale");
     hip_check(hipStreamSynchronize(s), "sync");

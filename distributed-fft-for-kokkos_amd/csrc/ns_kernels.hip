@@ -1,6 +1,8 @@
 // Pointwise kernels of the pseudo-spectral Navier-Stokes solver.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "ns_kernels.hpp"
 
@@ -26,10 +28,8 @@ __device__ __forceinline__ void block_coords(const NsBlock& b, int64_t m, int& i
   ix = static_cast<int>(q);
 }
 
-// wavenumbers of spectral point m (LayoutRight (ex, ey, ez) block)
-__device__ __forceinline__ Mode mode_of(const NsGrid& g, const NsBlock& b, int64_t m) {
-  int ix, iy, iz;
-  block_coords(b, m, ix, iy, iz);
+// wavenumbers of block-local spectral point (ix, iy, iz)
+__device__ __forceinline__ Mode mode_at(const NsGrid& g, const NsBlock& b, int ix, int iy, int iz) {
   const int sx = signed_index(ix + b.start[0], g.n);
   const int sy = signed_index(iy + b.start[1], g.n);
   const int sz = iz + b.start[2];
@@ -43,6 +43,28 @@ __device__ __forceinline__ Mode mode_of(const NsGrid& g, const NsBlock& b, int64
   md.mask = cut ? 0.0 : 1.0;
   md.kz0 = sz == 0;
   return md;
+}
+
+// the same for point m of the LayoutRight (ex, ey, ez) block
+__device__ __forceinline__ Mode mode_of(const NsGrid& g, const NsBlock& b, int64_t m) {
+  int ix, iy, iz;
+  block_coords(b, m, ix, iy, iz);
+  return mode_at(g, b, ix, iy, iz);
+}
+
+// visited mode i: its block-local coordinates; returns its index in the block
+__device__ __forceinline__ int64_t visited_mode(const NsBlock& b, const NsModes& k, int64_t i, int& ix, int& iy,
+                                                int& iz) {
+  const uint32_t ii = static_cast<uint32_t>(i);
+  const uint32_t r = k.div2.div(ii);
+  iz = static_cast<int>(ii - r * static_cast<uint32_t>(k.cnt[2]));
+  const uint32_t q = k.div1.div(r);
+  iy = static_cast<int>(r - q * static_cast<uint32_t>(k.cnt[1]));
+  ix = static_cast<int>(q);
+  ix += ix >= k.first[0] ? k.gap[0] : 0;
+  iy += iy >= k.first[1] ? k.gap[1] : 0;
+  iz += iz >= k.first[2] ? k.gap[2] : 0;
+  return (static_cast<int64_t>(ix) * b.ext[1] + iy) * b.ext[2] + iz;
 }
 
 __device__ __forceinline__ double2 cscale(double2 a, double s) { return double2{a.x * s, a.y * s}; }
@@ -64,6 +86,26 @@ inline unsigned blocks_for(int64_t n) {
 }
 
 }  // namespace
+
+NsModes ns_modes(const NsBlock& b, int n, int cut) {
+  NsModes k{};
+  for (int a = 0; a < 3; ++a) {
+    const int s = b.start[a], e = s + b.ext[a];
+    if (cut < 0) {
+      k.cnt[a] = k.first[a] = b.ext[a];
+    } else {
+      // kept global indices: 0 .. cut, and n - cut .. n - 1 along x and y
+      const int lo = std::max(0, std::min(e, cut + 1) - s);
+      const int from = std::max(s, n - cut), hi = a < 2 ? std::max(0, e - from) : 0;
+      k.cnt[a] = lo + hi;
+      k.first[a] = lo;
+      k.gap[a] = hi > 0 ? from - s - lo : 0;
+    }
+  }
+  k.div1 = FastDiv(static_cast<uint32_t>(k.cnt[1]));
+  k.div2 = FastDiv(static_cast<uint32_t>(k.cnt[2]));
+  return k;
+}
 
 __global__ void __launch_bounds__(256) products_kernel(const double* __restrict__ u, double* __restrict__ p,
                                                        int64_t npts) {
@@ -145,11 +187,14 @@ __device__ __forceinline__ void stream_store(double2* p, double2 x) {
   __builtin_nontemporal_store(v, reinterpret_cast<StreamD2*>(p));
 }
 
-__global__ void __launch_bounds__(256) rhs_rk_kernel(const NsGrid g, const NsBlock b, const NsStage st) {
+__global__ void __launch_bounds__(256) rhs_rk_kernel(const NsGrid g, const NsBlock b, const NsModes k, int64_t total,
+                                                     const NsStage st) {
   const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; m < m_tot; m += stride) {
-    const Mode md = mode_of(g, b, m);
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
+    int ix, iy, iz;
+    const int64_t m = visited_mode(b, k, i, ix, iy, iz);
+    const Mode md = mode_at(g, b, ix, iy, iz);
     double2 nl[3];
     if (st.form == 0) {
       // N_i = i sum_j k_j P_ij with P = [uu uv uw; uv vv vw; uw vw ww]
@@ -198,10 +243,10 @@ __global__ void __launch_bounds__(256) rhs_rk_kernel(const NsGrid g, const NsBlo
   }
 }
 
-hipError_t ns_rhs_rk(const NsGrid& g, const NsBlock& b, const NsStage& st, hipStream_t s) {
-  const int64_t m = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
+hipError_t ns_rhs_rk(const NsGrid& g, const NsBlock& b, const NsModes& k, const NsStage& st, hipStream_t s) {
+  const int64_t m = k.total();
   if (m <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rhs_rk_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, st);
+  hipLaunchKernelGGL(rhs_rk_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, k, m, st);
   return hipGetLastError();
 }
 
@@ -211,7 +256,7 @@ __global__ void __launch_bounds__(256) dealias_project_kernel(const NsGrid g, co
   for (int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; m < m_tot; m += stride) {
     const Mode md = mode_of(g, b, m);
     double2 v[3];
-    for (int c = 0; c < 3; ++c) v[c] = cscale(y[c * m_tot + m], md.mask);
+    for (int c = 0; c < 3; ++c) v[c] = md.mask != 0.0 ? y[c * m_tot + m] : double2{0.0, 0.0};
     project(md, v);
     for (int c = 0; c < 3; ++c) y[c * m_tot + m] = v[c];
   }
@@ -330,6 +375,10 @@ __global__ void __launch_bounds__(256) rhs_only_kernel(const NsGrid g, const NsB
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; m < m_tot; m += stride) {
     const Mode md = mode_of(g, b, m);
+    if (md.mask == 0.0) {
+      for (int c = 0; c < 3; ++c) out[c * m_tot + m] = double2{0.0, 0.0};
+      continue;
+    }
     const double2 p0 = nl[m], p1 = nl[m_tot + m], p2 = nl[2 * m_tot + m];
     const double2 p3 = nl[3 * m_tot + m], p4 = nl[4 * m_tot + m], p5 = nl[5 * m_tot + m];
     double2 n3[3];
@@ -355,12 +404,15 @@ hipError_t ns_rhs_only(const NsGrid& g, const NsBlock& b, const double2* nl6, co
   return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(256) adjoint_prepare_kernel(const NsGrid g, const NsBlock b, const double2* lam,
-                                                              double2* mu, double2* sig) {
+__global__ void __launch_bounds__(256) adjoint_prepare_kernel(const NsGrid g, const NsBlock b, const NsModes k,
+                                                              int64_t total, const double2* lam, double2* mu,
+                                                              double2* sig) {
   const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; m < m_tot; m += stride) {
-    const Mode md = mode_of(g, b, m);
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
+    int ix, iy, iz;
+    const int64_t m = visited_mode(b, k, i, ix, iy, iz);
+    const Mode md = mode_at(g, b, ix, iy, iz);
     double2 v[3];
     for (int c = 0; c < 3; ++c) v[c] = lam[c * m_tot + m];
     project(md, v);
@@ -368,12 +420,12 @@ __global__ void __launch_bounds__(256) adjoint_prepare_kernel(const NsGrid g, co
       v[c] = cscale(v[c], md.mask);
       mu[c * m_tot + m] = v[c];
     }
-    const double k[3] = {md.kx, md.ky, md.kz};
+    const double kk[3] = {md.kx, md.ky, md.kz};
     int f = 0;
-    for (int i = 0; i < 3; ++i) {
-      for (int j = i; j < 3; ++j) {
-        // -i (k_j mu_i + k_i mu_j)
-        const double2 s2 = cadd2(cscale(v[i], k[j]), cscale(v[j], k[i]));
+    for (int c = 0; c < 3; ++c) {
+      for (int j = c; j < 3; ++j) {
+        // -i (k_j mu_c + k_c mu_j)
+        const double2 s2 = cadd2(cscale(v[c], kk[j]), cscale(v[j], kk[c]));
         sig[f * m_tot + m] = double2{s2.y, -s2.x};
         ++f;
       }
@@ -381,11 +433,11 @@ __global__ void __launch_bounds__(256) adjoint_prepare_kernel(const NsGrid g, co
   }
 }
 
-hipError_t ns_adjoint_prepare(const NsGrid& g, const NsBlock& b, const double2* lam3, double2* mu3,
+hipError_t ns_adjoint_prepare(const NsGrid& g, const NsBlock& b, const NsModes& k, const double2* lam3, double2* mu3,
                               double2* sig6, hipStream_t s) {
-  const int64_t m = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
+  const int64_t m = k.total();
   if (m <= 0) return hipSuccess;
-  hipLaunchKernelGGL(adjoint_prepare_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, lam3, mu3, sig6);
+  hipLaunchKernelGGL(adjoint_prepare_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, k, m, lam3, mu3, sig6);
   return hipGetLastError();
 }
 
@@ -418,6 +470,10 @@ __global__ void __launch_bounds__(256) adjoint_finish_kernel(const NsGrid g, con
     const Mode md = mode_of(g, b, m);
     const double visc = -g.nu * md.ksq;
     for (int c = 0; c < 3; ++c) {
+      if (md.mask == 0.0) {
+        out[c * m_tot + m] = double2{0.0, 0.0};
+        continue;
+      }
       const double2 ch = chat[c * m_tot + m], u = mu[c * m_tot + m];
       out[c * m_tot + m] = double2{-md.mask * ch.x + visc * u.x, -md.mask * ch.y + visc * u.y};
     }
@@ -562,16 +618,19 @@ namespace dfft {
 //   mode 1: acc += t;  fb = dt (a lam + c t)   (the next stage's seed)
 //   mode 2: lam = D (acc + t)                  (the adjoint of the step input)
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) adjoint_finish_rk_kernel(const NsGrid g, const NsBlock b, const double2* chat,
+__global__ void __launch_bounds__(256) adjoint_finish_rk_kernel(const NsGrid g, const NsBlock b, const NsModes k,
+                                                                int64_t total, const double2* chat,
                                                                 const double2* mu, double2* acc, double2* lam,
                                                                 double2* fb, double a, double c, int mode) {
   const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; m < m_tot; m += stride) {
-    const Mode md = mode_of(g, b, m);
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
+    int ix, iy, iz;
+    const int64_t m = visited_mode(b, k, i, ix, iy, iz);
+    const Mode md = mode_at(g, b, ix, iy, iz);
     const double visc = -g.nu * md.ksq;
-    for (int k = 0; k < 3; ++k) {
-      const int64_t e = k * m_tot + m;
+    for (int f = 0; f < 3; ++f) {
+      const int64_t e = f * m_tot + m;
       const double2 ch = chat[e], u = mu[e];
       const double2 t{-md.mask * ch.x + visc * u.x, -md.mask * ch.y + visc * u.y};
       const double2 s = acc[e];
@@ -587,30 +646,38 @@ __global__ void __launch_bounds__(256) adjoint_finish_rk_kernel(const NsGrid g, 
   }
 }
 
-hipError_t ns_adjoint_finish_rk(const NsGrid& g, const NsBlock& b, const double2* chat3, const double2* mu3,
-                                double2* acc3, double2* lam3, double2* fb3, double a, double c, int mode,
-                                hipStream_t s) {
-  const int64_t m = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
+hipError_t ns_adjoint_finish_rk(const NsGrid& g, const NsBlock& b, const NsModes& k, const double2* chat3,
+                                const double2* mu3, double2* acc3, double2* lam3, double2* fb3, double a, double c,
+                                int mode, hipStream_t s) {
+  const int64_t m = k.total();
   if (m <= 0) return hipSuccess;
-  hipLaunchKernelGGL(adjoint_finish_rk_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, chat3, mu3, acc3, lam3,
-                     fb3, a, c, mode);
+  hipLaunchKernelGGL(adjoint_finish_rk_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, k, m, chat3, mu3, acc3,
+                     lam3, fb3, a, c, mode);
   return hipGetLastError();
 }
 
 // fb = c lam, acc = lam (start of a reverse RK4 step)
-__global__ void __launch_bounds__(256) rk_adjoint_init_kernel(int64_t n, const double2* lam, double2* fb,
-                                                              double2* acc, double c) {
+__global__ void __launch_bounds__(256) rk_adjoint_init_kernel(const NsBlock b, const NsModes k, int64_t total,
+                                                              const double2* lam, double2* fb, double2* acc,
+                                                              double c) {
+  const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const double2 l = lam[i];
-    fb[i] = double2{c * l.x, c * l.y};
-    acc[i] = l;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
+    int ix, iy, iz;
+    const int64_t m = visited_mode(b, k, i, ix, iy, iz);
+    for (int f = 0; f < 3; ++f) {
+      const double2 l = lam[f * m_tot + m];
+      fb[f * m_tot + m] = double2{c * l.x, c * l.y};
+      acc[f * m_tot + m] = l;
+    }
   }
 }
 
-hipError_t ns_rk_adjoint_init(int64_t n, const double2* lam, double2* fb, double2* acc, double c, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rk_adjoint_init_kernel, dim3(blocks_for(n)), dim3(256), 0, s, n, lam, fb, acc, c);
+hipError_t ns_rk_adjoint_init(const NsBlock& b, const NsModes& k, const double2* lam3, double2* fb3, double2* acc3,
+                              double c, hipStream_t s) {
+  const int64_t m = k.total();
+  if (m <= 0) return hipSuccess;
+  hipLaunchKernelGGL(rk_adjoint_init_kernel, dim3(blocks_for(m)), dim3(256), 0, s, b, k, m, lam3, fb3, acc3, c);
   return hipGetLastError();
 }
 

@@ -24,6 +24,20 @@ struct NsBlock {
   }
 };
 
+// The modes of a spectral block that a pointwise kernel visits: index i of
+// axis a stands for the block-local index i + (i >= first[a] ? gap[a] : 0).
+// Either every mode of the block or those within the dealias cutoff (two runs
+// along x and y, one along z).
+struct NsModes {
+  int32_t cnt[3];
+  int32_t first[3];
+  int32_t gap[3];
+  FastDiv div1, div2;
+  int64_t total() const { return int64_t(cnt[0]) * cnt[1] * cnt[2]; }
+};
+// n: grid points, cut: kept |k| along every axis (negative: all modes)
+NsModes ns_modes(const NsBlock& b, int n, int cut);
+
 struct NsGrid {
   int32_t n;       // grid points per direction
   int32_t cutoff;  // 2/3-rule cutoff on |integer wavenumber index|
@@ -55,9 +69,10 @@ struct NsStage {
   double2* k2;
   double2* k3;
 };
-hipError_t ns_rhs_rk(const NsGrid& g, const NsBlock& b, const NsStage& st, hipStream_t s);
+hipError_t ns_rhs_rk(const NsGrid& g, const NsBlock& b, const NsModes& k, const NsStage& st, hipStream_t s);
 
-// Projection u - k (k.u)/k^2 with the dealias mask (main.cpp:235-254, 214-225).
+// Projection u - k (k.u)/k^2 with the dealias mask (main.cpp:235-254, 214-225);
+// masked modes become zero and are not read.
 hipError_t ns_dealias_project(const NsGrid& g, const NsBlock& b, double2* y3, hipStream_t s);
 
 // Taylor-Green field on a physical block (main.cpp:349-353): grid spacing h.
@@ -72,16 +87,17 @@ hipError_t ns_sum(const double* partials, int n, double* out, hipStream_t s);
 // ---- tangent / adjoint pieces (divergence form) ---------------------------
 // p_ij = du_i u_j + u_i du_j (6 fields) from u (3) and du (3)
 hipError_t ns_products_tangent(const double* u3, const double* du3, double* p6, int64_t npts, hipStream_t s);
-// R(y) only (no RK update): out = P(-D N - nu k^2 D y), N from 6 product spectra
+// R(y) only (no RK update): out = P(-D N - nu k^2 D y), N from 6 product
+// spectra; zero at masked modes, whose inputs are not read
 hipError_t ns_rhs_only(const NsGrid& g, const NsBlock& b, const double2* nl6, const double2* y3, double2* out3,
                        hipStream_t s);
 // mu = D P lambda (written to mu3) and the 6 symmetric fields
 // sigma_mj = -i (k_j mu_m + k_m mu_j), m <= j (written to sig6)
-hipError_t ns_adjoint_prepare(const NsGrid& g, const NsBlock& b, const double2* lam3, double2* mu3,
+hipError_t ns_adjoint_prepare(const NsGrid& g, const NsBlock& b, const NsModes& k, const double2* lam3, double2* mu3,
                               double2* sig6, hipStream_t s);
 // c_m = sum_j u_j S_mj (physical)
 hipError_t ns_adjoint_contract(const double* u3, const double* S6, double* c3, int64_t npts, hipStream_t s);
-// out = -D chat - nu k^2 mu
+// out = -D chat - nu k^2 mu; zero at masked modes, whose inputs are not read
 hipError_t ns_adjoint_finish(const NsGrid& g, const NsBlock& b, const double2* chat3, const double2* mu3,
                              double2* out3, hipStream_t s);
 // x = a*x + b*y over n complex values; dealias / dealias+project helpers on 3 fields
@@ -93,11 +109,12 @@ hipError_t ns_scale(int64_t n, double a, double* x, hipStream_t s);
 
 // reverse RK4 step pieces: t = -D chat - nu k^2 mu; mode 1: acc += t,
 // fb = dt (a lam + c t); mode 2: lam = D (acc + t)
-hipError_t ns_adjoint_finish_rk(const NsGrid& g, const NsBlock& b, const double2* chat3, const double2* mu3,
-                                double2* acc3, double2* lam3, double2* fb3, double a, double c, int mode,
-                                hipStream_t s);
-// fb = c lam, acc = lam over n complex values
-hipError_t ns_rk_adjoint_init(int64_t n, const double2* lam, double2* fb, double2* acc, double c, hipStream_t s);
+hipError_t ns_adjoint_finish_rk(const NsGrid& g, const NsBlock& b, const NsModes& k, const double2* chat3,
+                                const double2* mu3, double2* acc3, double2* lam3, double2* fb3, double a, double c,
+                                int mode, hipStream_t s);
+// fb = c lam, acc = lam over 3 fields
+hipError_t ns_rk_adjoint_init(const NsBlock& b, const NsModes& k, const double2* lam3, double2* fb3, double2* acc3,
+                              double c, hipStream_t s);
 
 // diagnostics (main.cpp:781-910)
 constexpr int kMaxSpectrumBins = 256;

@@ -593,8 +593,90 @@ bool Plan::products_supported() const {
   return products_pass_supported(fwd_[0].n);
 }
 
-void Plan::execute_forward_products(void* const* u3, void* const* out, hipStream_t stream) {
-  if (!products_supported()) throw Error(DFFT_ERROR_UNSUPPORTED, "this plan cannot form the products in its R2C pass");
+bool Plan::band_supported(int cut) const {
+  if (!fp64_ || !real_ || d_.exec_mode != DFFT_EXEC_FUSED || view_layout_ != Layout::Right) return false;
+  if (rank_ != 4 || axes_ != Vec{1, 2, 3} || in_topo_[0] != 1 || out_topo_[0] != 1) return false;
+  if (cut < 1 || fwd_.size() != 3 || bwd_.size() != 3) return false;
+  for (const auto* passes : {&fwd_, &bwd_})
+    for (const PassSpec& s : *passes)
+      if (!band_pass_supported(s.n) || 2 * cut >= s.n || (s.kind != kC2C && (s.paired == 0 || s.axis != 3))) return false;
+  return fwd_[0].kind == kR2C && bwd_[2].kind == kC2R && in_topo_[fwd_[0].axis] == 1 &&
+         out_topo_[fwd_[2].axis] == 1 && out_topo_[bwd_[0].axis] == 1 && in_topo_[bwd_[2].axis] == 1;
+}
+
+// The plan scratch between the passes of kept modes: rows hold the kept
+// entries 0..cut of the half-spectrum axis, padded to 128 bytes.
+DDesc Plan::band_scratch(int cut) const {
+  DDesc d = scratch_desc(gout_, scratch_, 16);
+  d.pitch = (cut + 8) / 8 * 8;
+  return d;
+}
+
+void Plan::band_pass(LinePass& p, std::size_t i, bool forward, int cut) const {
+  const auto& passes = forward ? fwd_ : bwd_;
+  p.band = cut;
+  if (passes[i].values_per_thread != 0 && passes[i].values_per_thread != 8) p.lines_per_block = 0;
+  p.pad_axis = 0;
+  p.pad_real = 0;
+  int64_t nl = 1;
+  for (int j = 0; j < p.nbatch; ++j) {
+    const int a = p.batch_axis[j];
+    int32_t ext = static_cast<int32_t>(std::max(gin_[a], gout_[a]));
+    // spectral on this side of the pass: transformed before it (forward),
+    // not yet transformed back (backward)
+    bool spectral = false;
+    for (std::size_t k = 0; k < passes.size(); ++k)
+      if (passes[k].axis == a && (forward ? k < i : k > i)) spectral = true;
+    p.band_shift[j] = 0;
+    if (spectral && a == 3) {
+      ext = cut + 1;
+      // blocks of lines start on aligned scratch rows where that adds at most
+      // a sixteenth of padding lines (skipped in the kernel)
+      const int32_t row = (cut + 8) / 8 * 8;
+      if (j == p.nbatch - 1 && (row - ext) * 16 <= ext && row != ext) {
+        p.pad_axis = 3;
+        p.pad_real = ext;
+        ext = row;
+      }
+    } else if (spectral) {
+      p.band_shift[j] = ext - (2 * cut + 1);
+      ext = 2 * cut + 1;
+    }
+    p.batch_ext[j] = ext;
+    p.batch_div[j] = FastDiv(static_cast<uint32_t>(ext));
+    nl *= ext;
+  }
+  if (nl >= (int64_t(1) << 31)) throw Error(DFFT_ERROR_UNSUPPORTED, "too many lines in one pass");
+  p.nlines = static_cast<int32_t>(nl);
+}
+
+void Plan::execute_band(void* const* in, void* const* out, int direction, int cut, hipStream_t stream) {
+  if (!band_supported(cut)) throw Error(DFFT_ERROR_UNSUPPORTED, "this plan cannot transform kept modes only");
+  if (in == nullptr || out == nullptr) throw Error(DFFT_ERROR_INVALID_ARGUMENT, "null pointer table");
+  int cur = -1;
+  check_hip(hipGetDevice(&cur), "hipGetDevice");
+  if (cur != device_) check_hip(hipSetDevice(device_), "hipSetDevice");
+  if (total_size(gin_) == 0) return;
+  const bool forward = direction == DFFT_FORWARD;
+  TraceRange range("dfft::%s::execute %s (kept modes)", name_.c_str(), forward ? "forward" : "backward");
+  const auto& passes = forward ? fwd_ : bwd_;
+  DDesc src = forward ? user_desc(gin_, in_topo_, in_tl_, in) : user_desc(gout_, out_topo_, out_tl_, in);
+  DDesc dst = forward ? user_desc(gout_, out_topo_, out_tl_, out) : user_desc(gin_, in_topo_, in_tl_, out);
+  const DDesc scr = band_scratch(cut);
+  for (std::size_t i = 0; i < passes.size(); ++i) {
+    const bool first = i == 0, last = i + 1 == passes.size();
+    LinePass p = make_pass(passes[i], first ? src : scr, last ? dst : scr, !forward, last ? exec_scale(forward) : 1.0);
+    band_pass(p, i, forward, cut);
+    TraceRange pr("dfft::%s pass %zu axis %d (kept modes)", forward ? "forward" : "backward", i, passes[i].axis);
+    mark(stream);
+    check_hip(launch_band_pass(p, stream), "line pass");
+    mark(stream);
+  }
+}
+
+void Plan::execute_forward_products(void* const* u3, void* const* out, int cut, hipStream_t stream) {
+  if (!products_supported() || (cut > 0 && !band_supported(cut)))
+    throw Error(DFFT_ERROR_UNSUPPORTED, "this plan cannot form the products in its R2C pass");
   if (u3 == nullptr || out == nullptr) throw Error(DFFT_ERROR_INVALID_ARGUMENT, "null pointer table");
   int cur = -1;
   check_hip(hipGetDevice(&cur), "hipGetDevice");
@@ -614,12 +696,12 @@ void Plan::execute_forward_products(void* const* u3, void* const* out, hipStream
   src3.div_big[0] = FastDiv(4u);
   src3.div_small[0] = FastDiv(3u);
   DDesc dst = user_desc(gout_, out_topo_, out_tl_, out);
-  DDesc scr = scratch_desc(gout_, scratch_, 16);
+  DDesc scr = cut > 0 ? band_scratch(cut) : scratch_desc(gout_, scratch_, 16);
   for (std::size_t i = 0; i < passes.size(); ++i) {
     const bool first = i == 0, last = i + 1 == passes.size();
-    DDesc b = last ? dst : scr;
+    LinePass p = make_pass(passes[i], first ? src6 : scr, last ? dst : scr, false, last ? scale : 1.0);
+    if (cut > 0) band_pass(p, i, true, cut);
     if (first) {
-      LinePass p = make_pass(passes[0], src6, b, false, last ? scale : 1.0);
       p.in = src3;
       p.products = 1;
       p.prod_axis = 0;
@@ -641,16 +723,13 @@ void Plan::execute_forward_products(void* const* u3, void* const* out, hipStream
         p.batch_ext[p.nbatch - 1] = ex;
         p.batch_div[p.nbatch - 1] = dv;
       }
-      TraceRange pr("dfft::forward pass 0 axis %d (products of the velocity lines)", passes[0].axis);
-      mark(stream);
-      check_hip(launch_products_pass(p, stream), "products pass");
-      mark(stream);
-      continue;
     }
-    LinePass p = make_pass(passes[i], scr, b, false, last ? scale : 1.0);
-    TraceRange pr("dfft::forward pass %zu axis %d%s", i, passes[i].axis, last ? " (scatter to the output ranks)" : "");
+    TraceRange pr("dfft::forward pass %zu axis %d%s", i, passes[i].axis,
+                  first ? " (products of the velocity lines)" : last ? " (scatter to the output ranks)" : "");
     mark(stream);
-    check_hip(launch_pass(p, stream), "line pass");
+    if (cut > 0) check_hip(launch_band_pass(p, stream), "line pass");
+    else if (first) check_hip(launch_products_pass(p, stream), "products pass");
+    else check_hip(launch_pass(p, stream), "line pass");
     mark(stream);
   }
 }

@@ -53,16 +53,24 @@ class Plan {
   // adjoint of execute(direction) under the real inner product Re sum conj(a) b
   // of each side: in has the shape of that direction's output, out of its input
   void execute_adjoint(void* const* in, void* const* out, int direction, hipStream_t stream);
-  // Forward execute of a 6-field R2C plan over 4-D views (field axis first,
-  // not distributed, transform axes 1..3) whose input fields are the products
-  // u_i u_j of the 3 velocity fields in `u3` (per rank: 3 fields shaped like
-  // the plan's input blocks), (i, j) = (0,0) (0,1) (0,2) (1,1) (1,2) (2,2):
-  // the products are formed as the first (R2C) pass loads its lines, so the
-  // 6 product fields are never stored.  products_supported() says whether
-  // this plan can (FP64, fused executor, a paired R2C first pass of a
-  // power-of-two length 8..1024).
+  // Dealiased fields (4-D views, field axis first and not distributed, R2C
+  // over axes 1..3): only modes |k| <= cut along each axis are kept.
+  // band_supported: FP64, fused executor, LayoutRight, power-of-two lengths
+  // 8..1024, R2C lines in pairs.  execute_band(FORWARD) writes the kept modes
+  // of the spectra and leaves the others as they are; execute_band(BACKWARD)
+  // transforms spectra whose other modes count as zeros, whatever the arrays
+  // hold there.  Same results as execute on the masked spectra.
+  bool band_supported(int cut) const;
+  void execute_band(void* const* in, void* const* out, int direction, int cut, hipStream_t stream);
+  // Forward execute of a 6-field R2C plan over such views whose input fields
+  // are the products u_i u_j of the 3 velocity fields in `u3` (per rank: 3
+  // fields shaped like the plan's input blocks), (i, j) = (0,0) (0,1) (0,2)
+  // (1,1) (1,2) (2,2): the products are formed as the first (R2C) pass loads
+  // its lines, so the 6 product fields are never stored.  cut > 0: as
+  // execute_band.  products_supported() says whether this plan can (FP64,
+  // fused executor, a paired R2C first pass of a power-of-two length 8..1024).
   bool products_supported() const;
-  void execute_forward_products(void* const* u3, void* const* out, hipStream_t stream);
+  void execute_forward_products(void* const* u3, void* const* out, int cut, hipStream_t stream);
   // execute with a HIP event pair around every launch; durations in ms
   std::vector<float> execute_timed(void* const* in, void* const* out, int direction, hipStream_t stream);
   int num_passes(int direction) const;
@@ -99,6 +107,9 @@ class Plan {
   std::size_t scratch_elems(const Vec& ext, std::size_t elem_bytes) const;  // incl. padding
   LinePass make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, bool inverse, double scale,
                      int slow_axis = -1) const;
+  // restricts pass i of a direction to the kept modes
+  void band_pass(LinePass& p, std::size_t i, bool forward, int cut) const;
+  DDesc band_scratch(int cut) const;
   float time_direction(void* const* in, void* const* out, bool forward, hipStream_t s, int reps);
   void plan_fused();
   void run_fused(void* const* in, void* const* out, bool forward, hipStream_t s);

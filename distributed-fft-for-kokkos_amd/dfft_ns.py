@@ -91,7 +91,9 @@ class NavierStokes:
 
     def set_option(self, key, value):
         """"fuse_products" (1 default / 0): form the 6 products inside the
-        forward transform's first pass instead of storing them."""
+        forward transform's first pass instead of storing them.
+        "kept_modes" (1 default / 0): handle only the modes within the dealias
+        cutoff in the transforms and pointwise kernels (same results)."""
         _check(self._lib.dfft_ns_set_option(self._h, key.encode(), int(value)))
 
     def get_option(self, key):

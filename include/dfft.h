@@ -271,7 +271,10 @@ int dfft_ns_autotune(dfft_ns* ns, void* stream);
 /* "fuse_products" (1 default, 0): form the divergence form's 6 products in
  * the forward transform's first pass from the velocity lines (no product
  * fields stored) where the plan allows it; "products_fused" (read only): 1
- * when the step runs that way.  No counterpart in the reference. */
+ * when the step runs that way.  "kept_modes" (1 default, 0): transforms and
+ * pointwise kernels of the divergence form handle only the modes within the
+ * 2/3-rule cutoff where the plans allow it (same results; reads 1 then).
+ * No counterpart in the reference. */
 int dfft_ns_set_option(dfft_ns* ns, const char* key, long value);
 int dfft_ns_get_option(const dfft_ns* ns, const char* key, long* value);
 /* kinetic energy, FP64 reduction (diag_energy, main.cpp:855-910) */
