@@ -30,6 +30,7 @@ struct LinePass {
   int32_t lines_per_block;              // 0: launcher heuristic
   int32_t values_per_thread;            // 0: default (8); compile-time kernels exist for 4, 8, 16,
                                         // the runtime-radix kernel takes it as an upper bound
+  int32_t fit_block;                    // 1: lines_per_block is a default the launcher may halve to fit
   const void* tw;                       // exp(-2 pi i e / n), e in [0, n), Real precision
   double scale;
   // 1: an R2C (forward) or C2R (inverse) pass on the fast kernel transforms

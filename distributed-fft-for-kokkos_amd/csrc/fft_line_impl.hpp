@@ -1577,7 +1577,9 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
   constexpr int T = Cfg::T;
   if constexpr (dual_kernel_exists<Real, N>()) {
     // default: 32 lines (256-byte row segments) or as many as 1024 lanes hold
-    const int Bd = p.lines_per_block > 0 ? p.lines_per_block : (T <= 64 ? 32 : 2 * (1024 / T));
+    int Bd = p.lines_per_block > 0 ? p.lines_per_block : (T <= 64 ? 32 : 2 * (1024 / T));
+    if (p.fit_block)
+      while (Bd > 2 && Bd / 2 * T > 1024) Bd /= 2;
     const int mode = dual_lines_mode(p, Bd);
     if (mode >= 0) {
       p.dual_split = mode;
@@ -1602,6 +1604,10 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
     }
     while (B > 1 && static_cast<size_t>(B) * line_bytes > 160 * 1024) B /= 2;
   }
+  if (p.fit_block)  // at least two blocks resident on a CU, two blocks per CU in the grid
+    while (B > 1 && (B * T > 1024 || static_cast<size_t>(B) * line_bytes > 80 * 1024 ||
+                     (B > 4 && B * T > 64 && p.nlines / B < 512)))
+      B /= 2;
   const size_t smem = static_cast<size_t>(B) * line_bytes;
   if (B * T > 1024 || smem > 160 * 1024) return hipErrorInvalidConfiguration;
   p.lines_per_block = B;
@@ -1714,6 +1720,8 @@ hipError_t launch_band(LinePass p, hipStream_t s) {
     B = p.lines_fast ? 8 : (T >= 256 ? 1 : 256 / T);
     while (B * T > 1024) B /= 2;
   }
+  if (p.fit_block && !p.products)  // as launch_fast
+    while (B > 1 && (B * T > 1024 || (B > 4 && B * T > 64 && p.nlines / B < 512))) B /= 2;
   const size_t smem = static_cast<size_t>(B) * line_bytes;
   if (B * T > 1024 || smem > 160 * 1024) return hipErrorInvalidConfiguration;
   p.lines_per_block = B;

@@ -427,7 +427,6 @@ LinePass Plan::make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, b
   p.scale = scale;
   p.herm_weight = s.kind == kC2C ? 0.0 : adj_herm_;
   p.paired = s.kind == kC2C ? 0 : s.paired;
-  p.xcd_remap = s.xcd;
   p.swizzle = s.swz;
   p.split_lds = s.split;
   p.dual_lines = s.dual;
@@ -490,16 +489,90 @@ LinePass Plan::make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, b
   }
   p.line_begin = 0;
   p.lines_fast = s.lines_fast >= 0 ? s.lines_fast : (s.axis != innermost ? 1 : 0);
+  default_shape(p, s);
+  return p;
+}
+
+// Launch shapes by rule.  Each line was measured pass by pass on slab and
+// pencil plans of 64^3 to 1024^3 and 32 x 2048^2 in both precisions, C2C and
+// R2C, over 4, 8 and 16 values per lane, 2 to 32 lines per block, both block
+// numberings and both kinds of access (6,480 timings): over those 90 passes
+// the rule is 3 % behind the best shape of each pass, 8 values per lane and
+// 128-byte blocks of lines throughout were 17 % behind (us per pass, that ->
+// rule: FP64 512^3 x 917 -> 817, 1024^3 R2C y 4760 -> 3170 and x 6120 -> 3620,
+// 512^3 pencil R2C x 1470 -> 652; FP32 512^3 y 434 -> 360, 1024^3 R2C x 3510
+// -> 1960).
+//  * Lanes across lines: 128-byte row segments need 8 FP64 lines per block;
+//    wider ones pay off as long as two blocks stay resident on a CU, which 16
+//    values per lane allow from 512 points on (fewer lanes per line).
+//  * Blocks in XCD order: consecutive blocks touch the same rows, and rows
+//    that do not start on 128 bytes (odd half spectra) share lines that only
+//    one L2 should write: 787 -> 652 us for the 512^3 R2C x pass.  Aligned
+//    lines that step 1 MiB or more per element run up to 4 % faster in plain
+//    order, and arrays below 64 MiB up to 8 %.
+//  * Nontemporal accesses from 512 MiB on (round trips over three rotating
+//    sets of arrays, all cached -> all nontemporal: 512^3 FP32 2437 -> 2289
+//    us).  Smaller arrays are read back from the 256 MiB last-level cache by
+//    the next pass, so only the last pass, whose output nothing reads soon,
+//    streams (256^3 R2C FP64: all cached 355, all nontemporal 441, last
+//    backward pass only 337 us; 256^3 C2C FP64: 610, 612, last passes only 540
+//    us).  Never where two blocks write parts of one line of memory.
+void Plan::default_shape(LinePass& p, const PassSpec& s) const {
+  constexpr double kMiB = 1024.0 * 1024.0;
+  const int es = fp64_ ? 16 : 8;
+  const bool fast = has_fast_line_kernel(p.n);
+  // half-spectrum bytes, row alignment of both sides, distance of a line's elements
+  double elems = 1.0, stride = es;
+  for (std::size_t a = 0; a < rank_; ++a) elems *= static_cast<double>(std::min(p.in.ext[a], p.out.ext[a]));
+  bool odd = false;
+  for (const DDesc* d : {&p.in, &p.out}) {
+    const int inner = d->layout_left ? d->map[0] : d->map[d->ndim - 1];
+    if (inner == p.axis) continue;
+    const int rows = d->pitch > 0 ? d->pitch : d->base[inner];  // base + 1 on the first ranks of an uneven split
+    if (static_cast<int64_t>(rows) * es % 128 != 0 || (d->pitch <= 0 && d->rem[inner] > 0)) odd = true;
+  }
+  for (int k = 0; k < p.in.ndim; ++k) {
+    const int at = p.in.layout_left ? p.in.ndim - 1 - k : k;
+    if (p.in.map[at] == p.axis) {
+      stride = es;
+      continue;
+    }
+    stride *= p.in.ext[p.in.map[at]];
+  }
+  const double bytes = elems * es;
+  const bool across = p.lines_fast != 0;
+  const bool far = stride >= kMiB;
+  int vpt = 8, lines = 0;
+  if (!fast) {
+    vpt = 0;  // the runtime-radix kernel has its own rule
+  } else if (!across) {
+    // blocks of 128 lanes for short lines (256^3 R2C 69 -> 58 us)
+    lines = p.n <= 512 ? std::max(1, 1024 / p.n) : 0;
+  } else if (p.n <= 64) {
+    lines = p.n <= 32 ? 32 : fp64_ ? 8 : 16;
+  } else if (fp64_) {
+    if (p.n >= 512) vpt = 16;
+    lines = p.n <= 256 ? 8 : p.n == 512 ? 16 : p.n == 1024 ? 8 : 4;
+  } else {
+    if (p.n >= 1024 || (p.n == 512 && far)) vpt = 16;
+    lines = p.n == 128 ? (odd ? 16 : 32) : p.n <= 512 ? (p.n == 512 && far ? 32 : 16) : p.n == 1024 ? 16 : 8;
+  }
+  const bool narrow = across && lines > 0 && lines * es < 128;  // blocks share lines of memory
+  if (p.values_per_thread == 0 && p.lines_per_block == 0) {
+    p.values_per_thread = vpt;
+    p.lines_per_block = lines;
+    p.fit_block = 1;
+  }
+  if (s.xcd >= 0) p.xcd_remap = s.xcd;
+  else p.xcd_remap = across && (odd || narrow || (bytes >= 64 * kMiB && !far)) ? 1 : 0;
   if (s.nontemporal >= 0) {
     p.nontemporal = s.nontemporal;
+  } else if (across && (odd || narrow)) {
+    p.nontemporal = 0;
   } else {
-    // streaming accesses pay off once the array no longer fits the caches
-    double elems = 1.0;
-    for (std::size_t a = 0; a < rank_; ++a) elems *= static_cast<double>(in.ext[a]);
-    const double es = (s.kind == kR2C ? 0.5 : 1.0) * (fp64_ ? 16.0 : 8.0);
-    p.nontemporal = elems * es >= 1024.0 * 1024 * 1024 ? 1 : 0;
+    const bool last = p.in.ptr[0] == scratch_ && p.out.ptr[0] != scratch_;
+    p.nontemporal = bytes >= 512 * kMiB || last ? 1 : 0;
   }
-  return p;
 }
 
 void Plan::run_fused(void* const* in, void* const* out, bool forward, hipStream_t stream) {
@@ -615,7 +688,7 @@ DDesc Plan::band_scratch(int cut) const {
 void Plan::band_pass(LinePass& p, std::size_t i, bool forward, int cut) const {
   const auto& passes = forward ? fwd_ : bwd_;
   p.band = cut;
-  if (passes[i].values_per_thread != 0 && passes[i].values_per_thread != 8) p.lines_per_block = 0;
+  if (passes[i].values_per_thread != 0) p.lines_per_block = 0;  // tuned for the kernels of all modes
   p.pad_axis = 0;
   p.pad_real = 0;
   int64_t nl = 1;

@@ -21,13 +21,13 @@ struct PassSpec {
   int axis;
   int kind;  // LineKind
   int n;     // transform length
-  // launch shape (0 / -1 = launcher heuristic); set by options or the autotuner
+  // launch shape (0 / -1: Plan::default_shape); set by options or the autotuner
   int lines_per_block = 0;
   int values_per_thread = 0;
   int lines_fast = -1;
-  int nontemporal = -1;  // -1: on for arrays of at least 1 GiB
+  int nontemporal = -1;  // -1: by shape
   int paired = 1;        // R2C / C2R: two real lines per complex FFT
-  int xcd = 0;           // XCD-contiguous block numbering
+  int xcd = -1;          // XCD-contiguous block numbering (-1: by shape)
   int swz = 0;           // column-major walk of the block grid
   int split = 1;         // exchanges in real / imaginary halves (half the LDS; FP64, FP32 n >= 1024)
   int dual = 1;          // FP32 C2C: two adjacent lines per lane (16-byte accesses) where they apply
@@ -110,6 +110,8 @@ class Plan {
   // restricts pass i of a direction to the kept modes
   void band_pass(LinePass& p, std::size_t i, bool forward, int cut) const;
   DDesc band_scratch(int cut) const;
+  // launch shape of a pass where its spec leaves it open
+  void default_shape(LinePass& p, const PassSpec& s) const;
   float time_direction(void* const* in, void* const* out, bool forward, hipStream_t s, int reps);
   void plan_fused();
   void run_fused(void* const* in, void* const* out, bool forward, hipStream_t s);
