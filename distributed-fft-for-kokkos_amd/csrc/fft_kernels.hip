@@ -33,7 +33,7 @@ namespace dfft {
 // the line's LDS buffer.
 // ---------------------------------------------------------------------------
 template <typename Real, bool NT, bool DUAL, bool STAGE = false>
-__global__ void __launch_bounds__(kGroupThreads) fft_group_pass(const LinePass* __restrict__ items,
+__global__ void __launch_bounds__(kGroupThreads) fft_group_pass(const FastPass* __restrict__ items,
                                                                 const int32_t* __restrict__ first_block,
                                                                 int32_t count, int32_t total_blocks) {
   extern __shared__ unsigned char smem_raw[];
@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(kGroupThreads) fft_group_pass(const LinePass* 
       else hi = mid - 1;
     }
     const int32_t i = lo;
-    const LinePass& p = items[i];
+    const FastPass& p = items[i];
     const int32_t blk = vb - first_block[i];
     if constexpr (DUAL) {
       // DUAL instances hold the FP32 members taken two lines per lane (their
@@ -78,6 +78,29 @@ __global__ void __launch_bounds__(kGroupThreads) fft_group_pass(const LinePass* 
     }
     __syncthreads();  // the next virtual block reuses the LDS lines
   }
+}
+
+// Global indices of a line (per-element kernels)
+__device__ __forceinline__ void decode_line(const LinePass& p, int32_t line, int32_t* idx) {
+#pragma unroll
+  for (int a = 0; a < kMaxDim; ++a) idx[a] = 0;
+  uint32_t rem = static_cast<uint32_t>(line + p.line_begin);
+#pragma unroll
+  for (int j = kMaxDim - 2; j >= 0; --j) {
+    if (j < p.nbatch) {
+      uint32_t q = p.batch_div[j].div(rem);
+      idx[p.batch_axis[j]] = static_cast<int32_t>(rem - q * static_cast<uint32_t>(p.batch_ext[j]));
+      rem = q;
+    }
+  }
+}
+
+// true if line `line` of a pass enumerated over a padded extent is padding
+__device__ __forceinline__ bool padding_line(const LinePass& p, int32_t line) {
+  if (p.pad_real <= 0) return false;
+  int32_t idx[kMaxDim];
+  decode_line(p, line, idx);
+  return idx[p.pad_axis] >= p.pad_real;
 }
 
 // ---------------------------------------------------------------------------
@@ -138,7 +161,7 @@ __device__ __forceinline__ cplx_t<Real> generic_load(const LinePass& p, int32_t 
   using C = cplx_t<Real>;
   const int32_t n = p.n;
   int32_t idx[kMaxDim];
-  decode_line<Real>(p, line, idx);
+  decode_line(p, line, idx);
   const bool mirror = p.kind == kC2R && pos >= n / 2 + 1;
   idx[p.axis] = mirror ? n - pos : pos;
   int64_t st;
@@ -174,7 +197,7 @@ __device__ __forceinline__ void generic_store(const LinePass& p, int32_t line, i
   Real sc = static_cast<Real>(p.scale);
   if (p.kind == kR2C && pos != 0 && 2 * pos != n && p.herm_weight != 0.0) sc *= static_cast<Real>(p.herm_weight);
   int32_t idx[kMaxDim];
-  decode_line<Real>(p, line, idx);
+  decode_line(p, line, idx);
   idx[p.axis] = pos;
   int64_t st;
   const int64_t oes = p.kind == kC2R ? sizeof(Real) : sizeof(C);
@@ -208,7 +231,7 @@ __global__ void __launch_bounds__(256) fft_long_first(const LinePass p, const Ge
     C v{Real(0), Real(0)};
     if (sub < nsub) {
       const int32_t line = static_cast<int32_t>(sub / n2), i2 = static_cast<int32_t>(sub % n2);
-      if (!padding_line<Real>(p, line)) v = generic_load<Real>(p, line, i1 * n2 + i2);
+      if (!padding_line(p, line)) v = generic_load<Real>(p, line, i1 * n2 + i2);
     }
     bufA[b * n1 + i1] = v;
   }
@@ -255,7 +278,7 @@ __global__ void __launch_bounds__(256) fft_long_second(const LinePass p, const G
     const int64_t sub = sub0 + b;
     if (sub >= nsub) continue;
     const int32_t line = static_cast<int32_t>(sub / n1), k1 = static_cast<int32_t>(sub % n1);
-    if (padding_line<Real>(p, line)) continue;
+    if (padding_line(p, line)) continue;
     generic_store<Real>(p, line, k1 + n1 * k2, res[b * n2 + k2]);
   }
 }
@@ -280,7 +303,7 @@ __global__ void __launch_bounds__(256) bluestein_pre(const LinePass p, int32_t l
     const int32_t line = static_cast<int32_t>(g >> log2m);
     const int64_t j = g & (m - 1);
     C v{Real(0), Real(0)};
-    if (j < p.n && !padding_line<Real>(p, line)) {
+    if (j < p.n && !padding_line(p, line)) {
       const C x = generic_load<Real>(p, line, static_cast<int32_t>(j));
       v = cmul(x, to_prec<C>(chirp[(j * j) % n2]));
     }
@@ -310,7 +333,7 @@ __global__ void __launch_bounds__(256) bluestein_post(const LinePass p, int32_t 
        g += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int32_t line = static_cast<int32_t>(g / p.n);
     const int64_t k = g - static_cast<int64_t>(line) * p.n;
-    if (padding_line<Real>(p, line)) continue;
+    if (padding_line(p, line)) continue;
     const C y = s1[(static_cast<int64_t>(line) << log2m) + k];
     generic_store<Real>(p, line, static_cast<int32_t>(k), cmul(y, to_prec<C>(chirp[(k * k) % n2])));
   }
@@ -333,9 +356,9 @@ __global__ void __launch_bounds__(256) fft_line_generic(const LinePass p, const 
     const int32_t b = e / n, pos = e - b * n;
     const int32_t line = blockIdx.x * B + b;
     C v{Real(0), Real(0)};
-    if (line < p.nlines && !padding_line<Real>(p, line)) {
+    if (line < p.nlines && !padding_line(p, line)) {
       int32_t idx[kMaxDim];
-      decode_line<Real>(p, line, idx);
+      decode_line(p, line, idx);
       LineIO<Real> io;
       io.kind = p.kind;
       io.n = n;
@@ -373,10 +396,10 @@ __global__ void __launch_bounds__(256) fft_line_generic(const LinePass p, const 
   for (int32_t e = threadIdx.x; e < total; e += blockDim.x) {
     const int32_t b = e / n, pos = e - b * n;
     const int32_t line = blockIdx.x * B + b;
-    if (line >= p.nlines || padding_line<Real>(p, line)) continue;
+    if (line >= p.nlines || padding_line(p, line)) continue;
     if (p.kind == kR2C && 2 * pos > n) continue;
     int32_t idx[kMaxDim];
-    decode_line<Real>(p, line, idx);
+    decode_line(p, line, idx);
     idx[p.axis] = pos;
     int64_t st;
     LineIO<Real> io;
@@ -573,7 +596,7 @@ int group_grid(size_t lds_bytes, bool fp64, bool dual, int lanes) {
   return cus * (per_cu > 0 ? per_cu : 1);
 }
 
-hipError_t launch_group_pass(const LinePass* items, const int32_t* first_block, int count, int total_blocks,
+hipError_t launch_group_pass(const FastPass* items, const int32_t* first_block, int count, int total_blocks,
                              int grid, size_t lds_bytes, bool fp64, bool nontemporal, bool dual, int lanes,
                              bool stage, hipStream_t s) {
   if (total_blocks <= 0 || count <= 0) return hipSuccess;
@@ -612,6 +635,87 @@ hipError_t launch_group_pass(const LinePass* items, const int32_t* first_block, 
                          total_blocks);
   }
   return hipGetLastError();
+}
+
+namespace {
+void fast_side(Side& s, char** tab, const DDesc& d, const LinePass& p, int shift) {
+  s.shift = shift;
+  int ranks = 1;
+  for (int a = 0; a < d.ndim; ++a) ranks *= d.ntopo[a];
+  s.multi = ranks > 1 ? 1 : 0;
+  s.ptr = d.ptr[0];
+  // batch axis of an array axis, right-aligned in the three of a FastPass
+  auto batch_of = [&](int axis) {
+    for (int j = 0; j < p.nbatch; ++j)
+      if (p.batch_axis[j] == axis) return j + (kMaxDim - 1 - p.nbatch);
+    return -1;
+  };
+  int64_t acc = 1;
+  for (int k = 0; k < kMaxDim; ++k) {
+    SideAxis& x = s.ax[k];
+    x = SideAxis{};
+    x.base = 1;
+    x.m_small = 1;
+    if (k >= d.ndim) continue;
+    const int a = d.map[d.layout_left ? k : d.ndim - 1 - k];
+    const int row = (k == 0 && d.pitch > 0 && !d.layout_left) ? d.pitch : d.ext[a];
+    if (a == p.axis) {
+      s.line = acc;
+      x.base = 0;
+      x.line_len = row;
+      x.line_sel = -1;
+    } else {
+      const int j = batch_of(a);
+      if (j >= 0) s.stride[j] = acc;
+      x.sel0 = j == 0 ? -1 : 0;
+      x.sel1 = j == 1 ? -1 : 0;
+      x.sel2 = j == 2 ? -1 : 0;
+      x.base = d.base[a];
+      x.rem = d.rem[a];
+      x.split = d.rem[a] * (d.base[a] + 1);
+      x.rstride = d.rstride[a];
+      x.m_small = d.div_small[a].m;
+      x.m_xor = d.div_small[a].m ^ d.div_big[a].m;
+      x.l_small = d.div_small[a].l;
+      x.l_xor = d.div_small[a].l ^ d.div_big[a].l;
+    }
+    acc *= row;
+  }
+  if (s.multi)
+    for (int r = 0; r < ranks && r < kMaxRanks; ++r) tab[r] = d.ptr[r];
+}
+}  // namespace
+
+FastPass fast_pass(const LinePass& p, bool fp64) {
+  FastPass f;
+  f.nlines = p.nlines;
+  f.line_begin = p.line_begin;
+  f.kind = p.kind;
+  f.n = p.n;
+  f.inverse = p.inverse;
+  f.lines_fast = p.lines_fast;
+  f.lines_per_block = p.lines_per_block;
+  f.xcd_remap = p.xcd_remap;
+  f.swizzle = p.swizzle;
+  f.pad_real = p.pad_real > 0 ? p.pad_real : INT32_MAX;  // padded axes are the fastest batch axis
+  f.band = p.band;
+  f.dual_split = p.dual_split;
+  const int first = kMaxDim - 1 - p.nbatch;
+  for (int j = 0; j < kMaxDim - 1; ++j) {
+    const bool used = j >= first;
+    f.ext[j] = used ? p.batch_ext[j - first] : 1;
+    f.div[j] = used ? p.batch_div[j - first] : FastDiv(1u);
+    f.band_shift[j] = used ? p.band_shift[j - first] : 0;
+  }
+  f.bdiv = FastDiv(static_cast<uint32_t>(std::max(p.lines_per_block, 1)));
+  f.tw = p.tw;
+  f.scale = p.scale;
+  f.herm_weight = p.herm_weight;
+  const int cs = fp64 ? 4 : 3;  // a complex element; a real one is half of it
+  for (Side* d : {&f.in, &f.out}) d->stride[0] = d->stride[1] = d->stride[2] = d->line = 0;
+  fast_side(f.in, f.in_ptr, p.in, p, p.kind == kR2C ? cs - 1 : cs);
+  fast_side(f.out, f.out_ptr, p.out, p, p.kind == kC2R ? cs - 1 : cs);
+  return f;
 }
 
 bool has_fast_line_kernel(int n) {

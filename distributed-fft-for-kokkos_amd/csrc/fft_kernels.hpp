@@ -99,6 +99,50 @@ struct LinePass {
   void* long_scratch;
 };
 
+// The form of a line pass that the register kernels read (fast_pass).  A wave
+// has to know its lines' addresses before it can issue its first load, and
+// evaluating a DDesc costs some sixty dependent scalar loads and branches (a
+// LinePass spans 26 cache lines), 4 to 6 us before the first line load.  Here
+// the few fields of a side lie together, nothing branches on an axis, and a
+// single-rank side is three strides.  Round trips, DDesc -> this: 64^3 C2C
+// 42.5 -> 34 us, 50x42x36 R2C FP32 61 -> 51 us, 256^3 R2C FP64 336 -> 307 us,
+// 384^3 R2C FP64 1.50 -> 1.32 ms, 1024^3 R2C FP64 20.5 -> 19.8 ms.
+struct SideAxis {  // one storage axis of a multi-rank side; index 0 of extent 1 if unused
+  int32_t sel0, sel1, sel2;  // all ones for the batch axis it holds, else 0 (line axis: none)
+  int32_t base;              // ext / ntopo (line axis: 0)
+  int32_t split;             // rem * (base + 1): indices below it lie in ranks one longer
+  int32_t rem;
+  int32_t rstride;
+  uint32_t m_small, m_xor;   // multiplier of the division by base, and what turns it into that by base + 1
+  uint32_t l_small, l_xor;   // likewise the shift
+  int32_t line_len;          // of the line axis: its extent, else 0
+  int64_t line_sel;          // all ones for the line axis
+};
+struct Side {
+  char* ptr;          // single rank: its buffer
+  int64_t stride[3];  // single rank: elements between neighbours along each batch axis
+  int64_t line;       // single rank: elements between neighbours of a line
+  int32_t multi;      // more than one rank
+  int32_t shift;      // log2 of the element size in bytes
+  SideAxis ax[kMaxDim];  // storage axes, fastest first
+};
+struct FastPass {
+  int32_t nlines, line_begin, kind, n;
+  int32_t inverse, lines_fast, lines_per_block, xcd_remap;
+  int32_t swizzle, pad_real;  // pad_real: lines whose index along the fastest batch axis is >= it are padding
+  int32_t band, dual_split;
+  int32_t ext[3];         // batch axes, slowest first; unused ones come first with extent 1
+  int32_t band_shift[3];
+  FastDiv div[3];
+  FastDiv bdiv;           // lines_per_block
+  const void* tw;
+  double scale, herm_weight;
+  Side in, out;
+  char* in_ptr[kMaxRanks];   // multi-rank sides only
+  char* out_ptr[kMaxRanks];
+};
+FastPass fast_pass(const LinePass& p, bool fp64);
+
 // Element-wise permuted copy between two distributions of the same logical
 // array (one-GPU form of pack -> all-to-all -> unpack, and of local
 // transposes).  Iterates the destination in its storage order.
@@ -132,7 +176,7 @@ int group_grid(size_t lds_bytes, bool fp64, bool dual, int lanes);
 // dual: the launch holds only members with dual_lines set (FP32, kGroupThreads
 // lanes); lanes: lanes per block of a one-line launch; stage (FP32 one-line):
 // contiguous aligned lines move 16 bytes per lane through LDS
-hipError_t launch_group_pass(const LinePass* items, const int32_t* first_block, int count, int total_blocks,
+hipError_t launch_group_pass(const FastPass* items, const int32_t* first_block, int count, int total_blocks,
                              int grid, size_t lds_bytes, bool fp64, bool nontemporal, bool dual, int lanes,
                              bool stage, hipStream_t s);
 bool has_fast_line_kernel(int n);

@@ -273,96 +273,111 @@ template <typename Real, bool NT = false> struct PairIO {
   }
 };
 
-// BAND: a pass over the kept modes of a dealiased field only (LinePass::band)
-template <typename Real, bool BAND = false>
-__device__ __forceinline__ void decode_line(const LinePass& p, int32_t line, int32_t* idx) {
-#pragma unroll
-  for (int a = 0; a < kMaxDim; ++a) idx[a] = 0;
-  uint32_t rem = static_cast<uint32_t>(line + p.line_begin);
-#pragma unroll
-  for (int j = kMaxDim - 2; j >= 0; --j) {
-    if (j < p.nbatch) {
-      uint32_t q = p.batch_div[j].div(rem);
-      int32_t i = static_cast<int32_t>(rem - q * static_cast<uint32_t>(p.batch_ext[j]));
-      if constexpr (BAND) i += i > p.band ? p.band_shift[j] : 0;
-      idx[p.batch_axis[j]] = i;
-      rem = q;
-    }
+// Batch indices of a line (slowest axis first).  BAND: a pass over the kept
+// modes of a dealiased field only (FastPass::band).
+struct BatchIdx {
+  int32_t i0, i1, i2;
+};
+template <bool BAND = false>
+__device__ __forceinline__ BatchIdx batch_index(const FastPass& p, int32_t line) {
+  const uint32_t l = static_cast<uint32_t>(line + p.line_begin);
+  const uint32_t q2 = p.div[2].div(l);
+  const uint32_t q1 = p.div[1].div(q2);
+  BatchIdx x;
+  x.i2 = static_cast<int32_t>(l - q2 * static_cast<uint32_t>(p.ext[2]));
+  x.i1 = static_cast<int32_t>(q2 - q1 * static_cast<uint32_t>(p.ext[1]));
+  x.i0 = static_cast<int32_t>(q1);
+  if constexpr (BAND) {
+    x.i0 += x.i0 > p.band ? p.band_shift[0] : 0;
+    x.i1 += x.i1 > p.band ? p.band_shift[1] : 0;
+    x.i2 += x.i2 > p.band ? p.band_shift[2] : 0;
   }
+  return x;
 }
 
-// true if line `line` of a pass enumerated over a padded extent is padding
-template <typename Real, bool BAND = false>
-__device__ __forceinline__ bool padding_line(const LinePass& p, int32_t line) {
-  if (p.pad_real <= 0) return false;
-  int32_t idx[kMaxDim];
-  decode_line<Real, BAND>(p, line, idx);
-  return idx[p.pad_axis] >= p.pad_real;
+// Address of element 0 of line x on one side of a pass, and the line's
+// element stride.  Multi-rank sides: per storage axis, fastest first, the
+// owner bin and local index of the index (first rem bins one longer --
+// KokkosFFT_Distributed_MPI_Extents.hpp:195-235).  Every choice is a mask or
+// an exclusive or with a field: selects between two fields compile to
+// per-lane loads of the chosen one, selects on an axis to branches.
+__device__ __forceinline__ char* side_line(const Side& s, char* const* tab, const BatchIdx& x, int64_t& line) {
+  if (!s.multi) {
+    line = s.line;
+    return s.ptr + ((x.i0 * s.stride[0] + x.i1 * s.stride[1] + x.i2 * s.stride[2]) << s.shift);
+  }
+  int64_t acc = 1, off = 0, ls = 0;
+  int32_t rank = 0;
+#pragma unroll
+  for (int k = 0; k < kMaxDim; ++k) {
+    const SideAxis& a = s.ax[k];
+    const int32_t i = (x.i0 & a.sel0) | (x.i1 & a.sel1) | (x.i2 & a.sel2);
+    const int32_t low = i < a.split ? -1 : 0;  // in a rank one longer
+    const uint32_t t = static_cast<uint32_t>(i - (a.split & ~low));
+    const uint32_t q = (__umulhi(t, a.m_small ^ (a.m_xor & static_cast<uint32_t>(low))) + t) >>
+                       (a.l_small ^ (a.l_xor & static_cast<uint32_t>(low)));
+    const int32_t len = a.base - low;
+    rank += (static_cast<int32_t>(q) + (a.rem & ~low)) * a.rstride;
+    ls |= acc & a.line_sel;
+    off += (static_cast<int32_t>(t) - static_cast<int32_t>(q) * len) * acc;
+    acc *= len | a.line_len;
+  }
+  line = ls;
+  return tab[rank] + (off << s.shift);
 }
 
+// The line's addresses; false if it is padding (a pass enumerated over padded
+// rows)
 template <typename Real, bool NT = false, bool BAND = false>
-__device__ __forceinline__ LineIO<Real, NT> make_line_io(const LinePass& p, int32_t line) {
-  using C = cplx_t<Real>;
-  int32_t idx[kMaxDim];
-  decode_line<Real, BAND>(p, line, idx);
-  LineIO<Real, NT> io;
-  const int64_t ies = p.kind == kR2C ? sizeof(Real) : sizeof(C);
-  const int64_t oes = p.kind == kC2R ? sizeof(Real) : sizeof(C);
-  io.ib = element_ptr(p.in, idx, ies, p.axis, io.is);
-  io.ob = element_ptr(p.out, idx, oes, p.axis, io.os);
+__device__ __forceinline__ bool make_line_io(const FastPass& p, int32_t line, LineIO<Real, NT>& io) {
+  const BatchIdx x = batch_index<BAND>(p, line);
+  if (x.i2 >= p.pad_real) return false;
+  io.ib = side_line(p.in, p.in_ptr, x, io.is);
+  io.ob = side_line(p.out, p.out_ptr, x, io.os);
   io.kind = p.kind;
   io.n = p.n;
   io.inverse = p.inverse;
   io.scale = static_cast<Real>(p.scale);
   io.hw = p.herm_weight != 0.0 ? static_cast<Real>(p.herm_weight) : Real(1);
-  return io;
+  return true;
+}
+
+// true if line `line` is padding
+__device__ __forceinline__ bool padding_line(const FastPass& p, int32_t line) {
+  const uint32_t l = static_cast<uint32_t>(line + p.line_begin);
+  return static_cast<int32_t>(l - p.div[2].div(l) * static_cast<uint32_t>(p.ext[2])) >= p.pad_real;
 }
 
 // factors of product field f (0..5) of the divergence-form products
 __device__ __forceinline__ int32_t prod_first(int32_t f) { return f < 3 ? 0 : (f < 5 ? 1 : 2); }
 __device__ __forceinline__ int32_t prod_second(int32_t f) { return f < 3 ? f : (f < 5 ? f - 2 : 2); }
 
-// Products pass: line `idx` is product field f = idx[prod_axis] of one
-// position; the velocity field (f / 2) of that position, which the slot of
-// the pair (f, f + 1) stages for the position's three slots.  Selects over the
-// unrolled axes keep idx in registers.
-__device__ __forceinline__ const char* product_source(const LinePass& p, const int32_t* idx, int64_t ies,
-                                                      int64_t& is) {
-  int32_t f = 0;
-#pragma unroll
-  for (int a = 0; a < kMaxDim; ++a)
-    if (a == p.prod_axis) f = idx[a];
-  int32_t j[kMaxDim];
-#pragma unroll
-  for (int a = 0; a < kMaxDim; ++a) j[a] = a == p.prod_axis ? f / 2 : idx[a];
-  return element_ptr(p.in, j, ies, p.axis, is);
-}
-
+// PROD (products pass): the field axis is the fastest batch axis, and the
+// slot of the pair of fields (f, f + 1) stages velocity line f / 2 of its
+// position for the position's three slots.
 template <typename Real, bool NT, bool PROD = false, bool BAND = false>
-__device__ __forceinline__ PairIO<Real, NT> make_pair_io(const LinePass& p, int32_t pair) {
-  using C = cplx_t<Real>;
+__device__ __forceinline__ PairIO<Real, NT> make_pair_io(const FastPass& p, int32_t pair) {
   PairIO<Real, NT> io;
-  const int64_t ies = p.kind == kR2C ? sizeof(Real) : sizeof(C);
-  const int64_t oes = p.kind == kC2R ? sizeof(Real) : sizeof(C);
-  int32_t idx[kMaxDim];
   const int32_t la = 2 * pair;
-  decode_line<Real, BAND>(p, la, idx);
+  BatchIdx x = batch_index<BAND>(p, la);
+  io.ob[0] = side_line(p.out, p.out_ptr, x, io.os[0]);
   if constexpr (PROD) {
-    io.ib[0] = product_source(p, idx, ies, io.is[0]);
+    BatchIdx u = x;
+    u.i2 >>= 1;
+    io.ib[0] = side_line(p.in, p.in_ptr, u, io.is[0]);
   } else {
-    io.ib[0] = element_ptr(p.in, idx, ies, p.axis, io.is[0]);
+    io.ib[0] = side_line(p.in, p.in_ptr, x, io.is[0]);
   }
-  io.ob[0] = element_ptr(p.out, idx, oes, p.axis, io.os[0]);
   io.has_b = la + 1 < p.nlines;
   if (io.has_b) {
-    decode_line<Real, BAND>(p, la + 1, idx);
+    x = batch_index<BAND>(p, la + 1);
     if constexpr (PROD) {
       io.ib[1] = io.ib[0];
       io.is[1] = io.is[0];
     } else {
-      io.ib[1] = element_ptr(p.in, idx, ies, p.axis, io.is[1]);
+      io.ib[1] = side_line(p.in, p.in_ptr, x, io.is[1]);
     }
-    io.ob[1] = element_ptr(p.out, idx, oes, p.axis, io.os[1]);
+    io.ob[1] = side_line(p.out, p.out_ptr, x, io.os[1]);
   } else {
     io.ib[1] = io.ib[0];
     io.ob[1] = io.ob[0];
@@ -705,7 +720,7 @@ template <typename Real, int N, int RM, int S> struct StageLoop2 {
 // pair whose second line is padding (the next row's first element there, or
 // past the end of the rank's array) is not loaded.
 template <typename Real, int N, int RM, bool NT, int SPLIT_IN = 0>
-__device__ __forceinline__ void fast_line2_body(const LinePass& p, int32_t blk, int B, unsigned char* lds) {
+__device__ __forceinline__ void fast_line2_body(const FastPass& p, int32_t blk, int B, unsigned char* lds) {
   using C = cplx_t<Real>;
   using Cfg = FastCfg<Real, N, RM>;
   typedef Real V4 __attribute__((ext_vector_type(4)));
@@ -716,22 +731,24 @@ __device__ __forceinline__ void fast_line2_body(const LinePass& p, int32_t blk, 
   // lanes beyond P2*T (grouped launches of 256 lanes) run the stages on zeros
   // in two spare LDS slots (2*P2, 2*P2 + 1) and load and store nothing
   const bool active = tid < P2 * T;
-  const int b = active ? tid % P2 : P2, t = active ? tid / P2 : 0;
+  int t = static_cast<int>(p.bdiv.div(static_cast<uint32_t>(2 * tid)));  // tid / (B / 2): B is even
+  const int b = active ? tid - t * P2 : P2;
+  if (!active) t = 0;
   const int32_t la = blk * B + 2 * b;  // lines la, la + 1 (nlines is even)
-  const bool valid = active && la < p.nlines && !padding_line<Real>(p, la);
   const double2* tw = reinterpret_cast<const double2*>(p.tw);
   Real* ba = reinterpret_cast<Real*>(lds + (2 * b) * LB);
   Real* bb = reinterpret_cast<Real*>(lds + (2 * b + 1) * LB);
   LineIO<Real, NT> io;
-  if (valid) io = make_line_io<Real, NT>(p, la);
+  bool valid = active && la < p.nlines;
+  if (valid) valid = make_line_io<Real, NT>(p, la, io);
 
   bool second = false;
-  if constexpr (SPLIT_IN == 1) second = valid && !padding_line<Real>(p, la + 1);
+  if constexpr (SPLIT_IN == 1) second = valid && !padding_line(p, la + 1);
   // SPLIT_IN == 2: line la + 1 has addresses of its own on both sides
   [[maybe_unused]] LineIO<Real, NT> io2 = io;
   if constexpr (SPLIT_IN == 2) {
-    second = valid && la + 1 < p.nlines && !padding_line<Real>(p, la + 1);
-    if (second) io2 = make_line_io<Real, NT>(p, la + 1);
+    second = valid && la + 1 < p.nlines;
+    if (second) second = make_line_io<Real, NT>(p, la + 1, io2);
   }
   C va[R], vb[R];
   constexpr int r0 = Cfg::P.rad[0];
@@ -829,15 +846,15 @@ __device__ __forceinline__ void fast_line2_body(const LinePass& p, int32_t blk, 
 // BAND: a C2C pass over kept modes: inverse lines read positions outside the
 // band as zeros, forward lines store only the band.
 template <typename Real, int N, int RM, bool NT, bool SPLIT, bool STAGE = false, bool BAND = false>
-__device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, int B, unsigned char* lds) {
+__device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, int B, unsigned char* lds) {
   using C = cplx_t<Real>;
   using Cfg = FastCfg<Real, N, RM>;
   constexpr int R = Cfg::R, T = Cfg::T;
   const int tid = threadIdx.x;
   int b, t;
   if (p.lines_fast) {
-    b = tid % B;
-    t = tid / B;
+    t = static_cast<int>(p.bdiv.div(static_cast<uint32_t>(tid)));
+    b = tid - t * B;
   } else {
     t = tid % T;
     b = tid / T;
@@ -858,11 +875,11 @@ __device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, i
     // spare lanes), so the line index is wave-uniform and the descriptor
     // arithmetic of make_line_io runs once per wave on the scalar unit
     const int32_t wl = __builtin_amdgcn_readfirstlane(line);
-    valid = active && wl < p.nlines && !padding_line<Real, BAND>(p, wl);
-    if (valid) io = make_line_io<Real, NT, BAND>(p, wl);
+    valid = active && wl < p.nlines;
+    if (valid) valid = make_line_io<Real, NT, BAND>(p, wl, io);
   } else {
-    valid = active && line < p.nlines && !padding_line<Real, BAND>(p, line);
-    if (valid) io = make_line_io<Real, NT, BAND>(p, line);
+    valid = active && line < p.nlines;
+    if (valid) valid = make_line_io<Real, NT, BAND>(p, line, io);
   }
 
   C v[R];
@@ -1042,15 +1059,15 @@ __device__ __forceinline__ void fast_line_body(const LinePass& p, int32_t blk, i
 // product of the two factor lines' values at that position.
 // BAND: half-spectrum entries above p.band are neither read (zeros) nor stored.
 template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false, bool BAND = false>
-__device__ __forceinline__ void fast_pair_body(const LinePass& p, int32_t blk, int B, unsigned char* lds) {
+__device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, int B, unsigned char* lds) {
   using C = cplx_t<Real>;
   using Cfg = FastCfg<Real, N, RM>;
   constexpr int R = Cfg::R, T = Cfg::T;
   const int tid = threadIdx.x;
   int b, t;
   if (p.lines_fast) {
-    b = tid % B;
-    t = tid / B;
+    t = static_cast<int>(p.bdiv.div(static_cast<uint32_t>(tid)));
+    b = tid - t * B;
   } else {
     t = tid % T;
     b = tid / T;
@@ -1329,7 +1346,7 @@ __device__ __forceinline__ int32_t xcd_block(int32_t b, int32_t nb) {
 // then an optional column-major walk of the (nb / C) x C block grid, where C
 // blocks cover one row of the fastest batch axis (p.swizzle = C; the launcher
 // sets it only when it divides the grid).
-__device__ __forceinline__ int32_t pass_block(const LinePass& p, int32_t b, int32_t nb) {
+__device__ __forceinline__ int32_t pass_block(const FastPass& p, int32_t b, int32_t nb) {
   if (p.xcd_remap) b = xcd_block(b, nb);
   if (p.swizzle > 1) {
     const int32_t rows = nb / p.swizzle;
@@ -1339,21 +1356,21 @@ __device__ __forceinline__ int32_t pass_block(const LinePass& p, int32_t b, int3
 }
 
 template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false, bool BAND = false>
-__global__ void __launch_bounds__(1024) fft_pair_fast(const LinePass p) {
+__global__ void __launch_bounds__(1024) fft_pair_fast(const FastPass p) {
   extern __shared__ unsigned char smem_raw[];
   const int32_t blk = pass_block(p, blockIdx.x, gridDim.x);
   fast_pair_body<Real, N, RM, NT, SPLIT, PROD, BAND>(p, blk, p.lines_per_block, smem_raw);
 }
 
 template <typename Real, int N, int RM, bool NT, bool SPLIT, bool BAND = false>
-__global__ void __launch_bounds__(1024) fft_line_fast(const LinePass p) {
+__global__ void __launch_bounds__(1024) fft_line_fast(const FastPass p) {
   extern __shared__ unsigned char smem_raw[];
   const int32_t blk = pass_block(p, blockIdx.x, gridDim.x);
   fast_line_body<Real, N, RM, NT, SPLIT, false, BAND>(p, blk, p.lines_per_block, smem_raw);
 }
 
 template <typename Real, int N, int RM, bool NT, int SPLIT_IN>
-__global__ void __launch_bounds__(1024) fft_line2_fast(const LinePass p) {
+__global__ void __launch_bounds__(1024) fft_line2_fast(const FastPass p) {
   extern __shared__ unsigned char smem_raw[];
   const int32_t blk = pass_block(p, blockIdx.x, gridDim.x);
   fast_line2_body<Real, N, RM, NT, SPLIT_IN>(p, blk, p.lines_per_block, smem_raw);
@@ -1393,11 +1410,11 @@ template <typename Real, int N, int RM, bool NT, bool SPLIT> struct FastVariant 
   static void launch(bool pair, unsigned grid, unsigned threads, size_t smem, hipStream_t s, const LinePass& p) {
     if constexpr (kPairs) {
       if (pair) {
-        hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, SPLIT>), dim3(grid), dim3(threads), smem, s, p);
+        hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, SPLIT>), dim3(grid), dim3(threads), smem, s, fast_pass(p, sizeof(Real) == 8));
         return;
       }
     }
-    hipLaunchKernelGGL((fft_line_fast<Real, N, RM, NT, SPLIT>), dim3(grid), dim3(threads), smem, s, p);
+    hipLaunchKernelGGL((fft_line_fast<Real, N, RM, NT, SPLIT>), dim3(grid), dim3(threads), smem, s, fast_pass(p, sizeof(Real) == 8));
   }
 };
 
@@ -1558,13 +1575,13 @@ hipError_t launch_dual(LinePass p, int B, hipStream_t s) {
     }
     const dim3 g(grid), b(P2 * T);
     if (nt) {
-      if (mode == 2) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, true, 2>), g, b, smem, s, p);
-      else if (mode == 1) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, true, 1>), g, b, smem, s, p);
-      else hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, true, 0>), g, b, smem, s, p);
+      if (mode == 2) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, true, 2>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+      else if (mode == 1) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, true, 1>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+      else hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, true, 0>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
     } else {
-      if (mode == 2) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, false, 2>), g, b, smem, s, p);
-      else if (mode == 1) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, false, 1>), g, b, smem, s, p);
-      else hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, false, 0>), g, b, smem, s, p);
+      if (mode == 2) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, false, 2>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+      else if (mode == 1) hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, false, 1>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+      else hipLaunchKernelGGL((fft_line2_fast<Real, N, RM, false, 0>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
     }
     return hipGetLastError();
   }
@@ -1690,11 +1707,11 @@ hipError_t launch_products(LinePass p, hipStream_t s) {
   if (grid == 0) return hipSuccess;
   const dim3 g(grid), b(static_cast<unsigned>(T * B));
   if (split) {
-    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, true, true>), g, b, smem, s, p);
-    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, true, true>), g, b, smem, s, p);
+    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, true, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, true, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
   } else {
-    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, false, true>), g, b, smem, s, p);
-    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, false, true>), g, b, smem, s, p);
+    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, false, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, false, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
   }
   return hipGetLastError();
 }
@@ -1735,9 +1752,9 @@ hipError_t launch_band(LinePass p, hipStream_t s) {
   const int k = p.products ? 2 : (pair ? 1 : 0);
   const hipError_t e = raise_lds_limit(limit[k], fns[k], smem);
   if (e != hipSuccess) return e;
-  if (k == 2) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, true, true>), grid, block, smem, s, p);
-  else if (k == 1) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, false, true>), grid, block, smem, s, p);
-  else hipLaunchKernelGGL((fft_line_fast<Real, N, 8, NT, true, true>), grid, block, smem, s, p);
+  if (k == 2) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, true, true>), grid, block, smem, s, fast_pass(p, sizeof(Real) == 8));
+  else if (k == 1) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, false, true>), grid, block, smem, s, fast_pass(p, sizeof(Real) == 8));
+  else hipLaunchKernelGGL((fft_line_fast<Real, N, 8, NT, true, true>), grid, block, smem, s, fast_pass(p, sizeof(Real) == 8));
   return hipGetLastError();
 }
 

@@ -442,7 +442,7 @@ __device__ __forceinline__ void mix_stages(Real* re, Real* im, const MixPlan& m,
 // KIND kC2C: one complex line per T lanes.  kR2C / kC2R: two real lines 2q,
 // 2q+1 per T lanes as one complex line (PairIO).
 template <typename Real, int V, bool NT, int KIND>
-__global__ void __launch_bounds__(1024) fft_mixed(const LinePass p, const MixPlan m) {
+__global__ void __launch_bounds__(1024) fft_mixed(const FastPass p, const MixPlan m) {
   using C = cplx_t<Real>;
   extern __shared__ unsigned char smem_raw[];
   const int tid = threadIdx.x;
@@ -475,10 +475,10 @@ __global__ void __launch_bounds__(1024) fft_mixed(const LinePass p, const MixPla
   }
 
   if constexpr (KIND == kC2C) {
-    const bool valid = active && unit < p.nlines && !padding_line<Real>(p, unit);
     LineIO<Real, NT> io;
+    bool valid = active && unit < p.nlines;
+    if (valid) valid = make_line_io<Real, NT>(p, unit, io);
     if (valid) {
-      io = make_line_io<Real, NT>(p, unit);
 #define DFFT_MIX_CALL(r) mix_load_c2c<r, V, NT, Real>(re, im, s0, t, T, io.ib, io.is, p.inverse != 0)
       DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
 #undef DFFT_MIX_CALL

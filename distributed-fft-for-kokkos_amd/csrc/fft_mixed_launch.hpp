@@ -116,7 +116,7 @@ hipError_t launch_mixed_kernel(const LinePass& p, const MixPlan& m, unsigned gri
   static std::atomic<size_t> limit{64 * 1024};
   const hipError_t e = raise_lds_limit(limit, reinterpret_cast<const void*>(&fft_mixed<Real, V, NT, KIND>), smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((fft_mixed<Real, V, NT, KIND>), dim3(grid), dim3(threads), smem, s, p, m);
+  hipLaunchKernelGGL((fft_mixed<Real, V, NT, KIND>), dim3(grid), dim3(threads), smem, s, fast_pass(p, sizeof(Real) == 8), m);
   return hipGetLastError();
 }
 

@@ -277,7 +277,7 @@ void Group::build_tables(const std::vector<void*>& in, const std::vector<void*>&
       const int resident = group_grid(lds[v], fp64_, v == 1, lanes);
       if (resident <= 0) throw Error(DFFT_ERROR_HIP, "occupancy query of the grouped kernel failed");
       t.grid[slot] = grid_mult_ > 0 ? resident * grid_mult_ : first[v].back();
-      t.items[slot] = std::move(grouped[v]);
+      for (const LinePass& p : grouped[v]) t.items[slot].push_back(fast_pass(p, fp64_));
       t.first[slot] = std::move(first[v]);
     }
   }
@@ -293,10 +293,10 @@ void Group::upload(const std::vector<void*>& in, const std::vector<void*>& out, 
   for (std::size_t slot = 0; slot < ns; ++slot) {
     if (ds.tables.count[slot] == 0) continue;
     if (!ds.items[slot]) {
-      check(hipMalloc(&ds.items[slot], sizeof(LinePass) * members_.size()), "hipMalloc");
+      check(hipMalloc(&ds.items[slot], sizeof(FastPass) * members_.size()), "hipMalloc");
       check(hipMalloc(&ds.first[slot], sizeof(int32_t) * (members_.size() + 1)), "hipMalloc");
     }
-    check(hipMemcpy(ds.items[slot], ds.tables.items[slot].data(), sizeof(LinePass) * ds.tables.items[slot].size(),
+    check(hipMemcpy(ds.items[slot], ds.tables.items[slot].data(), sizeof(FastPass) * ds.tables.items[slot].size(),
                     hipMemcpyHostToDevice),
           "hipMemcpy");
     check(hipMemcpy(ds.first[slot], ds.tables.first[slot].data(), sizeof(int32_t) * ds.tables.first[slot].size(),
@@ -308,7 +308,7 @@ void Group::upload(const std::vector<void*>& in, const std::vector<void*>& out, 
   ds.built = true;
 }
 
-void Group::launch_tables(const Tables& t, LinePass* const* items, int32_t* const* first, int dir,
+void Group::launch_tables(const Tables& t, FastPass* const* items, int32_t* const* first, int dir,
                           hipStream_t s) const {
   TraceRange range("dfft::Group %s (%zu members)", dir == 0 ? "forward" : "backward", members_.size());
   for (int k = 0; k < max_passes_; ++k) {

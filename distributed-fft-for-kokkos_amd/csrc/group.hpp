@@ -59,7 +59,7 @@ class Group {
   // host form of one direction's launches: slot 2k + v holds the grouped
   // members of pass k taken one (v = 0) or two (v = 1) lines per lane
   struct Tables {
-    std::vector<std::vector<LinePass>> items;
+    std::vector<std::vector<FastPass>> items;
     std::vector<std::vector<int32_t>> first;  // virtual-block prefix per slot
     std::vector<int> count, total, grid, nt, lanes;
     std::vector<size_t> lds;
@@ -73,7 +73,7 @@ class Group {
   void launch_all(int dir, hipStream_t s);
   // launches of one direction from tables whose slots sit at items[slot] /
   // first[slot] on the device
-  void launch_tables(const Tables& t, LinePass* const* items, int32_t* const* first, int dir, hipStream_t s) const;
+  void launch_tables(const Tables& t, FastPass* const* items, int32_t* const* first, int dir, hipStream_t s) const;
   void invalidate();
 
   std::vector<Member> members_;
@@ -89,13 +89,13 @@ class Group {
   int contig_nt_ = -1;  // nontemporal accesses of launches of contiguous lines (-1: as nt_)
   std::map<int, void*> tw_;
   // per direction: the pointer set the device tables were built for, the
-  // tables of every pass (LinePass items + virtual-block prefix), members
+  // tables of every pass (FastPass items + virtual-block prefix), members
   // whose length has no grouped kernel (launched one by one), and a graph
   struct DirState {
     std::vector<void*> in, out;
     bool built = false;
     Tables tables;                    // host form of the launches
-    std::vector<LinePass*> items;     // device copies of tables.items, one array per slot
+    std::vector<FastPass*> items;     // device copies of tables.items, one array per slot
     std::vector<int32_t*> first;      // device copies of tables.first
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;

@@ -1,5 +1,5 @@
 // Group execution without device allocation (dfft_group_execute_noalloc):
-// the per-call pass tables (LinePass records and virtual-block prefixes of
+// the per-call pass tables (FastPass records and virtual-block prefixes of
 // every grouped launch) live in one static device array per GPU instead of
 // hipMalloc'ed tables, for callers that cannot allocate (code under stream
 // capture, serving loops, harnesses that forbid hipMalloc).
@@ -68,7 +68,7 @@ void Group::execute_static(void* const* in, void* const* out, int direction, hip
   for (std::size_t slot = 0; slot < ns; ++slot) {
     if (t.count[slot] == 0) continue;
     off_items[slot] = used;
-    used = align256(used + sizeof(LinePass) * t.items[slot].size());
+    used = align256(used + sizeof(FastPass) * t.items[slot].size());
     off_first[slot] = used;
     used = align256(used + sizeof(int32_t) * t.first[slot].size());
   }
@@ -77,7 +77,7 @@ void Group::execute_static(void* const* in, void* const* out, int direction, hip
                                             " bytes; the static table area holds " +
                                             std::to_string(kStaticTableBytes));
   if (used == 0) {  // nothing grouped: every pass is launched on its own
-    std::vector<LinePass*> none(ns, nullptr);
+    std::vector<FastPass*> none(ns, nullptr);
     std::vector<int32_t*> nonef(ns, nullptr);
     launch_tables(t, none.data(), nonef.data(), dir, s);
     return;
@@ -85,7 +85,7 @@ void Group::execute_static(void* const* in, void* const* out, int direction, hip
   std::vector<unsigned char> host(used, 0);
   for (std::size_t slot = 0; slot < ns; ++slot) {
     if (t.count[slot] == 0) continue;
-    std::memcpy(host.data() + off_items[slot], t.items[slot].data(), sizeof(LinePass) * t.items[slot].size());
+    std::memcpy(host.data() + off_items[slot], t.items[slot].data(), sizeof(FastPass) * t.items[slot].size());
     std::memcpy(host.data() + off_first[slot], t.first[slot].data(), sizeof(int32_t) * t.first[slot].size());
   }
   char* base = scratch_on(device_);
@@ -93,11 +93,11 @@ void Group::execute_static(void* const* in, void* const* out, int direction, hip
   // the host copy is released once the stream has taken it
   check(hipMemcpyAsync(base, host.data(), used, hipMemcpyHostToDevice, s), "hipMemcpyAsync of the pass tables");
   check(hipStreamSynchronize(s), "hipStreamSynchronize");
-  std::vector<LinePass*> items(ns, nullptr);
+  std::vector<FastPass*> items(ns, nullptr);
   std::vector<int32_t*> first(ns, nullptr);
   for (std::size_t slot = 0; slot < ns; ++slot) {
     if (t.count[slot] == 0) continue;
-    items[slot] = reinterpret_cast<LinePass*>(base + off_items[slot]);
+    items[slot] = reinterpret_cast<FastPass*>(base + off_items[slot]);
     first[slot] = reinterpret_cast<int32_t*>(base + off_first[slot]);
   }
   launch_tables(t, items.data(), first.data(), dir, s);

@@ -660,7 +660,7 @@ void Plan::run_fused(void* const* in, void* const* out, bool forward, hipStream_
 bool Plan::products_supported() const {
   if (!fp64_ || !real_ || d_.exec_mode != DFFT_EXEC_FUSED || view_layout_ != Layout::Right) return false;
   if (rank_ != 4 || gin_[0] != 6 || in_topo_[0] != 1 || out_topo_[0] != 1) return false;
-  if (fwd_.empty() || fwd_[0].kind != kR2C || fwd_[0].axis != 3 || fwd_[0].paired == 0) return false;
+  if (fwd_.empty() || fwd_[0].kind != kR2C || fwd_[0].axis != 3) return false;
   for (int a : {1, 2, 3})
     if (std::find(axes_.begin(), axes_.end(), static_cast<std::size_t>(a)) == axes_.end()) return false;
   return products_pass_supported(fwd_[0].n);
@@ -672,7 +672,7 @@ bool Plan::band_supported(int cut) const {
   if (cut < 1 || fwd_.size() != 3 || bwd_.size() != 3) return false;
   for (const auto* passes : {&fwd_, &bwd_})
     for (const PassSpec& s : *passes)
-      if (!band_pass_supported(s.n) || 2 * cut >= s.n || (s.kind != kC2C && (s.paired == 0 || s.axis != 3))) return false;
+      if (!band_pass_supported(s.n) || 2 * cut >= s.n || (s.kind != kC2C && s.axis != 3)) return false;
   return fwd_[0].kind == kR2C && bwd_[2].kind == kC2R && in_topo_[fwd_[0].axis] == 1 &&
          out_topo_[fwd_[2].axis] == 1 && out_topo_[bwd_[0].axis] == 1 && in_topo_[bwd_[2].axis] == 1;
 }
