@@ -526,62 +526,61 @@ namespace {
 // lines per block: as many as the block's lanes hold, capped so the lines
 // plus the spare slot fit `cap` bytes of dynamic LDS (at most 64 KB)
 template <typename Real, int N>
-void group_shape_of(size_t cap, int lanes, int* B, size_t* lds) {
+void group_shape_of(size_t cap, int lanes, bool across, GroupShape* g) {
   using Cfg = FastCfg<Real, N, 8>;
   static_assert(Cfg::T <= 64, "a grouped line fits the smallest block");
-  const size_t line_bytes = static_cast<size_t>(Cfg::LDSN) * sizeof(cplx_t<Real>);
-  if (cap > kGroupLds) cap = kGroupLds;
+  constexpr int elem = static_cast<int>(sizeof(cplx_t<Real>));
   int b = lanes / Cfg::T;
-  while (b > 1 && static_cast<size_t>(b + 1) * line_bytes > cap) --b;
-  *B = b;
-  *lds = static_cast<size_t>(b + 1) * line_bytes;
+  const size_t line = line_stride(static_cast<size_t>(Cfg::LDSN) * elem, elem, across, b, Cfg::T);
+  if (cap > kGroupLds) cap = kGroupLds;
+  while (b > 1 && static_cast<size_t>(b + 1) * line > cap) --b;
+  g->lines_per_block = b;
+  g->line_bytes = static_cast<int>(line);
+  g->lds_bytes = static_cast<size_t>(b + 1) * line;
 }
 template <typename Real>
-bool group_shape(int n, size_t cap, int lanes, int* B, size_t* lds) {
+bool group_shape(int n, size_t cap, int lanes, bool across, GroupShape* g) {
   switch (n) {
-    case 16: group_shape_of<Real, 16>(cap, lanes, B, lds); return true;
-    case 32: group_shape_of<Real, 32>(cap, lanes, B, lds); return true;
-    case 64: group_shape_of<Real, 64>(cap, lanes, B, lds); return true;
-    case 96: group_shape_of<Real, 96>(cap, lanes, B, lds); return true;
-    case 128: group_shape_of<Real, 128>(cap, lanes, B, lds); return true;
-    case 160: group_shape_of<Real, 160>(cap, lanes, B, lds); return true;
-    case 256: group_shape_of<Real, 256>(cap, lanes, B, lds); return true;
+    case 16: group_shape_of<Real, 16>(cap, lanes, across, g); return true;
+    case 32: group_shape_of<Real, 32>(cap, lanes, across, g); return true;
+    case 64: group_shape_of<Real, 64>(cap, lanes, across, g); return true;
+    case 96: group_shape_of<Real, 96>(cap, lanes, across, g); return true;
+    case 128: group_shape_of<Real, 128>(cap, lanes, across, g); return true;
+    case 160: group_shape_of<Real, 160>(cap, lanes, across, g); return true;
+    case 256: group_shape_of<Real, 256>(cap, lanes, across, g); return true;
     default: return false;
   }
 }
-}  // namespace
-
-namespace {
 // two lines per lane: pairs = lanes / T, lines = 2 * pairs, LDS for the
 // lines and the two spare slots (real / imaginary halves of each line)
-template <int N> void group_dual_shape_of(size_t cap, int* B, size_t* lds) {
+template <int N> void group_dual_shape_of(size_t cap, GroupShape* g) {
   using Cfg = FastCfg<float, N, 8>;
-  const size_t line_bytes = dual_line_bytes<float, N, 8>();
-  if (cap > kGroupLds) cap = kGroupLds;
   int pairs = kGroupThreads / Cfg::T;
-  while (pairs > 1 && static_cast<size_t>(2 * pairs + 2) * line_bytes > cap) --pairs;
-  *B = 2 * pairs;
-  *lds = static_cast<size_t>(2 * pairs + 2) * line_bytes;
+  const size_t line = dual_stride(dual_line_bytes<float, N, 8>(), 2 * pairs);
+  if (cap > kGroupLds) cap = kGroupLds;
+  while (pairs > 1 && static_cast<size_t>(2 * pairs + 2) * line > cap) --pairs;
+  g->lines_per_block = 2 * pairs;
+  g->line_bytes = static_cast<int>(line);
+  g->lds_bytes = static_cast<size_t>(2 * pairs + 2) * line;
 }
 }  // namespace
 
-bool group_dual_shape(int n, size_t lds_cap, int* lines_per_block, size_t* lds_bytes) {
+bool group_dual_shape(int n, size_t lds_cap, GroupShape* g) {
   switch (n) {
-    case 64: group_dual_shape_of<64>(lds_cap, lines_per_block, lds_bytes); return true;
-    case 96: group_dual_shape_of<96>(lds_cap, lines_per_block, lds_bytes); return true;
-    case 128: group_dual_shape_of<128>(lds_cap, lines_per_block, lds_bytes); return true;
-    case 160: group_dual_shape_of<160>(lds_cap, lines_per_block, lds_bytes); return true;
-    case 256: group_dual_shape_of<256>(lds_cap, lines_per_block, lds_bytes); return true;
+    case 64: group_dual_shape_of<64>(lds_cap, g); return true;
+    case 96: group_dual_shape_of<96>(lds_cap, g); return true;
+    case 128: group_dual_shape_of<128>(lds_cap, g); return true;
+    case 160: group_dual_shape_of<160>(lds_cap, g); return true;
+    case 256: group_dual_shape_of<256>(lds_cap, g); return true;
     default: return false;
   }
 }
 
 bool dual_lines_apply(const LinePass& p, int lines_per_block) { return dual_lines_apply_impl(p, lines_per_block); }
 
-bool group_line_shape(int n, bool fp64, size_t lds_cap, int lanes, int* lines_per_block, size_t* lds_bytes) {
+bool group_line_shape(int n, bool fp64, size_t lds_cap, int lanes, bool across, GroupShape* g) {
   if (lanes != 64 && lanes != 128 && lanes != kGroupThreads) return false;
-  return fp64 ? group_shape<double>(n, lds_cap, lanes, lines_per_block, lds_bytes)
-              : group_shape<float>(n, lds_cap, lanes, lines_per_block, lds_bytes);
+  return fp64 ? group_shape<double>(n, lds_cap, lanes, across, g) : group_shape<float>(n, lds_cap, lanes, across, g);
 }
 
 int group_grid(size_t lds_bytes, bool fp64, bool dual, int lanes) {
@@ -700,6 +699,7 @@ FastPass fast_pass(const LinePass& p, bool fp64) {
   f.pad_real = p.pad_real > 0 ? p.pad_real : INT32_MAX;  // padded axes are the fastest batch axis
   f.band = p.band;
   f.dual_split = p.dual_split;
+  f.line_bytes = p.line_bytes;
   const int first = kMaxDim - 1 - p.nbatch;
   for (int j = 0; j < kMaxDim - 1; ++j) {
     const bool used = j >= first;

@@ -30,6 +30,7 @@ struct LinePass {
   int32_t lines_per_block;              // 0: launcher heuristic
   int32_t values_per_thread;            // 0: default (8); compile-time kernels exist for 4, 8, 16,
                                         // the runtime-radix kernel takes it as an upper bound
+  int32_t line_bytes;                   // LDS bytes from a line's buffer to the next (set by launchers)
   int32_t fit_block;                    // 1: lines_per_block is a default the launcher may halve to fit
   const void* tw;                       // exp(-2 pi i e / n), e in [0, n), Real precision
   double scale;
@@ -131,6 +132,7 @@ struct FastPass {
   int32_t inverse, lines_fast, lines_per_block, xcd_remap;
   int32_t swizzle, pad_real;  // pad_real: lines whose index along the fastest batch axis is >= it are padding
   int32_t band, dual_split;
+  int32_t line_bytes;
   int32_t ext[3];         // batch axes, slowest first; unused ones come first with extent 1
   int32_t band_shift[3];
   FastDiv div[3];
@@ -161,12 +163,18 @@ struct RemapArgs {
 constexpr int kGroupThreads = 256;
 constexpr size_t kGenericLdsMax = 160 * 1024;  // LDS of one gfx950 workgroup
 constexpr size_t kGroupLds = 64 * 1024;  // dynamic LDS of a grouped launch, at most
-// lines per block and dynamic LDS bytes of the grouped kernel for length n
-// in blocks of `lanes` lanes (64, 128 or kGroupThreads) with at most lds_cap
-// bytes of LDS per block; false if n has no grouped kernel
-bool group_line_shape(int n, bool fp64, size_t lds_cap, int lanes, int* lines_per_block, size_t* lds_bytes);
+// lines per block, LDS bytes from line to line and dynamic LDS bytes of the
+// grouped kernel for length n in blocks of `lanes` lanes (64, 128 or
+// kGroupThreads, across the lines or along them) with at most lds_cap bytes of
+// LDS per block; false if n has no grouped kernel
+struct GroupShape {
+  int lines_per_block = 0;
+  int line_bytes = 0;
+  size_t lds_bytes = 0;
+};
+bool group_line_shape(int n, bool fp64, size_t lds_cap, int lanes, bool across, GroupShape* g);
 // the same for FP32 lines taken two per lane (false if n has no such kernel)
-bool group_dual_shape(int n, size_t lds_cap, int* lines_per_block, size_t* lds_bytes);
+bool group_dual_shape(int n, size_t lds_cap, GroupShape* g);
 // true if two adjacent lines per lane apply to pass p with that many lines per
 // block (FP32 C2C, lanes across lines, consecutive lines adjacent row
 // elements on both sides, 16-byte aligned rank buffers; grouped passes)

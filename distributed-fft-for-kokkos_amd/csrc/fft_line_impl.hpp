@@ -13,6 +13,7 @@
 
 #include "fft_kernels.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <mutex>
@@ -447,49 +448,86 @@ template <typename Real, int N, int RM, int S> struct StageTwiddles {
   using Cfg = FastCfg<Real, N, RM>;
   static constexpr int r = Cfg::P.rad[S];
   static constexpr int L = span_before(N, S);
+  static constexpr int T = Cfg::T;
   static constexpr int NB = Cfg::R / r;
   static constexpr int ts = N / (L * r);
-  static constexpr bool kAhead = L > 1 && NB <= 4;
-  // more entries per lane (the last radix-2 stage of 16 values per thread):
-  // when NB divides L they are the consecutive entries k0 .. k0 + NB - 1,
-  // k0 = t*NB mod L, and entry k0 + q is entry k0 times entry q, the same for
-  // every lane (a scalar load): one entry per lane is loaded ahead
-  static constexpr bool kBase = L > 1 && NB > 4 && L % NB == 0;
+  // butterfly q of lane t is beta = t + q*T and needs entry beta mod L: where L
+  // divides T that is the same one for every q
+  static constexpr bool kShared = L > 1 && T % L == 0;
+  static constexpr bool kAhead = L > 1 && !kShared && NB <= 4;
+  // more entries per lane (the last radix-2 stage of 16-value lanes): where T
+  // divides L, entry (t + q*T) mod L is entry t times entry q*T mod L, the
+  // same for every lane (a scalar load): one entry per lane is loaded ahead
+  static constexpr bool kBase = L > 1 && !kShared && NB > 4 && L % T == 0;
   double2 w[kAhead ? NB : 1];
   __device__ __forceinline__ void load(int t, const double2* tw) {
     if constexpr (kAhead) {
 #pragma unroll
-      for (int q = 0; q < NB; ++q) w[q] = twiddle_load(tw + ((t * NB + q) % L) * ts);
-    } else if constexpr (kBase) {
-      w[0] = twiddle_load(tw + ((t * NB) % L) * ts);
+      for (int q = 0; q < NB; ++q) w[q] = twiddle_load(tw + entry(t, q) * ts);
+    } else if constexpr (kBase || kShared) {
+      w[0] = twiddle_load(tw + entry(t, 0) * ts);
     }
+  }
+  // (t + q*T) mod L: T divides L or L divides T
+  __device__ static __forceinline__ unsigned entry(int t, int q) {
+    return T % L == 0 ? static_cast<unsigned>(t) % L : static_cast<unsigned>(t) + q * T % L;
   }
   __device__ __forceinline__ double2 get(int t, const double2* tw, int q) const {
     if constexpr (kAhead) return w[q];
-    else if constexpr (kBase) return q == 0 ? w[0] : cmul(w[0], twiddle_load(tw + q * ts));
-    else return twiddle_load(tw + ((t * NB + q) % L) * ts);
+    else if constexpr (kShared) return w[0];
+    else if constexpr (kBase) return q * T % L == 0 ? w[0] : cmul(w[0], twiddle_load(tw + (q * T % L) * ts));
+    else return twiddle_load(tw + entry(t, q) * ts);
   }
 };
+
+// Multiplies the lane's values by the stage's twiddles; `sets` register sets
+// of the same positions.  Where every butterfly of the lane has the same
+// twiddles each power is formed once and used up before the next (all powers
+// held over the lane's butterflies spilled the two-line kernel of 16 values).
+template <typename Real, int N, int RM, int S, int SETS>
+__device__ __forceinline__ void stage_twiddle(cplx_t<Real>* const (&v)[SETS], int t, const double2* tw,
+                                              const StageTwiddles<Real, N, RM, S>& pre) {
+  using C = cplx_t<Real>;
+  using Tw = StageTwiddles<Real, N, RM, S>;
+  constexpr int r = Tw::r, NB = Tw::NB;
+  if constexpr (Tw::L > 1) {
+    if constexpr (Tw::kShared) {
+      double2 pw[8];
+      twiddle_powers<r>(pre.get(t, tw, 0), pw);
+#pragma unroll
+      for (int j = 1; j < r; ++j) {
+        const C w = to_prec<C>(pw[j]);
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+#pragma unroll
+          for (int k = 0; k < SETS; ++k) v[k][q * r + j] = cmul(v[k][q * r + j], w);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        double2 pw[8];
+        twiddle_powers<r>(pre.get(t, tw, q), pw);
+#pragma unroll
+        for (int j = 1; j < r; ++j) {
+          const C w = to_prec<C>(pw[j]);
+#pragma unroll
+          for (int k = 0; k < SETS; ++k) v[k][q * r + j] = cmul(v[k][q * r + j], w);
+        }
+      }
+    }
+  }
+}
 
 template <typename Real, int N, int RM, int S>
 __device__ __forceinline__ void stage_compute(cplx_t<Real>* v, int t, const double2* tw,
                                               const StageTwiddles<Real, N, RM, S>& pre) {
   using Cfg = FastCfg<Real, N, RM>;
-  using C = cplx_t<Real>;
   constexpr int r = Cfg::P.rad[S];
-  constexpr int L = span_before(N, S);
-  constexpr int R = Cfg::R;
-  constexpr int NB = R / r;
+  cplx_t<Real>* const set[1] = {v};
+  stage_twiddle<Real, N, RM, S, 1>(set, t, tw, pre);
 #pragma unroll
-  for (int q = 0; q < NB; ++q) {
-    if constexpr (L > 1) {
-      double2 pw[8];
-      twiddle_powers<r>(pre.get(t, tw, q), pw);
-#pragma unroll
-      for (int j = 1; j < r; ++j) v[q * r + j] = cmul(v[q * r + j], to_prec<C>(pw[j]));
-    }
-    bfly<r>(v + q * r);
-  }
+  for (int q = 0; q < Cfg::R / r; ++q) bfly<r>(v + q * r);
 }
 
 // Bytes of one line's LDS buffer: LDSN complex values, or LDSN reals when
@@ -498,100 +536,120 @@ template <typename Real, int N, int RM, bool SPLIT> constexpr size_t line_lds_by
   return static_cast<size_t>(FastCfg<Real, N, RM>::LDSN) * (SPLIT ? sizeof(Real) : sizeof(cplx_t<Real>));
 }
 
-// Line buffer of the two-lines-per-lane kernel (reals): LDSN plus a pad
-// measured per length.  1024-point FP32 lines: one more float per line moves
-// the 16 line buffers a wave touches onto different banks (lane pairs read
-// and write 4 positions of each of 16 lines per access); the y pass of a
-// 1024^3 R2C plan took 1.80 instead of 2.08 ms with it, while the same pad
-// made 512-point lines 5-8 % slower.
-template <typename Real, int N> constexpr int dual_lds_extra() {
-  return (sizeof(Real) == 4 && N == 1024) ? 1 : 0;
-}
 template <typename Real, int N, int RM> constexpr size_t dual_line_bytes() {
-  return static_cast<size_t>(FastCfg<Real, N, RM>::LDSN + dual_lds_extra<Real, N>()) * sizeof(Real);
+  return static_cast<size_t>(FastCfg<Real, N, RM>::LDSN) * sizeof(Real);
 }
 
-// Register <-> LDS permutation of one line: every lane stores its values
-// v[q*RW + j] at positions wpos(q, j), then loads v[q*RR + j] from positions
-// rpos(q, j) (NW*RW = NR*RR = R).  SPLIT moves the real parts first and the
-// imaginary parts second through a buffer of reals: after the first half a
-// lane's old real parts are in LDS and can be overwritten, its old imaginary
-// parts are still in registers for the second half.
-template <typename Real, int N, int RM, bool SPLIT, int NW, int RW, int NR, int RR, typename WPos, typename RPos>
-__device__ __forceinline__ void lds_permute(cplx_t<Real>* v, void* line, WPos wpos, RPos rpos) {
+// LDS bytes from one line buffer to the next.  A cycle serves 128 bytes, 16
+// lanes of 8 or 32 of 4: lanes that access one position of `across`
+// neighbouring buffers together should lie 128 / across bytes apart (mod
+// `cycle`).  Buffers of n + n/8 + 1 reals alone left 61 % of the LDS cycles of
+// a strided 256-point FP64 pass in bank conflicts.  Lines below 256 bytes stay
+// as they are.
+inline size_t bank_stride(size_t bytes, int elem, int across, int cycle = 128) {
+  if (bytes < 256 || across <= 1) return bytes;
+  const size_t want = static_cast<size_t>(std::max(elem, 128 / across / elem * elem) % cycle);
+  while (bytes % static_cast<size_t>(cycle) != want) bytes += static_cast<size_t>(elem);
+  return bytes;
+}
+// lanes across the lines: B buffers share a position; along them: a line's T
+// lanes cover T elements of the 128 bytes
+inline size_t line_stride(size_t bytes, int elem, bool lanes_across, int B, int T) {
+  return bank_stride(bytes, elem, lanes_across ? B : 128 / std::min(128, T * elem));
+}
+// two lines per lane: neighbouring lanes access every second buffer
+inline size_t dual_stride(size_t bytes, int B) { return bank_stride(bytes, 4, B, 64); }
+
+// LDS positions of the exchange after stage S.  Lane t writes the outputs of
+// its butterflies t + q*T, (beta / L) L r + beta % L + j L, and reads the inputs
+// t + q*T + j*(N/r2) of stage S + 1.  T divides L or L divides T, so each is a
+// position of the lane plus a constant of (q, j), and the padding of the two
+// adds up (the constant never carries into the lane's part): one index per
+// lane and immediate offsets.
+template <typename Real, int N, int RM, int S> struct Exchange {
   using Cfg = FastCfg<Real, N, RM>;
+  static constexpr int R = Cfg::R, T = Cfg::T;
+  static constexpr int r = Cfg::P.rad[S], L = span_before(N, S), NB = R / r;
+  static constexpr int r2 = Cfg::P.rad[S + 1], NB2 = R / r2;
+  static_assert(T % L == 0 || L % T == 0, "butterflies of a lane");
+  static constexpr int padded(int c) { return c + (c >> LdsPad<Real>::shift); }
+  __device__ static __forceinline__ int write_base(unsigned t) {
+    return Cfg::lidx(static_cast<int>(T % L == 0 ? t / L * (L * r) + t % L : t));
+  }
+  static constexpr int write_at(int q, int j) {
+    return padded((T % L == 0 ? q * T * r : q * T / L * (L * r) + q * T % L) + j * L);
+  }
+  __device__ static __forceinline__ int read_base(unsigned t) { return Cfg::lidx(static_cast<int>(t)); }
+  static constexpr int read_at(int q, int j) { return padded(q * T + j * (N / r2)); }
+};
+
+// Write the outputs of stage S, read the inputs of stage S+1.  SPLIT moves the
+// real parts first and the imaginary parts second through a buffer of reals:
+// after the first half a lane's old real parts are in LDS and can be
+// overwritten, its old imaginary parts are still in registers for the second
+// half.
+template <typename Real, int N, int RM, bool SPLIT, int S>
+__device__ __forceinline__ void stage_exchange(cplx_t<Real>* v, int t, void* line) {
+  using X = Exchange<Real, N, RM, S>;
+  const int wb = X::write_base(static_cast<unsigned>(t)), rb = X::read_base(static_cast<unsigned>(t));
   if constexpr (SPLIT) {
-    Real* lr = static_cast<Real*>(line);
+    Real* lw = static_cast<Real*>(line) + wb;
+    const Real* lr = static_cast<const Real*>(line) + rb;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       __syncthreads();
 #pragma unroll
-      for (int q = 0; q < NW; ++q) {
+      for (int q = 0; q < X::NB; ++q) {
 #pragma unroll
-        for (int j = 0; j < RW; ++j) lr[Cfg::lidx(wpos(q, j))] = h ? v[q * RW + j].y : v[q * RW + j].x;
+        for (int j = 0; j < X::r; ++j) lw[X::write_at(q, j)] = h ? v[q * X::r + j].y : v[q * X::r + j].x;
       }
       __syncthreads();
 #pragma unroll
-      for (int q = 0; q < NR; ++q) {
+      for (int q = 0; q < X::NB2; ++q) {
 #pragma unroll
-        for (int j = 0; j < RR; ++j) {
-          const Real x = lr[Cfg::lidx(rpos(q, j))];
+        for (int j = 0; j < X::r2; ++j) {
+          const Real x = lr[X::read_at(q, j)];
           if (h) {
-            v[q * RR + j].y = x;
+            v[q * X::r2 + j].y = x;
           } else {
-            v[q * RR + j].x = x;
+            v[q * X::r2 + j].x = x;
           }
         }
       }
     }
   } else {
-    cplx_t<Real>* lc = static_cast<cplx_t<Real>*>(line);
+    cplx_t<Real>* lw = static_cast<cplx_t<Real>*>(line) + wb;
+    const cplx_t<Real>* lr = static_cast<const cplx_t<Real>*>(line) + rb;
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NW; ++q) {
+    for (int q = 0; q < X::NB; ++q) {
 #pragma unroll
-      for (int j = 0; j < RW; ++j) lc[Cfg::lidx(wpos(q, j))] = v[q * RW + j];
+      for (int j = 0; j < X::r; ++j) lw[X::write_at(q, j)] = v[q * X::r + j];
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NR; ++q) {
+    for (int q = 0; q < X::NB2; ++q) {
 #pragma unroll
-      for (int j = 0; j < RR; ++j) v[q * RR + j] = lc[Cfg::lidx(rpos(q, j))];
+      for (int j = 0; j < X::r2; ++j) v[q * X::r2 + j] = lr[X::read_at(q, j)];
     }
   }
 }
 
-// write the outputs of stage S, read the inputs of stage S+1
-template <typename Real, int N, int RM, bool SPLIT, int S>
-__device__ __forceinline__ void stage_exchange(cplx_t<Real>* v, int t, void* line) {
+// After the last stage, of radix rl with NBl butterflies per lane, value
+// q*rl + j is output t + q*T + j*(N/rl) = t + (q + j*NBl)*T: reordered, value
+// k of lane t is output t + k*T.  (With consecutive butterflies t*NBl + q
+// this took one more exchange through LDS, a third of all for 256 points.)
+template <typename Real, int N, int RM> __device__ __forceinline__ void final_order(cplx_t<Real>* v) {
   using Cfg = FastCfg<Real, N, RM>;
-  constexpr int r = Cfg::P.rad[S];
-  constexpr int L = span_before(N, S);
   constexpr int R = Cfg::R;
-  constexpr int NB = R / r;
-  constexpr int r2 = Cfg::P.rad[S + 1];
-  constexpr int NB2 = R / r2;
-  lds_permute<Real, N, RM, SPLIT, NB, r, NB2, r2>(
-      v, line,
-      [t](int q, int j) {
-        const int beta = t * NB + q;
-        return (beta / L) * L * r + beta % L + j * L;
-      },
-      [t](int q, int j) { return t * NB2 + q + j * (N / r2); });
-}
-
-// after the last stage the outputs sit at positions beta + j*(N/rl)
-// (beta = t*(R/rl) + q); regroup them to positions t + j*T
-template <typename Real, int N, int RM, bool SPLIT>
-__device__ __forceinline__ void final_regroup(cplx_t<Real>* v, int t, void* line) {
-  using Cfg = FastCfg<Real, N, RM>;
-  constexpr int R = Cfg::R, T = Cfg::T;
   constexpr int rl = Cfg::P.rad[Cfg::NST - 1];
   if constexpr (rl != R) {
     constexpr int NBl = R / rl;
-    lds_permute<Real, N, RM, SPLIT, NBl, rl, 1, R>(
-        v, line, [t](int q, int j) { return t * NBl + q + j * (N / rl); },
-        [t](int, int j) { return t + j * T; });
+    cplx_t<Real> u[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) u[k] = v[(k % NBl) * rl + k / NBl];
+#pragma unroll
+    for (int k = 0; k < R; ++k) v[k] = u[k];
   }
 }
 
@@ -625,58 +683,46 @@ template <typename Real, int N, int RM, int S>
 __device__ __forceinline__ void stage_compute2(cplx_t<Real>* va, cplx_t<Real>* vb, int t, const double2* tw,
                                                const StageTwiddles<Real, N, RM, S>& pre) {
   using Cfg = FastCfg<Real, N, RM>;
-  using C = cplx_t<Real>;
   constexpr int r = Cfg::P.rad[S];
-  constexpr int L = span_before(N, S);
-  constexpr int R = Cfg::R;
-  constexpr int NB = R / r;
+  cplx_t<Real>* const set[2] = {va, vb};
+  stage_twiddle<Real, N, RM, S, 2>(set, t, tw, pre);
 #pragma unroll
-  for (int q = 0; q < NB; ++q) {
-    if constexpr (L > 1) {
-      double2 pw[8];
-      twiddle_powers<r>(pre.get(t, tw, q), pw);
-#pragma unroll
-      for (int j = 1; j < r; ++j) {
-        const C w = to_prec<C>(pw[j]);
-        va[q * r + j] = cmul(va[q * r + j], w);
-        vb[q * r + j] = cmul(vb[q * r + j], w);
-      }
-    }
+  for (int q = 0; q < Cfg::R / r; ++q) {
     bfly<r>(va + q * r);
     bfly<r>(vb + q * r);
   }
 }
 
-// lds_permute for the two register sets of a lane (buffers la, lb of reals)
-template <typename Real, int N, int RM, int NW, int RW, int NR, int RR, typename WPos, typename RPos>
-__device__ __forceinline__ void lds_permute2(cplx_t<Real>* va, cplx_t<Real>* vb, Real* la, Real* lb, WPos wpos,
-                                             RPos rpos) {
-  using Cfg = FastCfg<Real, N, RM>;
+// stage_exchange for the two register sets of a lane (buffers la, lb of reals)
+template <typename Real, int N, int RM, int S>
+__device__ __forceinline__ void stage_exchange2(cplx_t<Real>* va, cplx_t<Real>* vb, int t, Real* la, Real* lb) {
+  using X = Exchange<Real, N, RM, S>;
+  const int wb = X::write_base(static_cast<unsigned>(t)), rb = X::read_base(static_cast<unsigned>(t));
+  Real *wa = la + wb, *wl = lb + wb;
+  const Real *ra = la + rb, *rl = lb + rb;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NW; ++q) {
+    for (int q = 0; q < X::NB; ++q) {
 #pragma unroll
-      for (int j = 0; j < RW; ++j) {
-        const int i = Cfg::lidx(wpos(q, j));
-        la[i] = h ? va[q * RW + j].y : va[q * RW + j].x;
-        lb[i] = h ? vb[q * RW + j].y : vb[q * RW + j].x;
+      for (int j = 0; j < X::r; ++j) {
+        wa[X::write_at(q, j)] = h ? va[q * X::r + j].y : va[q * X::r + j].x;
+        wl[X::write_at(q, j)] = h ? vb[q * X::r + j].y : vb[q * X::r + j].x;
       }
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NR; ++q) {
+    for (int q = 0; q < X::NB2; ++q) {
 #pragma unroll
-      for (int j = 0; j < RR; ++j) {
-        const int i = Cfg::lidx(rpos(q, j));
-        const Real xa = la[i], xb = lb[i];
+      for (int j = 0; j < X::r2; ++j) {
+        const Real xa = ra[X::read_at(q, j)], xb = rl[X::read_at(q, j)];
         if (h) {
-          va[q * RR + j].y = xa;
-          vb[q * RR + j].y = xb;
+          va[q * X::r2 + j].y = xa;
+          vb[q * X::r2 + j].y = xb;
         } else {
-          va[q * RR + j].x = xa;
-          vb[q * RR + j].x = xb;
+          va[q * X::r2 + j].x = xa;
+          vb[q * X::r2 + j].x = xb;
         }
       }
     }
@@ -692,24 +738,11 @@ template <typename Real, int N, int RM, int S> struct StageLoop2 {
   }
   __device__ static __forceinline__ void run(cplx_t<Real>* va, cplx_t<Real>* vb, int t, const double2* tw, Real* la,
                                              Real* lb, const StageTwiddles<Real, N, RM, S>& pre) {
-    using Cfg = FastCfg<Real, N, RM>;
     stage_compute2<Real, N, RM, S>(va, vb, t, tw, pre);
-    if constexpr (S + 1 < Cfg::NST) {
+    if constexpr (S + 1 < FastCfg<Real, N, RM>::NST) {
       StageTwiddles<Real, N, RM, S + 1> next;
       next.load(t, tw);
-      constexpr int r = Cfg::P.rad[S];
-      constexpr int L = span_before(N, S);
-      constexpr int R = Cfg::R;
-      constexpr int NB = R / r;
-      constexpr int r2 = Cfg::P.rad[S + 1];
-      constexpr int NB2 = R / r2;
-      lds_permute2<Real, N, RM, NB, r, NB2, r2>(
-          va, vb, la, lb,
-          [t](int q, int j) {
-            const int beta = t * NB + q;
-            return (beta / L) * L * r + beta % L + j * L;
-          },
-          [t](int q, int j) { return t * NB2 + q + j * (N / r2); });
+      stage_exchange2<Real, N, RM, S>(va, vb, t, la, lb);
       StageLoop2<Real, N, RM, S + 1>::run(va, vb, t, tw, la, lb, next);
     }
   }
@@ -725,7 +758,7 @@ __device__ __forceinline__ void fast_line2_body(const FastPass& p, int32_t blk, 
   using Cfg = FastCfg<Real, N, RM>;
   typedef Real V4 __attribute__((ext_vector_type(4)));
   constexpr int R = Cfg::R, T = Cfg::T;
-  constexpr size_t LB = dual_line_bytes<Real, N, RM>();
+  const size_t LB = static_cast<size_t>(p.line_bytes);
   const int P2 = B >> 1;
   const int tid = threadIdx.x;
   // lanes beyond P2*T (grouped launches of 256 lanes) run the stages on zeros
@@ -755,12 +788,12 @@ __device__ __forceinline__ void fast_line2_body(const FastPass& p, int32_t blk, 
   constexpr int NB0 = R / r0;
 #pragma unroll
   for (int q = 0; q < NB0; ++q) {
-    const C* src = reinterpret_cast<const C*>(io.ib) + static_cast<int64_t>(t * NB0 + q) * io.is;
+    const C* src = reinterpret_cast<const C*>(io.ib) + static_cast<int64_t>(t + q * T) * io.is;
     const int64_t step = static_cast<int64_t>(N / r0) * io.is;
     [[maybe_unused]] const C* src2 = nullptr;
     [[maybe_unused]] int64_t step2 = 0;
     if constexpr (SPLIT_IN == 2) {
-      src2 = reinterpret_cast<const C*>(io2.ib) + static_cast<int64_t>(t * NB0 + q) * io2.is;
+      src2 = reinterpret_cast<const C*>(io2.ib) + static_cast<int64_t>(t + q * T) * io2.is;
       step2 = static_cast<int64_t>(N / r0) * io2.is;
     }
 #pragma unroll
@@ -784,13 +817,8 @@ __device__ __forceinline__ void fast_line2_body(const FastPass& p, int32_t blk, 
     }
   }
   StageLoop2<Real, N, RM, 0>::run(va, vb, t, tw, ba, bb);
-  constexpr int rl = Cfg::P.rad[Cfg::NST - 1];
-  if constexpr (rl != R) {
-    constexpr int NBl = R / rl;
-    lds_permute2<Real, N, RM, NBl, rl, 1, R>(
-        va, vb, ba, bb, [t](int q, int j) { return t * NBl + q + j * (N / rl); },
-        [t](int, int j) { return t + j * T; });
-  }
+  final_order<Real, N, RM>(va);
+  final_order<Real, N, RM>(vb);
   // SPLIT_IN == 2: the pair is stored as one 16-byte element pair where the
   // second line's output follows the first's on a 16-byte boundary at every
   // position (even element stride), else as two elements
@@ -866,7 +894,7 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
   }
   const int32_t line = blk * B + b;
   const double2* tw = reinterpret_cast<const double2*>(p.tw);
-  void* buf = lds + b * line_lds_bytes<Real, N, RM, SPLIT>();
+  void* buf = lds + b * p.line_bytes;
 
   bool valid;
   LineIO<Real, NT> io;
@@ -911,7 +939,7 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
       for (int q = 0; q < NB0; ++q) {
 #pragma unroll
         for (int j = 0; j < r0; ++j) {
-          const C x = lc[Cfg::lidx(t * NB0 + q + j * (N / r0))];
+          const C x = lc[Cfg::lidx(t + q * T + j * (N / r0))];
           v[q * r0 + j] = p.inverse ? cconj(x) : x;
         }
       }
@@ -932,7 +960,7 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
         if (j * S > p.band && (j + 1) * S - 1 < N - p.band) continue;
 #pragma unroll
         for (int q = 0; q < NB0; ++q) {
-          const int pos = t * NB0 + q + j * S;
+          const int pos = t + q * T + j * S;
           const bool keep = pos <= p.band || pos >= N - p.band;
           const C x = gload_c<NT, Real>(reinterpret_cast<const C*>(io.ib) +
                                         static_cast<int64_t>(keep ? pos : p.band) * io.is);
@@ -948,7 +976,7 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
     if (valid) {
 #pragma unroll
       for (int q = 0; q < NB0; ++q) {
-        const C* src = reinterpret_cast<const C*>(io.ib) + static_cast<int64_t>(t * NB0 + q) * io.is;
+        const C* src = reinterpret_cast<const C*>(io.ib) + static_cast<int64_t>(t + q * T) * io.is;
         const int64_t step = static_cast<int64_t>(N / r0) * io.is;
 #pragma unroll
         for (int j = 0; j < r0; ++j) {
@@ -970,13 +998,13 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
 #pragma unroll
       for (int q = 0; q < NB0; ++q) {
 #pragma unroll
-        for (int j = 0; j < r0; ++j) v[q * r0 + j] = io.template load_kind<kR2C>(t * NB0 + q + j * (N / r0));
+        for (int j = 0; j < r0; ++j) v[q * r0 + j] = io.template load_kind<kR2C>(t + q * T + j * (N / r0));
       }
     } else {
 #pragma unroll
       for (int q = 0; q < NB0; ++q) {
 #pragma unroll
-        for (int j = 0; j < r0; ++j) v[q * r0 + j] = io.template load_kind<kC2R>(t * NB0 + q + j * (N / r0));
+        for (int j = 0; j < r0; ++j) v[q * r0 + j] = io.template load_kind<kC2R>(t + q * T + j * (N / r0));
       }
     }
   } else {
@@ -996,7 +1024,7 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
 #pragma unroll
     for (int q = 0; q < NBl; ++q) {
 #pragma unroll
-      for (int j = 0; j < rl; ++j) lc[Cfg::lidx(t * NBl + q + j * (N / rl))] = v[q * rl + j];
+      for (int j = 0; j < rl; ++j) lc[Cfg::lidx(t + q * T + j * (N / rl))] = v[q * rl + j];
     }
     __syncthreads();
     vout = valid && p.kind == kC2C && io.os == 1 && (reinterpret_cast<uintptr_t>(io.ob) & 15) == 0;
@@ -1022,7 +1050,7 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
       for (int j = 0; j < R; ++j) v[j] = lc[Cfg::lidx(t + j * T)];
     }
   } else {
-    final_regroup<Real, N, RM, SPLIT>(v, t, buf);
+    final_order<Real, N, RM>(v);
   }
 
   if (valid && !vout) {
@@ -1080,7 +1108,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
   const int32_t pair = blk * B + b;
   const bool valid = active && 2 * pair < p.nlines;  // paired passes never enumerate padding
   const double2* tw = reinterpret_cast<const double2*>(p.tw);
-  void* buf = lds + b * line_lds_bytes<Real, N, RM, SPLIT>();
+  void* buf = lds + b * p.line_bytes;
 
   PairIO<Real, NT> io{};
   if (T >= 64 && !p.lines_fast) {
@@ -1103,7 +1131,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
   [[maybe_unused]] int pq = 0;
   if constexpr (PROD) {
     pq = b % 3;
-    Real* st = reinterpret_cast<Real*>(lds + (b - pq) * line_lds_bytes<Real, N, RM, SPLIT>());
+    Real* st = reinterpret_cast<Real*>(lds + (b - pq) * p.line_bytes);
     if (valid) {
       const Real* src = reinterpret_cast<const Real*>(io.ib[0]) + static_cast<int64_t>(t) * io.is[0];
       const int64_t step = static_cast<int64_t>(T) * io.is[0];
@@ -1129,7 +1157,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
     const int64_t sa = static_cast<int64_t>(S) * io.is[0], sb = static_cast<int64_t>(S) * io.is[1];
 #pragma unroll
     for (int q = 0; q < NB0; ++q) {
-      const int beta = t * NB0 + q;
+      const int beta = t + q * T;
       if (p.kind == kR2C) {
         const Real* pa = reinterpret_cast<const Real*>(io.ib[0]) + static_cast<int64_t>(beta) * io.is[0];
         const Real* pb = reinterpret_cast<const Real*>(io.ib[1]) + static_cast<int64_t>(beta) * io.is[1];
@@ -1220,7 +1248,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
           for (int q = 0; q < NB0; ++q) {
 #pragma unroll
             for (int j = 0; j < r0; ++j) {
-              const int pos = t * NB0 + q + j * S;
+              const int pos = t + q * T + j * S;
               if (pos > 0 && 2 * pos < N) lr[Cfg::lidx(N - pos)] = h ? mirror[q * r0 + j].y : mirror[q * r0 + j].x;
             }
           }
@@ -1229,7 +1257,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
           for (int q = 0; q < NB0; ++q) {
 #pragma unroll
             for (int j = 0; j < r0; ++j) {
-              const int pos = t * NB0 + q + j * S;
+              const int pos = t + q * T + j * S;
               if (2 * pos > N) {
                 const Real x = lr[Cfg::lidx(pos)];
                 if (h) {
@@ -1247,7 +1275,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
         for (int q = 0; q < NB0; ++q) {
 #pragma unroll
           for (int j = 0; j < r0; ++j) {
-            const int pos = t * NB0 + q + j * S;
+            const int pos = t + q * T + j * S;
             if (pos > 0 && 2 * pos < N) lc[Cfg::lidx(N - pos)] = mirror[q * r0 + j];
           }
         }
@@ -1256,7 +1284,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
         for (int q = 0; q < NB0; ++q) {
 #pragma unroll
           for (int j = 0; j < r0; ++j) {
-            const int pos = t * NB0 + q + j * S;
+            const int pos = t + q * T + j * S;
             if (2 * pos > N) v[q * r0 + j] = lc[Cfg::lidx(pos)];
           }
         }
@@ -1265,7 +1293,7 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
   }
   if constexpr (PROD) __syncthreads();  // the staged lines share LDS with the exchanges
   StageLoop<Real, N, RM, SPLIT, 0>::run(v, t, tw, buf);
-  final_regroup<Real, N, RM, SPLIT>(v, t, buf);
+  final_order<Real, N, RM>(v);
   const int64_t ta = static_cast<int64_t>(T) * io.os[0], tb = static_cast<int64_t>(T) * io.os[1];
   if (p.kind == kC2R) {
     // w = FFT(conj Z) at each position, so a + i b = conj(w)
@@ -1549,7 +1577,10 @@ hipError_t launch_dual(LinePass p, int B, hipStream_t s) {
     using Cfg = FastCfg<Real, N, RM>;
     constexpr int T = Cfg::T;
     const int P2 = B / 2;
-    const size_t smem = static_cast<size_t>(B) * dual_line_bytes<Real, N, RM>();
+    size_t line = dual_stride(dual_line_bytes<Real, N, RM>(), B);
+    if (B * line > 160 * 1024) line = dual_line_bytes<Real, N, RM>();
+    p.line_bytes = static_cast<int32_t>(line);
+    const size_t smem = B * line;
     if (P2 * T > 1024 || smem > 160 * 1024) return hipErrorInvalidConfiguration;
     p.lines_per_block = B;
     static std::atomic<size_t> lds_limit[6] = {64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024};
@@ -1611,6 +1642,7 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
   }
   const bool split = split_available<Real, N>() && p.split_lds != 0;
   const size_t line_bytes = split ? line_lds_bytes<Real, N, RM, true>() : line_lds_bytes<Real, N, RM, false>();
+  const int elem = static_cast<int>(split ? sizeof(Real) : sizeof(C));
   int B = p.lines_per_block;
   if (B <= 0) {
     if (p.lines_fast) {
@@ -1625,7 +1657,10 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
     while (B > 1 && (B * T > 1024 || static_cast<size_t>(B) * line_bytes > 80 * 1024 ||
                      (B > 4 && B * T > 64 && p.nlines / B < 512)))
       B /= 2;
-  const size_t smem = static_cast<size_t>(B) * line_bytes;
+  size_t line = line_stride(line_bytes, elem, p.lines_fast != 0, B, T);
+  if (B * line > 160 * 1024) line = line_bytes;
+  p.line_bytes = static_cast<int32_t>(line);
+  const size_t smem = B * line;
   if (B * T > 1024 || smem > 160 * 1024) return hipErrorInvalidConfiguration;
   p.lines_per_block = B;
   // two real lines per complex FFT for forward R2C and inverse C2R passes
@@ -1687,6 +1722,7 @@ hipError_t launch_products(LinePass p, hipStream_t s) {
   int B = 3;
   while (B * T < 192 || (B * T) % 64) B += 3;
   while (B > 3 && (B * T > 1024 || static_cast<size_t>(B) * line_bytes > 160 * 1024)) B -= 3;
+  p.line_bytes = static_cast<int32_t>(line_bytes);
   const size_t smem = static_cast<size_t>(B) * line_bytes;
   if (B * T > 1024 || smem > 160 * 1024 || p.nlines % 6 != 0 || p.line_begin % 6 != 0)
     return hipErrorInvalidConfiguration;
@@ -1739,7 +1775,10 @@ hipError_t launch_band(LinePass p, hipStream_t s) {
   }
   if (p.fit_block && !p.products)  // as launch_fast
     while (B > 1 && (B * T > 1024 || (B > 4 && B * T > 64 && p.nlines / B < 512))) B /= 2;
-  const size_t smem = static_cast<size_t>(B) * line_bytes;
+  size_t line = p.products ? line_bytes : line_stride(line_bytes, sizeof(Real), p.lines_fast != 0, B, T);
+  if (B * line > 160 * 1024) line = line_bytes;
+  p.line_bytes = static_cast<int32_t>(line);
+  const size_t smem = B * line;
   if (B * T > 1024 || smem > 160 * 1024) return hipErrorInvalidConfiguration;
   p.lines_per_block = B;
   p.swizzle = 0;

@@ -62,22 +62,26 @@ inline std::vector<int> mix_radices(int n) {
 
 // Padding of the exchange after a stage of radix r over L positions: lanes
 // write runs of L positions, one run every L r + pad.  Of the paddings up to
-// an eighth of the run distance (at least one), the one whose runs spread
-// best over the LDS banks: a wave writes 64 reals, `across` of them adjacent
-// for every position, into 64 banks of 4 bytes, 256 bytes a cycle.
+// an eighth of the run distance (at least one), the one with the fewest bank
+// conflicts: a cycle serves 128 bytes, 16 lanes of 8 or 32 of 4, `across` of
+// them adjacent for every position.
 template <typename Real>
 inline int mix_pad(int L, int r, int across) {
-  constexpr int kSlots = 256 / static_cast<int>(sizeof(Real));
-  int best = 0, best_most = 1 << 30;
-  for (int pad = 0; pad <= std::min(std::max(1, L * r / 8), kSlots - 1) && best_most > 64 / kSlots; ++pad) {
-    int hits[kSlots] = {}, most = 0;
-    for (int lane = 0; lane < 64; ++lane) {
-      const int b = lane % across, beta = lane / across;
-      const int at = ((beta / L) * (L * r + pad) + beta % L) * across + b;
-      most = std::max(most, ++hits[at % kSlots]);
+  constexpr int kSlots = 128 / static_cast<int>(sizeof(Real));
+  int best = 0, best_sum = 1 << 30;
+  for (int pad = 0; pad <= std::min(std::max(1, L * r / 8), kSlots - 1) && best_sum > 64 / kSlots; ++pad) {
+    int sum = 0;
+    for (int first = 0; first < 64; first += kSlots) {
+      int hits[kSlots] = {}, most = 0;
+      for (int lane = first; lane < first + kSlots; ++lane) {
+        const int b = lane % across, beta = lane / across;
+        const int at = ((beta / L) * (L * r + pad) + beta % L) * across + b;
+        most = std::max(most, ++hits[at % kSlots]);
+      }
+      sum += most;
     }
-    if (most < best_most) {
-      best_most = most;
+    if (sum < best_sum) {
+      best_sum = sum;
       best = pad;
     }
   }
@@ -166,7 +170,9 @@ hipError_t launch_mixed(LinePass p, hipStream_t s) {
       L *= rad[i];
       most = std::max(most, n + (n / L - 1) * len.pad[i][k]);
     }
-    return most;
+    constexpr int kReal = static_cast<int>(sizeof(Real));
+    return p.lines_fast ? most
+                        : static_cast<int>(line_stride(static_cast<size_t>(most) * kReal, kReal, false, lines, T)) / kReal;
   };
   while (B > 1 && (B * T > 1024 || static_cast<size_t>(B) * ldsn(B) * sizeof(Real) > kGenericLdsMax)) B /= 2;
   const int line = ldsn(B);

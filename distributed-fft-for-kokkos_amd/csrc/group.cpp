@@ -190,16 +190,16 @@ std::vector<LinePass> Group::build_pass(const std::vector<void*>& in, const std:
     p.nlines = static_cast<int32_t>(nl);
     p.line_begin = 0;
     p.lines_fast = axis != m.rank - 1 ? 1 : 0;
-    int B = 0;
-    std::size_t lds = 0;
+    GroupShape g;
     p.values_per_thread = 8;
-    p.lines_per_block = group_line_shape(p.n, fp64_, lds_cap_, kGroupThreads, &B, &lds) ? B : 0;
-    if (!fp64_ && dual_ && kind == kC2C && p.lines_fast && group_dual_shape(p.n, lds_cap_, &B, &lds)) {
+    p.lines_per_block =
+        group_line_shape(p.n, fp64_, lds_cap_, kGroupThreads, p.lines_fast != 0, &g) ? g.lines_per_block : 0;
+    if (!fp64_ && dual_ && kind == kC2C && p.lines_fast && group_dual_shape(p.n, lds_cap_, &g)) {
       LinePass q = p;
       q.dual_lines = 1;
-      if (dual_lines_apply(q, B)) {
+      if (dual_lines_apply(q, g.lines_per_block)) {
         p = q;
-        p.lines_per_block = B;
+        p.lines_per_block = g.lines_per_block;
       }
     }
     passes.push_back(p);
@@ -234,12 +234,11 @@ void Group::build_tables(const std::vector<void*>& in, const std::vector<void*>&
     std::size_t lds[2] = {0, 0};
     bool contiguous = true;  // every one-line member walks its lines with lanes along the line
     for (const LinePass& p : all) {
-      int B = 0;
-      std::size_t l = 0;
+      GroupShape g;
       if (p.nlines == 0) continue;
       const int v = p.dual_lines ? 1 : 0;
-      const bool shaped = v ? group_dual_shape(p.n, lds_cap_, &B, &l)
-                            : group_line_shape(p.n, fp64_, lds_cap_, kGroupThreads, &B, &l);
+      const bool shaped = v ? group_dual_shape(p.n, lds_cap_, &g)
+                            : group_line_shape(p.n, fp64_, lds_cap_, kGroupThreads, p.lines_fast != 0, &g);
       if (shaped) {
         grouped[v].push_back(p);
         if (v == 0 && p.lines_fast) contiguous = false;
@@ -257,15 +256,16 @@ void Group::build_tables(const std::vector<void*>& in, const std::vector<void*>&
       // strided lines keep full blocks (more adjacent lines per access)
       const int lanes = v == 0 && contiguous ? lanes_ : kGroupThreads;
       for (LinePass& p : grouped[v]) {
-        int B = 0;
-        std::size_t l = 0;
-        if (v) group_dual_shape(p.n, lds_cap_, &B, &l);
-        else group_line_shape(p.n, fp64_, lds_cap_, lanes, &B, &l);
+        GroupShape g;
+        if (v) group_dual_shape(p.n, lds_cap_, &g);
+        else group_line_shape(p.n, fp64_, lds_cap_, lanes, p.lines_fast != 0, &g);
+        const int B = g.lines_per_block;
         p.lines_per_block = B;
+        p.line_bytes = g.line_bytes;
         const int64_t nb = first[v].back() + (static_cast<int64_t>(p.nlines) + B - 1) / B;
         if (nb >= (int64_t(1) << 31)) throw Error(DFFT_ERROR_UNSUPPORTED, "too many blocks in one grouped pass");
         first[v].push_back(static_cast<int32_t>(nb));
-        lds[v] = std::max(lds[v], l);
+        lds[v] = std::max(lds[v], g.lds_bytes);
       }
       const std::size_t slot = 2 * k + static_cast<std::size_t>(v);
       t.nt[slot] = v == 0 && contiguous && contig_nt_ >= 0 ? contig_nt_ : nt;
@@ -345,9 +345,8 @@ int Group::num_launches(int direction) const {
     for (const Member& m : members_) {
       if (k >= static_cast<int>(m.fwd_axes.size())) continue;
       const std::vector<int>& order = direction == DFFT_FORWARD ? m.fwd_axes : m.bwd_axes;
-      int B = 0;
-      std::size_t l = 0;
-      if (group_line_shape(static_cast<int>(m.gin[order[k]]), fp64_, lds_cap_, kGroupThreads, &B, &l)) grouped = true;
+      GroupShape g;
+      if (group_line_shape(static_cast<int>(m.gin[order[k]]), fp64_, lds_cap_, kGroupThreads, true, &g)) grouped = true;
       else ++n;
     }
     if (grouped) ++n;
