@@ -266,12 +266,6 @@ template <typename Real, bool NT = false> struct PairIO {
     // conj(A + i B)
     return C{A.x - Bv.y, -(A.y + Bv.x)};
   }
-  // R2C: spectra of both lines at pos <= n/2 from Z_pos and Z_{n-pos}
-  __device__ __forceinline__ void r2c_values(int32_t pos, C zk, C zm, C& A, C& Bv) const {
-    const Real h = Real(0.5) * scale * ((pos != 0 && 2 * pos != n) ? hw : Real(1));
-    A = C{(zk.x + zm.x) * h, (zk.y - zm.y) * h};
-    Bv = C{(zk.y + zm.y) * h, (zm.x - zk.x) * h};
-  }
 };
 
 // Batch indices of a line (slowest axis first).  BAND: a pass over the kept
@@ -1081,16 +1075,18 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
   }
 }
 
-// Paired R2C / C2R: slot b of the block transforms lines 2q and 2q+1
+// Paired R2C / C2R (KIND): slot b of the block transforms lines 2q and 2q+1
 // (q = blk*B + b) as one complex line; same stage code as fast_line_body.
+// Lane t holds positions t + k*T throughout.
 // PROD: a products pass (LinePass::products): each loaded real value is the
 // product of the two factor lines' values at that position.
 // BAND: half-spectrum entries above p.band are neither read (zeros) nor stored.
-template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false, bool BAND = false>
+template <typename Real, int N, int RM, bool NT, bool SPLIT, int KIND, bool PROD = false, bool BAND = false>
 __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, int B, unsigned char* lds) {
   using C = cplx_t<Real>;
   using Cfg = FastCfg<Real, N, RM>;
-  constexpr int R = Cfg::R, T = Cfg::T;
+  constexpr int R = Cfg::R, T = Cfg::T, H = R / 2;
+  static_assert(R % 2 == 0 && (KIND == kR2C || KIND == kC2R), "real lines");
   const int tid = threadIdx.x;
   int b, t;
   if (p.lines_fast) {
@@ -1120,243 +1116,241 @@ __device__ __forceinline__ void fast_pair_body(const FastPass& p, int32_t blk, i
   } else {
     if (valid) io = make_pair_io<Real, NT, PROD, BAND>(p, pair);
   }
+  const bool vb = valid && io.has_b;
 
-  // Products pass: the block holds whole positions (B is a multiple of 3 and
-  // the field axis is enumerated fastest, so slots 3m..3m+2 are the pairs
-  // (0,1), (2,3), (4,5) of one position).  Slot 3m+q stages velocity line q of
-  // the position into the LDS of the position's three slots; each slot then
-  // forms its two product lines from LDS.  Global loads: 3 lines per
-  // position instead of 2 per product line.
-  [[maybe_unused]] const Real* stage = nullptr;
-  [[maybe_unused]] int pq = 0;
+  // LDS index of position t + k*T, and of the mirrored N - t - k*T: both a
+  // lane part and a constant where the padding interval divides T
+  constexpr bool kLinear = T % (1 << LdsPad<Real>::shift) == 0;
+  const int at0 = Cfg::lidx(t), mir0 = Cfg::lidx(N - t);
+  auto at = [&](int k) { return kLinear ? at0 + k * T + (k * T >> LdsPad<Real>::shift) : Cfg::lidx(t + k * T); };
+  auto mir = [&](int k) { return kLinear ? mir0 - k * T - (k * T >> LdsPad<Real>::shift) : Cfg::lidx(N - t - k * T); };
+
+  // input k of lane t (position t + k*T) is value (k % NB0)*r0 + k / NB0 of
+  // the first stage
+  constexpr int r0 = Cfg::P.rad[0];
+  constexpr int NB0 = R / r0;
+  C v[R];
+  auto in = [](int k) { return (k % NB0) * r0 + k / NB0; };
   if constexpr (PROD) {
-    pq = b % 3;
+    // Products pass: the block holds whole positions (B is a multiple of 3 and
+    // the field axis is enumerated fastest, so slots 3m..3m+2 are the pairs
+    // (0,1), (2,3), (4,5) of one position).  Slot 3m+q stages velocity line q
+    // of the position into the LDS of the position's three slots; each slot
+    // then forms its two product lines from LDS.  Global loads: 3 lines per
+    // position instead of 2 per product line.
+    const int pq = b % 3;
     Real* st = reinterpret_cast<Real*>(lds + (b - pq) * p.line_bytes);
     if (valid) {
       const Real* src = reinterpret_cast<const Real*>(io.ib[0]) + static_cast<int64_t>(t) * io.is[0];
       const int64_t step = static_cast<int64_t>(T) * io.is[0];
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
-        st[pq * N + t + j * T] = gload<NT>(src);
+      for (int k = 0; k < R; ++k) {
+        st[pq * N + t + k * T] = gload<NT>(src);
         src += step;
       }
     }
     __syncthreads();
-    stage = st;
-  }
-
-  // line elements are walked with pointer increments (positions beta + j*S
-  // on load, t + j*T on store): no 64-bit product per element
-  C v[R];
-  C mirror[R];  // C2R: input at position n - pos, formed by the lane that loads X[pos]
-  {
-    constexpr int r0 = Cfg::P.rad[0];
-    constexpr int NB0 = R / r0;
-    constexpr int S = N / r0;
-    const bool vb = valid && io.has_b;
-    const int64_t sa = static_cast<int64_t>(S) * io.is[0], sb = static_cast<int64_t>(S) * io.is[1];
+    // pair q = fields 2q, 2q + 1: (0,0) (0,1) | (0,2) (1,1) | (1,2) (2,2)
+    const Real* fa0 = st + prod_first(2 * pq) * N + t;
+    const Real* fa1 = st + prod_second(2 * pq) * N + t;
+    const Real* fb0 = st + prod_first(2 * pq + 1) * N + t;
+    const Real* fb1 = st + prod_second(2 * pq + 1) * N + t;
 #pragma unroll
-    for (int q = 0; q < NB0; ++q) {
-      const int beta = t + q * T;
-      if (p.kind == kR2C) {
-        const Real* pa = reinterpret_cast<const Real*>(io.ib[0]) + static_cast<int64_t>(beta) * io.is[0];
-        const Real* pb = reinterpret_cast<const Real*>(io.ib[1]) + static_cast<int64_t>(beta) * io.is[1];
+    for (int k = 0; k < R; ++k) v[in(k)] = C{fa0[k * T] * fa1[k * T], fb0[k * T] * fb1[k * T]};
+    __syncthreads();  // the staged lines share LDS with the exchanges
+  } else if constexpr (KIND == kR2C) {
 #pragma unroll
-        for (int j = 0; j < r0; ++j) {
-          Real xa, xb;
-          if constexpr (PROD) {
-            const int pos = beta + j * S;
-            const int fa = 2 * pq, fb = 2 * pq + 1;
-            xa = valid ? stage[prod_first(fa) * N + pos] * stage[prod_second(fa) * N + pos] : Real(0);
-            xb = vb ? stage[prod_first(fb) * N + pos] * stage[prod_second(fb) * N + pos] : Real(0);
-          } else {
-            xa = valid ? gload<NT>(pa) : Real(0);
-            xb = vb ? gload<NT>(pb) : Real(0);
-          }
-          v[q * r0 + j] = C{xa, xb};
-          pa += sa;
-          pb += sb;
-        }
-      } else {
-        // C2R: each half-spectrum entry X[m], m <= n/2, is loaded once, by the
-        // lane holding position m; that lane also forms the input at the
-        // mirrored position n - m (from conj X[m]) and hands it over through
-        // LDS below
-        // beta < S, so positions beta + j*S with j < r0/2 are below n/2, the
-        // one with j = r0/2 reaches n/2 only for beta = 0 and the others lie
-        // above: the loads of the first r0/2 positions are unconditional and
-        // sit under one branch per line (a branch per load would wait for
-        // each pair of loads before the next)
-        constexpr int JH = r0 / 2;
-        const C* la = reinterpret_cast<const C*>(io.ib[0]) + static_cast<int64_t>(beta) * io.is[0];
-        const C* lb = reinterpret_cast<const C*>(io.ib[1]) + static_cast<int64_t>(beta) * io.is[1];
-        const bool mid = !BAND && 2 * (beta + JH * S) <= N;
-        C A[JH + 1], Bv[JH + 1];
-#pragma unroll
-        for (int j = 0; j <= JH; ++j) {
-          A[j] = C{Real(0), Real(0)};
-          Bv[j] = C{Real(0), Real(0)};
-        }
-        if constexpr (BAND) {
-          // as in fast_line_body: whole runs above the band are skipped, lanes
-          // beyond its edge repeat the edge's address
-#pragma unroll
-          for (int j = 0; j < JH; ++j) {
-            if (j * S > p.band) continue;
-            const int pos = beta + j * S;
-            const bool keep = pos <= p.band;
-            const int64_t at = keep ? pos : p.band;
-            if (valid) {
-              const C x = gload_c<NT, Real>(reinterpret_cast<const C*>(io.ib[0]) + at * io.is[0]);
-              A[j] = keep ? x : C{Real(0), Real(0)};
-            }
-            if (vb) {
-              const C x = gload_c<NT, Real>(reinterpret_cast<const C*>(io.ib[1]) + at * io.is[1]);
-              Bv[j] = keep ? x : C{Real(0), Real(0)};
-            }
-          }
-        } else {
-          if (valid) {
-#pragma unroll
-            for (int j = 0; j < JH; ++j) A[j] = gload_c<NT, Real>(la + j * sa);
-            if (mid) A[JH] = gload_c<NT, Real>(la + JH * sa);
-          }
-          if (vb) {
-#pragma unroll
-            for (int j = 0; j < JH; ++j) Bv[j] = gload_c<NT, Real>(lb + j * sb);
-            if (mid) Bv[JH] = gload_c<NT, Real>(lb + JH * sb);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j <= JH; ++j) {
-          const int pos = beta + j * S;
-          if (j < JH || mid || BAND) {
-            v[q * r0 + j] = io.c2r_value(pos, true, A[j], Bv[j]);
-            mirror[q * r0 + j] = io.c2r_value(N - pos, false, A[j], Bv[j]);
-          }
-        }
-      }
-    }
-    if (p.kind == kC2R) {
-      // positions above n/2 receive the value formed by the lane holding n - pos
-      if constexpr (SPLIT) {
-        Real* lr = static_cast<Real*>(buf);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (h) __syncthreads();
-#pragma unroll
-          for (int q = 0; q < NB0; ++q) {
-#pragma unroll
-            for (int j = 0; j < r0; ++j) {
-              const int pos = t + q * T + j * S;
-              if (pos > 0 && 2 * pos < N) lr[Cfg::lidx(N - pos)] = h ? mirror[q * r0 + j].y : mirror[q * r0 + j].x;
-            }
-          }
-          __syncthreads();
-#pragma unroll
-          for (int q = 0; q < NB0; ++q) {
-#pragma unroll
-            for (int j = 0; j < r0; ++j) {
-              const int pos = t + q * T + j * S;
-              if (2 * pos > N) {
-                const Real x = lr[Cfg::lidx(pos)];
-                if (h) {
-                  v[q * r0 + j].y = x;
-                } else {
-                  v[q * r0 + j].x = x;
-                }
-              }
-            }
-          }
-        }
-      } else {
-        C* lc = static_cast<C*>(buf);
-#pragma unroll
-        for (int q = 0; q < NB0; ++q) {
-#pragma unroll
-          for (int j = 0; j < r0; ++j) {
-            const int pos = t + q * T + j * S;
-            if (pos > 0 && 2 * pos < N) lc[Cfg::lidx(N - pos)] = mirror[q * r0 + j];
-          }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < NB0; ++q) {
-#pragma unroll
-          for (int j = 0; j < r0; ++j) {
-            const int pos = t + q * T + j * S;
-            if (2 * pos > N) v[q * r0 + j] = lc[Cfg::lidx(pos)];
-          }
-        }
-      }
-    }
-  }
-  if constexpr (PROD) __syncthreads();  // the staged lines share LDS with the exchanges
-  StageLoop<Real, N, RM, SPLIT, 0>::run(v, t, tw, buf);
-  final_order<Real, N, RM>(v);
-  const int64_t ta = static_cast<int64_t>(T) * io.os[0], tb = static_cast<int64_t>(T) * io.os[1];
-  if (p.kind == kC2R) {
-    // w = FFT(conj Z) at each position, so a + i b = conj(w)
+    for (int k = 0; k < R; ++k) v[k] = C{Real(0), Real(0)};
     if (valid) {
-      Real* pa = reinterpret_cast<Real*>(io.ob[0]) + static_cast<int64_t>(t) * io.os[0];
-      Real* pb = reinterpret_cast<Real*>(io.ob[1]) + static_cast<int64_t>(t) * io.os[1];
+      const Real* pa = reinterpret_cast<const Real*>(io.ib[0]) + static_cast<int64_t>(t) * io.is[0];
+      const int64_t sa = static_cast<int64_t>(T) * io.is[0];
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
-        gstore<NT>(pa, v[j].x * io.scale);
-        if (io.has_b) gstore<NT>(pb, -v[j].y * io.scale);
-        pa += ta;
-        pb += tb;
+      for (int k = 0; k < R; ++k) {
+        v[in(k)].x = gload<NT>(pa);
+        pa += sa;
       }
     }
-    return;
-  }
-  // R2C: Z_{n-pos} lives in another lane; exchange the whole line through LDS
-  C w[R];  // w[j] = Z_{(n - pos) mod n} for pos = t + j*T
-  if constexpr (SPLIT) {
-    Real* lr = static_cast<Real*>(buf);
+    if (vb) {
+      const Real* pb = reinterpret_cast<const Real*>(io.ib[1]) + static_cast<int64_t>(t) * io.is[1];
+      const int64_t sb = static_cast<int64_t>(T) * io.is[1];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < R; ++j) lr[Cfg::lidx(t + j * T)] = h ? v[j].y : v[j].x;
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        const int pos = t + j * T;
-        const Real x = lr[Cfg::lidx(pos == 0 ? 0 : N - pos)];
-        if (h) {
-          w[j].y = x;
-        } else {
-          w[j].x = x;
-        }
+      for (int k = 0; k < R; ++k) {
+        v[in(k)].y = gload<NT>(pb);
+        pb += sb;
       }
     }
   } else {
-    C* lc = static_cast<C*>(buf);
-    __syncthreads();
+    // C2R: each half-spectrum entry X[m], m <= n/2, is loaded once, by the
+    // lane holding position m; that lane also forms the input at the mirrored
+    // position n - m (from conj X[m]) and hands it over through LDS.  The
+    // positions of k < R/2 are below n/2, the one of k = R/2 reaches n/2 only
+    // for t = 0; the loads sit under one branch per line (a branch per load
+    // would wait for each pair of loads before the next).
+    C A[H + 1], Bv[H + 1];
 #pragma unroll
-    for (int j = 0; j < R; ++j) lc[Cfg::lidx(t + j * T)] = v[j];
-    __syncthreads();
+    for (int k = 0; k <= H; ++k) {
+      A[k] = C{Real(0), Real(0)};
+      Bv[k] = C{Real(0), Real(0)};
+    }
+    const C* la = reinterpret_cast<const C*>(io.ib[0]) + static_cast<int64_t>(t) * io.is[0];
+    const C* lb = reinterpret_cast<const C*>(io.ib[1]) + static_cast<int64_t>(t) * io.is[1];
+    const int64_t sa = static_cast<int64_t>(T) * io.is[0], sb = static_cast<int64_t>(T) * io.is[1];
+    if constexpr (BAND) {
+      // as in fast_line_body: whole runs above the band are skipped, lanes
+      // beyond its edge repeat the edge's address
+      const C* ea = reinterpret_cast<const C*>(io.ib[0]) + p.band * io.is[0];
+      const C* eb = reinterpret_cast<const C*>(io.ib[1]) + p.band * io.is[1];
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const int pos = t + j * T;
-      w[j] = lc[Cfg::lidx(pos == 0 ? 0 : N - pos)];
+      for (int k = 0; k < H; ++k) {
+        if (k * T > p.band) continue;
+        const bool keep = t + k * T <= p.band;
+        if (valid) {
+          const C x = gload_c<NT, Real>(keep ? la + k * sa : ea);
+          A[k] = keep ? x : C{Real(0), Real(0)};
+        }
+        if (vb) {
+          const C x = gload_c<NT, Real>(keep ? lb + k * sb : eb);
+          Bv[k] = keep ? x : C{Real(0), Real(0)};
+        }
+      }
+    } else {
+      if (valid) {
+#pragma unroll
+        for (int k = 0; k < H; ++k) A[k] = gload_c<NT, Real>(la + k * sa);
+        if (t == 0) A[H] = gload_c<NT, Real>(la + H * sa);
+      }
+      if (vb) {
+#pragma unroll
+        for (int k = 0; k < H; ++k) Bv[k] = gload_c<NT, Real>(lb + k * sb);
+        if (t == 0) Bv[H] = gload_c<NT, Real>(lb + H * sb);
+      }
+    }
+    C mirror[H];
+#pragma unroll
+    for (int k = 0; k <= H; ++k) {
+      v[in(k)] = io.c2r_value(t + k * T, true, A[k], Bv[k]);
+      if (k < H) mirror[k] = io.c2r_value(N - t - k * T, false, A[k], Bv[k]);
+    }
+    // positions above n/2 receive the value formed by the lane holding n - pos
+    if constexpr (SPLIT) {
+      Real* lr = static_cast<Real*>(buf);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (h) __syncthreads();
+#pragma unroll
+        for (int k = 0; k < H; ++k)
+          if (k > 0 || t > 0) lr[mir(k)] = h ? mirror[k].y : mirror[k].x;
+        __syncthreads();
+#pragma unroll
+        for (int k = H; k < R; ++k) {
+          if (k > H || t > 0) {
+            const Real x = lr[at(k)];
+            if (h) {
+              v[in(k)].y = x;
+            } else {
+              v[in(k)].x = x;
+            }
+          }
+        }
+      }
+    } else {
+      C* lc = static_cast<C*>(buf);
+#pragma unroll
+      for (int k = 0; k < H; ++k)
+        if (k > 0 || t > 0) lc[mir(k)] = mirror[k];
+      __syncthreads();
+#pragma unroll
+      for (int k = H; k < R; ++k)
+        if (k > H || t > 0) v[in(k)] = lc[at(k)];
     }
   }
-  if (valid) {
-    C* pa = reinterpret_cast<C*>(io.ob[0]) + static_cast<int64_t>(t) * io.os[0];
-    C* pb = reinterpret_cast<C*>(io.ob[1]) + static_cast<int64_t>(t) * io.os[1];
+  StageLoop<Real, N, RM, SPLIT, 0>::run(v, t, tw, buf);
+  final_order<Real, N, RM>(v);
+  const int64_t ta = static_cast<int64_t>(T) * io.os[0], tb = static_cast<int64_t>(T) * io.os[1];
+  if constexpr (KIND == kC2R) {
+    // w = FFT(conj Z) at each position, so a + i b = conj(w)
+    if (valid) {
+      Real* pa = reinterpret_cast<Real*>(io.ob[0]) + static_cast<int64_t>(t) * io.os[0];
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const int pos = t + j * T;
-      if (BAND ? pos <= p.band : 2 * pos <= N) {
-        C A, Bv;
-        io.r2c_values(pos, v[j], w[j], A, Bv);
-        gstore_c<NT, Real>(pa, A);
-        if (io.has_b) gstore_c<NT, Real>(pb, Bv);
+      for (int k = 0; k < R; ++k) {
+        gstore<NT>(pa, v[k].x * io.scale);
+        pa += ta;
       }
-      pa += ta;
-      pb += tb;
+    }
+    if (vb) {
+      Real* pb = reinterpret_cast<Real*>(io.ob[1]) + static_cast<int64_t>(t) * io.os[1];
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        gstore<NT>(pb, -v[k].y * io.scale);
+        pb += tb;
+      }
+    }
+  } else {
+    // R2C: entry m = t + k*T <= n/2 of both spectra from Z_m and Z_{n-m}.  The
+    // lanes hand out the upper half of Z; Z_0 and Z_{n/2} are their own
+    // mirrors.
+    C A[H + 1], Bv[H + 1];
+    const bool own = t == 0;
+    if constexpr (SPLIT) {
+      Real* lr = static_cast<Real*>(buf);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int k = H; k < R; ++k) lr[at(k)] = h ? v[k].y : v[k].x;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k <= H; ++k) {
+          const Real z = h ? v[k].y : v[k].x;
+          Real m = z;
+          if (k < H) {
+            m = lr[mir(k)];
+            if (k == 0 && own) m = z;
+          }
+          if (h) {
+            A[k].y = z - m;
+            Bv[k].x = z + m;
+          } else {
+            A[k].x = z + m;
+            Bv[k].y = m - z;
+          }
+        }
+      }
+    } else {
+      C* lc = static_cast<C*>(buf);
+      __syncthreads();
+#pragma unroll
+      for (int k = H; k < R; ++k) lc[at(k)] = v[k];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k <= H; ++k) {
+        C m = v[k];
+        if (k < H) {
+          m = lc[mir(k)];
+          if (k == 0 && own) m = v[0];
+        }
+        A[k] = C{v[k].x + m.x, v[k].y - m.y};
+        Bv[k] = C{v[k].y + m.y, m.x - v[k].x};
+      }
+    }
+    const Real h0 = Real(0.5) * io.scale, hw = h0 * io.hw;
+    if (valid) {
+      C* pa = reinterpret_cast<C*>(io.ob[0]) + static_cast<int64_t>(t) * io.os[0];
+#pragma unroll
+      for (int k = 0; k <= H; ++k) {
+        const Real h = k == H || (k == 0 && own) ? h0 : hw;
+        if (BAND ? k < H && t + k * T <= p.band : k < H || own) gstore_c<NT, Real>(pa, C{A[k].x * h, A[k].y * h});
+        pa += ta;
+      }
+    }
+    if (vb) {
+      C* pb = reinterpret_cast<C*>(io.ob[1]) + static_cast<int64_t>(t) * io.os[1];
+#pragma unroll
+      for (int k = 0; k <= H; ++k) {
+        const Real h = k == H || (k == 0 && own) ? h0 : hw;
+        if (BAND ? k < H && t + k * T <= p.band : k < H || own) gstore_c<NT, Real>(pb, C{Bv[k].x * h, Bv[k].y * h});
+        pb += tb;
+      }
     }
   }
 }
@@ -1383,11 +1377,11 @@ __device__ __forceinline__ int32_t pass_block(const FastPass& p, int32_t b, int3
   return b;
 }
 
-template <typename Real, int N, int RM, bool NT, bool SPLIT, bool PROD = false, bool BAND = false>
+template <typename Real, int N, int RM, bool NT, bool SPLIT, int KIND, bool PROD = false, bool BAND = false>
 __global__ void __launch_bounds__(1024) fft_pair_fast(const FastPass p) {
   extern __shared__ unsigned char smem_raw[];
   const int32_t blk = pass_block(p, blockIdx.x, gridDim.x);
-  fast_pair_body<Real, N, RM, NT, SPLIT, PROD, BAND>(p, blk, p.lines_per_block, smem_raw);
+  fast_pair_body<Real, N, RM, NT, SPLIT, KIND, PROD, BAND>(p, blk, p.lines_per_block, smem_raw);
 }
 
 template <typename Real, int N, int RM, bool NT, bool SPLIT, bool BAND = false>
@@ -1429,20 +1423,26 @@ inline hipError_t raise_lds_limit(std::atomic<size_t>& limit, const void* fn, si
 // nontemporal or cached accesses, split or complex LDS exchanges.
 template <typename Real, int N, int RM, bool NT, bool SPLIT> struct FastVariant {
   static constexpr bool kPairs = !(std::is_same<Real, double>::value && (N % 3 == 0 || N % 5 == 0));
-  static const void* fn(bool pair) {
+  // pair: 0 single lines, else kR2C or kC2R
+  static const void* fn(int pair) {
     if constexpr (kPairs) {
-      if (pair) return reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, SPLIT>);
+      if (pair == kR2C) return reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, SPLIT, kR2C>);
+      if (pair == kC2R) return reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, SPLIT, kC2R>);
     }
     return reinterpret_cast<const void*>(&fft_line_fast<Real, N, RM, NT, SPLIT>);
   }
-  static void launch(bool pair, unsigned grid, unsigned threads, size_t smem, hipStream_t s, const LinePass& p) {
+  static void launch(int pair, unsigned grid, unsigned threads, size_t smem, hipStream_t s, const FastPass& f) {
     if constexpr (kPairs) {
-      if (pair) {
-        hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, SPLIT>), dim3(grid), dim3(threads), smem, s, fast_pass(p, sizeof(Real) == 8));
+      if (pair == kR2C) {
+        hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, SPLIT, kR2C>), dim3(grid), dim3(threads), smem, s, f);
+        return;
+      }
+      if (pair == kC2R) {
+        hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, SPLIT, kC2R>), dim3(grid), dim3(threads), smem, s, f);
         return;
       }
     }
-    hipLaunchKernelGGL((fft_line_fast<Real, N, RM, NT, SPLIT>), dim3(grid), dim3(threads), smem, s, fast_pass(p, sizeof(Real) == 8));
+    hipLaunchKernelGGL((fft_line_fast<Real, N, RM, NT, SPLIT>), dim3(grid), dim3(threads), smem, s, f);
   }
 };
 
@@ -1453,8 +1453,8 @@ template <typename Real, int N> constexpr bool split_available() {
 }
 
 template <typename Real, int N, int RM, bool NT>
-void launch_fast_variant(bool split, bool pair, unsigned grid, unsigned threads, size_t smem, hipStream_t s,
-                         const LinePass& p) {
+void launch_fast_variant(bool split, int pair, unsigned grid, unsigned threads, size_t smem, hipStream_t s,
+                         const FastPass& p) {
   if constexpr (split_available<Real, N>()) {
     if (split) {
       FastVariant<Real, N, RM, NT, true>::launch(pair, grid, threads, smem, s, p);
@@ -1465,7 +1465,7 @@ void launch_fast_variant(bool split, bool pair, unsigned grid, unsigned threads,
 }
 
 template <typename Real, int N, int RM>
-const void* fast_variant_fn(bool split, bool pair, bool nt) {
+const void* fast_variant_fn(bool split, int pair, bool nt) {
   if constexpr (split_available<Real, N>()) {
     if (split) return nt ? FastVariant<Real, N, RM, true, true>::fn(pair) : FastVariant<Real, N, RM, false, true>::fn(pair);
   }
@@ -1670,12 +1670,13 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
   const bool pair = FastVariant<Real, N, RM, false, false>::kPairs && RM == 8 && p.paired &&
                     ((p.kind == kR2C && !p.inverse) || (p.kind == kC2R && p.inverse));
   const bool nt = p.nontemporal != 0;
-  const int v = 4 * (split ? 1 : 0) + 2 * (pair ? 1 : 0) + (nt ? 1 : 0);
+  const int kind = pair ? p.kind : 0;
+  const int v = 6 * (split ? 1 : 0) + 2 * kind + (nt ? 1 : 0);
   // raise the dynamic-LDS limit once per kernel instance
-  static std::atomic<size_t> lds_limit[8] = {64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024,
-                                             64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024};
+  static std::atomic<size_t> lds_limit[12] = {64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024,
+                                              64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024};
   {
-    const hipError_t e = raise_lds_limit(lds_limit[v], fast_variant_fn<Real, N, RM>(split, pair, nt), smem);
+    const hipError_t e = raise_lds_limit(lds_limit[v], fast_variant_fn<Real, N, RM>(split, kind, nt), smem);
     if (e != hipSuccess) return e;
   }
   const int64_t units = pair ? (static_cast<int64_t>(p.nlines) + 1) / 2 : p.nlines;
@@ -1688,10 +1689,11 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
     const int32_t C = (inner > 0 && inner % per == 0) ? inner / per : 0;
     p.swizzle = (C > 1 && grid % static_cast<unsigned>(C) == 0 && grid / C > 1) ? C : 0;
   }
+  const FastPass f = fast_pass(p, sizeof(Real) == 8);
   if (nt) {
-    launch_fast_variant<Real, N, RM, true>(split, pair, grid, static_cast<unsigned>(T * B), smem, s, p);
+    launch_fast_variant<Real, N, RM, true>(split, kind, grid, static_cast<unsigned>(T * B), smem, s, f);
   } else {
-    launch_fast_variant<Real, N, RM, false>(split, pair, grid, static_cast<unsigned>(T * B), smem, s, p);
+    launch_fast_variant<Real, N, RM, false>(split, kind, grid, static_cast<unsigned>(T * B), smem, s, f);
   }
   return hipGetLastError();
 }
@@ -1732,10 +1734,10 @@ hipError_t launch_products(LinePass p, hipStream_t s) {
   p.swizzle = 0;
   const bool nt = p.nontemporal != 0;
   static std::atomic<size_t> lds_limit[4] = {64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024};
-  const void* fn = split ? (nt ? reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, true, true, true>)
-                               : reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, false, true, true>))
-                         : (nt ? reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, true, false, true>)
-                               : reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, false, false, true>));
+  const void* fn = split ? (nt ? reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, true, true, kR2C, true>)
+                               : reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, false, true, kR2C, true>))
+                         : (nt ? reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, true, false, kR2C, true>)
+                               : reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, false, false, kR2C, true>));
   const hipError_t e = raise_lds_limit(lds_limit[2 * (split ? 1 : 0) + (nt ? 1 : 0)], fn, smem);
   if (e != hipSuccess) return e;
   const int64_t units = (static_cast<int64_t>(p.nlines) + 1) / 2;
@@ -1743,11 +1745,11 @@ hipError_t launch_products(LinePass p, hipStream_t s) {
   if (grid == 0) return hipSuccess;
   const dim3 g(grid), b(static_cast<unsigned>(T * B));
   if (split) {
-    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, true, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
-    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, true, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, true, kR2C, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, true, kR2C, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
   } else {
-    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, false, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
-    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, false, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+    if (nt) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, true, false, kR2C, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
+    else hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, false, false, kR2C, true>), g, b, smem, s, fast_pass(p, sizeof(Real) == 8));
   }
   return hipGetLastError();
 }
@@ -1784,16 +1786,19 @@ hipError_t launch_band(LinePass p, hipStream_t s) {
   p.swizzle = 0;
   const int64_t units = pair ? (static_cast<int64_t>(p.nlines) + 1) / 2 : p.nlines;
   const dim3 grid(static_cast<unsigned>((units + B - 1) / B)), block(static_cast<unsigned>(T * B));
-  static std::atomic<size_t> limit[3] = {64 * 1024, 64 * 1024, 64 * 1024};
-  const void* fns[3] = {reinterpret_cast<const void*>(&fft_line_fast<Real, N, 8, NT, true, true>),
-                        reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, true, false, true>),
-                        reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, true, true, true>)};
-  const int k = p.products ? 2 : (pair ? 1 : 0);
+  static std::atomic<size_t> limit[4] = {64 * 1024, 64 * 1024, 64 * 1024, 64 * 1024};
+  const void* fns[4] = {reinterpret_cast<const void*>(&fft_line_fast<Real, N, 8, NT, true, true>),
+                        reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, true, kR2C, false, true>),
+                        reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, true, kC2R, false, true>),
+                        reinterpret_cast<const void*>(&fft_pair_fast<Real, N, 8, NT, true, kR2C, true, true>)};
+  const int k = p.products ? 3 : p.kind == kC2R ? 2 : pair ? 1 : 0;
   const hipError_t e = raise_lds_limit(limit[k], fns[k], smem);
   if (e != hipSuccess) return e;
-  if (k == 2) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, true, true>), grid, block, smem, s, fast_pass(p, sizeof(Real) == 8));
-  else if (k == 1) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, false, true>), grid, block, smem, s, fast_pass(p, sizeof(Real) == 8));
-  else hipLaunchKernelGGL((fft_line_fast<Real, N, 8, NT, true, true>), grid, block, smem, s, fast_pass(p, sizeof(Real) == 8));
+  const FastPass f = fast_pass(p, true);
+  if (k == 3) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, kR2C, true, true>), grid, block, smem, s, f);
+  else if (k == 2) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, kC2R, false, true>), grid, block, smem, s, f);
+  else if (k == 1) hipLaunchKernelGGL((fft_pair_fast<Real, N, 8, NT, true, kR2C, false, true>), grid, block, smem, s, f);
+  else hipLaunchKernelGGL((fft_line_fast<Real, N, 8, NT, true, true>), grid, block, smem, s, f);
   return hipGetLastError();
 }
 
