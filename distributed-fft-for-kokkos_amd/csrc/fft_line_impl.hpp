@@ -1422,7 +1422,7 @@ inline hipError_t raise_lds_limit(std::atomic<size_t>& limit, const void* fn, si
 // One compile-time variant of the fast kernels: paired or single lines,
 // nontemporal or cached accesses, split or complex LDS exchanges.
 template <typename Real, int N, int RM, bool NT, bool SPLIT> struct FastVariant {
-  static constexpr bool kPairs = !(std::is_same<Real, double>::value && (N % 3 == 0 || N % 5 == 0));
+  static constexpr bool kPairs = N % 3 != 0 && N % 5 != 0;
   // pair: 0 single lines, else kR2C or kC2R
   static const void* fn(int pair) {
     if constexpr (kPairs) {
@@ -1665,8 +1665,7 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
   p.lines_per_block = B;
   // two real lines per complex FFT for forward R2C and inverse C2R passes
   // (kernels for 8 values per thread)
-  // (not for FP64 lengths with an odd factor: the pair kernel's two sets of
-  // 20-40 complex values per lane spill registers there)
+  // (lengths with an odd factor run their pairs on fft_smooth)
   const bool pair = FastVariant<Real, N, RM, false, false>::kPairs && RM == 8 && p.paired &&
                     ((p.kind == kR2C && !p.inverse) || (p.kind == kC2R && p.inverse));
   const bool nt = p.nontemporal != 0;

@@ -7,8 +7,8 @@ bool mixed_length(int n, bool fp64) {
   return n >= 2 && line_length_single_pass(n, fp64) && (fp64 ? mixed_lanes_f64(n) : mixed_lanes_f32(n)) > 0;
 }
 
-bool mixed_pass_supported(const LinePass& p, bool fp64) {
-  if (!mixed_length(p.n, fp64) || p.long_n1 > 0 || p.products) return false;
+bool whole_line_pass(const LinePass& p) {
+  if (p.long_n1 > 0 || p.products) return false;
   if (p.in.ntopo[p.axis] != 1 || p.out.ntopo[p.axis] != 1) return false;
   if (p.kind == kC2C) return true;
   if (!p.paired || p.pad_real > 0) return false;

@@ -1,21 +1,19 @@
 // Line passes of any length n = product of radices 2..13, 15, 16 (every n
 // without a prime factor above 13): a Stockham kernel whose radices are read
 // from the launch's plan and whose butterflies are straight-line code on
-// registers.  It serves the lengths without a compile-time kernel
-// (fft_line_impl.hpp), e.g. 36, 50, 100, 162, 250, 360, 375, 384, 1000.
+// registers.  It serves the lengths without a compiled kernel
+// (fft_line_impl.hpp, fft_smooth_impl.hpp): those with a factor 7, 11 or 13
+// and those above 1024, e.g. 42, 504, 1155, 1536.
 //
 // Why this shape: the per-element kernel (fft_line_generic) forms every output
 // of a radix-r stage as an r-term sum read from LDS, 4 to 16 LDS reads and
 // complex products per element and stage, and moved 0.25 to 0.6 TB/s.  Here a
 // lane reads a butterfly's r inputs once, so LDS traffic and arithmetic drop
-// by about r and a pass is bound by its line loads and stores (contiguous
-// FP64 lines: 4.7 to 5.5 TB/s read and written) or, in FP32 and in real
-// pairs, by instruction issue (2.4 to 4.7 TB/s).  An LDS index with a shift
-// per element instead of one constant step per exchange cost 5-10 % there.
-// Measured, per-element kernel -> this one (forward + backward unless stated):
-// R2C 384^3 FP64 7.16 -> 1.55 ms, C2C 375x250x162 FP32 forward 1.16 -> 0.29 ms,
-// inverse 2-D of 32x1000x1000 FP64 2.43 -> 0.49 ms, R2C 50x42x36 FP32
-// 124 -> 62 us.
+// by about r; a pass is bound by instruction issue (100 to 160 vector
+// instructions per element) at 2.4 to 5 TB/s.  An LDS index with a shift per
+// element instead of one constant step per exchange cost 5-10 % there.
+// Per-element kernel -> this one, forward and backward: R2C 384^3 FP64 7.16 ->
+// 1.30 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -11,6 +11,7 @@
 //    PencilPlan.hpp:1444-1598): FFT blocks on each rank's mapped local array
 //    and one exchange remap per transpose block.
 #include "plan.hpp"
+#include "fft_smooth.hpp"
 #include "trace.hpp"
 
 #include "buffer_check.hpp"
@@ -520,7 +521,7 @@ LinePass Plan::make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, b
 void Plan::default_shape(LinePass& p, const PassSpec& s) const {
   constexpr double kMiB = 1024.0 * 1024.0;
   const int es = fp64_ ? 16 : 8;
-  const bool fast = has_fast_line_kernel(p.n);
+  const bool fast = has_fast_line_kernel(p.n) && !smooth_length(p.n);
   // half-spectrum bytes, row alignment of both sides, distance of a line's elements
   double elems = 1.0, stride = es;
   for (std::size_t a = 0; a < rank_; ++a) elems *= static_cast<double>(std::min(p.in.ext[a], p.out.ext[a]));
@@ -544,7 +545,7 @@ void Plan::default_shape(LinePass& p, const PassSpec& s) const {
   const bool far = stride >= kMiB;
   int vpt = 8, lines = 0;
   if (!fast) {
-    vpt = 0;  // the runtime-radix kernel has its own rule
+    vpt = 0;  // the kernels of the other lengths have rules of their own
   } else if (!across) {
     // blocks of 128 lanes for short lines (256^3 R2C 69 -> 58 us)
     lines = p.n <= 512 ? std::max(1, 1024 / p.n) : 0;
