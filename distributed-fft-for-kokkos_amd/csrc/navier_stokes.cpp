@@ -76,8 +76,13 @@ NavierStokes::NavierStokes(int n, int px, int py, double lx, double nu, double d
     sblk_.push_back(sb);
     pblk_.push_back(pb);
   }
+  kblk_ = NsBlock{3, {n, n, Plan::band_row(g_.cutoff)}, {0, 0, 0}};
+  kblk_.set_divisors();
+  kept_supported_ = form == 0 && int64_t(n) * n * kblk_.ext[2] < (int64_t(1) << 31);
+  for (const Plan* p : {plan_b_.get(), plan_f_.get(), plan_f3_.get()})
+    if (p && !p->band_supported(g_.cutoff)) kept_supported_ = false;
   y_ = alloc_set(true, 3);
-  yc_ = alloc_set(true, 3);
+  ys_ = alloc_set(true, 3);
   k1_ = alloc_set(true, 3);
   k2_ = alloc_set(true, 3);
   k3_ = alloc_set(true, 3);
@@ -115,45 +120,76 @@ void NavierStokes::check_fields(void* const* f3, bool spectral, const char* what
   }
 }
 
+// Spectral sets are one allocation (256-byte aligned rank blocks) that also
+// holds the packed form at the first rank's pointer.
 std::vector<void*> NavierStokes::alloc_set(bool spectral, int nf) {
   std::vector<void*> out(P_, nullptr);
-  for (int r = 0; r < P_; ++r) {
-    const size_t bytes = size_t(nf) * (spectral ? spec_pts(r) * 16 : phys_pts(r) * 8);
-    if (bytes == 0) continue;
+  auto fresh = [&](size_t bytes) {
     void* p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) throw Error(DFFT_ERROR_OUT_OF_MEMORY, "hipMalloc of NS field failed");
     all_.push_back(p);
-    out[r] = p;
+    return p;
+  };
+  if (!spectral) {
+    for (int r = 0; r < P_; ++r)
+      if (phys_pts(r) > 0) out[r] = fresh(size_t(nf) * phys_pts(r) * 8);
+    return out;
   }
+  std::vector<size_t> at(P_, 0);
+  size_t total = 0;
+  for (int r = 0; r < P_; ++r) {
+    at[r] = total;
+    total += (size_t(nf) * spec_pts(r) * 16 + 255) / 256 * 256;
+  }
+  if (kept_supported_) total = std::max(total, size_t(nf) * kblk_.ext[0] * kblk_.ext[1] * kblk_.ext[2] * 16);
+  char* base = static_cast<char*>(fresh(std::max<size_t>(total, 256)));
+  for (int r = 0; r < P_; ++r) out[r] = base + at[r];
   return out;
 }
 
-bool NavierStokes::kept_only() const {
-  if (form_ != 0 || !kept_modes_) return false;
-  for (const Plan* p : {plan_b_.get(), plan_f_.get(), plan_f3_.get()})
-    if (!p->band_supported(g_.cutoff)) return false;
-  return true;
+NavierStokes::Part NavierStokes::part(bool packed, int r) const {
+  const NsBlock& b = packed ? kblk_ : sblk_[r];
+  return Part{b, ns_modes(b, n_, packed || kept_only() ? g_.cutoff : -1)};
 }
 
-void NavierStokes::forward(Plan& p, void* const* in, void* const* out, hipStream_t s) {
-  if (kept_only()) p.execute_band(in, out, DFFT_FORWARD, g_.cutoff, s);
+void NavierStokes::pack(void* const* blocks, void* const* packed, hipStream_t s) const {
+  for (int r = 0; r < P_; ++r)
+    hip_check(ns_pack(g_, sblk_[r], kblk_, static_cast<const double2*>(blocks[r]), static_cast<double2*>(packed[0]), s),
+              "ns_pack");
+}
+
+void NavierStokes::unpack(void* const* packed, void* const* blocks, hipStream_t s) const {
+  for (int r = 0; r < P_; ++r)
+    hip_check(ns_unpack(g_, sblk_[r], kblk_, static_cast<const double2*>(packed[0]), static_cast<double2*>(blocks[r]), s),
+              "ns_unpack");
+}
+
+const std::vector<void*>& NavierStokes::state_blocks(hipStream_t s) {
+  if (!kept_only()) return y_;
+  ensure_aux();
+  unpack(y_.data(), aux_s3b_.data(), s);
+  return aux_s3b_;
+}
+
+void NavierStokes::forward(Plan& p, void* const* in, void* const* out, bool packed, hipStream_t s) {
+  if (kept_only()) p.execute_band(in, out, DFFT_FORWARD, g_.cutoff, packed, s);
   else p.execute(in, out, DFFT_FORWARD, s);
 }
 
-void NavierStokes::backward(Plan& p, void* const* in, void* const* out, hipStream_t s) {
-  if (kept_only()) p.execute_band(in, out, DFFT_BACKWARD, g_.cutoff, s);
+void NavierStokes::backward(Plan& p, void* const* in, void* const* out, bool packed, hipStream_t s) {
+  if (kept_only()) p.execute_band(in, out, DFFT_BACKWARD, g_.cutoff, packed, s);
   else p.execute(in, out, DFFT_BACKWARD, s);
 }
 
-void NavierStokes::forward_products(void* const* u, hipStream_t s) {
+void NavierStokes::forward_products(void* const* u, bool packed, hipStream_t s) {
   if (fuse_products_ && plan_f_->products_supported()) {
-    plan_f_->execute_forward_products(u, nl_.data(), kept_only() ? g_.cutoff : 0, s);
+    plan_f_->execute_forward_products(u, nl_.data(), kept_only() ? g_.cutoff : 0, packed, s);
     return;
   }
   for (int r = 0; r < P_; ++r)
     hip_check(ns_products(static_cast<const double*>(u[r]), static_cast<double*>(pf_[r]), phys_pts(r), s),
               "ns_products");
-  forward(*plan_f_, pf_.data(), nl_.data(), s);
+  forward(*plan_f_, pf_.data(), nl_.data(), packed, s);
 }
 
 void NavierStokes::set_option(const std::string& key, long value) {
@@ -169,7 +205,16 @@ void NavierStokes::set_option(const std::string& key, long value) {
     (void)hipGraphDestroy(graph_);
     graph_ = nullptr;
   }
+  if (*flag == (value != 0)) return;
+  const bool was = kept_only();
   *flag = value != 0;
+  if (kept_only() == was) return;
+  // the state changes its form (ys_ holds nothing between steps)
+  hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
+  if (was) unpack(y_.data(), ys_.data(), nullptr);
+  else pack(y_.data(), ys_.data(), nullptr);
+  hip_check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+  std::swap(y_, ys_);
 }
 
 long NavierStokes::get_option(const std::string& key) const {
@@ -180,13 +225,15 @@ long NavierStokes::get_option(const std::string& key) const {
 }
 
 void NavierStokes::rk_stage(int stage, hipStream_t s, void* const* u_keep) {
+  const bool packed = kept_only();
+  const std::vector<void*>& z = stage == 0 ? y_ : ys_;  // the value this stage starts from
   if (form_ == 0) {
     void* const* u = u_keep ? u_keep : pb_.data();
-    backward(*plan_b_, y_.data(), u, s);
-    forward_products(u, s);
+    backward(*plan_b_, z.data(), u, packed, s);
+    forward_products(u, packed, s);
   } else {
     for (int r = 0; r < P_; ++r)
-      hip_check(ns_gradients(g_, sblk_[r], static_cast<double2*>(y_[r]), static_cast<double2*>(bin_[r]), s),
+      hip_check(ns_gradients(g_, sblk_[r], static_cast<double2*>(z[r]), static_cast<double2*>(bin_[r]), s),
                 "ns_gradients");
     plan_b_->execute(bin_.data(), pb_.data(), DFFT_BACKWARD, s);
     for (int r = 0; r < P_; ++r)
@@ -194,11 +241,12 @@ void NavierStokes::rk_stage(int stage, hipStream_t s, void* const* u_keep) {
                 "ns_advection");
     plan_f_->execute(pf_.data(), nl_.data(), DFFT_FORWARD, s);
   }
-  for (int r = 0; r < P_; ++r) {
+  for (int r = 0; r < parts(packed); ++r) {
     NsStage st{form_, stage, static_cast<const double2*>(nl_[r]), static_cast<double2*>(y_[r]),
-               static_cast<double2*>(yc_[r]), static_cast<double2*>(k1_[r]), static_cast<double2*>(k2_[r]),
+               static_cast<double2*>(ys_[r]), static_cast<double2*>(k1_[r]), static_cast<double2*>(k2_[r]),
                static_cast<double2*>(k3_[r])};
-    hip_check(ns_rhs_rk(g_, sblk_[r], modes(r), st, s), "ns_rhs_rk");
+    const Part p = part(packed, r);
+    hip_check(ns_rhs_rk(g_, p.b, p.k, st, s), "ns_rhs_rk");
   }
 }
 
@@ -252,27 +300,30 @@ void NavierStokes::autotune(hipStream_t s) {
     (void)hipGraphDestroy(graph_);
     graph_ = nullptr;
   }
-  // scratch only: yc_ and bin_ / nl_ / pb_ / pf_ are rewritten by every stage.
+  // scratch only: ys_ and bin_ / nl_ / pb_ / pf_ are rewritten by every stage.
   // Plan::autotune(in, out) takes the plan's input (physical, real) first and
   // its output (spectral, complex) second, whatever direction the solver uses
   // the plan in: each buffer must hold the side it is passed as.
   if (form_ == 0) {
-    plan_b_->autotune(pb_.data(), yc_.data(), s);  // 3 fields: pb_ holds >= 3 physical, yc_ 3 spectral
+    plan_b_->autotune(pb_.data(), ys_.data(), s);  // 3 fields: pb_ holds >= 3 physical, ys_ 3 spectral
     plan_f_->autotune(pf_.data(), nl_.data(), s);  // 6 fields: pf_ physical, nl_ spectral
-    if (plan_f3_) plan_f3_->autotune(pb_.data(), yc_.data(), s);
+    if (plan_f3_) plan_f3_->autotune(pb_.data(), ys_.data(), s);
   } else {
     plan_b_->autotune(pb_.data(), bin_.data(), s);  // 12 fields: pb_ 12 physical, bin_ 12 spectral
     plan_f_->autotune(pf_.data(), nl_.data(), s);   // 3 fields
-    if (plan_b3_) plan_b3_->autotune(pb_.data(), yc_.data(), s);
+    if (plan_b3_) plan_b3_->autotune(pb_.data(), ys_.data(), s);
   }
   hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 
 void NavierStokes::set_physical(void* const* u3, hipStream_t s) {
+  const bool packed = kept_only();
   Plan* pf = plan_f3_ ? plan_f3_.get() : plan_f_.get();
-  forward(*pf, u3, y_.data(), s);
-  for (int r = 0; r < P_; ++r)  // also clears the modes beyond the cutoff
-    hip_check(ns_dealias_project(g_, sblk_[r], static_cast<double2*>(y_[r]), s), "ns_dealias_project");
+  forward(*pf, u3, y_.data(), packed, s);
+  for (int r = 0; r < parts(packed); ++r) {  // in rank blocks also clears the modes beyond the cutoff
+    const Part p = part(packed, r);
+    hip_check(ns_dealias_project(g_, p.b, p.k, static_cast<double2*>(y_[r]), s), "ns_dealias_project");
+  }
 }
 
 void NavierStokes::init_taylor_green(double v0, hipStream_t s) {
@@ -283,10 +334,13 @@ void NavierStokes::init_taylor_green(double v0, hipStream_t s) {
 }
 
 double NavierStokes::energy(hipStream_t s) {
-  for (int r = 0; r < P_; ++r)
-    hip_check(ns_energy_partials(g_, sblk_[r], static_cast<const double2*>(y_[r]), partials_ + 256 * r, 256, s),
+  const bool packed = kept_only();
+  for (int r = 0; r < parts(packed); ++r) {
+    const Part p = part(packed, r);
+    hip_check(ns_energy_partials(g_, p.b, p.k, static_cast<const double2*>(y_[r]), partials_ + 256 * r, 256, s),
               "ns_energy");
-  hip_check(ns_sum(partials_, 256 * P_, esum_, s), "ns_sum");
+  }
+  hip_check(ns_sum(partials_, 256 * parts(packed), esum_, s), "ns_sum");
   double e = 0.0;
   hip_check(hipMemcpyAsync(&e, esum_, sizeof(double), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
   hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
@@ -294,6 +348,10 @@ double NavierStokes::energy(hipStream_t s) {
 }
 
 void NavierStokes::get_state(void* const* dst, hipStream_t s) const {
+  if (kept_only()) {
+    unpack(y_.data(), dst, s);
+    return;
+  }
   for (int r = 0; r < P_; ++r)
     if (spec_pts(r) > 0)
       hip_check(hipMemcpyAsync(dst[r], y_[r], size_t(3 * spec_pts(r)) * 16, hipMemcpyDeviceToDevice, s),
@@ -303,6 +361,10 @@ void NavierStokes::get_state(void* const* dst, hipStream_t s) const {
 // The stored state is kept dealiased: the reference's rhs dealiases its
 // argument in place first (main.cpp:576-578), so this changes no result.
 void NavierStokes::set_state(void* const* src, hipStream_t s) {
+  if (kept_only()) {
+    pack(src, y_.data(), s);
+    return;
+  }
   for (int r = 0; r < P_; ++r)
     hip_check(ns_dealias(g_, sblk_[r], static_cast<const double2*>(src[r]), static_cast<double2*>(y_[r]), s),
               "ns_dealias");

@@ -79,8 +79,9 @@ class NavierStokes {
     void* const* fb = nullptr;  // mode 1: written (may alias l3)
     double a = 0.0, c = 0.0;
   };
+  // packed: l3 and f's fields lie packed (y3 null), else in rank blocks
   void adjoint_core(const void* const* y3, const void* const* l3, const void* const* u3, const AdjFinish& f,
-                    hipStream_t s);
+                    bool packed, hipStream_t s);
   void one_step(hipStream_t s);
   int64_t spec_pts(int r) const;
   int64_t phys_pts(int r) const;
@@ -90,20 +91,40 @@ class NavierStokes {
   // Kept modes only: the spectra this solver reads and writes are dealiased,
   // so in the divergence form its transforms and pointwise kernels handle the
   // modes within the cutoff alone (0.30 of them) where every plan supports
-  // that.  The state y_ is zero at the others; scratch spectra (nl_, k1_, ...,
-  // the adjoint's fields) hold anything there.  The passes are bound by HBM,
+  // that.  A state in rank blocks is zero at the others; a packed one (below)
+  // and scratch spectra (nl_, k1_, ..., the adjoint's fields) hold anything there.  The passes are bound by HBM,
   // and a stage at 256^3 moves 4.6 GB instead of 9.3 GB: four steps from a
   // physical field 39.8 -> 21.7 ms, the gradient of four 128^3 steps 16.5 ->
   // 13.3 ms, results bit for bit the same.
-  bool kept_only() const;
-  NsModes modes(int r) const { return ns_modes(sblk_[r], n_, kept_only() ? g_.cutoff : -1); }
-  void forward(Plan& p, void* const* in, void* const* out, hipStream_t s);
-  void backward(Plan& p, void* const* in, void* const* out, hipStream_t s);
-  // forward transform of the 6 products of the velocity blocks u (fused into
-  // the R2C pass when enabled and supported, else products kernel + transform)
-  void forward_products(void* const* u, hipStream_t s);
+  bool kept_only() const { return kept_modes_ && kept_supported_; }
+  // With the kept modes alone, the state and every spectrum between a step's or
+  // a gradient's transforms lie packed: one array of all ranks with aligned
+  // rows of the kept entries (Plan::execute_band), which the x passes and the
+  // pointwise kernels walk without rank blocks.  Spectra of the caller stay in
+  // rank blocks.  A set of fields is one allocation that either form fits
+  // (256^3 in 2 x 2 ranks: x pass of the products 156 -> 130 us, of the velocity
+  // 64 -> 60, stage update 184 -> 150; four steps 16.7 -> 15.3 ms).
+  // A Part is what a pointwise kernel visits: a rank's block or the packed array.
+  struct Part {
+    NsBlock b;
+    NsModes k;
+    int64_t pts() const { return int64_t(b.ext[0]) * b.ext[1] * b.ext[2]; }
+  };
+  int parts(bool packed) const { return packed ? 1 : P_; }
+  Part part(bool packed, int r) const;
+  // the state in rank blocks (aux_s3b_ if it lies packed)
+  const std::vector<void*>& state_blocks(hipStream_t s);
+  void pack(void* const* blocks, void* const* packed, hipStream_t s) const;
+  void unpack(void* const* packed, void* const* blocks, hipStream_t s) const;
+  void forward(Plan& p, void* const* in, void* const* out, bool packed, hipStream_t s);
+  void backward(Plan& p, void* const* in, void* const* out, bool packed, hipStream_t s);
+  // forward transform of the 6 products of the velocity blocks u into nl_
+  // (fused into the R2C pass when enabled and supported, else products kernel
+  // + transform)
+  void forward_products(void* const* u, bool packed, hipStream_t s);
   bool fuse_products_ = true;
   bool kept_modes_ = true;
+  bool kept_supported_ = false;
   int n_, px_, py_, P_, form_;
   NsGrid g_{};
   double lx_;
@@ -112,8 +133,9 @@ class NavierStokes {
   std::unique_ptr<Plan> plan_b6_;            // 6-field backward (adjoint)
   int nf_b_, nf_f_;
   std::vector<NsBlock> sblk_, pblk_;  // per rank (3-field blocks; nf is set per use)
+  NsBlock kblk_{};                    // the packed array
   // device buffers, one pointer per rank
-  std::vector<void*> y_, yc_, k1_, k2_, k3_, nl_, bin_, pb_, pf_;
+  std::vector<void*> y_, ys_, k1_, k2_, k3_, nl_, bin_, pb_, pf_;
   std::vector<void*> aux_s3a_, aux_s3b_, aux_p3_;  // tangent/adjoint work fields (allocated on first use)
   std::vector<void*> all_;
   double* partials_ = nullptr;

@@ -41,8 +41,8 @@ void NavierStokes::apply_rhs(void* const* y3, void* const* out3, hipStream_t s) 
   for (int r = 0; r < P_; ++r)
     hip_check(ns_dealias(g_, sblk_[r], static_cast<const double2*>(y3[r]), static_cast<double2*>(ym[r]), s),
               "dealias");
-  backward(*plan_b_, ym.data(), pb_.data(), s);
-  forward_products(pb_.data(), s);
+  backward(*plan_b_, ym.data(), pb_.data(), false, s);
+  forward_products(pb_.data(), false, s);
   for (int r = 0; r < P_; ++r)
     hip_check(ns_rhs_only(g_, sblk_[r], static_cast<const double2*>(nl_[r]), static_cast<const double2*>(ym[r]),
                           static_cast<double2*>(out3[r]), s),
@@ -61,13 +61,13 @@ void NavierStokes::apply_rhs_tangent(void* const* y3, void* const* d3, void* con
     hip_check(ns_dealias(g_, sblk_[r], static_cast<const double2*>(y3[r]), static_cast<double2*>(ym[r]), s),
               "dealias");
   }
-  backward(*plan_b_, ym.data(), pb_.data(), s);
-  backward(*plan_b_, dm.data(), du.data(), s);
+  backward(*plan_b_, ym.data(), pb_.data(), false, s);
+  backward(*plan_b_, dm.data(), du.data(), false, s);
   for (int r = 0; r < P_; ++r)
     hip_check(ns_products_tangent(static_cast<double*>(pb_[r]), static_cast<double*>(du[r]),
                                   static_cast<double*>(pf_[r]), phys_pts(r), s),
               "products_tangent");
-  forward(*plan_f_, pf_.data(), nl_.data(), s);
+  forward(*plan_f_, pf_.data(), nl_.data(), false, s);
   for (int r = 0; r < P_; ++r)
     hip_check(ns_rhs_only(g_, sblk_[r], static_cast<const double2*>(nl_[r]), static_cast<const double2*>(dm[r]),
                           static_cast<double2*>(out3[r]), s),
@@ -78,40 +78,43 @@ void NavierStokes::apply_rhs_adjoint(void* const* y3, void* const* l3, void* con
   AdjFinish f;
   f.mode = 0;
   f.out3 = out3;
-  adjoint_core(y3, l3, nullptr, f, s);
+  adjoint_core(y3, l3, nullptr, f, false, s);
 }
 
 void NavierStokes::adjoint_core(const void* const* y3, const void* const* l3, const void* const* u3,
-                                const AdjFinish& f, hipStream_t s) {
+                                const AdjFinish& f, bool packed, hipStream_t s) {
   if (form_ != 0) throw Error(DFFT_ERROR_UNSUPPORTED, "adjoint needs the divergence form");
   ensure_aux();
   std::vector<void*>& mu = aux_s3a_;
   std::vector<void*>& ch = aux_s3b_;
   std::vector<void*>& c = aux_p3_;
-  for (int r = 0; r < P_; ++r)
-    hip_check(ns_adjoint_prepare(g_, sblk_[r], modes(r), static_cast<const double2*>(l3[r]), static_cast<double2*>(mu[r]),
+  for (int r = 0; r < parts(packed); ++r) {
+    const Part p = part(packed, r);
+    hip_check(ns_adjoint_prepare(g_, p.b, p.k, static_cast<const double2*>(l3[r]), static_cast<double2*>(mu[r]),
                                  static_cast<double2*>(nl_[r]), s),
               "adjoint_prepare");
-  backward(*plan_f_, nl_.data(), pf_.data(), s);  // S_mj (6 fields)
+  }
+  backward(*plan_f_, nl_.data(), pf_.data(), packed, s);  // S_mj (6 fields)
   if (!u3) {
     for (int r = 0; r < P_; ++r)  // D y into ch, which is free until the forward transform of c
       hip_check(ns_dealias(g_, sblk_[r], static_cast<const double2*>(y3[r]), static_cast<double2*>(ch[r]), s),
                 "dealias");
-    backward(*plan_b_, ch.data(), pb_.data(), s);  // u = IFFT(D y)
+    backward(*plan_b_, ch.data(), pb_.data(), false, s);  // u = IFFT(D y)
     u3 = pb_.data();
   }
   for (int r = 0; r < P_; ++r)
     hip_check(ns_adjoint_contract(static_cast<const double*>(u3[r]), static_cast<double*>(pf_[r]),
                                   static_cast<double*>(c[r]), phys_pts(r), s),
               "adjoint_contract");
-  forward(*plan_f3_, c.data(), ch.data(), s);
-  for (int r = 0; r < P_; ++r) {
+  forward(*plan_f3_, c.data(), ch.data(), packed, s);
+  for (int r = 0; r < parts(packed); ++r) {
+    const Part p = part(packed, r);
     const auto* chr = static_cast<const double2*>(ch[r]);
     const auto* mur = static_cast<const double2*>(mu[r]);
     if (f.mode == 0)
-      hip_check(ns_adjoint_finish(g_, sblk_[r], chr, mur, static_cast<double2*>(f.out3[r]), s), "adjoint_finish");
+      hip_check(ns_adjoint_finish(g_, p.b, chr, mur, static_cast<double2*>(f.out3[r]), s), "adjoint_finish");
     else
-      hip_check(ns_adjoint_finish_rk(g_, sblk_[r], modes(r), chr, mur, static_cast<double2*>(f.acc[r]),
+      hip_check(ns_adjoint_finish_rk(g_, p.b, p.k, chr, mur, static_cast<double2*>(f.acc[r]),
                                      static_cast<double2*>(f.lam[r]), f.fb ? static_cast<double2*>(f.fb[r]) : nullptr,
                                      f.a, f.c, f.mode, s),
                 "adjoint_finish_rk");
@@ -138,15 +141,25 @@ double NavierStokes::gradient(int nsteps, int ck, void* const* u0, void* const* 
   if (form_ != 0) throw Error(DFFT_ERROR_UNSUPPORTED, "gradient needs the divergence form");
   if (nsteps < 0 || ck < 1) throw Error(DFFT_ERROR_INVALID_ARGUMENT, "bad step counts");
   const double dt = g_.dt;
+  const bool packed = kept_only();
   std::vector<std::vector<void*>> owned;
   auto fresh = [&](bool spectral, int nf) {
     owned.push_back(alloc_set(spectral, nf));
     return owned.back();
   };
+  auto release = [&] {
+    for (auto& v : owned)
+      for (void* p : v) {
+        const auto it = std::find(all_.begin(), all_.end(), p);  // a spectral set has one allocation
+        if (it == all_.end()) continue;
+        all_.erase(it);
+        (void)hipFree(p);
+      }
+  };
   auto copy3 = [&](const std::vector<void*>& dst, const std::vector<void*>& src) {
-    for (int r = 0; r < P_; ++r)
-      if (spec_pts(r) > 0)
-        hip_check(hipMemcpyAsync(dst[r], src[r], size_t(3 * spec_pts(r)) * 16, hipMemcpyDeviceToDevice, s), "copy");
+    for (int r = 0; r < parts(packed); ++r)
+      if (const int64_t pts = part(packed, r).pts())
+        hip_check(hipMemcpyAsync(dst[r], src[r], size_t(3 * pts) * 16, hipMemcpyDeviceToDevice, s), "copy");
   };
   double J = 0.0;
   try {
@@ -169,8 +182,8 @@ double NavierStokes::gradient(int nsteps, int ck, void* const* u0, void* const* 
     J = energy(s);
     std::vector<void*> lam = fresh(true, 3), acc = fresh(true, 3), fb = fresh(true, 3);
     copy3(lam, y_);
-    for (int r = 0; r < P_; ++r)
-      hip_check(ns_axpby(3 * spec_pts(r), g_.coef, static_cast<double2*>(lam[r]), 0.0,
+    for (int r = 0; r < parts(packed); ++r)
+      hip_check(ns_axpby(3 * part(packed, r).pts(), g_.coef, static_cast<double2*>(lam[r]), 0.0,
                          static_cast<const double2*>(lam[r]), s),
                 "axpby");
     AdjFinish f;
@@ -186,45 +199,39 @@ double NavierStokes::gradient(int nsteps, int ck, void* const* u0, void* const* 
       }
       for (int st = last - 1; st >= first; --st) {
         const int base = 4 * (st - first);
-        for (int r = 0; r < P_; ++r)
-          hip_check(ns_rk_adjoint_init(sblk_[r], modes(r), static_cast<const double2*>(lam[r]),
-                                       static_cast<double2*>(fb[r]), static_cast<double2*>(acc[r]), dt / 6.0, s),
+        for (int r = 0; r < parts(packed); ++r) {
+          const Part p = part(packed, r);
+          hip_check(ns_rk_adjoint_init(p.b, p.k, static_cast<const double2*>(lam[r]), static_cast<double2*>(fb[r]),
+                                       static_cast<double2*>(acc[r]), dt / 6.0, s),
                     "rk_adjoint_init");
+        }
         const double a[3] = {1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0}, c[3] = {1.0, 0.5, 0.5};
         for (int k = 3; k >= 1; --k) {
           f.mode = 1;
           f.a = a[3 - k];
           f.c = c[3 - k];
-          adjoint_core(nullptr, fb.data(), stage_u[base + k].data(), f, s);
+          adjoint_core(nullptr, fb.data(), stage_u[base + k].data(), f, packed, s);
         }
         f.mode = 2;
-        adjoint_core(nullptr, fb.data(), stage_u[base].data(), f, s);
+        adjoint_core(nullptr, fb.data(), stage_u[base].data(), f, packed, s);
       }
     }
     // x0 = D P FFT(u0)  =>  dJ/du0 = n^3 IFFT(D P lam_0)
-    for (int r = 0; r < P_; ++r)
-      hip_check(ns_dealias_project(g_, sblk_[r], static_cast<double2*>(lam[r]), s), "dealias_project");
+    for (int r = 0; r < parts(packed); ++r) {
+      const Part p = part(packed, r);
+      hip_check(ns_dealias_project(g_, p.b, p.k, static_cast<double2*>(lam[r]), s), "dealias_project");
+    }
     Plan* pb3 = plan_b3_ ? plan_b3_.get() : plan_b_.get();
-    backward(*pb3, lam.data(), grad, s);
+    backward(*pb3, lam.data(), grad, packed, s);
     const double n3 = std::pow(static_cast<double>(n_), 3);
     for (int r = 0; r < P_; ++r) hip_check(ns_scale(3 * phys_pts(r), n3, static_cast<double*>(grad[r]), s), "scale");
     hip_check(hipStreamSynchronize(s), "sync");
   } catch (...) {
     (void)hipStreamSynchronize(s);
-    for (auto& v : owned)
-      for (void* p : v)
-        if (p) {
-          all_.erase(std::find(all_.begin(), all_.end(), p));
-          (void)hipFree(p);
-        }
+    release();
     throw;
   }
-  for (auto& v : owned)
-    for (void* p : v)
-      if (p) {
-        all_.erase(std::find(all_.begin(), all_.end(), p));
-        (void)hipFree(p);
-      }
+  release();
   return J;
 }
 

@@ -35,13 +35,14 @@ void write_raw(const std::string& name, const void* data, std::size_t bytes) {
 
 void NavierStokes::velocity(void* const* u3, hipStream_t s) {
   Plan* pb3 = plan_b3_ ? plan_b3_.get() : plan_b_.get();
-  pb3->execute(y_.data(), u3, DFFT_BACKWARD, s);
+  backward(*pb3, y_.data(), u3, kept_only(), s);
 }
 
 void NavierStokes::vorticity(void* const* w3, hipStream_t s) {
   ensure_aux();
+  const std::vector<void*>& y = state_blocks(s);
   for (int r = 0; r < P_; ++r)
-    hip_check(ns_vorticity(g_, sblk_[r], static_cast<const double2*>(y_[r]), static_cast<double2*>(aux_s3a_[r]), s),
+    hip_check(ns_vorticity(g_, sblk_[r], static_cast<const double2*>(y[r]), static_cast<double2*>(aux_s3a_[r]), s),
               "ns_vorticity");
   Plan* pb3 = plan_b3_ ? plan_b3_.get() : plan_b_.get();
   pb3->execute(aux_s3a_.data(), w3, DFFT_BACKWARD, s);
@@ -65,8 +66,9 @@ void NavierStokes::energy_spectrum(int nb, double* e_spec, double* k_vals, hipSt
   hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
   hip_check(hipMemcpy(spec_bins_, bins.data(), sizeof(double) * (nb + 1), hipMemcpyHostToDevice), "hipMemcpy");
   double* sums = spec_bins_ + kMaxSpectrumBins + 1;
+  const std::vector<void*>& y = state_blocks(s);
   for (int r = 0; r < P_; ++r)
-    hip_check(ns_energy_spectrum_partials(g_, sblk_[r], static_cast<const double2*>(y_[r]), spec_bins_, nb,
+    hip_check(ns_energy_spectrum_partials(g_, sblk_[r], static_cast<const double2*>(y[r]), spec_bins_, nb,
                                           spec_partials_ + static_cast<std::size_t>(r) * kSpecBlocks * nb,
                                           kSpecBlocks, s),
               "ns_energy_spectrum");

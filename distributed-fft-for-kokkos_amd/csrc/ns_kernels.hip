@@ -172,9 +172,10 @@ hipError_t ns_gradients(const NsGrid& g, const NsBlock& b, const double2* y3, do
 }
 
 // Streaming (nontemporal) element access of the spectral fields: the stage
-// update reads and writes 18-24 fields once each (2.4-3.2 GB at 256^3), far
-// beyond the caches, so its lines need not displace anything (256^3 step
-// 9.17 -> 8.89 ms; the 128^3 adjoint unchanged).
+// update reads and writes 15-24 fields once each, far beyond the caches, so
+// its lines need not displace anything.  The next stage's values are stored
+// through the caches (four 256^3 steps: all streaming 15.4 ms, values cached
+// 15.3, everything cached 15.8).
 typedef double StreamD2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ double2 stream_load(const double2* p) {
   const StreamD2 v = __builtin_nontemporal_load(reinterpret_cast<const StreamD2*>(p));
@@ -187,58 +188,75 @@ __device__ __forceinline__ void stream_store(double2* p, double2 x) {
   __builtin_nontemporal_store(v, reinterpret_cast<StreamD2*>(p));
 }
 
+// Bound by memory: 15 to 24 fields pass through once.  Stage and form are
+// compile-time constants so that every load of a mode is issued before the
+// first is waited for, the state is read where it lies instead of being copied
+// first, and a packed spectrum is one launch for all ranks: 256^3 in 2 x 2
+// ranks, a stage's update 184 us in four launches (4.2 TB/s) -> 150 us (4.8).
+template <int STAGE, int FORM>
 __global__ void __launch_bounds__(256) rhs_rk_kernel(const NsGrid g, const NsBlock b, const NsModes k, int64_t total,
                                                      const NsStage st) {
   const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  constexpr int NL = FORM == 0 ? 6 : 3;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
     int ix, iy, iz;
     const int64_t m = visited_mode(b, k, i, ix, iy, iz);
+    double2 p[NL], z[3], y[3], k1[3], k2[3], k3[3];
+#pragma unroll
+    for (int f = 0; f < NL; ++f) p[f] = stream_load(st.nl + (f * m_tot + m));
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int64_t e = c * m_tot + m;
+      y[c] = stream_load(st.y + e);
+      if constexpr (STAGE > 0) z[c] = stream_load(st.ys + e);
+      if constexpr (STAGE == 3) {
+        k1[c] = stream_load(st.k1 + e);
+        k2[c] = stream_load(st.k2 + e);
+        k3[c] = stream_load(st.k3 + e);
+      }
+    }
     const Mode md = mode_at(g, b, ix, iy, iz);
     double2 nl[3];
-    if (st.form == 0) {
+    if constexpr (FORM == 0) {
       // N_i = i sum_j k_j P_ij with P = [uu uv uw; uv vv vw; uw vw ww]
-      const double2 p0 = stream_load(st.nl + m), p1 = stream_load(st.nl + (m_tot + m));
-      const double2 p2 = stream_load(st.nl + (2 * m_tot + m)), p3 = stream_load(st.nl + (3 * m_tot + m));
-      const double2 p4 = stream_load(st.nl + (4 * m_tot + m)), p5 = stream_load(st.nl + (5 * m_tot + m));
-      nl[0] = ci(cadd2(cadd2(cscale(p0, md.kx), cscale(p1, md.ky)), cscale(p2, md.kz)));
-      nl[1] = ci(cadd2(cadd2(cscale(p1, md.kx), cscale(p3, md.ky)), cscale(p4, md.kz)));
-      nl[2] = ci(cadd2(cadd2(cscale(p2, md.kx), cscale(p4, md.ky)), cscale(p5, md.kz)));
+      nl[0] = ci(cadd2(cadd2(cscale(p[0], md.kx), cscale(p[1], md.ky)), cscale(p[2], md.kz)));
+      nl[1] = ci(cadd2(cadd2(cscale(p[1], md.kx), cscale(p[3], md.ky)), cscale(p[4], md.kz)));
+      nl[2] = ci(cadd2(cadd2(cscale(p[2], md.kx), cscale(p[4], md.ky)), cscale(p[5], md.kz)));
     } else {
-      nl[0] = stream_load(st.nl + m);
-      nl[1] = stream_load(st.nl + (m_tot + m));
-      nl[2] = stream_load(st.nl + (2 * m_tot + m));
+#pragma unroll
+      for (int c = 0; c < 3; ++c) nl[c] = p[c];
     }
     // dealias, combine (-adv - nu k^2 u), project (main.cpp:655-665, 780-810)
-    double2 y[3], r[3];
+    double2 r[3];
     const double visc = -g.nu * md.ksq;
+#pragma unroll
     for (int c = 0; c < 3; ++c) {
-      y[c] = cscale(stream_load(st.y + (c * m_tot + m)), md.mask);
-      r[c] = double2{-md.mask * nl[c].x + visc * y[c].x, -md.mask * nl[c].y + visc * y[c].y};
+      const double2 v = cscale(STAGE > 0 ? z[c] : y[c], md.mask);
+      r[c] = double2{-md.mask * nl[c].x + visc * v.x, -md.mask * nl[c].y + visc * v.y};
     }
     project(md, r);
     // RK4th::advance (math_utils.hpp:96-137)
+#pragma unroll
     for (int c = 0; c < 3; ++c) {
       const int64_t e = c * m_tot + m;
-      const double2 kk = cscale(r[c], g.dt);
+      const double2 kk = cscale(r[c], g.dt), y0 = cscale(y[c], md.mask);
       double2 yn;
-      if (st.stage == 0) {
-        stream_store(st.yc + e, y[c]);
+      if constexpr (STAGE == 0) {
         stream_store(st.k1 + e, kk);
-        yn = cadd2(y[c], cscale(kk, 0.5));
-      } else if (st.stage == 1) {
+        yn = cadd2(y0, cscale(kk, 0.5));
+      } else if constexpr (STAGE == 1) {
         stream_store(st.k2 + e, kk);
-        yn = cadd2(stream_load(st.yc + e), cscale(kk, 0.5));
-      } else if (st.stage == 2) {
+        yn = cadd2(y0, cscale(kk, 0.5));
+      } else if constexpr (STAGE == 2) {
         stream_store(st.k3 + e, kk);
-        yn = cadd2(stream_load(st.yc + e), kk);
+        yn = cadd2(y0, kk);
       } else {
-        const double2 k1 = stream_load(st.k1 + e), k2 = stream_load(st.k2 + e), k3 = stream_load(st.k3 + e);
-        const double2 sum = double2{(k1.x + 2.0 * k2.x + 2.0 * k3.x + kk.x) / 6.0,
-                                    (k1.y + 2.0 * k2.y + 2.0 * k3.y + kk.y) / 6.0};
-        yn = cadd2(stream_load(st.yc + e), sum);
+        const double2 sum = double2{(k1[c].x + 2.0 * k2[c].x + 2.0 * k3[c].x + kk.x) / 6.0,
+                                    (k1[c].y + 2.0 * k2[c].y + 2.0 * k3[c].y + kk.y) / 6.0};
+        yn = cadd2(y0, sum);
       }
-      stream_store(st.y + e, cscale(yn, md.mask));
+      (STAGE == 3 ? st.y : st.ys)[e] = cscale(yn, md.mask);  // read by the next transform
     }
   }
 }
@@ -246,15 +264,21 @@ __global__ void __launch_bounds__(256) rhs_rk_kernel(const NsGrid g, const NsBlo
 hipError_t ns_rhs_rk(const NsGrid& g, const NsBlock& b, const NsModes& k, const NsStage& st, hipStream_t s) {
   const int64_t m = k.total();
   if (m <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rhs_rk_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, k, m, st);
+  static void (*const kernel[2][4])(NsGrid, NsBlock, NsModes, int64_t, NsStage) = {
+      {rhs_rk_kernel<0, 0>, rhs_rk_kernel<1, 0>, rhs_rk_kernel<2, 0>, rhs_rk_kernel<3, 0>},
+      {rhs_rk_kernel<0, 1>, rhs_rk_kernel<1, 1>, rhs_rk_kernel<2, 1>, rhs_rk_kernel<3, 1>}};
+  hipLaunchKernelGGL(kernel[st.form == 0 ? 0 : 1][st.stage], dim3(blocks_for(m)), dim3(256), 0, s, g, b, k, m, st);
   return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(256) dealias_project_kernel(const NsGrid g, const NsBlock b, double2* y) {
+__global__ void __launch_bounds__(256) dealias_project_kernel(const NsGrid g, const NsBlock b, const NsModes k,
+                                                              int64_t total, double2* y) {
   const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; m < m_tot; m += stride) {
-    const Mode md = mode_of(g, b, m);
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
+    int ix, iy, iz;
+    const int64_t m = visited_mode(b, k, i, ix, iy, iz);
+    const Mode md = mode_at(g, b, ix, iy, iz);
     double2 v[3];
     for (int c = 0; c < 3; ++c) v[c] = md.mask != 0.0 ? y[c * m_tot + m] : double2{0.0, 0.0};
     project(md, v);
@@ -262,10 +286,50 @@ __global__ void __launch_bounds__(256) dealias_project_kernel(const NsGrid g, co
   }
 }
 
-hipError_t ns_dealias_project(const NsGrid& g, const NsBlock& b, double2* y3, hipStream_t s) {
-  const int64_t m = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
+hipError_t ns_dealias_project(const NsGrid& g, const NsBlock& b, const NsModes& k, double2* y3, hipStream_t s) {
+  const int64_t m = k.total();
   if (m <= 0) return hipSuccess;
-  hipLaunchKernelGGL(dealias_project_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, y3);
+  hipLaunchKernelGGL(dealias_project_kernel, dim3(blocks_for(m)), dim3(256), 0, s, g, b, k, m, y3);
+  return hipGetLastError();
+}
+
+// mode i of the visited ones of rank block b <-> the same mode of the packed
+// array p (one copy of the kept modes; bound by memory)
+template <bool UNPACK>
+__global__ void __launch_bounds__(256) repack_kernel(const NsGrid g, const NsBlock b, const NsBlock p, const NsModes k,
+                                                     int64_t total, const double2* src, double2* dst) {
+  const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
+  const int64_t p_tot = static_cast<int64_t>(p.ext[0]) * p.ext[1] * p.ext[2];
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
+    int ix, iy, iz;
+    const int64_t m = visited_mode(b, k, i, ix, iy, iz);
+    const int gx = ix + b.start[0], gy = iy + b.start[1], gz = iz + b.start[2];
+    const int64_t e = (static_cast<int64_t>(gx) * p.ext[1] + gy) * p.ext[2] + gz;
+    const int sx = signed_index(gx, g.n), sy = signed_index(gy, g.n);
+    const bool cut = (sx < 0 ? -sx : sx) > g.cutoff || (sy < 0 ? -sy : sy) > g.cutoff || gz > g.cutoff;
+    for (int c = 0; c < 3; ++c) {
+      if constexpr (UNPACK) stream_store(dst + (c * m_tot + m), cut ? double2{0.0, 0.0} : stream_load(src + (c * p_tot + e)));
+      else if (!cut) dst[c * p_tot + e] = src[c * m_tot + m];
+    }
+  }
+}
+
+hipError_t ns_pack(const NsGrid& g, const NsBlock& b, const NsBlock& p, const double2* src3, double2* dst3,
+                   hipStream_t s) {
+  const NsModes k = ns_modes(b, g.n, g.cutoff);
+  const int64_t m = k.total();
+  if (m <= 0) return hipSuccess;
+  hipLaunchKernelGGL(repack_kernel<false>, dim3(blocks_for(m)), dim3(256), 0, s, g, b, p, k, m, src3, dst3);
+  return hipGetLastError();
+}
+
+hipError_t ns_unpack(const NsGrid& g, const NsBlock& b, const NsBlock& p, const double2* src3, double2* dst3,
+                     hipStream_t s) {
+  const NsModes k = ns_modes(b, g.n, -1);
+  const int64_t m = k.total();
+  if (m <= 0) return hipSuccess;
+  hipLaunchKernelGGL(repack_kernel<true>, dim3(blocks_for(m)), dim3(256), 0, s, g, b, p, k, m, src3, dst3);
   return hipGetLastError();
 }
 
@@ -294,15 +358,15 @@ hipError_t ns_taylor_green(const NsBlock& b, double h, double v0, double* u3, hi
 }
 
 // block-level tree reduction in LDS; deterministic for a fixed launch shape
-__global__ void __launch_bounds__(256) energy_kernel(const NsGrid g, const NsBlock b, const double2* y,
-                                                     double* partials) {
+__global__ void __launch_bounds__(256) energy_kernel(const NsGrid g, const NsBlock b, const NsModes k, int64_t total,
+                                                     const double2* y, double* partials) {
   __shared__ double red[256];
   const int64_t m_tot = static_cast<int64_t>(b.ext[0]) * b.ext[1] * b.ext[2];
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   double acc = 0.0;
-  for (int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; m < m_tot; m += stride) {
-    const uint32_t mm = static_cast<uint32_t>(m);
-    const int iz = static_cast<int>(mm - b.div2.div(mm) * static_cast<uint32_t>(b.ext[2]));
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
+    int ix, iy, iz;
+    const int64_t m = visited_mode(b, k, i, ix, iy, iz);
     const double f = (iz + b.start[2]) == 0 ? 1.0 : 2.0;
     double s = 0.0;
     for (int c = 0; c < 3; ++c) {
@@ -320,9 +384,9 @@ __global__ void __launch_bounds__(256) energy_kernel(const NsGrid g, const NsBlo
   if (threadIdx.x == 0) partials[blockIdx.x] = red[0] * g.coef;
 }
 
-hipError_t ns_energy_partials(const NsGrid& g, const NsBlock& b, const double2* y3, double* partials,
-                              int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(energy_kernel, dim3(nblocks), dim3(256), 0, s, g, b, y3, partials);
+hipError_t ns_energy_partials(const NsGrid& g, const NsBlock& b, const NsModes& k, const double2* y3,
+                              double* partials, int nblocks, hipStream_t s) {
+  hipLaunchKernelGGL(energy_kernel, dim3(nblocks), dim3(256), 0, s, g, b, k, k.total(), y3, partials);
   return hipGetLastError();
 }
 

@@ -57,14 +57,14 @@ hipError_t ns_gradients(const NsGrid& g, const NsBlock& b, const double2* y3, do
 // Right-hand side of the RK stage and the RK4 update (main.cpp:572-666 and
 // math_utils.hpp:89-141).  form 0: `nl` holds the 6 product spectra
 // (divergence form, N_i = i k_j (u_i u_j)^); form 1: `nl` holds the 3
-// advection spectra.  y is the stage value (updated in place), yc/k1/k2/k3
-// the RK registers.
+// advection spectra.  y is the step's state (written by the last stage), ys
+// the value the next stage starts from, k1..k3 the RK registers.
 struct NsStage {
   int32_t form;
   int32_t stage;
   const double2* nl;
   double2* y;
-  double2* yc;
+  double2* ys;
   double2* k1;
   double2* k2;
   double2* k3;
@@ -72,16 +72,24 @@ struct NsStage {
 hipError_t ns_rhs_rk(const NsGrid& g, const NsBlock& b, const NsModes& k, const NsStage& st, hipStream_t s);
 
 // Projection u - k (k.u)/k^2 with the dealias mask (main.cpp:235-254, 214-225);
-// masked modes become zero and are not read.
-hipError_t ns_dealias_project(const NsGrid& g, const NsBlock& b, double2* y3, hipStream_t s);
+// masked modes among the visited ones become zero and are not read.
+hipError_t ns_dealias_project(const NsGrid& g, const NsBlock& b, const NsModes& k, double2* y3, hipStream_t s);
+
+// The kept modes of 3 fields between a rank's spectral block b and the packed
+// array p of all ranks: dst = D src.  pack visits the block's kept modes,
+// unpack every mode (zero beyond the cutoff).
+hipError_t ns_pack(const NsGrid& g, const NsBlock& b, const NsBlock& p, const double2* src3, double2* dst3,
+                   hipStream_t s);
+hipError_t ns_unpack(const NsGrid& g, const NsBlock& b, const NsBlock& p, const double2* src3, double2* dst3,
+                     hipStream_t s);
 
 // Taylor-Green field on a physical block (main.cpp:349-353): grid spacing h.
 hipError_t ns_taylor_green(const NsBlock& b, double h, double v0, double* u3, hipStream_t s);
 
 // Kinetic energy partial sums of a spectral block (main.cpp:855-910, global kz
 // index for the Hermitian weight); partials has `nblocks` doubles.
-hipError_t ns_energy_partials(const NsGrid& g, const NsBlock& b, const double2* y3, double* partials,
-                              int nblocks, hipStream_t s);
+hipError_t ns_energy_partials(const NsGrid& g, const NsBlock& b, const NsModes& k, const double2* y3,
+                              double* partials, int nblocks, hipStream_t s);
 hipError_t ns_sum(const double* partials, int n, double* out, hipStream_t s);
 
 // ---- tangent / adjoint pieces (divergence form) ---------------------------

@@ -61,8 +61,13 @@ class Plan {
   // of the spectra and leaves the others as they are; execute_band(BACKWARD)
   // transforms spectra whose other modes count as zeros, whatever the arrays
   // hold there.  Same results as execute on the masked spectra.
+  // packed: the spectral side is one array of all ranks in the layout of the
+  // plan's scratch (its one pointer first in the table): (fields, n, n,
+  // band_row(cut)) elements, entry (f, x, y, z) of the global spectrum at that
+  // index, nothing beyond the cutoff touched.
   bool band_supported(int cut) const;
-  void execute_band(void* const* in, void* const* out, int direction, int cut, hipStream_t stream);
+  static int32_t band_row(int cut) { return (cut + 8) / 8 * 8; }
+  void execute_band(void* const* in, void* const* out, int direction, int cut, bool packed, hipStream_t stream);
   // Forward execute of a 6-field R2C plan over such views whose input fields
   // are the products u_i u_j of the 3 velocity fields in `u3` (per rank: 3
   // fields shaped like the plan's input blocks), (i, j) = (0,0) (0,1) (0,2)
@@ -71,7 +76,7 @@ class Plan {
   // execute_band.  products_supported() says whether this plan can (FP64,
   // fused executor, an R2C first pass of a power-of-two length 8..1024).
   bool products_supported() const;
-  void execute_forward_products(void* const* u3, void* const* out, int cut, hipStream_t stream);
+  void execute_forward_products(void* const* u3, void* const* out, int cut, bool packed, hipStream_t stream);
   // execute with a HIP event pair around every launch; durations in ms
   std::vector<float> execute_timed(void* const* in, void* const* out, int direction, hipStream_t stream);
   int num_passes(int direction) const;
@@ -110,7 +115,8 @@ class Plan {
                      int slow_axis = -1) const;
   // restricts pass i of a direction to the kept modes
   void band_pass(LinePass& p, std::size_t i, bool forward, int cut) const;
-  DDesc band_scratch(int cut) const;
+  static void packed_stores(LinePass& p, const PassSpec& s);
+  DDesc band_array(int cut, void* p) const;
   // launch shape of a pass where its spec leaves it open
   void default_shape(LinePass& p, const PassSpec& s) const;
   float time_direction(void* const* in, void* const* out, bool forward, hipStream_t s, int reps);
