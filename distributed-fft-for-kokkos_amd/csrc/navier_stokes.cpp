@@ -120,31 +120,33 @@ void NavierStokes::check_fields(void* const* f3, bool spectral, const char* what
   }
 }
 
-// Spectral sets are one allocation (256-byte aligned rank blocks) that also
-// holds the packed form at the first rank's pointer.
-std::vector<void*> NavierStokes::alloc_set(bool spectral, int nf) {
-  std::vector<void*> out(P_, nullptr);
-  auto fresh = [&](size_t bytes) {
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) throw Error(DFFT_ERROR_OUT_OF_MEMORY, "hipMalloc of NS field failed");
-    all_.push_back(p);
-    return p;
-  };
-  if (!spectral) {
-    for (int r = 0; r < P_; ++r)
-      if (phys_pts(r) > 0) out[r] = fresh(size_t(nf) * phys_pts(r) * 8);
-    return out;
-  }
-  std::vector<size_t> at(P_, 0);
+// A set of fields is one allocation: rank blocks on 256-byte boundaries; a
+// spectral set also holds the packed form at the first rank's pointer.
+size_t NavierStokes::set_bytes(bool spectral, int nf) const {
   size_t total = 0;
+  for (int r = 0; r < P_; ++r)
+    total += (size_t(nf) * (spectral ? spec_pts(r) * 16 : phys_pts(r) * 8) + 255) / 256 * 256;
+  if (spectral && kept_supported_)
+    total = std::max(total, (size_t(nf) * kblk_.ext[0] * kblk_.ext[1] * kblk_.ext[2] * 16 + 255) / 256 * 256);
+  return total;
+}
+
+std::vector<void*> NavierStokes::place_set(void* base, bool spectral, int nf) const {
+  std::vector<void*> out(P_, nullptr);
+  char* at = static_cast<char*>(base);
   for (int r = 0; r < P_; ++r) {
-    at[r] = total;
-    total += (size_t(nf) * spec_pts(r) * 16 + 255) / 256 * 256;
+    out[r] = at;
+    at += (size_t(nf) * (spectral ? spec_pts(r) * 16 : phys_pts(r) * 8) + 255) / 256 * 256;
   }
-  if (kept_supported_) total = std::max(total, size_t(nf) * kblk_.ext[0] * kblk_.ext[1] * kblk_.ext[2] * 16);
-  char* base = static_cast<char*>(fresh(std::max<size_t>(total, 256)));
-  for (int r = 0; r < P_; ++r) out[r] = base + at[r];
   return out;
+}
+
+std::vector<void*> NavierStokes::alloc_set(bool spectral, int nf) {
+  void* p = nullptr;
+  if (hipMalloc(&p, std::max<size_t>(set_bytes(spectral, nf), 256)) != hipSuccess)
+    throw Error(DFFT_ERROR_OUT_OF_MEMORY, "hipMalloc of NS field failed");
+  all_.push_back(p);
+  return place_set(p, spectral, nf);
 }
 
 NavierStokes::Part NavierStokes::part(bool packed, int r) const {

@@ -85,6 +85,8 @@ class NavierStokes {
   void one_step(hipStream_t s);
   int64_t spec_pts(int r) const;
   int64_t phys_pts(int r) const;
+  size_t set_bytes(bool spectral, int nf) const;
+  std::vector<void*> place_set(void* base, bool spectral, int nf) const;  // a set at base
   std::vector<void*> alloc_set(bool spectral, int nf);
   void ensure_aux();
 
