@@ -175,6 +175,11 @@ struct GroupShape {
 bool group_line_shape(int n, bool fp64, size_t lds_cap, int lanes, bool across, GroupShape* g);
 // the same for FP32 lines taken two per lane (false if n has no such kernel)
 bool group_dual_shape(int n, size_t lds_cap, GroupShape* g);
+// true if the staged instance is the better one for contiguous lines of n: a
+// lane of more than 16 values leaves 8 lanes to a line, 64 bytes per access
+// (fields of 160^3 there and back 1884 -> 1755 us); elsewhere its registers (168
+// against 90) cost more than the wider accesses give (128^3 1304 -> 1366 us)
+bool group_stage_pays(int n);
 // true if two adjacent lines per lane apply to pass p with that many lines per
 // block (FP32 C2C, lanes across lines, consecutive lines adjacent row
 // elements on both sides, 16-byte aligned rank buffers; grouped passes)

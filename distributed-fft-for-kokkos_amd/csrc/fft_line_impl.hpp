@@ -33,10 +33,12 @@ struct FPlan {
 
 constexpr int cgcd(int a, int b) { return b == 0 ? a : cgcd(b, a % b); }
 
-// Power-of-two stages first, then 3s and 5s.  R (values per thread) is the
-// least common multiple of the radices, doubled while below `rmin` and still
-// a divisor of n.  With an odd factor the power-of-two part uses radix 4 (not
-// 8) so R stays small: 160 = 4*4*2*5 holds 20 values per thread, not 40.
+// Power-of-two stages first, then 3s and 5s, the first of them together with a
+// single 2 left over as a radix 6 or 10 (96 = 4*4*6, 160 = 4*4*10: an exchange
+// less than 4*4*2*5 at the same values per thread).  R (values per thread) is
+// the least common multiple of the radices, doubled while below `rmin` and
+// still a divisor of n.  With an odd factor the power-of-two part uses radix 4
+// (not 8) so R stays small: 160 holds 20 values per thread, not 40.
 constexpr FPlan make_plan(int n, int rmin = 1) {
   FPlan p;
   if (n <= 1) return p;
@@ -47,7 +49,9 @@ constexpr FPlan make_plan(int n, int rmin = 1) {
     while (m % 8 == 0) { p.rad[p.nst++] = 8; m /= 8; }
   }
   while (m % 4 == 0) { p.rad[p.nst++] = 4; m /= 4; }
-  if (m % 2 == 0) { p.rad[p.nst++] = 2; m /= 2; }
+  if (m % 6 == 0) { p.rad[p.nst++] = 6; m /= 6; }
+  else if (m % 10 == 0) { p.rad[p.nst++] = 10; m /= 10; }
+  else if (m % 2 == 0) { p.rad[p.nst++] = 2; m /= 2; }
   while (m % 3 == 0) { p.rad[p.nst++] = 3; m /= 3; }
   while (m % 5 == 0) { p.rad[p.nst++] = 5; m /= 5; }
   p.ok = (m == 1);
@@ -135,12 +139,43 @@ template <typename C> __device__ __forceinline__ void bfly5(C* a) {
   a[3] = csub(A2, X2);
 }
 
+template <int r, typename C> __device__ __forceinline__ void bfly(C* a);
+
+// r = r1 * r2, coprime: input r2 i + r1 j and output e1 k1 + e2 k2 (mod r)
+// with e1 = 1 (mod r1), 0 (mod r2) and e2 the other way round need no
+// twiddles between the two dimensions (Good 1958, Thomas 1963)
+template <int r1, int r2, typename C> __device__ __forceinline__ void bfly_coprime(C* a) {
+  constexpr int r = r1 * r2;
+  constexpr int e1 = [] { for (int v = r2;; v += r2) if (v % r1 == 1) return v; }();
+  constexpr int e2 = [] { for (int v = r1;; v += r1) if (v % r2 == 1) return v; }();
+  C g[r2][r1];
+#pragma unroll
+  for (int j = 0; j < r2; ++j) {
+#pragma unroll
+    for (int i = 0; i < r1; ++i) g[j][i] = a[(r2 * i + r1 * j) % r];
+    bfly<r1>(g[j]);
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < r1; ++k1) {
+    C t[r2];
+#pragma unroll
+    for (int j = 0; j < r2; ++j) t[j] = g[j][k1];
+    bfly<r2>(t);
+#pragma unroll
+    for (int k2 = 0; k2 < r2; ++k2) a[(e1 * k1 + e2 * k2) % r] = t[k2];
+  }
+}
+
 template <int r, typename C> __device__ __forceinline__ void bfly(C* a) {
   if constexpr (r == 2) bfly2(a);
   else if constexpr (r == 3) bfly3(a);
   else if constexpr (r == 4) bfly4(a);
   else if constexpr (r == 5) bfly5(a);
   else if constexpr (r == 8) bfly8(a);
+  else if constexpr (r == 6) bfly_coprime<2, 3>(a);
+  else if constexpr (r == 10) bfly_coprime<2, 5>(a);
+  else if constexpr (r == 12) bfly_coprime<4, 3>(a);
+  else if constexpr (r == 15) bfly_coprime<3, 5>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -416,6 +451,8 @@ __device__ __forceinline__ void twiddle_powers(double2 w, double2* p) {
   if constexpr (r > 5) p[5] = cmul(p[4], w);
   if constexpr (r > 6) p[6] = cmul(p[3], p[3]);
   if constexpr (r > 7) p[7] = cmul(p[4], p[3]);
+  if constexpr (r > 8) p[8] = cmul(p[4], p[4]);
+  if constexpr (r > 9) p[9] = cmul(p[5], p[4]);
 }
 
 template <typename C> __device__ __forceinline__ C to_prec(double2 w);
@@ -486,7 +523,7 @@ __device__ __forceinline__ void stage_twiddle(cplx_t<Real>* const (&v)[SETS], in
   constexpr int r = Tw::r, NB = Tw::NB;
   if constexpr (Tw::L > 1) {
     if constexpr (Tw::kShared) {
-      double2 pw[8];
+      double2 pw[10];
       twiddle_powers<r>(pre.get(t, tw, 0), pw);
 #pragma unroll
       for (int j = 1; j < r; ++j) {
@@ -500,7 +537,7 @@ __device__ __forceinline__ void stage_twiddle(cplx_t<Real>* const (&v)[SETS], in
     } else {
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
-        double2 pw[8];
+        double2 pw[10];
         twiddle_powers<r>(pre.get(t, tw, q), pw);
 #pragma unroll
         for (int j = 1; j < r; ++j) {

@@ -135,31 +135,6 @@ template <int p, typename C> __device__ __forceinline__ void bfly_prime(C* a) {
 
 template <int r, typename C> __device__ __forceinline__ void mix_bfly(C* a);
 
-// r = r1 * r2, coprime: input r2 i + r1 j and output e1 k1 + e2 k2 (mod r)
-// with e1 = 1 (mod r1), 0 (mod r2) and e2 the other way round need no
-// twiddles between the two dimensions (Good 1958, Thomas 1963)
-template <int r1, int r2, typename C> __device__ __forceinline__ void bfly_coprime(C* a) {
-  constexpr int r = r1 * r2;
-  constexpr int e1 = [] { for (int v = r2;; v += r2) if (v % r1 == 1) return v; }();
-  constexpr int e2 = [] { for (int v = r1;; v += r1) if (v % r2 == 1) return v; }();
-  C g[r2][r1];
-#pragma unroll
-  for (int j = 0; j < r2; ++j) {
-#pragma unroll
-    for (int i = 0; i < r1; ++i) g[j][i] = a[(r2 * i + r1 * j) % r];
-    mix_bfly<r1>(g[j]);
-  }
-#pragma unroll
-  for (int k1 = 0; k1 < r1; ++k1) {
-    C t[r2];
-#pragma unroll
-    for (int j = 0; j < r2; ++j) t[j] = g[j][k1];
-    mix_bfly<r2>(t);
-#pragma unroll
-    for (int k2 = 0; k2 < r2; ++k2) a[(e1 * k1 + e2 * k2) % r] = t[k2];
-  }
-}
-
 // r = q * q: q sub-transforms of the inputs q i + j, a twiddle, q across
 template <int q, typename C> __device__ __forceinline__ void bfly_square(C* a) {
   using R = decltype(a[0].x);
@@ -191,14 +166,10 @@ template <int q, typename C> __device__ __forceinline__ void bfly_square(C* a) {
 }
 
 template <int r, typename C> __device__ __forceinline__ void mix_bfly(C* a) {
-  if constexpr (r == 2 || r == 3 || r == 4 || r == 5 || r == 8) bfly<r>(a);
-  else if constexpr (r == 6) bfly_coprime<2, 3>(a);
-  else if constexpr (r == 9) bfly_square<3>(a);
-  else if constexpr (r == 10) bfly_coprime<2, 5>(a);
-  else if constexpr (r == 12) bfly_coprime<4, 3>(a);
-  else if constexpr (r == 15) bfly_coprime<3, 5>(a);
+  if constexpr (r == 9) bfly_square<3>(a);
   else if constexpr (r == 16) bfly_square<4>(a);
-  else bfly_prime<r>(a);
+  else if constexpr (r == 7 || r == 11 || r == 13) bfly_prime<r>(a);
+  else bfly<r>(a);
 }
 
 // Twiddle-table entries a butterfly loads: w, and for FP64 also w^4 and w^8,

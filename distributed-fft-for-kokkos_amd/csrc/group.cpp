@@ -218,6 +218,7 @@ void Group::build_tables(const std::vector<void*>& in, const std::vector<void*>&
   t.nt.assign(ns, 0);
   t.lds.assign(ns, 0);
   t.lanes.assign(ns, kGroupThreads);
+  t.stage.assign(ns, 0);
   t.single.assign(np, {});
   for (std::size_t k = 0; k < np; ++k) {
     std::vector<LinePass> all = build_pass(in, out, dir == 0, static_cast<int>(k));
@@ -227,7 +228,11 @@ void Group::build_tables(const std::vector<void*>& in, const std::vector<void*>&
       for (int a = 0; a < p.in.ndim; ++a) e *= static_cast<double>(p.in.ext[a]);
       bytes += e * (p.kind == kR2C ? 0.5 : 1.0) * (fp64_ ? 16.0 : 8.0);
     }
-    const int nt = nt_ >= 0 ? nt_ : (bytes >= 1024.0 * 1024 * 1024 ? 1 : 0);
+    // streaming accesses where the arrays do not stay in the 256 MB Infinity
+    // Cache from pass to pass (there and back, cached / streaming: 32 fields of
+    // 128^3 FP32 1362 / 1304 us, 24 of 160^3 1950 / 1755, 16 of 160^3 FP64 2519 /
+    // 2364; 130 MB of real fields 608 / 726)
+    const int nt = nt_ >= 0 ? nt_ : (bytes >= 256.0 * 1024 * 1024 ? 1 : 0);
     for (LinePass& p : all) p.nontemporal = nt;
     std::vector<LinePass> grouped[2];
     std::vector<int32_t> first[2] = {{0}, {0}};
@@ -268,6 +273,13 @@ void Group::build_tables(const std::vector<void*>& in, const std::vector<void*>&
         lds[v] = std::max(lds[v], g.lds_bytes);
       }
       const std::size_t slot = 2 * k + static_cast<std::size_t>(v);
+      double elems = 0.0, gain = 0.0;
+      for (const LinePass& p : grouped[v]) {
+        const double e = static_cast<double>(p.nlines) * p.n;
+        elems += e;
+        if (group_stage_pays(p.n)) gain += e;
+      }
+      t.stage[slot] = stage_ != 0 && (!stage_auto_ || 2.0 * gain >= elems) ? 1 : 0;
       t.nt[slot] = v == 0 && contiguous && contig_nt_ >= 0 ? contig_nt_ : nt;
       t.lanes[slot] = lanes;
       t.count[slot] = static_cast<int>(grouped[v].size());
@@ -316,7 +328,7 @@ void Group::launch_tables(const Tables& t, FastPass* const* items, int32_t* cons
       const int slot = 2 * k + v;
       if (t.count[slot] > 0)
         check(launch_group_pass(items[slot], first[slot], t.count[slot], t.total[slot], t.grid[slot], t.lds[slot],
-                                fp64_, t.nt[slot] != 0, v == 1, t.lanes[slot], stage_ != 0, s),
+                                fp64_, t.nt[slot] != 0, v == 1, t.lanes[slot], t.stage[slot] != 0, s),
               "grouped line pass");
     }
     for (const LinePass& p : t.single[k]) check(launch_line_pass(p, fp64_, s), "line pass");
@@ -389,6 +401,7 @@ void Group::set_option(const std::string& key, long value) {
   } else if (key == "stage") {
     if (value < 0 || value > 1) throw Error(DFFT_ERROR_INVALID_ARGUMENT, "stage must be 0 or 1");
     stage_ = static_cast<int>(value);
+    stage_auto_ = false;
   } else if (key == "lanes") {
     if (value != 64 && value != 128 && value != kGroupThreads)
       throw Error(DFFT_ERROR_INVALID_ARGUMENT, "lanes must be 64, 128 or 256");

@@ -61,7 +61,7 @@ class Group {
   struct Tables {
     std::vector<std::vector<FastPass>> items;
     std::vector<std::vector<int32_t>> first;  // virtual-block prefix per slot
-    std::vector<int> count, total, grid, nt, lanes;
+    std::vector<int> count, total, grid, nt, lanes, stage;
     std::vector<size_t> lds;
     std::vector<std::vector<LinePass>> single;  // per pass: individually launched passes
   };
@@ -81,11 +81,12 @@ class Group {
   int device_ = 0;
   int max_passes_ = 0;
   std::size_t lds_cap_ = kGroupLds;
-  int grid_mult_ = 1;
+  int grid_mult_ = 0;  // 0: a block per virtual block, else that many resident blocks walk them
   int nt_ = -1;
   int dual_ = 1;  // FP32: two adjacent lines per lane where they apply
-  int lanes_ = kGroupThreads;  // lanes per block of launches that hold only contiguous lines
+  int lanes_ = 128;  // lanes per block of launches that hold only contiguous lines
   int stage_ = 1;  // FP32: contiguous aligned lines 16 bytes per lane through LDS
+  bool stage_auto_ = true;  // ... where most of a launch's elements gain by it; until the option is set
   int contig_nt_ = -1;  // nontemporal accesses of launches of contiguous lines (-1: as nt_)
   std::map<int, void*> tw_;
   // per direction: the pointer set the device tables were built for, the
