@@ -775,7 +775,7 @@ bool line_length_supported(int n, bool fp64) {
 // 2053: 79 / 3.4 ms.  Bluestein is taken where it models at least 20 %
 // cheaper than every other kernel that can run the length.
 bool bluestein_preferred(int n, bool fp64) {
-  if (n < 2 || has_fast_line_kernel(n) || mixed_length(n, fp64)) return false;
+  if (n < 2 || has_fast_line_kernel(n) || smooth_length(n) || mixed_length(n, fp64)) return false;
   if (!line_length_supported(n, fp64)) return true;
   auto generic = [](int len) {
     GenPlan g;
