@@ -67,17 +67,12 @@ struct LinePass {
   // a row's end has its second line in the padding (that element is then not
   // loaded)
   int32_t dual_split;
-  // 1 (one-line lanes-across-lines C2C passes from a padded scratch into odd
-  // unpadded output rows): lines enumerated over the real elements only, so a
-  // block writes whole, aligned output segments (see lines_linear_unpadded)
-  int32_t linear_lines;
-  // FP64 R2C passes only (pair kernel): 1 = the line of field f (the batch
-  // axis prod_axis, six fields) is the pointwise product u_I * u_J of two of
+  // FP64 R2C passes only (pair kernel): 1 = the line of field f (array axis 0,
+  // six fields) is the pointwise product u_I * u_J of two of
   // the three fields that the input descriptor holds along that axis, (I, J)
   // = (0,0) (0,1) (0,2) (1,1) (1,2) (2,2) for f = 0..5 -- the products of the
   // divergence-form Navier-Stokes right-hand side formed as the lines load
   int32_t products;
-  int32_t prod_axis;
   // band > 0: a pass over the kept modes |k| <= band of a dealiased field
   // (FP64, power-of-two lengths 8..1024; launch_band_pass).  Index i of batch
   // axis j stands for i + (i > band ? band_shift[j] : 0) (the kept indices of

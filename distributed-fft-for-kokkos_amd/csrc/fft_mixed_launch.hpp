@@ -131,10 +131,6 @@ hipError_t launch_mixed(LinePass p, hipStream_t s) {
   const std::vector<int>& rad = len.rad;
   if (rad.empty()) return hipErrorNotSupported;
   int T = len.lanes;
-  {
-    LinePass q;
-    if (p.linear_lines && lines_linear_unpadded(p, q)) p = q;
-  }
   const int64_t units = p.kind == kC2C ? p.nlines : (static_cast<int64_t>(p.nlines) + 1) / 2;
   if (units <= 0) return hipSuccess;
 

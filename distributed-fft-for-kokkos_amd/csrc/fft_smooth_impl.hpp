@@ -591,13 +591,17 @@ template <typename Real, int N>
 hipError_t launch_smooth(LinePass p, hipStream_t s) {
   using Cfg = SmoothCfg<Real, N>;
   constexpr int T = Cfg::T;
-  {
-    LinePass q;
-    if (p.linear_lines && lines_linear_unpadded(p, q)) p = q;
-  }
   const int64_t units = p.kind == kC2C ? p.nlines : (static_cast<int64_t>(p.nlines) + 1) / 2;
   if (units <= 0) return hipSuccess;
   int B = p.lines_per_block;
+  if constexpr (N == 96 || N == 160) {
+    // a caller's block shape beyond a workgroup of the grouped launches' kernel
+    // of these lengths is refused, as it is for powers of two
+    const bool split = split_available<Real, N>() && p.split_lds != 0;
+    const size_t line = split ? line_lds_bytes<Real, N, 8, true>() : line_lds_bytes<Real, N, 8, false>();
+    if (!p.fit_block && B > 0 && (B * FastCfg<Real, N, 8>::T > 1024 || B * line > kGenericLdsMax))
+      return hipErrorInvalidConfiguration;
+  }
   if (B <= 0) {
     if (p.lines_fast) {
       B = 32;

@@ -431,7 +431,6 @@ LinePass Plan::make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, b
   p.swizzle = s.swz;
   p.split_lds = s.split;
   p.dual_lines = s.dual;
-  p.linear_lines = s.lin;
   p.tw = twiddles(s.n);
   p.lines_per_block = s.lines_per_block;
   p.values_per_thread = s.values_per_thread;
@@ -461,7 +460,7 @@ LinePass Plan::make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, b
   // a padded scratch row axis is enumerated over its pitch (padding lines are
   // skipped in the kernel) so each block of lines starts on an aligned row;
   // paired R2C / C2R passes keep the plain enumeration.  So do passes that
-  // write the user's arrays: there blocks then follow each other through the
+  // write the user's arrays (unless option lin is 0): there blocks then follow each other through the
   // rows without a gap and write whole lines of memory together (x passes onto
   // a 2 x 2 pencil grid: 512^3 R2C FP64 690 -> 553 us, 512 x 512 x 405 FP32 504 ->
   // 450; slabs unchanged).  Reading the user's arrays that way costs more than
@@ -471,7 +470,7 @@ LinePass Plan::make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, b
   const int32_t pitch = in.pitch > 0 ? in.pitch : out.pitch;
   const int inner = static_cast<int>(rank_) - 1;  // padded storage axis of the scratch (LayoutRight)
   const bool pairable = s.kind != kC2C && s.paired;
-  if (pitch > 0 && out.pitch > 0 && s.axis != inner && !pairable) {
+  if (pitch > 0 && (out.pitch > 0 || s.lin == 0) && s.axis != inner && !pairable) {
     for (int j = 0; j < p.nbatch; ++j) {
       if (p.batch_axis[j] != inner) continue;
       nl = nl / p.batch_ext[j] * pitch;
@@ -796,7 +795,6 @@ void Plan::execute_forward_products(void* const* u3, void* const* out, int cut, 
     if (first) {
       p.in = src3;
       p.products = 1;
-      p.prod_axis = 0;
       // enumerate the field axis fastest: the six product lines of one
       // position sit in neighbouring pairs and read the same three velocity
       // lines, which the caches serve after the first read

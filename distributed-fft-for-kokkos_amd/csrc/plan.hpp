@@ -31,7 +31,7 @@ struct PassSpec {
   int swz = 0;           // column-major walk of the block grid
   int split = 1;         // exchanges in real / imaginary halves (half the LDS; FP64, FP32 n >= 1024)
   int dual = 1;          // FP32 C2C: two adjacent lines per lane (16-byte accesses) where they apply
-  int lin = 1;           // one-line C2C passes into odd unpadded rows: lines enumerated over real elements
+  int lin = 1;           // passes that write the user's arrays enumerate real lines only (0: padded scratch rows)
 };
 
 // device table exp(-2 pi i e / n), e in [0, n): evaluated in long double,

@@ -150,18 +150,19 @@ int dfft_execute_timed(dfft_plan* plan, void* const* in, void* const* out, int d
  * 1/16, 0 off, 1 on); "fwd.<i>.lpb",
  * "fwd.<i>.vpt", "fwd.<i>.lf", "fwd.<i>.nt", "fwd.<i>.pair", "fwd.<i>.xcd",
  * "fwd.<i>.swz", "fwd.<i>.split" (and "bwd.…") = lines per block, values
- * per thread (4, 8, 16), lane order, nontemporal global accesses (-1 = on
- * for arrays of at least 1 GiB), two real lines per complex FFT in an R2C /
+ * per thread (4, 8, 16), lane order, nontemporal global accesses (-1 = by
+ * size and pass), two real lines per complex FFT in an R2C /
  * C2R pass (default on), XCD-contiguous block numbering, a column-major walk
  * of the block grid, radix-stage exchanges through LDS in real and
  * imaginary halves (default on; half the LDS per line; FP64 lines and FP32
  * lines of 1024 points or more), and "fwd.<i>.dual" = two adjacent FP32
  * lines per lane with 16-byte accesses (default on; C2C lanes-across-lines
  * passes whose consecutive lines are adjacent row elements; elsewhere
- * ignored), "fwd.<i>.lin" = lines of a one-line C2C lanes-across-lines pass
- * from the padded plan scratch into odd unpadded rows enumerated over the
- * real elements, so blocks write whole aligned segments (default on;
- * elsewhere ignored) of pass i.  A shape that does not fit a workgroup makes
+ * ignored), "fwd.<i>.lin" = the last pass's lines, which leave the padded plan
+ * scratch for the caller's rows, enumerated over the real elements, so blocks
+ * write whole segments (default on; elsewhere ignored) of pass i.  A shape
+ * that does not fit a workgroup (or, for lengths that are no power of two,
+ * that the kernel of the length cannot make fit) makes
  * execute return DFFT_ERROR_HIP without launching. */
 int dfft_plan_set_option(dfft_plan* plan, const char* key, long value);
 int dfft_plan_get_option(const dfft_plan* plan, const char* key, long* value);
