@@ -805,14 +805,14 @@ hipError_t launch_products_pass(const LinePass& p, hipStream_t s) {
   return dispatch_products_f64(p, s);
 }
 
-bool band_pass_supported(int n) { return products_pass_supported(n); }
+bool band_pass_supported(int n) { return products_pass_supported(n) || smooth_band_length(n); }
 
 hipError_t launch_band_pass(const LinePass& p, hipStream_t s) {
   if (p.nlines <= 0) return hipSuccess;
   if (!band_pass_supported(p.n) || p.band <= 0 || 2 * p.band >= p.n || p.in.ntopo[p.axis] != 1 ||
       p.out.ntopo[p.axis] != 1)
     return hipErrorNotSupported;
-  return dispatch_band_f64(p, s);
+  return smooth_band_length(p.n) ? launch_smooth_band(p, s) : dispatch_band_f64(p, s);
 }
 
 hipError_t launch_bluestein_pre(const LinePass& p, int log2m, const void* chirp, void* s1, bool fp64,

@@ -74,7 +74,7 @@ struct LinePass {
   // divergence-form Navier-Stokes right-hand side formed as the lines load
   int32_t products;
   // band > 0: a pass over the kept modes |k| <= band of a dealiased field
-  // (FP64, power-of-two lengths 8..1024; launch_band_pass).  Index i of batch
+  // (FP64, band_pass_supported lengths; launch_band_pass).  Index i of batch
   // axis j stands for i + (i > band ? band_shift[j] : 0) (the kept indices of
   // a whole spectral axis wrap around), inverse lines read the positions
   // beyond the band as zeros, forward lines store none of them.

@@ -9,6 +9,9 @@ namespace dfft {
 bool smooth_length(int n);
 hipError_t launch_smooth_f64(const LinePass& p, hipStream_t s);
 hipError_t launch_smooth_f32(const LinePass& p, hipStream_t s);
+// kept-mode passes (launch_band_pass), FP64: even such lengths from 36 to 384
+bool smooth_band_length(int n);
+hipError_t launch_smooth_band(const LinePass& p, hipStream_t s);
 
 // one per instantiation unit; hipErrorNotSupported for other lengths
 hipError_t smooth_f64_a(const LinePass& p, hipStream_t s);
@@ -19,5 +22,8 @@ hipError_t smooth_f32_a(const LinePass& p, hipStream_t s);
 hipError_t smooth_f32_b(const LinePass& p, hipStream_t s);
 hipError_t smooth_f32_c(const LinePass& p, hipStream_t s);
 hipError_t smooth_f32_d(const LinePass& p, hipStream_t s);
+hipError_t smooth_band_a(const LinePass& p, hipStream_t s);
+hipError_t smooth_band_b(const LinePass& p, hipStream_t s);
+hipError_t smooth_band_c(const LinePass& p, hipStream_t s);
 
 }  // namespace dfft

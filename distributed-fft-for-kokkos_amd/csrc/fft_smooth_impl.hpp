@@ -285,7 +285,12 @@ __device__ __forceinline__ void smooth_stages(cplx_t<Real>* v, int t, void* buf,
 
 // KIND kC2C: one complex line per T lanes.  kR2C / kC2R: the two real lines
 // 2 unit, 2 unit + 1 per T lanes as one complex line (PairIO).
-template <typename Real, int N, bool NT, int KIND>
+// BAND: a pass of a dealiased field's kept modes (LinePass::band): modes beyond
+// are neither read (zeros) nor stored (Navier-Stokes solver on 2 ranks, all
+// modes -> kept modes: three steps at 48^3 0.85 -> 0.69 ms, 96^3 1.92 -> 1.34,
+// 160^3 6.7 -> 3.4; gradient of four 96^3 steps 7.3 -> 5.0).  PROD: a products pass
+// (LinePass::products) as in fast_pair_body.
+template <typename Real, int N, bool NT, int KIND, bool PROD = false, bool BAND = false>
 __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const FastPass p) {
   using C = cplx_t<Real>;
   using Cfg = SmoothCfg<Real, N>;
@@ -314,7 +319,7 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
   if constexpr (KIND == kC2C) {
     LineIO<Real, NT> io;
     bool valid = unit < p.nlines;
-    if (valid) valid = make_line_io<Real, NT>(p, unit, io);
+    if (valid) valid = make_line_io<Real, NT, BAND>(p, unit, io);
     if (valid) {
 #pragma unroll
       for (int q = 0; q < S0::NB; ++q) {
@@ -323,7 +328,15 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
           const int64_t step = S0::nr * io.is;
 #pragma unroll
           for (int j = 0; j < S0::r; ++j) {
-            v[q * S0::r + j] = gload_c<NT, Real>(src);
+            if constexpr (BAND) {
+              // lanes beyond the band repeat the line's first address
+              const int at = t + q * T + j * S0::nr;
+              const bool keep = !p.inverse || at <= p.band || at >= N - p.band;
+              const C x = gload_c<NT, Real>(keep ? src : reinterpret_cast<const C*>(io.ib));
+              v[q * S0::r + j] = keep ? x : C{Real(0), Real(0)};
+            } else {
+              v[q * S0::r + j] = gload_c<NT, Real>(src);
+            }
             src += step;
           }
         }
@@ -343,7 +356,9 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
           const int64_t step = Sl::nr * io.os;
 #pragma unroll
           for (int j = 0; j < Sl::r; ++j) {
-            gstore_c<NT, Real>(dst, C{v[q * Sl::r + j].x * io.scale, v[q * Sl::r + j].y * sy});
+            const int at = t + q * T + j * Sl::nr;
+            if (!BAND || p.inverse || at <= p.band || at >= N - p.band)
+              gstore_c<NT, Real>(dst, C{v[q * Sl::r + j].x * io.scale, v[q * Sl::r + j].y * sy});
             dst += step;
           }
         }
@@ -352,8 +367,42 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
   } else if constexpr (KIND == kR2C) {
     const bool valid = 2 * unit < p.nlines;  // paired passes never enumerate padding
     PairIO<Real, NT> io{};
-    if (valid) {
-      io = make_pair_io<Real, NT>(p, unit);
+    if (valid) io = make_pair_io<Real, NT, PROD, BAND>(p, unit);
+    if constexpr (PROD) {
+      // slots 3m..3m+2 are the pairs of one position: slot 3m+q stages velocity
+      // line q, each slot then forms its two product lines from LDS
+      const int pq = b % 3;
+      Real* st = reinterpret_cast<Real*>(smem_raw + (b - pq) * p.line_bytes);
+      if (valid) {
+#pragma unroll
+        for (int q = 0; q < S0::NB; ++q) {
+          if (S0::on(t, q)) {
+            const Real* src = reinterpret_cast<const Real*>(io.ib[0]) + (t + q * T) * io.is[0];
+            const int64_t step = S0::nr * io.is[0];
+#pragma unroll
+            for (int j = 0; j < S0::r; ++j) {
+              st[pq * N + t + q * T + j * S0::nr] = gload<NT>(src);
+              src += step;
+            }
+          }
+        }
+      }
+      __syncthreads();
+      const Real* fa0 = st + prod_first(2 * pq) * N;
+      const Real* fa1 = st + prod_second(2 * pq) * N;
+      const Real* fb0 = st + prod_first(2 * pq + 1) * N;
+      const Real* fb1 = st + prod_second(2 * pq + 1) * N;
+#pragma unroll
+      for (int q = 0; q < S0::NB; ++q) {
+        if (S0::on(t, q)) {
+#pragma unroll
+          for (int j = 0; j < S0::r; ++j) {
+            const int at = t + q * T + j * S0::nr;
+            v[q * S0::r + j] = C{fa0[at] * fa1[at], fb0[at] * fb1[at]};
+          }
+        }
+      }
+    } else if (valid) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         if (h && !io.has_b) continue;
@@ -376,7 +425,7 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
         }
       }
     }
-    smooth_stages<Real, N, 0, true>(v, t, buf, tw, nullptr);
+    smooth_stages<Real, N, 0, !PROD>(v, t, buf, tw, nullptr);  // the staged lines share LDS with the exchanges
     // Spectra at m = t + q T + j nr <= n/2 from Z_m and Z_{n-m}: A = (Z_m +
     // conj Z_{n-m}) / 2, B = (Z_m - conj Z_{n-m}) / (2 i).  The lanes hand out
     // the upper half of Z; Z_0 and Z_{n/2} are their own mirrors.
@@ -455,7 +504,7 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
               const bool self = (j == 0 && q == 0 && t == 0) || (j >= LOW && 2 * at == N);
               const C w = self ? z : m[q * (TOP + 1) + j];
               const Real h = self ? h0 : hw;
-              if (j < LOW || 2 * at <= N)
+              if (BAND ? at <= p.band : j < LOW || 2 * at <= N)
                 gstore_c<NT, Real>(dst, line ? C{(z.y + w.y) * h, (w.x - z.x) * h} : C{(z.x + w.x) * h, (z.y - w.y) * h});
               dst += step;
             }
@@ -477,7 +526,7 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
       Bv[k] = C{Real(0), Real(0)};
     }
     if (valid) {
-      io = make_pair_io<Real, NT>(p, unit);
+      io = make_pair_io<Real, NT, false, BAND>(p, unit);
 #pragma unroll
       for (int line = 0; line < 2; ++line) {
         if (line && !io.has_b) continue;
@@ -490,8 +539,9 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
 #pragma unroll
             for (int j = 0; j <= TOP; ++j) {
               // above n/2 (only lanes of the middle output): the first entry again, not used
-              const bool low = j < LOW || 2 * (beta + j * S0::nr) <= N;
-              const C x = gload_c<NT, Real>(low ? src : reinterpret_cast<const C*>(io.ib[line]));
+              const bool low = BAND ? beta + j * S0::nr <= p.band : j < LOW || 2 * (beta + j * S0::nr) <= N;
+              C x = gload_c<NT, Real>(low ? src : reinterpret_cast<const C*>(io.ib[line]));
+              if (BAND && !low) x = C{Real(0), Real(0)};
               if (line) {
                 Bv[q * (TOP + 1) + j] = x;
               } else {
@@ -632,6 +682,58 @@ hipError_t launch_smooth(LinePass p, hipStream_t s) {
       return nt ? launch_smooth_kernel<Real, N, true, kC2R>(p, grid, threads, smem, s)
                 : launch_smooth_kernel<Real, N, false, kC2R>(p, grid, threads, smem, s);
   }
+}
+
+template <int N, int KIND, bool PROD>
+hipError_t launch_smooth_band_kernel(const LinePass& p, unsigned grid, unsigned threads, size_t smem, hipStream_t s) {
+  static std::atomic<size_t> limit{64 * 1024};
+  const void* fn = reinterpret_cast<const void*>(&fft_smooth<double, N, false, KIND, PROD, true>);
+  const hipError_t e = raise_lds_limit(limit, fn, smem);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((fft_smooth<double, N, false, KIND, PROD, true>), dim3(grid), dim3(threads), smem, s,
+                     fast_pass(p, true));
+  return hipGetLastError();
+}
+
+// a kept-mode pass (launch_band_pass)
+template <int N>
+hipError_t launch_smooth_band(LinePass p, hipStream_t s) {
+  using Cfg = SmoothCfg<double, N>;
+  constexpr int T = Cfg::T;
+  if (p.kind != kC2C && (p.kind == kR2C) == (p.inverse != 0)) return hipErrorInvalidValue;
+  if (p.products && (p.kind != kR2C || p.nlines % 6 != 0 || p.line_begin % 6 != 0)) return hipErrorInvalidConfiguration;
+  const int64_t units = p.kind == kC2C ? p.nlines : (static_cast<int64_t>(p.nlines) + 1) / 2;
+  if (units <= 0) return hipSuccess;
+  int B;
+  if (p.products) {
+    B = std::max(1, 128 / (3 * T)) * 3;  // whole positions
+  } else if (p.lines_fast) {
+    B = 32;
+    while (B > Cfg::LEAST && B * T > 256) B /= 2;
+  } else {
+    B = T >= 64 ? 1 : 64 / T;
+  }
+  if (!p.products)
+    while (B > 1 && (units + B - 1) / B < 512 && B * T > 64) B = (B + 1) / 2;
+  constexpr size_t kLine = static_cast<size_t>(Cfg::LDSN) * Cfg::ELEM;
+  const size_t stride = line_stride(kLine, Cfg::ELEM, p.lines_fast != 0, B, T);
+  if (B * T > Cfg::LANES || B * stride > kGenericLdsMax) return hipErrorInvalidConfiguration;
+  p.lines_per_block = B;
+  p.line_bytes = static_cast<int32_t>(stride);
+  p.swizzle = 0;
+  const size_t smem = B * stride;
+  const unsigned grid = static_cast<unsigned>((units + B - 1) / B), threads = static_cast<unsigned>(B * T);
+  if (p.kind == kC2C) return launch_smooth_band_kernel<N, kC2C, false>(p, grid, threads, smem, s);
+  if (p.kind == kC2R) return launch_smooth_band_kernel<N, kC2R, false>(p, grid, threads, smem, s);
+  return p.products ? launch_smooth_band_kernel<N, kR2C, true>(p, grid, threads, smem, s)
+                    : launch_smooth_band_kernel<N, kR2C, false>(p, grid, threads, smem, s);
+}
+
+template <int... Ns>
+hipError_t dispatch_smooth_band(const LinePass& p, hipStream_t s) {
+  hipError_t e = hipErrorNotSupported;
+  static_cast<void>(((p.n == Ns ? (e = launch_smooth_band<Ns>(p, s), true) : false) || ...));
+  return e;
 }
 
 // runs p on the kernel of its length if it is one of Ns

@@ -184,7 +184,7 @@ void NavierStokes::backward(Plan& p, void* const* in, void* const* out, bool pac
 }
 
 void NavierStokes::forward_products(void* const* u, bool packed, hipStream_t s) {
-  if (fuse_products_ && plan_f_->products_supported()) {
+  if (fuse_products_ && plan_f_->products_supported(kept_only() ? g_.cutoff : 0)) {
     plan_f_->execute_forward_products(u, nl_.data(), kept_only() ? g_.cutoff : 0, packed, s);
     return;
   }
@@ -221,7 +221,7 @@ void NavierStokes::set_option(const std::string& key, long value) {
 
 long NavierStokes::get_option(const std::string& key) const {
   if (key == "fuse_products") return fuse_products_ ? 1 : 0;
-  if (key == "products_fused") return (form_ == 0 && fuse_products_ && plan_f_->products_supported()) ? 1 : 0;
+  if (key == "products_fused") return (form_ == 0 && fuse_products_ && plan_f_->products_supported(kept_only() ? g_.cutoff : 0)) ? 1 : 0;
   if (key == "kept_modes") return kept_only() ? 1 : 0;
   throw Error(DFFT_ERROR_INVALID_ARGUMENT, "unknown NS option " + key);
 }

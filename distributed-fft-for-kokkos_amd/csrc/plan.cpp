@@ -662,13 +662,13 @@ void Plan::run_fused(void* const* in, void* const* out, bool forward, hipStream_
   }
 }
 
-bool Plan::products_supported() const {
+bool Plan::products_supported(int cut) const {
   if (!fp64_ || !real_ || d_.exec_mode != DFFT_EXEC_FUSED || view_layout_ != Layout::Right) return false;
   if (rank_ != 4 || gin_[0] != 6 || in_topo_[0] != 1 || out_topo_[0] != 1) return false;
   if (fwd_.empty() || fwd_[0].kind != kR2C || fwd_[0].axis != 3) return false;
   for (int a : {1, 2, 3})
     if (std::find(axes_.begin(), axes_.end(), static_cast<std::size_t>(a)) == axes_.end()) return false;
-  return products_pass_supported(fwd_[0].n);
+  return cut > 0 ? band_supported(cut) : products_pass_supported(fwd_[0].n);
 }
 
 bool Plan::band_supported(int cut) const {
@@ -765,7 +765,7 @@ void Plan::execute_band(void* const* in, void* const* out, int direction, int cu
 }
 
 void Plan::execute_forward_products(void* const* u3, void* const* out, int cut, bool packed, hipStream_t stream) {
-  if (!products_supported() || (cut > 0 ? !band_supported(cut) : packed))
+  if (!products_supported(cut) || (cut <= 0 && packed))
     throw Error(DFFT_ERROR_UNSUPPORTED, "this plan cannot form the products in its R2C pass");
   if (u3 == nullptr || out == nullptr) throw Error(DFFT_ERROR_INVALID_ARGUMENT, "null pointer table");
   int cur = -1;

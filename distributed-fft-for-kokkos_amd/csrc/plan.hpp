@@ -56,8 +56,8 @@ class Plan {
   // Dealiased fields (4-D views, field axis first and not distributed, R2C
   // over axes 1..3): only modes |k| <= cut along each axis are kept.
   // band_supported: FP64, fused executor, LayoutRight, power-of-two lengths
-  // 8..1024 (their real lines run in pairs whatever the plan's own passes
-  // do).  execute_band(FORWARD) writes the kept modes
+  // 8..1024 and even 2^a 3^b 5^c from 36 to 384 (their real lines run in pairs
+  // whatever the plan's own passes do).  execute_band(FORWARD) writes the kept modes
   // of the spectra and leaves the others as they are; execute_band(BACKWARD)
   // transforms spectra whose other modes count as zeros, whatever the arrays
   // hold there.  Same results as execute on the masked spectra.
@@ -73,9 +73,10 @@ class Plan {
   // fields shaped like the plan's input blocks), (i, j) = (0,0) (0,1) (0,2)
   // (1,1) (1,2) (2,2): the products are formed as the first (R2C) pass loads
   // its lines, so the 6 product fields are never stored.  cut > 0: as
-  // execute_band.  products_supported() says whether this plan can (FP64,
-  // fused executor, an R2C first pass of a power-of-two length 8..1024).
-  bool products_supported() const;
+  // execute_band.  products_supported(cut) says whether this plan can (FP64,
+  // fused executor, an R2C first pass of a power-of-two length 8..1024, or with
+  // cut > 0 band_supported).
+  bool products_supported(int cut) const;
   void execute_forward_products(void* const* u3, void* const* out, int cut, bool packed, hipStream_t stream);
   // execute with a HIP event pair around every launch; durations in ms
   std::vector<float> execute_timed(void* const* in, void* const* out, int direction, hipStream_t stream);
