@@ -2,8 +2,8 @@
 // without a prime factor above 13): a Stockham kernel whose radices are read
 // from the launch's plan and whose butterflies are straight-line code on
 // registers.  It serves the lengths without a compiled kernel
-// (fft_line_impl.hpp, fft_smooth_impl.hpp): those with a factor 7, 11 or 13
-// and those above 1024, e.g. 42, 504, 1155, 1536.
+// (fft_line_impl.hpp, fft_smooth_impl.hpp): those with a factor 11 or 13,
+// those with a 7 above 256 and those above 1024, e.g. 143, 504, 1155, 1536.
 //
 // Why this shape: the per-element kernel (fft_line_generic) forms every output
 // of a radix-r stage as an r-term sum read from LDS, 4 to 16 LDS reads and

@@ -1,4 +1,5 @@
-// Host interface of the compiled kernels of lengths 2^a 3^b 5^c (fft_smooth_impl.hpp).
+// Host interface of the compiled kernels of lengths 2^a 3^b 5^c up to 1024, and
+// with factors 7 up to 256 (fft_smooth_impl.hpp).
 #pragma once
 
 #include "fft_kernels.hpp"
@@ -9,7 +10,7 @@ namespace dfft {
 bool smooth_length(int n);
 hipError_t launch_smooth_f64(const LinePass& p, hipStream_t s);
 hipError_t launch_smooth_f32(const LinePass& p, hipStream_t s);
-// kept-mode passes (launch_band_pass), FP64: even such lengths from 36 to 384
+// kept-mode passes (launch_band_pass), FP64: even 2^a 3^b 5^c from 36 to 384
 bool smooth_band_length(int n);
 hipError_t launch_smooth_band(const LinePass& p, hipStream_t s);
 
@@ -18,10 +19,12 @@ hipError_t smooth_f64_a(const LinePass& p, hipStream_t s);
 hipError_t smooth_f64_b(const LinePass& p, hipStream_t s);
 hipError_t smooth_f64_c(const LinePass& p, hipStream_t s);
 hipError_t smooth_f64_d(const LinePass& p, hipStream_t s);
+hipError_t smooth_f64_e(const LinePass& p, hipStream_t s);
 hipError_t smooth_f32_a(const LinePass& p, hipStream_t s);
 hipError_t smooth_f32_b(const LinePass& p, hipStream_t s);
 hipError_t smooth_f32_c(const LinePass& p, hipStream_t s);
 hipError_t smooth_f32_d(const LinePass& p, hipStream_t s);
+hipError_t smooth_f32_e(const LinePass& p, hipStream_t s);
 hipError_t smooth_band_a(const LinePass& p, hipStream_t s);
 hipError_t smooth_band_b(const LinePass& p, hipStream_t s);
 hipError_t smooth_band_c(const LinePass& p, hipStream_t s);

@@ -13,12 +13,16 @@ hipError_t smooth_f64_a(const LinePass& p, hipStream_t s) {
 
 bool smooth_length(int n) {
   if (n < 3 || n > 1024 || (n & (n - 1)) == 0) return false;
+  if (n <= 256)
+    while (n % 7 == 0) n /= 7;
+  if (n == 1) return true;
   for (int r : {2, 3, 5})
     while (n % r == 0) n /= r;
   return n == 1;
 }
 
 hipError_t launch_smooth_f64(const LinePass& p, hipStream_t s) {
+  if (p.n % 7 == 0) return smooth_f64_e(p, s);
   return p.n <= 100 ? smooth_f64_a(p, s) : p.n <= 250 ? smooth_f64_b(p, s) : p.n <= 500 ? smooth_f64_c(p, s) : smooth_f64_d(p, s);
 }
 

@@ -1,7 +1,7 @@
 // Line passes of the lengths 2^a 3^b 5^c up to 1024 (without the powers of two,
-// which fft_line_impl.hpp serves): a Stockham kernel compiled per
-// length, with the radices, lanes per line and LDS paddings worked out at
-// compile time.
+// which fft_line_impl.hpp serves) and 2^a 3^b 5^c 7^d up to 256: a Stockham
+// kernel compiled per length, with the radices, lanes per line and LDS
+// paddings worked out at compile time.
 //
 // What bounds it: the runtime-radix kernel (fft_mixed_impl.hpp) spent 100 to
 // 160 vector instructions per element on these lengths, most of them index
@@ -15,7 +15,9 @@
 // 36 to 1000, both precisions, complex and real: 1.32 times as fast.
 // 96 and 160 against the compiled power-of-two kernel, which has no FP64 pairs
 // there: real FP64 160 contiguous 3.9 -> 4.7 TB/s, 96 2.9 -> 4.0, complex FP32
-// 160 6.5 -> 6.8, 96 4.0 -> 4.3 (FP64 96 strided 4.4 -> 4.0).
+// 160 6.5 -> 6.8, 96 4.0 -> 4.3 (FP64 96 strided 4.4 -> 4.0).  With factors 7
+// (42 to 252 points, both precisions, complex and real) 1.34 times the
+// runtime-radix kernel; longer ones are left to it.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -72,7 +74,7 @@ constexpr void smooth_search(SmoothPlan& best, const SmoothPlan& cur, int n, int
     return;
   }
   if (cur.nst >= 4) return;
-  constexpr int kRadix[] = {16, 15, 12, 10, 9, 8, 6, 5, 4, 3, 2};
+  constexpr int kRadix[] = {16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
   for (int r : kRadix) {
     if (r > top || rest % r) continue;
     SmoothPlan next = cur;
