@@ -108,31 +108,59 @@ template <typename C> __device__ __forceinline__ void bfly8(C* a) {
   a[7] = csub(e[3], o3);
 }
 
+__device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// A constant of a butterfly as the rounded value and what the rounding took
+// away.  Every line multiplies by the same few constants, so their rounding
+// errors add up over the stages instead of averaging out: with sqrt(3)/2 alone
+// (off by half an ulp) a 243-point FP64 line was 2.3e-16 off, with its low part
+// 1.95e-16.  low is zero where it is less than a seventh of an ulp of one.
+template <typename R> struct Wide {
+  R high, low;
+};
+template <typename R> constexpr Wide<R> wide(double high, double low) {
+  const R h = static_cast<R>(high);
+  const double l = sizeof(R) == 8 ? low : high - static_cast<double>(h);
+  const double least = sizeof(R) == 8 ? 1.5e-17 : 8e-9;
+  return Wide<R>{h, l < least && l > -least ? R(0) : static_cast<R>(l)};
+}
+// a + c b and a - c b, the low part of c first
+template <typename R> __device__ __forceinline__ R add_wide(R a, const Wide<R>& c, R b) {
+  return fmadd(c.high, b, c.low != R(0) ? fmadd(c.low, b, a) : a);
+}
+template <typename R> __device__ __forceinline__ R sub_wide(R a, const Wide<R>& c, R b) {
+  return add_wide(a, Wide<R>{-c.high, -c.low}, b);
+}
+template <typename R> __device__ __forceinline__ R mul_wide(const Wide<R>& c, R b) {
+  return c.low != R(0) ? fmadd(c.low, b, c.high * b) : c.high * b;
+}
+
 template <typename C> __device__ __forceinline__ void bfly3(C* a) {
   using R = decltype(a[0].x);
-  const R s3 = static_cast<R>(0.86602540378443864676);  // sin(2 pi / 3)
-  C s = cadd(a[1], a[2]);
-  C d = csub(a[1], a[2]);
-  C m = C{a[0].x - static_cast<R>(0.5) * s.x, a[0].y - static_cast<R>(0.5) * s.y};
-  C t = cmul_mi(C{s3 * d.x, s3 * d.y});
+  constexpr Wide<R> s3 = wide<R>(0.86602540378443864676, 5.017542e-17);  // sin(2 pi / 3)
+  const C s = cadd(a[1], a[2]);
+  const C d = csub(a[1], a[2]);
+  const C m = C{fmadd(R(-0.5), s.x, a[0].x), fmadd(R(-0.5), s.y, a[0].y)};
   a[0] = cadd(a[0], s);
-  a[1] = cadd(m, t);
-  a[2] = csub(m, t);
+  a[1] = C{add_wide(m.x, s3, d.y), sub_wide(m.y, s3, d.x)};
+  a[2] = C{sub_wide(m.x, s3, d.y), add_wide(m.y, s3, d.x)};
 }
 
 template <typename C> __device__ __forceinline__ void bfly5(C* a) {
   using R = decltype(a[0].x);
-  const R c1 = static_cast<R>(0.30901699437494742410);   // cos(2 pi/5)
-  const R c2 = static_cast<R>(-0.80901699437494742410);  // cos(4 pi/5)
-  const R s1 = static_cast<R>(0.95105651629515357212);   // sin(2 pi/5)
-  const R s2 = static_cast<R>(0.58778525229247312917);   // sin(4 pi/5)
-  C b1 = cadd(a[1], a[4]), b2 = cadd(a[2], a[3]);
-  C d1 = csub(a[1], a[4]), d2 = csub(a[2], a[3]);
-  C A1 = C{a[0].x + c1 * b1.x + c2 * b2.x, a[0].y + c1 * b1.y + c2 * b2.y};
-  C A2 = C{a[0].x + c2 * b1.x + c1 * b2.x, a[0].y + c2 * b1.y + c1 * b2.y};
-  C X1 = cmul_mi(C{s1 * d1.x + s2 * d2.x, s1 * d1.y + s2 * d2.y});
-  C X2 = cmul_mi(C{s2 * d1.x - s1 * d2.x, s2 * d1.y - s1 * d2.y});
-  a[0] = cadd(a[0], cadd(b1, b2));
+  constexpr Wide<R> c1 = wide<R>(0.30901699437494742410, -2.716058e-17);  // cos(2 pi/5)
+  constexpr Wide<R> c2 = wide<R>(-0.80901699437494742410, 2.716058e-17);  // cos(4 pi/5)
+  constexpr Wide<R> s1 = wide<R>(0.95105651629515357212, 4.093450e-17);   // sin(2 pi/5)
+  constexpr Wide<R> s2 = wide<R>(0.58778525229247312917, -7.934751e-18);  // sin(4 pi/5)
+  const C b1 = cadd(a[1], a[4]), b2 = cadd(a[2], a[3]);
+  const C d1 = csub(a[1], a[4]), d2 = csub(a[2], a[3]);
+  // the smaller term of a sum first: its rounding errors are those of the partial sums
+  const C A1 = C{add_wide(add_wide(a[0].x, c1, b1.x), c2, b2.x), add_wide(add_wide(a[0].y, c1, b1.y), c2, b2.y)};
+  const C A2 = C{add_wide(add_wide(a[0].x, c1, b2.x), c2, b1.x), add_wide(add_wide(a[0].y, c1, b2.y), c2, b1.y)};
+  const C X1 = cmul_mi(C{add_wide(mul_wide(s2, d2.x), s1, d1.x), add_wide(mul_wide(s2, d2.y), s1, d1.y)});
+  const C X2 = cmul_mi(C{sub_wide(mul_wide(s2, d1.x), s1, d2.x), sub_wide(mul_wide(s2, d1.y), s1, d2.y)});
+  a[0] = cadd(cadd(a[0], b1), b2);
   a[1] = cadd(A1, X1);
   a[4] = csub(A1, X1);
   a[2] = cadd(A2, X2);

@@ -60,40 +60,40 @@ struct MixPlan {
 };
 
 // ---------------------------------------------------------------------------
-// Butterflies beyond 2, 3, 4, 5 and 8 (exponent -2 pi i jk / r).
+// Butterflies beyond 2, 3, 4 and 5 (exponent -2 pi i jk / r).
 // ---------------------------------------------------------------------------
-template <int r> struct Roots;  // c[k] = cos(2 pi k / r), s[k] = sin(2 pi k / r)
+template <int r> struct Roots;  // c[k] = cos(2 pi k / r), s[k] = sin(2 pi k / r), k <= r / 2; cl, sl: see Wide
 template <> struct Roots<7> {
-  static constexpr double c[7] = {1.0, 0.623489801858733530525, -0.222520933956314404289, -0.900968867902419126236,
-                                  -0.900968867902419126236, -0.222520933956314404289, 0.623489801858733530525};
-  static constexpr double s[7] = {0.0, 0.781831482468029808708, 0.974927912181823607018, 0.433883739117558120475,
-                                  -0.433883739117558120475, -0.974927912181823607018, -0.781831482468029808708};
+  static constexpr double c[4] = {1.0, 0.623489801858733530525, -0.222520933956314404289, -0.900968867902419126236};
+  static constexpr double cl[4] = {0.0, 4.716100e-17, -1.141249e-17, 1.976265e-17};
+  static constexpr double s[4] = {0.0, 0.781831482468029808708, 0.974927912181823607018, 0.433883739117558120475};
+  static constexpr double sl[4] = {0.0, 5.074320e-18, -1.232384e-17, 7.407189e-20};
 };
 template <> struct Roots<9> {
   static constexpr double c[5] = {1.0, 0.766044443118978035202, 0.173648177666930348852, -0.5,
                                   -0.939692620785908384054};
+  static constexpr double cl[5] = {0.0, 2.175071e-17, -1.009049e-17, 0.0, 4.385093e-17};
   static constexpr double s[5] = {0.0, 0.642787609686539326323, 0.984807753012208059367, 0.866025403784438646764,
                                   0.342020143325668733044};
+  static constexpr double sl[5] = {0.0, -3.659608e-17, 3.905109e-17, 5.017542e-17, 2.013602e-17};
 };
 template <> struct Roots<11> {
-  static constexpr double c[11] = {1.0, 0.841253532831181168862, 0.415415013001886425529, -0.142314838273285140443,
-                                   -0.654860733945285064056, -0.959492973614497389891, -0.959492973614497389891,
-                                   -0.654860733945285064056, -0.142314838273285140443, 0.415415013001886425529,
-                                   0.841253532831181168862};
-  static constexpr double s[11] = {0.0, 0.540640817455597582108, 0.909631995354518371412, 0.989821441880932732376,
-                                   0.755749574354258283774, 0.281732556841429697711, -0.281732556841429697711,
-                                   -0.755749574354258283774, -0.989821441880932732376, -0.909631995354518371412,
-                                   -0.540640817455597582108};
+  static constexpr double c[6] = {1.0, 0.841253532831181168862, 0.415415013001886425529, -0.142314838273285140443,
+                                  -0.654860733945285064056, -0.959492973614497389891};
+  static constexpr double cl[6] = {0.0, -3.664729e-17, -9.555212e-18, 3.133448e-18, 3.655315e-17, -2.123968e-17};
+  static constexpr double s[6] = {0.0, 0.540640817455597582108, 0.909631995354518371412, 0.989821441880932732376,
+                                  0.755749574354258283774, 0.281732556841429697711};
+  static constexpr double sl[6] = {0.0, 2.667779e-17, 4.130148e-17, 4.815530e-17, 1.486952e-17, 2.667630e-17};
 };
 template <> struct Roots<13> {
-  static constexpr double c[13] = {1.0, 0.885456025653209895900, 0.568064746731155775490, 0.12053668025532305335,
-                                   -0.354604887042535625970, -0.748510748171101098635, -0.970941817426052027156,
-                                   -0.970941817426052027156, -0.748510748171101098635, -0.354604887042535625970,
-                                   0.12053668025532305335, 0.568064746731155775490, 0.885456025653209895900};
-  static constexpr double s[13] = {0.0, 0.464723172043768546302, 0.82298386589365639458, 0.992708874098054009100,
-                                   0.935016242685414832420, 0.663122658240795206160, 0.23931566428755776715,
-                                   -0.23931566428755776715, -0.663122658240795206160, -0.935016242685414832420,
-                                   -0.992708874098054009100, -0.82298386589365639458, -0.464723172043768546302};
+  static constexpr double c[7] = {1.0, 0.885456025653209895900, 0.568064746731155775490, 0.12053668025532305335,
+                                  -0.354604887042535625970, -0.748510748171101098635, -0.970941817426052027156};
+  static constexpr double cl[7] = {0.0, -1.460830e-17, -9.353414e-18, 5.709930e-18, -4.547648e-18, -1.735159e-17,
+                                   -1.536013e-17};
+  static constexpr double s[7] = {0.0, 0.464723172043768546302, 0.82298386589365639458, 0.992708874098054009100,
+                                  0.935016242685414832420, 0.663122658240795206160, 0.23931566428755776715};
+  static constexpr double sl[7] = {0.0, -1.637795e-17, 4.233793e-17, 2.007753e-17, -9.984533e-18, 9.324777e-18,
+                                   4.947072e-19};
 };
 template <> struct Roots<16> {
   static constexpr double c[10] = {1.0, 0.923879532511286756128, 0.707106781186547524401, 0.382683432365089771728,
@@ -103,17 +103,46 @@ template <> struct Roots<16> {
                                    1.0, 0.923879532511286756128, 0.707106781186547524401, 0.382683432365089771728,
                                    0.0, -0.382683432365089771728};
 };
+// cos and sin(2 pi k / r), 0 <= k < r
+template <int r, typename R> __device__ __forceinline__ constexpr Wide<R> root_cos(int k) {
+  const int m = 2 * k <= r ? k : r - k;
+  return wide<R>(Roots<r>::c[m], Roots<r>::cl[m]);
+}
+template <int r, typename R> __device__ __forceinline__ constexpr Wide<R> root_sin(int k) {
+  const int m = 2 * k <= r ? k : r - k;
+  const Wide<R> w = wide<R>(Roots<r>::s[m], Roots<r>::sl[m]);
+  return 2 * k <= r ? w : Wide<R>{-w.high, -w.low};
+}
 
-// prime radix: the terms m and p - m share their cosine and sine products
-template <int p, typename C> __device__ __forceinline__ void bfly_prime(C* a) {
+// term m (1 <= m <= r / 2) with the i-th smallest factor (sine or cosine) in
+// output k: added in this order, a sum's partial sums and with them its
+// rounding errors are smallest
+template <int r> constexpr int root_order(int k, int i, bool sine) {
+  auto size = [=](int m) {
+    const int q = k * m % r, t = 2 * q <= r ? q : r - q;
+    const double v = sine ? Roots<r>::s[t] : Roots<r>::c[t];
+    return v < 0.0 ? -v : v;
+  };
+  for (int m = 1; 2 * m < r; ++m) {
+    int below = 0;
+    for (int o = 1; 2 * o < r; ++o) below += size(o) < size(m) || (size(o) == size(m) && o < m) ? 1 : 0;
+    if (below == i) return m;
+  }
+  return 0;
+}
+
+// odd radix: the terms m and r - m share their cosine and sine products.  For 9
+// too: as 3 x 3 it takes a third less arithmetic, but the twiddles between the
+// two add to the error (729 points FP64 2.2e-16, this way 2.0e-16).
+template <int r, typename C> __device__ __forceinline__ void bfly_odd(C* a) {
   using R = decltype(a[0].x);
-  constexpr int h = (p - 1) / 2;
+  constexpr int h = (r - 1) / 2;
   C s[h], d[h];
   C sum = a[0];
 #pragma unroll
   for (int m = 0; m < h; ++m) {
-    s[m] = cadd(a[m + 1], a[p - 1 - m]);
-    d[m] = csub(a[m + 1], a[p - 1 - m]);
+    s[m] = cadd(a[m + 1], a[r - 1 - m]);
+    d[m] = csub(a[m + 1], a[r - 1 - m]);
     sum = cadd(sum, s[m]);
   }
   const C a0 = a[0];
@@ -122,53 +151,75 @@ template <int p, typename C> __device__ __forceinline__ void bfly_prime(C* a) {
   for (int k = 1; k <= h; ++k) {
     C A = a0, B{R(0), R(0)};
 #pragma unroll
-    for (int m = 1; m <= h; ++m) {
-      const R c = static_cast<R>(Roots<p>::c[(k * m) % p]), sn = static_cast<R>(Roots<p>::s[(k * m) % p]);
-      A = C{A.x + c * s[m - 1].x, A.y + c * s[m - 1].y};
-      B = C{B.x + sn * d[m - 1].x, B.y + sn * d[m - 1].y};
+    for (int i = 0; i < h; ++i) {
+      const int mc = root_order<r>(k, i, false), ms = root_order<r>(k, i, true);
+      const Wide<R> c = root_cos<r, R>(k * mc % r), sn = root_sin<r, R>(k * ms % r);
+      const C x = s[mc - 1], y = d[ms - 1];
+      A = C{add_wide(A.x, c, x.x), add_wide(A.y, c, x.y)};
+      B = i == 0 ? C{mul_wide(sn, y.x), mul_wide(sn, y.y)} : C{add_wide(B.x, sn, y.x), add_wide(B.y, sn, y.y)};
     }
     const C t = cmul_mi(B);
     a[k] = cadd(A, t);
-    a[p - k] = csub(A, t);
+    a[r - k] = csub(A, t);
   }
 }
 
-template <int r, typename C> __device__ __forceinline__ void mix_bfly(C* a);
-
-// r = q * q: q sub-transforms of the inputs q i + j, a twiddle, q across
-template <int q, typename C> __device__ __forceinline__ void bfly_square(C* a) {
+// 8 points as 2 x 4, the two outputs of an odd position by fused products with
+// 1/sqrt(2)
+template <typename C> __device__ __forceinline__ void bfly8_wide(C* a) {
   using R = decltype(a[0].x);
-  constexpr int r = q * q;
-  C g[q][q];
+  constexpr Wide<R> h = wide<R>(0.70710678118654752440, -4.833647e-17);
+  C e[4] = {a[0], a[2], a[4], a[6]};
+  C o[4] = {a[1], a[3], a[5], a[7]};
+  bfly4(e);
+  bfly4(o);
+  // o[k] *= exp(-2 pi i k / 8), but for h
+  const C o1 = C{o[1].x + o[1].y, o[1].y - o[1].x};
+  const C o2 = cmul_mi(o[2]);
+  const C o3 = C{o[3].y - o[3].x, -(o[3].x + o[3].y)};
+  a[0] = cadd(e[0], o[0]);
+  a[4] = csub(e[0], o[0]);
+  a[1] = C{add_wide(e[1].x, h, o1.x), add_wide(e[1].y, h, o1.y)};
+  a[5] = C{sub_wide(e[1].x, h, o1.x), sub_wide(e[1].y, h, o1.y)};
+  a[2] = cadd(e[2], o2);
+  a[6] = csub(e[2], o2);
+  a[3] = C{add_wide(e[3].x, h, o3.x), add_wide(e[3].y, h, o3.y)};
+  a[7] = C{sub_wide(e[3].x, h, o3.x), sub_wide(e[3].y, h, o3.y)};
+}
+
+// 16 = 4 x 4: sub-transforms of the inputs 4 i + j, a twiddle, 4 across
+template <typename C> __device__ __forceinline__ void bfly16(C* a) {
+  using R = decltype(a[0].x);
+  C g[4][4];
 #pragma unroll
-  for (int j = 0; j < q; ++j) {
+  for (int j = 0; j < 4; ++j) {
 #pragma unroll
-    for (int i = 0; i < q; ++i) g[j][i] = a[q * i + j];
-    mix_bfly<q>(g[j]);
+    for (int i = 0; i < 4; ++i) g[j][i] = a[4 * i + j];
+    bfly4(g[j]);
 #pragma unroll
-    for (int k = 1; k < q; ++k) {
+    for (int k = 1; k < 4; ++k) {
       if (j > 0) {
-        const R c = static_cast<R>(Roots<r>::c[j * k]), s = static_cast<R>(Roots<r>::s[j * k]);
+        const R c = static_cast<R>(Roots<16>::c[j * k]), s = static_cast<R>(Roots<16>::s[j * k]);
         const C x = g[j][k];
         g[j][k] = C{x.x * c + x.y * s, x.y * c - x.x * s};
       }
     }
   }
 #pragma unroll
-  for (int k1 = 0; k1 < q; ++k1) {
-    C t[q];
+  for (int k1 = 0; k1 < 4; ++k1) {
+    C t[4];
 #pragma unroll
-    for (int j = 0; j < q; ++j) t[j] = g[j][k1];
-    mix_bfly<q>(t);
+    for (int j = 0; j < 4; ++j) t[j] = g[j][k1];
+    bfly4(t);
 #pragma unroll
-    for (int k2 = 0; k2 < q; ++k2) a[k1 + q * k2] = t[k2];
+    for (int k2 = 0; k2 < 4; ++k2) a[k1 + 4 * k2] = t[k2];
   }
 }
 
 template <int r, typename C> __device__ __forceinline__ void mix_bfly(C* a) {
-  if constexpr (r == 9) bfly_square<3>(a);
-  else if constexpr (r == 16) bfly_square<4>(a);
-  else if constexpr (r == 7 || r == 11 || r == 13) bfly_prime<r>(a);
+  if constexpr (r == 8) bfly8_wide(a);
+  else if constexpr (r == 16) bfly16(a);
+  else if constexpr (r == 7 || r == 9 || r == 11 || r == 13) bfly_odd<r>(a);
   else bfly<r>(a);
 }
 
