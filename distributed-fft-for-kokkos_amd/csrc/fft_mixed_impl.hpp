@@ -223,36 +223,35 @@ template <int r, typename C> __device__ __forceinline__ void mix_bfly(C* a) {
   else bfly<r>(a);
 }
 
-// Twiddle-table entries a butterfly loads: w, and for FP64 also w^4 and w^8,
-// which keeps every power at most two rounded products away from the table
-// (with w alone they are four away, and the error of a 1000-point FP64 line
-// grows from 5.2e-16 to 6.4e-16).  FP32 powers are FP64 products of w.
-template <int r, typename Real> constexpr int mix_ntw() { return sizeof(Real) == 8 ? (r + 3) / 4 : 1; }
+// Twiddle-table entries a butterfly loads: FP64 all its powers (products of w,
+// w^4 and w^8 left the error of a 504-point line 21 % larger), FP32 w alone,
+// whose powers are FP64 products.
+template <int r, typename Real> constexpr int mix_ntw() { return sizeof(Real) == 8 ? r - 1 : 1; }
 
-// v[j] *= w^j: each power is rounded once to the kernel's precision and used
-// before the next is formed
+// v[j] *= w^j
 template <int r, typename C> __device__ __forceinline__ void mix_twiddle(C* v, const double2* ww) {
-  constexpr bool kTable = sizeof(C) == 16;
-  const double2 w = ww[0];
-  double2 lo[4];
-  lo[1] = w;
-  if constexpr (r > 2) lo[2] = cmul(w, w);
-  if constexpr (r > 3) lo[3] = cmul(lo[2], w);
+  if constexpr (sizeof(C) == 16) {
 #pragma unroll
-  for (int j = 1; j < 4 && j < r; ++j) v[j] = cmul(v[j], to_prec<C>(lo[j]));
-  if constexpr (r > 4) {
-    double2 w4, hi;
-    if constexpr (kTable) hi = w4 = ww[1];
-    else hi = w4 = cmul(lo[2], lo[2]);
+    for (int j = 1; j < r; ++j) v[j] = cmul(v[j], ww[j - 1]);
+  } else {
+    // each power is rounded once to FP32 and used before the next is formed
+    const double2 w = ww[0];
+    double2 lo[4];
+    lo[1] = w;
+    if constexpr (r > 2) lo[2] = cmul(w, w);
+    if constexpr (r > 3) lo[3] = cmul(lo[2], w);
 #pragma unroll
-    for (int g = 4; g < r; g += 4) {
-      v[g] = cmul(v[g], to_prec<C>(hi));
+    for (int j = 1; j < 4 && j < r; ++j) v[j] = cmul(v[j], to_prec<C>(lo[j]));
+    if constexpr (r > 4) {
+      const double2 w4 = cmul(lo[2], lo[2]);
+      double2 hi = w4;
 #pragma unroll
-      for (int j = 1; j < 4; ++j)
-        if (g + j < r) v[g + j] = cmul(v[g + j], to_prec<C>(cmul(hi, lo[j])));
-      if (g + 4 < r) {
-        if constexpr (kTable) hi = ww[g / 4 + 1];
-        else hi = cmul(hi, w4);
+      for (int g = 4; g < r; g += 4) {
+        v[g] = cmul(v[g], to_prec<C>(hi));
+#pragma unroll
+        for (int j = 1; j < 4; ++j)
+          if (g + j < r) v[g + j] = cmul(v[g + j], to_prec<C>(cmul(hi, lo[j])));
+        if (g + 4 < r) hi = cmul(hi, w4);
       }
     }
   }
@@ -293,23 +292,27 @@ __device__ __forceinline__ void mix_scatter(const Real* v, const MixStage& st, i
     }
   }
 }
-// twiddle-table entries of the lane's butterflies of a stage
+// twiddle-table entries of butterfly beta of a stage
+template <int r, typename Real>
+__device__ __forceinline__ void mix_tw_entries(double2* w, const MixStage& st, int beta, const double2* tw) {
+  const int g = static_cast<int>(st.dL.div(static_cast<uint32_t>(beta)));
+  const int e = (beta - g * st.L) * st.ts;
+#pragma unroll
+  for (int i = 0; i < mix_ntw<r, Real>(); ++i) w[i] = twiddle_load(tw + (i + 1) * e);
+}
+// FP32: those of the lane's butterflies, ahead of the stage.  FP64 has r - 1 of
+// each, too many to hold beside the values: mix_compute loads them.
 template <int r, int V, typename Real>
 __device__ __forceinline__ void mix_tw_load(double2* w, const MixStage& st, int t, int T, const double2* tw) {
+  if constexpr (sizeof(Real) == 4) {
 #pragma unroll
-  for (int q = 0; q < mix_nb<V>(r); ++q) {
-    const int beta = t + q * T;
-    if (beta < st.nr) {
-      const int g = static_cast<int>(st.dL.div(static_cast<uint32_t>(beta)));
-      const int e = (beta - g * st.L) * st.ts;
-      constexpr int N = mix_ntw<r, Real>();
-#pragma unroll
-      for (int i = 0; i < N; ++i) w[q * N + i] = twiddle_load(tw + (i == 0 ? e : 4 * i * e));
-    }
+    for (int q = 0; q < mix_nb<V>(r); ++q)
+      if (t + q * T < st.nr) mix_tw_entries<r, Real>(w + q, st, t + q * T, tw);
   }
 }
 template <int r, int V, typename Real>
-__device__ __forceinline__ void mix_compute(Real* re, Real* im, const MixStage& st, int t, int T, const double2* w) {
+__device__ __forceinline__ void mix_compute(Real* re, Real* im, const MixStage& st, int t, int T, const double2* w,
+                                            const double2* tw) {
   using C = cplx_t<Real>;
 #pragma unroll
   for (int q = 0; q < mix_nb<V>(r); ++q) {
@@ -317,7 +320,15 @@ __device__ __forceinline__ void mix_compute(Real* re, Real* im, const MixStage& 
       C a[r];
 #pragma unroll
       for (int j = 0; j < r; ++j) a[j] = C{re[q * r + j], im[q * r + j]};
-      if (st.L > 1) mix_twiddle<r>(a, w + q * mix_ntw<r, Real>());
+      if (st.L > 1) {
+        if constexpr (sizeof(Real) == 4) {
+          mix_twiddle<r>(a, w + q);
+        } else {
+          double2 all[mix_ntw<r, Real>()];
+          mix_tw_entries<r, Real>(all, st, t + q * T, tw);
+          mix_twiddle<r>(a, all);
+        }
+      }
       mix_bfly<r>(a);
 #pragma unroll
       for (int j = 0; j < r; ++j) {
@@ -429,10 +440,10 @@ __device__ __forceinline__ void mix_store_real(const Real* v, const MixStage& st
 // the outputs of the last stage there.
 template <int V, typename Real>
 __device__ __forceinline__ void mix_stages(Real* re, Real* im, const MixPlan& m, int t, Real* lds, const double2* tw) {
-  double2 w[sizeof(Real) == 8 ? 4 : mix_nb_max<V>()];
+  double2 w[mix_nb_max<V>()];
   for (int s = 0;; ++s) {
     const MixStage& st = m.st[s];
-#define DFFT_MIX_CALL(r) mix_compute<r, V, Real>(re, im, st, t, m.T, w)
+#define DFFT_MIX_CALL(r) mix_compute<r, V, Real>(re, im, st, t, m.T, w, tw)
     DFFT_MIX_SWITCH(st.r, DFFT_MIX_CALL)
 #undef DFFT_MIX_CALL
     if (s + 1 >= m.nst) break;

@@ -144,31 +144,6 @@ template <typename Real, int N> struct SmoothCfg {
   static constexpr int LANES = T * LEAST <= 256 ? 256 : T * LEAST <= 512 ? 512 : 1024;  // most lanes of a block
 };
 
-// Twiddle-table entries a butterfly loads: w, and for FP64 also w^2, w^3, w^4
-// and w^8, so that every power is at most one rounded product of two table
-// entries (with w, w^4 and w^8 alone the error of a 384-point line was 2.4e-16
-// instead of 1.8e-16; the loads cost 1 to 3 %).  FP32 powers are
-// FP64 products of w.
-template <int r, typename Real> constexpr int smooth_ntw() {
-  if (sizeof(Real) == 4) return 1;
-  return r <= 4 ? r - 1 : r <= 8 ? 4 : 5;
-}
-constexpr int smooth_exponent(int i) { return i < 4 ? i + 1 : 8; }  // of table entry i
-
-// v[j] *= w^j
-template <int r, typename C> __device__ __forceinline__ void smooth_twiddle(C* v, const double2* ww) {
-  if constexpr (sizeof(C) == 16) {
-    static_assert(r <= 12, "one product of two table entries reaches w^11");
-#pragma unroll
-    for (int j = 1; j < r; ++j) {
-      const double2 w = j < 4 ? ww[j - 1] : j % 4 == 0 ? ww[j == 4 ? 3 : 4] : cmul(ww[j < 8 ? 3 : 4], ww[j % 4 - 1]);
-      v[j] = cmul(v[j], w);
-    }
-  } else {
-    mix_twiddle<r>(v, ww);
-  }
-}
-
 // Stage S: lane t carries butterflies beta = t + q T (q < NB); their inputs
 // are positions beta + j nr, their outputs (beta / L) L r + beta % L + j L.
 template <typename Real, int N, int S> struct SmoothStage {
@@ -178,7 +153,7 @@ template <typename Real, int N, int S> struct SmoothStage {
   static constexpr int out_group = L * r + Cfg::pad(S);
   static constexpr int in_pad = S > 0 ? Cfg::pad(S > 0 ? S - 1 : 0) : 0;
   static constexpr int in_step = nr + nr / L * in_pad;
-  static constexpr int NTW = smooth_ntw<r, Real>();
+  static constexpr int NTW = mix_ntw<r, Real>();
   static constexpr bool kShared = T % L == 0;  // every butterfly of the lane has the same twiddles
   __device__ static __forceinline__ bool on(int t, int q) { return (q + 1) * T <= nr || t + q * T < nr; }
   // beta / L (exact for beta < 1024)
@@ -199,7 +174,7 @@ template <typename Real, int N, int S> struct SmoothStage {
           const int beta = t + q * T;
           const int e = (beta - group(beta) * L) * ts;
 #pragma unroll
-          for (int i = 0; i < NTW; ++i) w[q * NTW + i] = twiddle_load(tw + smooth_exponent(i) * e);
+          for (int i = 0; i < NTW; ++i) w[q * NTW + i] = twiddle_load(tw + (i + 1) * e);
         }
       }
     }
@@ -208,7 +183,7 @@ template <typename Real, int N, int S> struct SmoothStage {
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
       if (on(t, q)) {
-        if constexpr (L > 1) smooth_twiddle<r>(v + q * r, w + (kShared ? 0 : q * NTW));
+        if constexpr (L > 1) mix_twiddle<r>(v + q * r, w + (kShared ? 0 : q * NTW));
         mix_bfly<r>(v + q * r);
       }
     }

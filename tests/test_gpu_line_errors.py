@@ -45,3 +45,10 @@ def _complex_errors(dev, n, fp64):
 def test_fp32_lines(dev, n):
     here, per_element = _complex_errors(dev, n, False)
     assert here < TOL * per_element, (here, per_element)
+
+
+@pytest.mark.parametrize("n", [20, 90, 98, 99, 140, 143, 162, 250, 300, 324, 375, 441, 504, 539, 648, 729, 900, 1000,
+                               1001, 1155, 1280, 1536, 1701, 2187, 2401, 3125, 4374, 4802, 5120])
+def test_fp64_lines(dev, n):
+    here, per_element = _complex_errors(dev, n, True)
+    assert here < TOL * per_element, (here, per_element)
