@@ -469,7 +469,10 @@ template <typename Real, int N, int RM> struct FastCfg {
 // Twiddles of a radix-r butterfly are the powers w^j (j = 1..r-1) of one
 // table entry w = exp(-2 pi i k / (L r)): one FP64 load, the other powers by
 // FP64 products (at most three multiplications deep), each rounded once to the
-// kernel's precision.
+// kernel's precision.  FP64 lines of 96 and 160 points read w to w^4 and w^8:
+// chains up to w^9, four products deep, left a 160-point line 2.8e-16 off
+// instead of 1.7e-16.
+template <typename Real, int N> constexpr bool powers_from_table() { return sizeof(Real) == 8 && (N & (N - 1)) != 0; }
 template <int r>
 __device__ __forceinline__ void twiddle_powers(double2 w, double2* p) {
   p[1] = w;
@@ -520,7 +523,9 @@ template <typename Real, int N, int RM, int S> struct StageTwiddles {
   static constexpr bool kBase = L > 1 && !kShared && NB > 4 && L % T == 0;
   double2 w[kAhead ? NB : 1];
   __device__ __forceinline__ void load(int t, const double2* tw) {
-    if constexpr (kAhead) {
+    if constexpr (powers_from_table<Real, N>()) {
+      // stage_twiddle loads them
+    } else if constexpr (kAhead) {
 #pragma unroll
       for (int q = 0; q < NB; ++q) w[q] = twiddle_load(tw + entry(t, q) * ts);
     } else if constexpr (kBase || kShared) {
@@ -550,7 +555,22 @@ __device__ __forceinline__ void stage_twiddle(cplx_t<Real>* const (&v)[SETS], in
   using Tw = StageTwiddles<Real, N, RM, S>;
   constexpr int r = Tw::r, NB = Tw::NB;
   if constexpr (Tw::L > 1) {
-    if constexpr (Tw::kShared) {
+    if constexpr (powers_from_table<Real, N>()) {
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const unsigned e = Tw::entry(t, q) * Tw::ts;
+        double2 lo[5], hi;
+#pragma unroll
+        for (int j = 1; j < 5 && j < r; ++j) lo[j] = twiddle_load(tw + j * e);
+        if constexpr (r > 8) hi = twiddle_load(tw + 8 * e);
+#pragma unroll
+        for (int j = 1; j < r; ++j) {
+          const double2 w = j < 5 ? lo[j] : j == 8 ? hi : cmul(j < 8 ? lo[4] : hi, lo[j % 4]);
+#pragma unroll
+          for (int k = 0; k < SETS; ++k) v[k][q * r + j] = cmul(v[k][q * r + j], w);
+        }
+      }
+    } else if constexpr (Tw::kShared) {
       double2 pw[10];
       twiddle_powers<r>(pre.get(t, tw, 0), pw);
 #pragma unroll

@@ -52,3 +52,21 @@ def test_fp32_lines(dev, n):
 def test_fp64_lines(dev, n):
     here, per_element = _complex_errors(dev, n, True)
     assert here < TOL * per_element, (here, per_element)
+
+
+@pytest.mark.parametrize("n", [96, 160])
+@pytest.mark.parametrize("real", [False, True])
+def test_fp64_grouped_lines(dev, n, real):
+    """Grouped lines of 96 and 160 points: the power-of-two kernel with a radix 6 or 10."""
+    import torch
+    import dfft
+    x = _lines(n)
+    x = np.ascontiguousarray((x.real if real else x).T)
+    a = torch.from_numpy(x).to(dev)
+    b = torch.empty((x.shape[0], n // 2 + 1 if real else n), dtype=torch.complex128, device=dev)
+    g = dfft.Group([a], [b], [1], norm="none")
+    g.execute([a], [b], dfft.Direction.forward)
+    ref = _exact(x.T)[:b.shape[1]]
+    per_element = _per_element(dev, x.T.astype(np.complex128), True)[:b.shape[1]]
+    here, there = rel_l2(b.cpu().numpy().T, ref), rel_l2(per_element, ref)
+    assert here < TOL * there, (here, there)
