@@ -852,8 +852,10 @@ hipError_t launch_line_pass(const LinePass& p, bool fp64, hipStream_t s) {
   if (p.nlines <= 0) return hipSuccess;
   if (p.long_n1 > 0) return fp64 ? launch_long<double>(p, s) : launch_long<float>(p, s);
   // the register kernels need the line axis undistributed on both sides
+  // (FP32 real lines of 96 and 160 points run in pairs on the power-of-two one)
   const bool whole = whole_line_pass(p);
-  if (whole && smooth_length(p.n)) return fp64 ? launch_smooth_f64(p, s) : launch_smooth_f32(p, s);
+  const bool pairs = !fp64 && p.kind != kC2C && p.paired && has_fast_line_kernel(p.n);
+  if (whole && smooth_length(p.n) && !pairs) return fp64 ? launch_smooth_f64(p, s) : launch_smooth_f32(p, s);
   const bool fast = has_fast_line_kernel(p.n) && p.in.ntopo[p.axis] == 1 && p.out.ntopo[p.axis] == 1;
   if (fast) return fp64 ? dispatch<double>(p, s) : dispatch<float>(p, s);
   if (whole && mixed_length(p.n, fp64)) return fp64 ? launch_mixed_f64(p, s) : launch_mixed_f32(p, s);

@@ -385,13 +385,15 @@ __device__ __forceinline__ char* side_line(const Side& s, char* const* tab, cons
 }
 
 // The line's addresses; false if it is padding (a pass enumerated over padded
-// rows)
-template <typename Real, bool NT = false, bool BAND = false>
+// rows).  PROD (products pass, the field axis the fastest batch axis): product
+// fields 0 to 2 read velocity lines 0 to 2; the others' input is not used.
+template <typename Real, bool NT = false, bool BAND = false, bool PROD = false>
 __device__ __forceinline__ bool make_line_io(const FastPass& p, int32_t line, LineIO<Real, NT>& io) {
-  const BatchIdx x = batch_index<BAND>(p, line);
+  BatchIdx x = batch_index<BAND>(p, line);
   if (x.i2 >= p.pad_real) return false;
-  io.ib = side_line(p.in, p.in_ptr, x, io.is);
   io.ob = side_line(p.out, p.out_ptr, x, io.os);
+  if constexpr (PROD) x.i2 = x.i2 < 2 ? x.i2 : 2;
+  io.ib = side_line(p.in, p.in_ptr, x, io.is);
   io.kind = p.kind;
   io.n = p.n;
   io.inverse = p.inverse;
@@ -1507,7 +1509,7 @@ inline hipError_t raise_lds_limit(std::atomic<size_t>& limit, const void* fn, si
 // One compile-time variant of the fast kernels: paired or single lines,
 // nontemporal or cached accesses, split or complex LDS exchanges.
 template <typename Real, int N, int RM, bool NT, bool SPLIT> struct FastVariant {
-  static constexpr bool kPairs = N % 3 != 0 && N % 5 != 0;
+  static constexpr bool kPairs = !(std::is_same<Real, double>::value && (N % 3 == 0 || N % 5 == 0));
   // pair: 0 single lines, else kR2C or kC2R
   static const void* fn(int pair) {
     if constexpr (kPairs) {
@@ -1720,7 +1722,7 @@ hipError_t launch_fast(LinePass p, hipStream_t s) {
   p.lines_per_block = B;
   // two real lines per complex FFT for forward R2C and inverse C2R passes
   // (kernels for 8 values per thread)
-  // (lengths with an odd factor run their pairs on fft_smooth)
+  // (FP64 lines of 96 and 160 points run one by one)
   const bool pair = FastVariant<Real, N, RM, false, false>::kPairs && RM == 8 && p.paired &&
                     ((p.kind == kR2C && !p.inverse) || (p.kind == kC2R && p.inverse));
   const bool nt = p.nontemporal != 0;

@@ -10,9 +10,7 @@ bool mixed_length(int n, bool fp64) {
 bool whole_line_pass(const LinePass& p) {
   if (p.long_n1 > 0 || p.products) return false;
   if (p.in.ntopo[p.axis] != 1 || p.out.ntopo[p.axis] != 1) return false;
-  if (p.kind == kC2C) return true;
-  if (!p.paired || p.pad_real > 0) return false;
-  return p.kind == kR2C ? !p.inverse : p.inverse != 0;
+  return p.kind == kC2C || (p.kind == kR2C ? !p.inverse : p.inverse != 0);
 }
 
 static bool wide(int n) { return n % 11 == 0 || n % 13 == 0; }

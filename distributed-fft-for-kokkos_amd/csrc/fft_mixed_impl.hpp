@@ -418,6 +418,28 @@ __device__ __forceinline__ void mix_store_c2c(const Real* re, const Real* im, co
     }
   }
 }
+// the outputs at positions up to n/2 (R2C)
+template <int r, int V, bool NT, typename Real>
+__device__ __forceinline__ void mix_store_half(const Real* re, const Real* im, const MixStage& st, int t, int T, int n,
+                                               const LineIO<Real, NT>& io) {
+  using C = cplx_t<Real>;
+  const Real hw = io.scale * io.hw;
+#pragma unroll
+  for (int q = 0; q < mix_nb<V>(r); ++q) {
+    const int beta = t + q * T;
+    if (beta < st.nr) {
+      C* dst = reinterpret_cast<C*>(io.ob) + beta * io.os;
+      const int64_t step = st.nr * io.os;
+#pragma unroll
+      for (int j = 0; j <= r / 2; ++j) {
+        const int at = beta + j * st.nr;
+        const Real h = at == 0 || 2 * at == n ? io.scale : hw;
+        if (2 * at <= n) gstore_c<NT, Real>(dst, C{re[q * r + j] * h, im[q * r + j] * h});
+        dst += step;
+      }
+    }
+  }
+}
 template <int r, int V, bool NT, typename Real>
 __device__ __forceinline__ void mix_store_real(const Real* v, const MixStage& st, int t, int T, char* ob, int64_t os,
                                                Real s) {
@@ -470,8 +492,7 @@ __device__ __forceinline__ void mix_stages(Real* re, Real* im, const MixPlan& m,
   }
 }
 
-// KIND kC2C: one complex line per T lanes.  kR2C / kC2R: two real lines 2q,
-// 2q+1 per T lanes as one complex line (PairIO).
+// One line per T lanes; real lines run one by one (why: fft_smooth).
 template <typename Real, int V, bool NT, int KIND>
 __global__ void __launch_bounds__(1024) fft_mixed(const FastPass p, const MixPlan m) {
   using C = cplx_t<Real>;
@@ -505,10 +526,10 @@ __global__ void __launch_bounds__(1024) fft_mixed(const FastPass p, const MixPla
     im[j] = Real(0);
   }
 
+  LineIO<Real, NT> io{};
+  bool valid = active && unit < p.nlines;
+  if (valid) valid = make_line_io<Real, NT>(p, unit, io);
   if constexpr (KIND == kC2C) {
-    LineIO<Real, NT> io;
-    bool valid = active && unit < p.nlines;
-    if (valid) valid = make_line_io<Real, NT>(p, unit, io);
     if (valid) {
 #define DFFT_MIX_CALL(r) mix_load_c2c<r, V, NT, Real>(re, im, s0, t, T, io.ib, io.is, p.inverse != 0)
       DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
@@ -522,105 +543,36 @@ __global__ void __launch_bounds__(1024) fft_mixed(const FastPass p, const MixPla
 #undef DFFT_MIX_CALL
     }
   } else if constexpr (KIND == kR2C) {
-    const bool valid = active && 2 * unit < p.nlines;  // paired passes never enumerate padding
-    PairIO<Real, NT> io{};
     if (valid) {
-      io = make_pair_io<Real, NT>(p, unit);
-#define DFFT_MIX_CALL(r) mix_load_real<r, V, NT, Real>(re, s0, t, T, io.ib[0], io.is[0])
+#define DFFT_MIX_CALL(r) mix_load_real<r, V, NT, Real>(re, s0, t, T, io.ib, io.is)
       DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
 #undef DFFT_MIX_CALL
-      if (io.has_b) {
-#define DFFT_MIX_CALL(r) mix_load_real<r, V, NT, Real>(im, s0, t, T, io.ib[1], io.is[1])
-        DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
-#undef DFFT_MIX_CALL
-      }
     }
     mix_stages<V, Real>(re, im, m, t, lds, tw);
-    // spectra of the two lines at k = t + q T <= n/2 from Z_k and Z_{n-k}:
-    // A = (Z_k + conj Z_{n-k}) / 2, B = (Z_k - conj Z_{n-k}) / (2 i)
-    Real ax[mix_half<V>()], by[mix_half<V>()], ay[mix_half<V>()], bx[mix_half<V>()];
-    __syncthreads();
-#define DFFT_MIX_CALL(r) mix_scatter<r, V, Real>(re, sl, t, T, lds, m.ps)
-    DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
-#undef DFFT_MIX_CALL
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < mix_half<V>(); ++q) {
-      const int k = t + q * T;
-      if (2 * k <= n) {
-        const Real u = lds[k * m.ps], v = lds[(k == 0 ? 0 : n - k) * m.ps];
-        ax[q] = u + v;
-        by[q] = v - u;
-      }
-    }
-    __syncthreads();
-#define DFFT_MIX_CALL(r) mix_scatter<r, V, Real>(im, sl, t, T, lds, m.ps)
-    DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
-#undef DFFT_MIX_CALL
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < mix_half<V>(); ++q) {
-      const int k = t + q * T;
-      if (2 * k <= n) {
-        const Real u = lds[k * m.ps], v = lds[(k == 0 ? 0 : n - k) * m.ps];
-        ay[q] = u - v;
-        bx[q] = u + v;
-      }
-    }
     if (valid) {
-      C* pa = reinterpret_cast<C*>(io.ob[0]) + t * io.os[0];
-      C* pb = reinterpret_cast<C*>(io.ob[1]) + t * io.os[1];
-#pragma unroll
-      for (int q = 0; q < mix_half<V>(); ++q) {
-        const int k = t + q * T;
-        if (2 * k <= n) {
-          const Real h = Real(0.5) * io.scale * ((k != 0 && 2 * k != n) ? io.hw : Real(1));
-          gstore_c<NT, Real>(pa + static_cast<int64_t>(q) * T * io.os[0], C{ax[q] * h, ay[q] * h});
-          if (io.has_b) gstore_c<NT, Real>(pb + static_cast<int64_t>(q) * T * io.os[1], C{bx[q] * h, by[q] * h});
-        }
-      }
+#define DFFT_MIX_CALL(r) mix_store_half<r, V, NT, Real>(re, im, sl, t, T, n, io)
+      DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
+#undef DFFT_MIX_CALL
     }
   } else {
-    // C2R: the lane that loads entry k <= n/2 of both half spectra forms the
-    // inputs conj(A + i B) at k and at n - k and hands them out through LDS
-    const bool valid = active && 2 * unit < p.nlines;
-    PairIO<Real, NT> io{};
-    Real xk[mix_half<V>()], xm[mix_half<V>()], yk[mix_half<V>()], ym[mix_half<V>()];
-    if (valid) {
-      io = make_pair_io<Real, NT>(p, unit);
-      C A[mix_half<V>()], Bv[mix_half<V>()];
-      const C* pa = reinterpret_cast<const C*>(io.ib[0]) + t * io.is[0];
-      const C* pb = reinterpret_cast<const C*>(io.ib[1]) + t * io.is[1];
+    // C2R: the lane that loads entry k <= n/2 of the half spectrum hands its
+    // conjugate out through LDS as the input at k and the entry as that at n - k
+    C x[mix_half<V>()];
 #pragma unroll
-      for (int q = 0; q < mix_half<V>(); ++q) {
-        const int k = t + q * T;
-        A[q] = C{Real(0), Real(0)};
-        Bv[q] = C{Real(0), Real(0)};
-        if (2 * k <= n) {
-          A[q] = gload_c<NT, Real>(pa + static_cast<int64_t>(q) * T * io.is[0]);
-          if (io.has_b) Bv[q] = gload_c<NT, Real>(pb + static_cast<int64_t>(q) * T * io.is[1]);
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < mix_half<V>(); ++q) {
-        const int k = t + q * T;
-        const C lo = io.c2r_value(k, true, A[q], Bv[q]);
-        const C hi = io.c2r_value(n - k, false, A[q], Bv[q]);
-        xk[q] = lo.x;
-        yk[q] = lo.y;
-        xm[q] = hi.x;
-        ym[q] = hi.y;
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < mix_half<V>(); ++q) xk[q] = xm[q] = yk[q] = ym[q] = Real(0);
+    for (int q = 0; q < mix_half<V>(); ++q) {
+      const int k = t + q * T;
+      x[q] = C{Real(0), Real(0)};
+      if (valid && 2 * k <= n) x[q] = gload_c<NT, Real>(reinterpret_cast<const C*>(io.ib) + static_cast<int64_t>(k) * io.is);
     }
 #pragma unroll
     for (int q = 0; q < mix_half<V>(); ++q) {
       const int k = t + q * T;
+      const bool self = k == 0 || 2 * k == n;
+      x[q].x *= self ? Real(1) : io.hw;
+      x[q].y = self ? Real(0) : x[q].y * io.hw;
       if (2 * k <= n) {
-        lds[k * m.ps] = xk[q];
-        if (k > 0 && 2 * k < n) lds[(n - k) * m.ps] = xm[q];
+        lds[k * m.ps] = x[q].x;
+        if (k > 0 && 2 * k < n) lds[(n - k) * m.ps] = x[q].x;
       }
     }
     __syncthreads();
@@ -632,8 +584,8 @@ __global__ void __launch_bounds__(1024) fft_mixed(const FastPass p, const MixPla
     for (int q = 0; q < mix_half<V>(); ++q) {
       const int k = t + q * T;
       if (2 * k <= n) {
-        lds[k * m.ps] = yk[q];
-        if (k > 0 && 2 * k < n) lds[(n - k) * m.ps] = ym[q];
+        lds[k * m.ps] = -x[q].y;
+        if (k > 0 && 2 * k < n) lds[(n - k) * m.ps] = x[q].y;
       }
     }
     __syncthreads();
@@ -641,16 +593,10 @@ __global__ void __launch_bounds__(1024) fft_mixed(const FastPass p, const MixPla
     DFFT_MIX_SWITCH(s0.r, DFFT_MIX_CALL)
 #undef DFFT_MIX_CALL
     mix_stages<V, Real>(re, im, m, t, lds, tw);
-    // w = FFT(conj Z), a + i b = conj(w)
     if (valid) {
-#define DFFT_MIX_CALL(r) mix_store_real<r, V, NT, Real>(re, sl, t, T, io.ob[0], io.os[0], io.scale)
+#define DFFT_MIX_CALL(r) mix_store_real<r, V, NT, Real>(re, sl, t, T, io.ob, io.os, io.scale)
       DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
 #undef DFFT_MIX_CALL
-      if (io.has_b) {
-#define DFFT_MIX_CALL(r) mix_store_real<r, V, NT, Real>(im, sl, t, T, io.ob[1], io.os[1], -io.scale)
-        DFFT_MIX_SWITCH(sl.r, DFFT_MIX_CALL)
-#undef DFFT_MIX_CALL
-      }
     }
   }
 }

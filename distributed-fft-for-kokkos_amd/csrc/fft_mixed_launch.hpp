@@ -131,7 +131,7 @@ hipError_t launch_mixed(LinePass p, hipStream_t s) {
   const std::vector<int>& rad = len.rad;
   if (rad.empty()) return hipErrorNotSupported;
   int T = len.lanes;
-  const int64_t units = p.kind == kC2C ? p.nlines : (static_cast<int64_t>(p.nlines) + 1) / 2;
+  const int64_t units = p.nlines;
   if (units <= 0) return hipSuccess;
 
   // Lanes per line: full registers, or one butterfly per lane where the pass

@@ -260,13 +260,15 @@ __device__ __forceinline__ void smooth_stages(cplx_t<Real>* v, int t, void* buf,
   }
 }
 
-// KIND kC2C: one complex line per T lanes.  kR2C / kC2R: the two real lines
-// 2 unit, 2 unit + 1 per T lanes as one complex line (PairIO).
+// One line per T lanes.  Real lines run one by one: two of them as one complex
+// line (as the power-of-two lengths do) take half the arithmetic, but then an
+// infinity or a large value of one line reaches the other, which may belong to
+// another transform, and the error of a C2R line is up to 1.35 times as large.
+// The zero imaginary parts of R2C inputs and the unused ones of C2R outputs
+// drop out of the first and the last stage.
 // BAND: a pass of a dealiased field's kept modes (LinePass::band): modes beyond
-// are neither read (zeros) nor stored (Navier-Stokes solver on 2 ranks, all
-// modes -> kept modes: three steps at 48^3 0.85 -> 0.69 ms, 96^3 1.92 -> 1.34,
-// 160^3 6.7 -> 3.4; gradient of four 96^3 steps 7.3 -> 5.0).  PROD: a products pass
-// (LinePass::products) as in fast_pair_body.
+// are neither read (zeros) nor stored.  PROD: a products pass
+// (LinePass::products): the field axis is the fastest batch axis.
 template <typename Real, int N, bool NT, int KIND, bool PROD = false, bool BAND = false>
 __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const FastPass p) {
   using C = cplx_t<Real>;
@@ -293,10 +295,10 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
 #pragma unroll
   for (int j = 0; j < Cfg::V; ++j) v[j] = C{Real(0), Real(0)};
 
+  LineIO<Real, NT> io{};
+  bool valid = unit < p.nlines;
+  if (valid) valid = make_line_io<Real, NT, BAND, PROD>(p, unit, io);
   if constexpr (KIND == kC2C) {
-    LineIO<Real, NT> io;
-    bool valid = unit < p.nlines;
-    if (valid) valid = make_line_io<Real, NT, BAND>(p, unit, io);
     if (valid) {
 #pragma unroll
       for (int q = 0; q < S0::NB; ++q) {
@@ -342,211 +344,111 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
       }
     }
   } else if constexpr (KIND == kR2C) {
-    const bool valid = 2 * unit < p.nlines;  // paired passes never enumerate padding
-    PairIO<Real, NT> io{};
-    if (valid) io = make_pair_io<Real, NT, PROD, BAND>(p, unit);
     if constexpr (PROD) {
-      // slots 3m..3m+2 are the pairs of one position: slot 3m+q stages velocity
-      // line q, each slot then forms its two product lines from LDS
-      const int pq = b % 3;
-      Real* st = reinterpret_cast<Real*>(smem_raw + (b - pq) * p.line_bytes);
-      if (valid) {
+      // slots 6m..6m+5 are the product fields of one position: the first three
+      // stage its velocity lines, each then forms its product line from LDS
+      const int f = b % 6;
+      Real* st = reinterpret_cast<Real*>(smem_raw + (b - f) * p.line_bytes);
+      if (valid && f < 3) {
 #pragma unroll
         for (int q = 0; q < S0::NB; ++q) {
           if (S0::on(t, q)) {
-            const Real* src = reinterpret_cast<const Real*>(io.ib[0]) + (t + q * T) * io.is[0];
-            const int64_t step = S0::nr * io.is[0];
+            const Real* src = reinterpret_cast<const Real*>(io.ib) + (t + q * T) * io.is;
+            const int64_t step = S0::nr * io.is;
 #pragma unroll
             for (int j = 0; j < S0::r; ++j) {
-              st[pq * N + t + q * T + j * S0::nr] = gload<NT>(src);
+              st[f * N + t + q * T + j * S0::nr] = gload<NT>(src);
               src += step;
             }
           }
         }
       }
       __syncthreads();
-      const Real* fa0 = st + prod_first(2 * pq) * N;
-      const Real* fa1 = st + prod_second(2 * pq) * N;
-      const Real* fb0 = st + prod_first(2 * pq + 1) * N;
-      const Real* fb1 = st + prod_second(2 * pq + 1) * N;
+      const Real* f0 = st + prod_first(f) * N;
+      const Real* f1 = st + prod_second(f) * N;
 #pragma unroll
       for (int q = 0; q < S0::NB; ++q) {
         if (S0::on(t, q)) {
 #pragma unroll
           for (int j = 0; j < S0::r; ++j) {
             const int at = t + q * T + j * S0::nr;
-            v[q * S0::r + j] = C{fa0[at] * fa1[at], fb0[at] * fb1[at]};
+            v[q * S0::r + j].x = f0[at] * f1[at];
           }
         }
       }
     } else if (valid) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (h && !io.has_b) continue;
+      for (int q = 0; q < S0::NB; ++q) {
+        if (S0::on(t, q)) {
+          const Real* src = reinterpret_cast<const Real*>(io.ib) + (t + q * T) * io.is;
+          const int64_t step = S0::nr * io.is;
 #pragma unroll
-        for (int q = 0; q < S0::NB; ++q) {
-          if (S0::on(t, q)) {
-            const Real* src = reinterpret_cast<const Real*>(io.ib[h]) + (t + q * T) * io.is[h];
-            const int64_t step = S0::nr * io.is[h];
-#pragma unroll
-            for (int j = 0; j < S0::r; ++j) {
-              const Real x = gload<NT>(src);
-              src += step;
-              if (h) {
-                v[q * S0::r + j].y = x;
-              } else {
-                v[q * S0::r + j].x = x;
-              }
-            }
+          for (int j = 0; j < S0::r; ++j) {
+            v[q * S0::r + j].x = gload<NT>(src);
+            src += step;
           }
         }
       }
     }
     smooth_stages<Real, N, 0, !PROD>(v, t, buf, tw, nullptr);  // the staged lines share LDS with the exchanges
-    // Spectra at m = t + q T + j nr <= n/2 from Z_m and Z_{n-m}: A = (Z_m +
-    // conj Z_{n-m}) / 2, B = (Z_m - conj Z_{n-m}) / (2 i).  The lanes hand out
-    // the upper half of Z; Z_0 and Z_{n/2} are their own mirrors.
-    constexpr int LOW = (N + 1) / (2 * Sl::nr);    // outputs j < LOW lie below n/2
-    constexpr int TOP = N / 2 / Sl::nr;            // outputs j > TOP above
-    C m[Sl::NB * (TOP + 1)];
-    __syncthreads();
-    if constexpr (Cfg::SPLIT) {
-      Real* lr = static_cast<Real*>(buf);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (h) __syncthreads();
-#pragma unroll
-        for (int q = 0; q < Sl::NB; ++q) {
-          if (Sl::on(t, q)) {
-            const int beta = t + q * T;
-#pragma unroll
-            for (int j = LOW; j < Sl::r; ++j)
-              if (j > TOP || 2 * (beta + j * Sl::nr) > N)
-                lr[beta + j * Sl::nr] = h ? v[q * Sl::r + j].y : v[q * Sl::r + j].x;
-          }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < Sl::NB; ++q) {
-          if (Sl::on(t, q)) {
-            const int beta = t + q * T;
-#pragma unroll
-            for (int j = 0; j <= TOP; ++j) {
-              const Real x = lr[N - beta - j * Sl::nr];
-              if (h) {
-                m[q * (TOP + 1) + j].y = x;
-              } else {
-                m[q * (TOP + 1) + j].x = x;
-              }
-            }
-          }
-        }
-      }
-    } else {
-      C* lc = static_cast<C*>(buf);
-#pragma unroll
-      for (int q = 0; q < Sl::NB; ++q) {
-        if (Sl::on(t, q)) {
-          const int beta = t + q * T;
-#pragma unroll
-          for (int j = LOW; j < Sl::r; ++j)
-            if (j > TOP || 2 * (beta + j * Sl::nr) > N) lc[beta + j * Sl::nr] = v[q * Sl::r + j];
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < Sl::NB; ++q) {
-        if (Sl::on(t, q)) {
-          const int beta = t + q * T;
-#pragma unroll
-          for (int j = 0; j <= TOP; ++j) m[q * (TOP + 1) + j] = lc[N - beta - j * Sl::nr];
-        }
-      }
-    }
     if (valid) {
-      const Real h0 = Real(0.5) * io.scale, hw = h0 * io.hw;
+      constexpr int LOW = (N + 1) / (2 * Sl::nr);  // outputs j < LOW lie below n/2
+      constexpr int TOP = N / 2 / Sl::nr;          // outputs j > TOP above
+      const Real hw = io.scale * io.hw;
 #pragma unroll
-      for (int line = 0; line < 2; ++line) {
-        if (line && !io.has_b) continue;
+      for (int q = 0; q < Sl::NB; ++q) {
+        if (Sl::on(t, q)) {
+          const int beta = t + q * T;
+          C* dst = reinterpret_cast<C*>(io.ob) + beta * io.os;
+          const int64_t step = Sl::nr * io.os;
 #pragma unroll
-        for (int q = 0; q < Sl::NB; ++q) {
-          if (Sl::on(t, q)) {
-            const int beta = t + q * T;
-            C* dst = reinterpret_cast<C*>(io.ob[line]) + beta * io.os[line];
-            const int64_t step = Sl::nr * io.os[line];
-#pragma unroll
-            for (int j = 0; j <= TOP; ++j) {
-              const int at = beta + j * Sl::nr;
-              const C z = v[q * Sl::r + j];
-              const bool self = (j == 0 && q == 0 && t == 0) || (j >= LOW && 2 * at == N);
-              const C w = self ? z : m[q * (TOP + 1) + j];
-              const Real h = self ? h0 : hw;
-              if (BAND ? at <= p.band : j < LOW || 2 * at <= N)
-                gstore_c<NT, Real>(dst, line ? C{(z.y + w.y) * h, (w.x - z.x) * h} : C{(z.x + w.x) * h, (z.y - w.y) * h});
-              dst += step;
-            }
+          for (int j = 0; j <= TOP; ++j) {
+            const int at = beta + j * Sl::nr;
+            const bool self = (j == 0 && q == 0 && t == 0) || (j >= LOW && 2 * at == N);
+            const C z = v[q * Sl::r + j];
+            const Real h = self ? io.scale : hw;
+            if (BAND ? at <= p.band : j < LOW || 2 * at <= N) gstore_c<NT, Real>(dst, C{z.x * h, z.y * h});
+            dst += step;
           }
         }
       }
     }
   } else {
-    // C2R: the lane that holds position m <= n/2 loads entry m of both half
-    // spectra, forms the inputs conj(A + i B) at m and at n - m and hands the
-    // latter over through LDS
-    const bool valid = 2 * unit < p.nlines;
-    PairIO<Real, NT> io{};
+    // C2R: the lane that holds position m <= n/2 loads entry m of the half
+    // spectrum, takes its conjugate as the input at m and hands the entry over
+    // through LDS as the input at n - m
     constexpr int LOW = (N + 1) / (2 * S0::nr), TOP = N / 2 / S0::nr;
-    C A[S0::NB * (TOP + 1)], Bv[S0::NB * (TOP + 1)];
+    C up[S0::NB * (TOP + 1)];
 #pragma unroll
-    for (int k = 0; k < S0::NB * (TOP + 1); ++k) {
-      A[k] = C{Real(0), Real(0)};
-      Bv[k] = C{Real(0), Real(0)};
-    }
+    for (int k = 0; k < S0::NB * (TOP + 1); ++k) up[k] = C{Real(0), Real(0)};
     if (valid) {
-      io = make_pair_io<Real, NT, false, BAND>(p, unit);
 #pragma unroll
-      for (int line = 0; line < 2; ++line) {
-        if (line && !io.has_b) continue;
+      for (int q = 0; q < S0::NB; ++q) {
+        if (S0::on(t, q)) {
+          const int beta = t + q * T;
+          const C* src = reinterpret_cast<const C*>(io.ib) + beta * io.is;
+          const int64_t step = S0::nr * io.is;
 #pragma unroll
-        for (int q = 0; q < S0::NB; ++q) {
-          if (S0::on(t, q)) {
-            const int beta = t + q * T;
-            const C* src = reinterpret_cast<const C*>(io.ib[line]) + beta * io.is[line];
-            const int64_t step = S0::nr * io.is[line];
-#pragma unroll
-            for (int j = 0; j <= TOP; ++j) {
-              // above n/2 (only lanes of the middle output): the first entry again, not used
-              const bool low = BAND ? beta + j * S0::nr <= p.band : j < LOW || 2 * (beta + j * S0::nr) <= N;
-              C x = gload_c<NT, Real>(low ? src : reinterpret_cast<const C*>(io.ib[line]));
-              if (BAND && !low) x = C{Real(0), Real(0)};
-              if (line) {
-                Bv[q * (TOP + 1) + j] = x;
-              } else {
-                A[q * (TOP + 1) + j] = x;
-              }
-              src += step;
-            }
+          for (int j = 0; j <= TOP; ++j) {
+            // above n/2 (only lanes of the middle output): the first entry again, not used
+            const bool low = BAND ? beta + j * S0::nr <= p.band : j < LOW || 2 * (beta + j * S0::nr) <= N;
+            const C x = gload_c<NT, Real>(low ? src : reinterpret_cast<const C*>(io.ib));
+            up[q * (TOP + 1) + j] = BAND && !low ? C{Real(0), Real(0)} : x;
+            src += step;
           }
         }
       }
     }
-    C up[S0::NB * (TOP + 1)];
 #pragma unroll
     for (int q = 0; q < S0::NB; ++q) {
 #pragma unroll
       for (int j = 0; j <= TOP; ++j) {
         const int at = t + q * T + j * S0::nr, k = q * (TOP + 1) + j;
         const bool self = (j == 0 && q == 0 && t == 0) || (j >= LOW && 2 * at == N);
-        C a = A[k], c = Bv[k];
-        a.y = self ? Real(0) : a.y;
-        c.y = self ? Real(0) : c.y;
         const Real hw = self ? Real(1) : io.hw;
-        a.x *= hw;
-        a.y *= hw;
-        c.x *= hw;
-        c.y *= hw;
-        v[q * S0::r + j] = C{a.x - c.y, -(a.y + c.x)};
-        up[k] = C{a.x + c.y, a.y - c.x};
+        up[k].x *= hw;
+        up[k].y = self ? Real(0) : up[k].y * hw;
+        v[q * S0::r + j] = cconj(up[k]);
       }
     }
     auto hand = [&](auto* lds, auto value, auto take) {
@@ -580,21 +482,16 @@ __global__ void __launch_bounds__((SmoothCfg<Real, N>::LANES)) fft_smooth(const 
       hand(static_cast<C*>(buf), [](const C& x) { return x; }, [](C& d, const C& x) { d = x; });
     }
     smooth_stages<Real, N, 0, false>(v, t, buf, tw, nullptr);
-    // w = FFT(conj Z), a + i b = conj(w)
     if (valid) {
 #pragma unroll
-      for (int line = 0; line < 2; ++line) {
-        if (line && !io.has_b) continue;
+      for (int q = 0; q < Sl::NB; ++q) {
+        if (Sl::on(t, q)) {
+          Real* dst = reinterpret_cast<Real*>(io.ob) + (t + q * T) * io.os;
+          const int64_t step = Sl::nr * io.os;
 #pragma unroll
-        for (int q = 0; q < Sl::NB; ++q) {
-          if (Sl::on(t, q)) {
-            Real* dst = reinterpret_cast<Real*>(io.ob[line]) + (t + q * T) * io.os[line];
-            const int64_t step = Sl::nr * io.os[line];
-#pragma unroll
-            for (int j = 0; j < Sl::r; ++j) {
-              gstore<NT>(dst, line ? -v[q * Sl::r + j].y * io.scale : v[q * Sl::r + j].x * io.scale);
-              dst += step;
-            }
+          for (int j = 0; j < Sl::r; ++j) {
+            gstore<NT>(dst, v[q * Sl::r + j].x * io.scale);
+            dst += step;
           }
         }
       }
@@ -618,7 +515,7 @@ template <typename Real, int N>
 hipError_t launch_smooth(LinePass p, hipStream_t s) {
   using Cfg = SmoothCfg<Real, N>;
   constexpr int T = Cfg::T;
-  const int64_t units = p.kind == kC2C ? p.nlines : (static_cast<int64_t>(p.nlines) + 1) / 2;
+  const int64_t units = p.nlines;
   if (units <= 0) return hipSuccess;
   int B = p.lines_per_block;
   if constexpr (N == 96 || N == 160) {
@@ -679,11 +576,11 @@ hipError_t launch_smooth_band(LinePass p, hipStream_t s) {
   constexpr int T = Cfg::T;
   if (p.kind != kC2C && (p.kind == kR2C) == (p.inverse != 0)) return hipErrorInvalidValue;
   if (p.products && (p.kind != kR2C || p.nlines % 6 != 0 || p.line_begin % 6 != 0)) return hipErrorInvalidConfiguration;
-  const int64_t units = p.kind == kC2C ? p.nlines : (static_cast<int64_t>(p.nlines) + 1) / 2;
+  const int64_t units = p.nlines;
   if (units <= 0) return hipSuccess;
   int B;
   if (p.products) {
-    B = std::max(1, 128 / (3 * T)) * 3;  // whole positions
+    B = std::max(1, 256 / (6 * T)) * 6;  // whole positions
   } else if (p.lines_fast) {
     B = 32;
     while (B > Cfg::LEAST && B * T > 256) B /= 2;
