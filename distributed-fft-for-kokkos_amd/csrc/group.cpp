@@ -252,7 +252,6 @@ void Group::build_tables(const std::vector<void*>& in, const std::vector<void*>&
         q.lines_per_block = 0;  // launcher heuristic
         q.values_per_thread = 0;
         q.dual_lines = 0;
-        q.paired = 1;  // real lines of an own launch run in pairs
         t.single[k].push_back(q);
       }
     }

@@ -107,3 +107,26 @@ def test_backward_errors(dev, n, fp64):
     ref = np.conj(_exact(np.conj(full))).real
     per_element = _per_element(dev, np.conj(full), fp64).real.astype(rdt)
     assert rel_l2(got, ref) < TOL * np.sqrt(1.25) * rel_l2(per_element, ref)
+
+
+@pytest.mark.parametrize("fp64", [True, False])
+@pytest.mark.parametrize("n", [8, 60, 512, 1024])
+def test_group_members_launched_on_their_own(dev, n, fp64):
+    """Lengths without a grouped kernel, 8, 512 and 1024 among them."""
+    import torch
+    import dfft
+    rdt, cdt = (torch.float64, torch.complex128) if fp64 else (torch.float32, torch.complex64)
+    rng = np.random.default_rng(n)
+    x = rng.uniform(-1, 1, (5, n))
+    x[1] *= 1e8
+    x[3, 0] = np.nan
+    a = torch.from_numpy(x).to(dev, rdt)
+    b = torch.empty((5, n // 2 + 1), dtype=cdt, device=dev)
+    c = torch.empty_like(a)
+    g = dfft.Group([a], [b], [1])
+    g.execute([a], [b], dfft.Direction.forward)
+    g.execute([b], [c], dfft.Direction.backward)
+    x, got, back = a.cpu().numpy(), b.cpu().numpy(), c.cpu().numpy()
+    for k in (0, 1, 2, 4):
+        assert rel_l2(got[k], F.fftn(x[k].astype(np.float64)[None], [1], True)[0]) < LINE_TOL[fp64], k
+        assert rel_l2(back[k], x[k]) < LINE_TOL[fp64], k
