@@ -389,11 +389,12 @@ __device__ __forceinline__ char* side_line(const Side& s, char* const* tab, cons
 // fields 0 to 2 read velocity lines 0 to 2; the others' input is not used.
 template <typename Real, bool NT = false, bool BAND = false, bool PROD = false>
 __device__ __forceinline__ bool make_line_io(const FastPass& p, int32_t line, LineIO<Real, NT>& io) {
-  BatchIdx x = batch_index<BAND>(p, line);
+  const BatchIdx x = batch_index<BAND>(p, line);
   if (x.i2 >= p.pad_real) return false;
+  BatchIdx u = x;
+  if constexpr (PROD) u.i2 = x.i2 < 2 ? x.i2 : 2;
+  io.ib = side_line(p.in, p.in_ptr, u, io.is);
   io.ob = side_line(p.out, p.out_ptr, x, io.os);
-  if constexpr (PROD) x.i2 = x.i2 < 2 ? x.i2 : 2;
-  io.ib = side_line(p.in, p.in_ptr, x, io.is);
   io.kind = p.kind;
   io.n = p.n;
   io.inverse = p.inverse;

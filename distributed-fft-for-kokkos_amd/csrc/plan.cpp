@@ -521,7 +521,17 @@ LinePass Plan::make_pass(const PassSpec& s, const DDesc& in, const DDesc& out, b
 //    the next pass, so only the last pass, whose output nothing reads soon,
 //    streams (256^3 R2C FP64: all cached 355, all nontemporal 441, last
 //    backward pass only 337 us; 256^3 C2C FP64: 610, 612, last passes only 540
-//    us).  Never where two blocks write parts of one line of memory.
+//    us).  Never where two blocks write parts of one line of memory, and not in
+//    real passes across lines: a pair's two lines are every other real of a
+//    row, two half-written lines of memory per access (LayoutLeft, us, streamed
+//    -> cached: 256^3 FP64 C2R 120 -> 50, FP32 50 -> 30, 1024^2 x 64 FP64 R2C 512 ->
+//    230, C2R 486 -> 225), and single lines stream well only as R2C rows of whole
+//    lines of memory (512^3 FP64 R2C 543 streamed, 574 cached, C2R 631, 542).
+//  * Real passes across lines with 16 values per lane run one line per FFT (the
+//    pair kernels hold 8).  Cached, best block of each, us, 8 values in pairs /
+//    16 values alone, R2C and C2R: FP64 512^3 629 / 574, 520 / 542, 256^2 x 1024
+//    341 / 322, 327 / 293, 128 x 64 x 2048 109 / 110, 81 / 71; FP32 256^2 x 1024
+//    253 / 189, 242 / 182, 512^3 339 / 359, 325 / 386.
 void Plan::default_shape(LinePass& p, const PassSpec& s) const {
   constexpr double kMiB = 1024.0 * 1024.0;
   const int es = fp64_ ? 16 : 8;
@@ -555,14 +565,17 @@ void Plan::default_shape(LinePass& p, const PassSpec& s) const {
     lines = p.n <= 512 ? std::max(1, 1024 / p.n) : 0;
   } else if (p.n <= 64) {
     lines = p.n <= 32 ? 32 : fp64_ ? 8 : 16;
+    if (p.kind != kC2C && p.n > 32) lines *= 2;  // 512^2 x 64 FP64 R2C 75 -> 65 us
   } else if (fp64_) {
     if (p.n >= 512) vpt = 16;
     lines = p.n <= 256 ? 8 : p.n == 512 ? 16 : p.n == 1024 ? 8 : 4;
   } else {
-    if (p.n >= 1024 || (p.n == 512 && far)) vpt = 16;
-    lines = p.n == 128 ? (odd ? 16 : 32) : p.n <= 512 ? (p.n == 512 && far ? 32 : 16) : p.n == 1024 ? 16 : 8;
+    const bool far512 = p.n == 512 && far && p.kind == kC2C;
+    if (p.n >= 1024 || far512) vpt = 16;
+    lines = p.n == 128 ? (odd ? 16 : 32) : p.n <= 512 ? (far512 ? 32 : 16) : p.n == 1024 ? 16 : 8;
   }
   const bool narrow = across && lines > 0 && lines * es < 128;  // blocks share lines of memory
+  const bool streams = !across || p.kind == kC2C || (p.kind == kR2C && vpt == 16 && lines * es >= 256);
   if (p.values_per_thread == 0 && p.lines_per_block == 0) {
     p.values_per_thread = vpt;
     p.lines_per_block = lines;
@@ -572,7 +585,7 @@ void Plan::default_shape(LinePass& p, const PassSpec& s) const {
   else p.xcd_remap = across && (odd || narrow || (bytes >= 64 * kMiB && !far)) ? 1 : 0;
   if (s.nontemporal >= 0) {
     p.nontemporal = s.nontemporal;
-  } else if (across && (odd || narrow)) {
+  } else if ((across && (odd || narrow)) || !streams) {
     p.nontemporal = 0;
   } else {
     const bool last = p.in.ptr[0] == scratch_ && p.out.ptr[0] != scratch_;
