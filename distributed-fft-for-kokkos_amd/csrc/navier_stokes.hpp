@@ -30,7 +30,7 @@ class NavierStokes {
   NavierStokes& operator=(const NavierStokes&) = delete;
 
   void init_taylor_green(double v0, hipStream_t s);
-  void autotune(hipStream_t s);  // tunes every plan on scratch buffers; keeps the state
+  void autotune(hipStream_t s);  // tunes the passes the options select on scratch buffers; keeps the state
   // "fuse_products" (1, default): the divergence form's 6 products are formed
   // in the forward transform's first pass from the 3 velocity fields where
   // the plan allows it; 0: a separate products kernel writes the 6 fields.

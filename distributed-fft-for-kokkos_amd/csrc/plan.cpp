@@ -342,6 +342,8 @@ void Plan::plan_fused() {
   };
   fwd_ = build(in_topo_, out_topo_, true);
   bwd_ = build(out_topo_, in_topo_, false);
+  band_fwd_ = fwd_;
+  band_bwd_ = bwd_;
 }
 
 DDesc Plan::user_desc(const Vec& ext, const Vec& topo, Layout tl, void* const* ptrs) const {
@@ -705,9 +707,8 @@ DDesc Plan::band_array(int cut, void* p) const {
 }
 
 void Plan::band_pass(LinePass& p, std::size_t i, bool forward, int cut) const {
-  const auto& passes = forward ? fwd_ : bwd_;
+  const auto& passes = forward ? band_fwd_ : band_bwd_;
   p.band = cut;
-  if (passes[i].values_per_thread != 0) p.lines_per_block = 0;  // tuned for the kernels of all modes
   p.pad_axis = 0;
   p.pad_real = 0;
   int64_t nl = 1;
@@ -758,7 +759,7 @@ void Plan::execute_band(void* const* in, void* const* out, int direction, int cu
   if (total_size(gin_) == 0) return;
   const bool forward = direction == DFFT_FORWARD;
   TraceRange range("dfft::%s::execute %s (kept modes)", name_.c_str(), forward ? "forward" : "backward");
-  const auto& passes = forward ? fwd_ : bwd_;
+  const auto& passes = forward ? band_fwd_ : band_bwd_;
   auto spectral = [&](void* const* ptrs) {
     return packed ? band_array(cut, ptrs[0]) : user_desc(gout_, out_topo_, out_tl_, ptrs);
   };
@@ -786,7 +787,7 @@ void Plan::execute_forward_products(void* const* u3, void* const* out, int cut, 
   if (cur != device_) check_hip(hipSetDevice(device_), "hipSetDevice");
   if (total_size(gin_) == 0) return;
   TraceRange range("dfft::%s::execute forward (products of 3 fields)", name_.c_str());
-  const auto& passes = fwd_;
+  const auto& passes = cut > 0 ? band_fwd_ : fwd_;
   const double scale = exec_scale(true);
   // the 6-field input distribution (line enumeration) and the 3-field one
   // the products are read from: the field axis is not distributed, so every
@@ -1119,6 +1120,71 @@ float Plan::time_direction(void* const* in, void* const* out, bool forward, hipS
   return ms / reps;
 }
 
+namespace {
+
+// The fastest of the candidate shapes of one pass by `time_spec` (ms, negative
+// if the launcher refuses the shape): each is timed once, then the six fastest
+// three more times, and the best single timing wins (one noisy sample does not
+// decide).  split: the six also with the other LDS exchange form (split halves
+// or complex; kernels without a split form ignore the option).
+template <typename Time>
+PassSpec fastest_shape(const std::vector<PassSpec>& candidates, const PassSpec& otherwise, bool split, Time&& time_spec) {
+  std::vector<std::pair<float, PassSpec>> timed;
+  for (const PassSpec& s : candidates) {
+    const float ms = time_spec(s);
+    if (ms >= 0.f) timed.emplace_back(ms, s);
+  }
+  std::stable_sort(timed.begin(), timed.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+  const std::size_t finalists = std::min<std::size_t>(6, timed.size());
+  float best = 1e30f;
+  PassSpec best_spec = otherwise;
+  for (std::size_t f = 0; f < finalists; ++f) {
+    for (int flip = 0; flip < (split ? 2 : 1); ++flip) {
+      PassSpec s = timed[f].second;
+      if (flip) s.split = s.split ? 0 : 1;
+      float ms = flip ? 1e30f : timed[f].first;
+      for (int trial = 0; trial < 3; ++trial) {
+        const float m = time_spec(s);
+        if (m >= 0.f) ms = std::min(ms, m);
+      }
+      if (ms < best) {
+        best = ms;
+        best_spec = s;
+      }
+    }
+  }
+  return best_spec;
+}
+
+// three launches between two events after an untimed one; ms, or -1 if refused
+struct LaunchTimer {
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  hipStream_t stream;
+  explicit LaunchTimer(hipStream_t s) : stream(s) {
+    check_hip(hipEventCreate(&e0), "hipEventCreate");
+    check_hip(hipEventCreate(&e1), "hipEventCreate");
+  }
+  ~LaunchTimer() {
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+  }
+  template <typename Launch> float operator()(Launch&& launch) const {
+    if (launch() != hipSuccess) {
+      (void)hipGetLastError();
+      return -1.f;
+    }
+    check_hip(hipEventRecord(e0, stream), "hipEventRecord");
+    for (int k = 0; k < 3; ++k) check_hip(launch(), "line pass");
+    check_hip(hipEventRecord(e1, stream), "hipEventRecord");
+    check_hip(hipEventSynchronize(e1), "hipEventSynchronize");
+    float ms = 0.f;
+    check_hip(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
+    return ms;
+  }
+};
+
+}  // namespace
+
 // Autotuner: per pass, every compile-time launch shape (values per thread x
 // lines per block x lane order) is timed on the pass's own descriptors; then
 // the chunk size of the first two passes.  Shapes the launcher rejects
@@ -1128,9 +1194,7 @@ void Plan::autotune(void* const* in, void* const* out, hipStream_t stream) {
   // the tuner writes both sides: refuse arrays that cannot hold them
   check_buffers(in, out, DFFT_FORWARD);
   check_hip(hipSetDevice(device_), "hipSetDevice");
-  hipEvent_t e0, e1;
-  check_hip(hipEventCreate(&e0), "hipEventCreate");
-  check_hip(hipEventCreate(&e1), "hipEventCreate");
+  const LaunchTimer timer(stream);
   const int vpts[] = {4, 8, 16};
   const int lpbs[] = {1, 2, 4, 8, 16, 32};
   for (int dir = 0; dir < 2; ++dir) {
@@ -1145,24 +1209,11 @@ void Plan::autotune(void* const* in, void* const* out, hipStream_t stream) {
       if (!has_fast_line_kernel(passes[i].n)) continue;
       DDesc a = i == 0 ? src : scr;
       DDesc b = i + 1 == passes.size() ? dst : scr;
-      // one timing of 3 launches per shape, then the six fastest shapes are
-      // timed three more times and the best single timing wins (one noisy
-      // sample does not decide)
-      auto time_spec = [&](const PassSpec& s) -> float {
-        LinePass p = make_pass(s, a, b, !forward, 1.0);
-        if (launch_pass(p, stream) != hipSuccess) {
-          (void)hipGetLastError();
-          return -1.f;
-        }
-        check_hip(hipEventRecord(e0, stream), "hipEventRecord");
-        for (int k = 0; k < 3; ++k) check_hip(launch_pass(p, stream), "line pass");
-        check_hip(hipEventRecord(e1, stream), "hipEventRecord");
-        check_hip(hipEventSynchronize(e1), "hipEventSynchronize");
-        float ms = 0.f;
-        check_hip(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
-        return ms;
+      auto time_spec = [&](const PassSpec& s) {
+        const LinePass p = make_pass(s, a, b, !forward, 1.0);
+        return timer([&] { return launch_pass(p, stream); });
       };
-      std::vector<std::pair<float, PassSpec>> timed;
+      std::vector<PassSpec> candidates;
       for (int vpt : vpts) {
         for (int lpb : lpbs) {
           // the column-major block walk ("swz") is left out of the search: it
@@ -1183,35 +1234,11 @@ void Plan::autotune(void* const* in, void* const* out, hipStream_t stream) {
             } else {
               s.paired = lfnt >> 3;
             }
-            const float ms = time_spec(s);
-            if (ms >= 0.f) timed.emplace_back(ms, s);
+            candidates.push_back(s);
           }
         }
       }
-      if (timed.empty()) continue;
-      std::stable_sort(timed.begin(), timed.end(),
-                       [](const auto& x, const auto& y) { return x.first < y.first; });
-      const std::size_t finalists = std::min<std::size_t>(6, timed.size());
-      float best = 1e30f;
-      PassSpec best_spec = passes[i];
-      for (std::size_t f = 0; f < finalists; ++f) {
-        // each finalist also with the other LDS exchange form (split halves
-        // or complex; kernels without a split form ignore the option)
-        for (int flip = 0; flip < 2; ++flip) {
-          PassSpec s = timed[f].second;
-          if (flip) s.split = s.split ? 0 : 1;
-          float ms = flip ? 1e30f : timed[f].first;
-          for (int trial = 0; trial < 3; ++trial) {
-            const float m = time_spec(s);
-            if (m >= 0.f) ms = std::min(ms, m);
-          }
-          if (ms < best) {
-            best = ms;
-            best_spec = s;
-          }
-        }
-      }
-      passes[i] = best_spec;
+      passes[i] = fastest_shape(candidates, passes[i], true, time_spec);
     }
     if (passes.size() == 3) {
       // a chunk size must beat the unchunked passes by 3 % (timing noise
@@ -1230,8 +1257,44 @@ void Plan::autotune(void* const* in, void* const* out, hipStream_t stream) {
       chunk_[dir] = best_chunk;
     }
   }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+}
+
+// The passes over kept modes: block shapes, lane order, block numbering and
+// kind of access (8 values per lane, split exchanges and pairs are fixed;
+// fft_smooth's kernels choose their blocks and cached accesses themselves).
+void Plan::autotune_band(void* const* in, void* const* out, int cut, hipStream_t stream) {
+  if (!band_supported(cut)) throw Error(DFFT_ERROR_UNSUPPORTED, "this plan cannot transform kept modes only");
+  check_hip(hipSetDevice(device_), "hipSetDevice");
+  const LaunchTimer timer(stream);
+  const DDesc phys = user_desc(gin_, in_topo_, in_tl_, in), spec = band_array(cut, out[0]);
+  const DDesc scr = band_array(cut, scratch_);
+  for (const bool forward : {true, false}) {
+    auto& passes = forward ? band_fwd_ : band_bwd_;
+    for (std::size_t i = 0; i < passes.size(); ++i) {
+      const bool first = i == 0, last = i + 1 == passes.size();
+      const DDesc& a = first ? (forward ? phys : spec) : scr;
+      const DDesc& b = last ? (forward ? spec : phys) : scr;
+      std::vector<PassSpec> candidates;
+      const bool fixed = smooth_band_length(passes[i].n);
+      for (int lpb : {0, 1, 2, 4, 8, 16, 32}) {
+        if (fixed && lpb > 0) break;
+        for (int k = 0; k < 8; ++k) {
+          if (fixed && (k & 2)) continue;
+          PassSpec s = passes[i];
+          s.lines_per_block = lpb;
+          s.lines_fast = k & 1;
+          s.nontemporal = k >> 1 & 1;
+          s.xcd = k >> 2;
+          candidates.push_back(s);
+        }
+      }
+      passes[i] = fastest_shape(candidates, passes[i], false, [&](const PassSpec& s) {
+        LinePass p = make_pass(s, a, b, !forward, 1.0);
+        band_pass(p, i, forward, cut);
+        return timer([&] { return launch_band_pass(p, stream); });
+      });
+    }
+  }
 }
 
 int Plan::num_passes(int direction) const {

@@ -94,6 +94,9 @@ class Plan {
   // measure candidate launch shapes and chunk sizes on the caller's arrays
   // (their contents are overwritten) and keep the fastest
   void autotune(void* const* in, void* const* out, hipStream_t stream);
+  // the same for the passes of execute_band on a packed spectral side (contents
+  // are overwritten), whose launch shapes are kept apart
+  void autotune_band(void* const* in, void* const* out, int cut, hipStream_t stream);
 
   const std::string& name() const { return name_; }
   std::size_t nranks() const { return P_; }
@@ -164,6 +167,7 @@ class Plan {
   std::size_t workspace_bytes_ = 0;
   std::map<int, void*> tw_;
   std::vector<PassSpec> fwd_, bwd_;
+  std::vector<PassSpec> band_fwd_, band_bwd_;  // launch shapes of the passes over kept modes
   int chunk_[2] = {0, 0};  // planes per chunk, forward / backward (0 = no chunking)
   int pad_ = -1;           // scratch row padding: -1 auto (<= 1/16 extra), 0 off, 1 on
   // set only while execute_adjoint runs: scale of the adjoint direction and

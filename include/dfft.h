@@ -266,8 +266,9 @@ int dfft_ns_get_state(dfft_ns* ns, void* const* y3, void* stream);
 /* RK4 steps (NavierStokes::solve, main.cpp:544-561); use_graph replays one
  * captured step as a hipGraph after an eager first step */
 int dfft_ns_step(dfft_ns* ns, int nsteps, int use_graph, void* stream);
-/* time the launch shapes of every plan the solver uses (on its scratch
- * buffers; the state is kept) and keep the fastest -- no counterpart in the
+/* time the launch shapes of the transforms that the solver's options select
+ * (on its scratch buffers; the state is kept) and keep the fastest: after a
+ * change of "kept_modes" the others are still untuned.  No counterpart in the
  * reference, whose plans are created once with vendor defaults */
 int dfft_ns_autotune(dfft_ns* ns, void* stream);
 /* "fuse_products" (1 default, 0): form the divergence form's 6 products in
