@@ -31,7 +31,8 @@ class Group {
   // every group on the device; no graph.  Throws DFFT_ERROR_UNSUPPORTED when
   // this call's tables do not fit.
   void execute_static(void* const* in, void* const* out, int direction, hipStream_t s);
-  static constexpr std::size_t kStaticTableBytes = std::size_t(4) << 20;
+  static constexpr std::size_t kStaticTableBytes = std::size_t(4300) << 10;  // 2,550 member passes
+  static_assert(sizeof(FastPass) <= 1720, "the records of 2,550 member passes and their block prefixes");
   int count() const { return static_cast<int>(members_.size()); }
   // launches one execute of `direction` issues
   int num_launches(int direction) const;

@@ -631,7 +631,7 @@ class Group:
 
     def execute_noalloc(self, ins, outs, direction, stream=None):
         """``execute`` without device allocation: the pass tables go into the
-        library's static table area (4 MiB per GPU, shared by every call on
+        library's static table area (4.2 MiB per GPU, shared by every call on
         the device; overlapping calls race)."""
         self.check_views(ins, outs, direction)
         _check(self._lib.dfft_group_execute_noalloc(self._h, _ptrs(ins), _ptrs(outs), int(direction),

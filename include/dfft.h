@@ -214,8 +214,8 @@ int dfft_group_execute(dfft_group* group, void* const* in, void* const* out, int
 /* dfft_group_execute (use_graph = 0) that allocates no device memory: no
  * counterpart in the reference; for callers that cannot call hipMalloc (code
  * under stream capture, serving loops, harnesses that forbid allocation).
- * The call's pass tables go into a static device array of 4 MiB per GPU
- * (about 2,600 member passes); a call whose tables need more returns
+ * The call's pass tables go into a static device array of 4.2 MiB per GPU
+ * (about 2,550 member passes); a call whose tables need more returns
  * DFFT_ERROR_UNSUPPORTED before launching anything.  The array is shared by
  * every group and every call on the device: calls that overlap on one GPU
  * race.  The call synchronises the stream once (after the table copy, before
