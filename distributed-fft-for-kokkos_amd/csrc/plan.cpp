@@ -1213,15 +1213,19 @@ void Plan::autotune(void* const* in, void* const* out, hipStream_t stream) {
         const LinePass p = make_pass(s, a, b, !forward, 1.0);
         return timer([&] { return launch_pass(p, stream); });
       };
+      // 96 and 160 points: fft_smooth has one form of a line (FP32 real lines
+      // run on the kernels of the powers of two)
+      const bool one_form = smooth_length(passes[i].n) && (fp64_ || passes[i].kind == kC2C);
       std::vector<PassSpec> candidates;
       for (int vpt : vpts) {
+        if (one_form && vpt != 8) continue;
         for (int lpb : lpbs) {
           // the column-major block walk ("swz") is left out of the search: it
           // measured slower on every pass shape tried (512^3 x pass +36 %)
           // bit 3: two real lines per complex FFT (R2C / C2R) or two adjacent
           // lines per lane (FP32 C2C lanes across lines)
           const bool c2c = passes[i].kind == kC2C;
-          for (int lfnt = 0; lfnt < (c2c && fp64_ ? 8 : 16); ++lfnt) {
+          for (int lfnt = 0; lfnt < (one_form || (c2c && fp64_) ? 8 : 16); ++lfnt) {
             if (c2c && (lfnt >> 3) && !(lfnt & 1)) continue;  // dual lines need lanes across lines
             PassSpec s = passes[i];
             s.values_per_thread = vpt;
@@ -1229,7 +1233,9 @@ void Plan::autotune(void* const* in, void* const* out, hipStream_t stream) {
             s.lines_fast = lfnt & 1;
             s.nontemporal = (lfnt >> 1) & 1;
             s.xcd = (lfnt >> 2) & 1;
-            if (c2c) {
+            if (one_form) {
+              // nothing else to choose
+            } else if (c2c) {
               s.dual = lfnt >> 3;
             } else {
               s.paired = lfnt >> 3;
@@ -1238,7 +1244,7 @@ void Plan::autotune(void* const* in, void* const* out, hipStream_t stream) {
           }
         }
       }
-      passes[i] = fastest_shape(candidates, passes[i], true, time_spec);
+      passes[i] = fastest_shape(candidates, passes[i], !one_form, time_spec);
     }
     if (passes.size() == 3) {
       // a chunk size must beat the unchunked passes by 3 % (timing noise
