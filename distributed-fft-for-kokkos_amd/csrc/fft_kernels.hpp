@@ -34,8 +34,9 @@ struct LinePass {
   int32_t fit_block;                    // 1: lines_per_block is a default the launcher may halve to fit
   const void* tw;                       // exp(-2 pi i e / n), e in [0, n), Real precision
   double scale;
-  // 1: an R2C (forward) or C2R (inverse) pass on the fast kernel transforms
-  // two real lines per complex FFT (lines 2q and 2q+1 of the pass)
+  // 1: an R2C (forward) or C2R (inverse) pass on the power-of-two kernels with
+  // 8 values per lane transforms two real lines per complex FFT (lines 2q and
+  // 2q+1 of the pass); other lengths run real lines one by one
   int32_t paired;
   // pad_real > 0: batch axis pad_axis is enumerated over a padded extent
   // (batch_ext, the row pitch of a padded array) and lines whose index along
@@ -213,7 +214,7 @@ hipError_t launch_bluestein_post(const LinePass& p, int log2m, const void* chirp
 hipError_t launch_products_pass(const LinePass& p, hipStream_t s);
 bool products_pass_supported(int n);
 // a pass with p.band set (and products, if set too): C2C lines, R2C / C2R
-// lines in pairs, undistributed line axis
+// lines (of a power of two in pairs), undistributed line axis
 hipError_t launch_band_pass(const LinePass& p, hipStream_t s);
 bool band_pass_supported(int n);
 hipError_t launch_remap(const RemapArgs& a, int esize, hipStream_t s);

@@ -115,7 +115,7 @@ __device__ __forceinline__ float fmadd(float a, float b, float c) { return __bui
 // away.  Every line multiplies by the same few constants, so their rounding
 // errors add up over the stages instead of averaging out: with sqrt(3)/2 alone
 // (off by half an ulp) a 243-point FP64 line was 2.3e-16 off, with its low part
-// 1.95e-16.  low is zero where it is less than a seventh of an ulp of one.
+// 1.95e-16.  low is zero where it is less than a seventh of the ulp below one.
 template <typename R> struct Wide {
   R high, low;
 };
@@ -471,7 +471,7 @@ template <typename Real, int N, int RM> struct FastCfg {
 
 // Twiddles of a radix-r butterfly are the powers w^j (j = 1..r-1) of one
 // table entry w = exp(-2 pi i k / (L r)): one FP64 load, the other powers by
-// FP64 products (at most three multiplications deep), each rounded once to the
+// FP64 products (three multiplications deep, w^9 four), each rounded once to the
 // kernel's precision.  FP64 lines of 96 and 160 points read w to w^4 and w^8:
 // chains up to w^9, four products deep, left a 160-point line 2.8e-16 off
 // instead of 1.7e-16.
@@ -1097,7 +1097,7 @@ __device__ __forceinline__ void fast_line_body(const FastPass& p, int32_t blk, i
   bool vout = false;
   if constexpr (STAGE) {
     // the last stage's outputs go to LDS in natural order (this replaces
-    // final_regroup); contiguous aligned C2C outputs are stored as element
+    // final_order); contiguous aligned C2C outputs are stored as element
     // pairs, any other line reads back positions t + j*T
     constexpr int rl = Cfg::P.rad[Cfg::NST - 1];
     constexpr int NBl = R / rl;

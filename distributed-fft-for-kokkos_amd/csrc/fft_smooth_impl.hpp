@@ -3,21 +3,22 @@
 // kernel compiled per length, with the radices, lanes per line and LDS
 // paddings worked out at compile time.
 //
-// What bounds it: the runtime-radix kernel (fft_mixed_impl.hpp) spent 100 to
+// What bounds it: the runtime-radix kernel (fft_mixed_impl.hpp) spends 100 to
 // 160 vector instructions per element on these lengths, most of them index
-// arithmetic on plan fields, against 50 of a compiled length; its passes were
+// arithmetic on plan fields, against 50 of a compiled length; its passes are
 // bound by instruction issue.  Compiled, with LDS indices of a lane part and
-// immediates and no radix branch, they take 45 to 70 and most passes are bound
-// by memory again (strided FP64 4.5 to 6 TB/s, contiguous 4.5 to 6.5).
-// Runtime radices -> this kernel: R2C 384^3 FP64 there and back 1.32 -> 1.13
-// ms, C2C 375x250x162 FP32 forward 251 -> 179 us, inverse 2-D of 32x1000x1000
-// FP64 488 -> 412 us, R2C 50x42x36 FP32 50.8 -> 41.2 us; over 39 lengths from
-// 36 to 1000, both precisions, complex and real: 1.32 times as fast.
-// 96 and 160 against the compiled power-of-two kernel, which has no FP64 pairs
-// there: real FP64 160 contiguous 3.9 -> 4.7 TB/s, 96 2.9 -> 4.0, complex FP32
-// 160 6.5 -> 6.8, 96 4.0 -> 4.3 (FP64 96 strided 4.4 -> 4.0).  With factors 7
-// (42 to 252 points, both precisions, complex and real) 1.34 times the
-// runtime-radix kernel; longer ones are left to it.
+// immediates and no radix branch, they take 45 to 75 and most complex passes
+// are bound by memory again (FP64 3.7 to 6.2 TB/s, FP32 2.8 to 6.3, the shorter
+// lines less); real lines, which run one by one, are bound by the latency of
+// the exchanges (3.1 to 5.3 TB/s across the lines, 2.0 to 4.4 along them).
+// Runtime radices -> this kernel over 39 lengths from 36 to 1000, both
+// precisions, complex and real: 1.40 times as fast (passes of 24M elements, us:
+// 384 real FP64 140 -> 106 along the lines, 104 -> 93 across; 375 FP32 95 -> 92,
+// 128 -> 97; 1000 FP64 148 -> 133, 209 -> 173).  With factors 7 (42 to 252
+// points) 1.39 times; longer ones are left to it.
+// 96 and 160 against the compiled power-of-two kernel: complex FP64 160 4.4 to
+// 6.0 -> 4.8 to 6.5 TB/s, FP32 160 5.0 -> 5.7 along the lines, real FP64 160 3.3 ->
+// 4.1 and 2.6 -> 3.6, 96 3.2 -> 3.4 and 2.5 -> 3.2 (complex FP64 96 5.7 -> 5.4).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -30,7 +31,7 @@ namespace dfft {
 
 constexpr int kSmoothStages = 6;
 // Complex values a lane holds at most.  FP64 with 16 (fewer lanes, 120
-// registers) ran real pairs 8 % slower, FP32 with 20 2-13 % slower.
+// registers) ran the 39 lengths 2.6 % slower, FP32 with 20 2-13 % slower.
 template <typename Real> constexpr int kSmoothValues = sizeof(Real) == 8 ? 12 : 16;
 struct SmoothPlan {
   int nst = 0;
@@ -42,7 +43,8 @@ struct SmoothPlan {
 
 constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
 // instructions a lane spends on one value of a radix-r stage, roughly: twiddle
-// and its powers, exchange, butterfly
+// and its powers, exchange, butterfly.  Counted, not fitted: the choices that
+// these figures lead to were timed as a whole (above), not each against others.
 constexpr int smooth_value_cost(int r) {
   return r >= 15 ? 26 : r >= 12 ? 25 : r >= 9 ? 24 : r == 8 ? 23 : r >= 5 ? 22 : r >= 4 ? 20 : 18;
 }
@@ -519,8 +521,8 @@ hipError_t launch_smooth(LinePass p, hipStream_t s) {
   if (units <= 0) return hipSuccess;
   int B = p.lines_per_block;
   if constexpr (N == 96 || N == 160) {
-    // a caller's block shape beyond a workgroup of the grouped launches' kernel
-    // of these lengths is refused, as it is for powers of two
+    // a caller's block shape beyond a workgroup of the power-of-two kernel,
+    // which runs these lengths too, is refused, as it always was
     const bool split = split_available<Real, N>() && p.split_lds != 0;
     const size_t line = split ? line_lds_bytes<Real, N, 8, true>() : line_lds_bytes<Real, N, 8, false>();
     if (!p.fit_block && B > 0 && (B * FastCfg<Real, N, 8>::T > 1024 || B * line > kGenericLdsMax))
@@ -531,7 +533,7 @@ hipError_t launch_smooth(LinePass p, hipStream_t s) {
       B = 32;
       while (B > Cfg::LEAST && B * T > 256) B /= 2;
     } else {
-      // one wave: its barriers cost least (real pairs 1 to 8 % over 256 lanes)
+      // one wave: its barriers cost least (1.1 % over 256 lanes, 39 lengths)
       B = T >= 64 ? 1 : 64 / T;
     }
     while (B > 1 && (units + B - 1) / B < 512 && B * T > 64) B = (B + 1) / 2;

@@ -97,7 +97,7 @@ class NavierStokes {
   // and scratch spectra (nl_, k1_, ..., the adjoint's fields) hold anything there.  The passes are bound by HBM,
   // and a stage at 256^3 moves 4.6 GB instead of 9.3 GB: four steps from a
   // physical field 39.8 -> 21.7 ms, the gradient of four 128^3 steps 16.5 ->
-  // 13.3 ms, results bit for bit the same.
+  // 13.3 ms, results equal to rounding.
   bool kept_only() const { return kept_modes_ && kept_supported_; }
   // With the kept modes alone, the state and every spectrum between a step's or
   // a gradient's transforms lie packed: one array of all ranks with aligned

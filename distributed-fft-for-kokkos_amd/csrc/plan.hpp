@@ -26,7 +26,7 @@ struct PassSpec {
   int values_per_thread = 0;
   int lines_fast = -1;
   int nontemporal = -1;  // -1: by shape
-  int paired = 1;        // R2C / C2R: two real lines per complex FFT
+  int paired = 1;        // R2C / C2R: two real lines per complex FFT where the length has such a kernel
   int xcd = -1;          // XCD-contiguous block numbering (-1: by shape)
   int swz = 0;           // column-major walk of the block grid
   int split = 1;         // exchanges in real / imaginary halves (half the LDS; FP64, FP32 n >= 1024)
@@ -56,8 +56,8 @@ class Plan {
   // Dealiased fields (4-D views, field axis first and not distributed, R2C
   // over axes 1..3): only modes |k| <= cut along each axis are kept.
   // band_supported: FP64, fused executor, LayoutRight, power-of-two lengths
-  // 8..1024 and even 2^a 3^b 5^c from 36 to 384 (their real lines run in pairs
-  // whatever the plan's own passes do).  execute_band(FORWARD) writes the kept modes
+  // 8..1024 (their real lines run in pairs whatever the plan's own passes do)
+  // and even 2^a 3^b 5^c from 36 to 384 (one by one).  execute_band(FORWARD) writes the kept modes
   // of the spectra and leaves the others as they are; execute_band(BACKWARD)
   // transforms spectra whose other modes count as zeros, whatever the arrays
   // hold there.  Same results as execute on the masked spectra.
@@ -85,10 +85,11 @@ class Plan {
   // "pad" (scratch rows padded to 128-byte multiples: -1 auto, 0 off, 1 on),
   // "fwd.<i>.lpb|vpt|lf|nt|pair|xcd|swz|split|dual|lin", "bwd.<i>.…" (lines
   // per block, values per thread, lanes-across-lines, nontemporal accesses,
-  // two real lines per complex FFT in an R2C / C2R pass, XCD-contiguous
+  // two real lines per complex FFT in an R2C / C2R pass of a power of two
+  // with 8 values per thread, XCD-contiguous
   // blocks, column-major block walk, LDS exchanges in real/imaginary halves,
-  // two adjacent FP32 lines per lane, one-line passes into odd unpadded rows
-  // enumerated over the real elements) of pass i
+  // two adjacent FP32 lines per lane, the last pass enumerated over the real
+  // elements) of pass i
   void set_option(const std::string& key, long value);
   long get_option(const std::string& key) const;
   // measure candidate launch shapes and chunk sizes on the caller's arrays

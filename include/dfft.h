@@ -152,7 +152,11 @@ int dfft_execute_timed(dfft_plan* plan, void* const* in, void* const* out, int d
  * "fwd.<i>.swz", "fwd.<i>.split" (and "bwd.…") = lines per block, values
  * per thread (4, 8, 16), lane order, nontemporal global accesses (-1 = by
  * size and pass), two real lines per complex FFT in an R2C /
- * C2R pass (default on), XCD-contiguous block numbering, a column-major walk
+ * C2R pass (default on; power-of-two lengths, and FP32 96 and 160, with 8 values
+ * per thread, which passes across the lines of 512 FP64 or 1024 FP32 points
+ * and more do not take by default; a line's error is then relative to the
+ * larger of the two, and an infinity or NaN reaches both; other lengths run
+ * real lines one by one), XCD-contiguous block numbering, a column-major walk
  * of the block grid, radix-stage exchanges through LDS in real and
  * imaginary halves (default on; half the LDS per line; FP64 lines and FP32
  * lines of 1024 points or more), and "fwd.<i>.dual" = two adjacent FP32
@@ -161,9 +165,9 @@ int dfft_execute_timed(dfft_plan* plan, void* const* in, void* const* out, int d
  * ignored), "fwd.<i>.lin" = the last pass's lines, which leave the padded plan
  * scratch for the caller's rows, enumerated over the real elements, so blocks
  * write whole segments (default on; elsewhere ignored) of pass i.  A shape
- * that does not fit a workgroup (or, for lengths that are no power of two,
- * that the kernel of the length cannot make fit) makes
- * execute return DFFT_ERROR_HIP without launching. */
+ * that does not fit a workgroup makes execute return DFFT_ERROR_HIP without
+ * launching; for lengths other than powers of two, 96 and 160 "vpt" is an upper
+ * bound at most and "lpb" is halved until the block fits. */
 int dfft_plan_set_option(dfft_plan* plan, const char* key, long value);
 int dfft_plan_get_option(const dfft_plan* plan, const char* key, long* value);
 /* Autotuner: times every launch shape of every pass and the chunk sizes on the
