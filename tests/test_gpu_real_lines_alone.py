@@ -80,11 +80,11 @@ def test_forward_errors(dev, n, fp64):
 @pytest.mark.parametrize("n", [20, 54, 81, 96, 160, 162, 243, 375, 504, 625, 729, 1155, 1536, 2187, 3125])
 def test_backward_errors(dev, n, fp64):
     """The per-element kernel runs the Hermitian extension as a complex line; the
-    real part of its output is the C2R line.  A real output keeps only the real
-    part of the error, half of it if the parts are alike.  With power-of-two
-    radices mirrored inputs are rounded alike, which keeps more of it in the real
-    part than sums in order do: up to 1.25 of the half allowed (as two lines of a
-    pair, both parts count: 2)."""
+    real part of its output is the C2R line.  Of the early stages' errors half
+    falls into the imaginary part, which a real output does not keep; the values
+    of the last stage lie in the real part, and all of its errors count.  With
+    fewer, larger radices that stage has a larger share: 1.25 times the squared
+    error allowed (two lines of a pair keep both parts: 2)."""
     if _pairs(n, fp64):
         pytest.skip("in pairs")
     import torch
